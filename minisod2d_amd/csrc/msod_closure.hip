@@ -15,7 +15,7 @@
 // through the MLP with bf16 MFMA products and FP32 accumulation.
 #include <cmath>
 
-#include "msod_kernels.h"
+#include "msod_columns.h"
 #include "msod_mlp.h"
 #include "msod_closure.h"
 
@@ -46,7 +46,7 @@ __global__ void __launch_bounds__(Shape<P>::NT) k_closure_elem(ClosureElemArgs a
     const int I = l % Q, J = (l / Q) % Q, K = l / (Q * Q);
     double r = 0, uu[3] = {0, 0, 0}, rerr_ener = 0;
     if (active) {
-        const int64_t g = a.conn[e * NN + l];
+        const int64_t g = a.conn[ElemEntry<P>{e, l}.entry()];
         const int64_t np = a.npoin;
         r = a.rho[g];
         sA[le][0][l] = r;
@@ -65,7 +65,11 @@ __global__ void __launch_bounds__(Shape<P>::NT) k_closure_elem(ClosureElemArgs a
     double h[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
     double gT[3] = {0, 0, 0}, V[4][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, gv = 0;
     if (active) {
-        const GeoNode<double> gn = load_geo<NN, false>(a.geo, e, l);
+        const ElemEntry<P> en{e, l};
+        const GeoPair<double> *gp = reinterpret_cast<const GeoPair<double> *>(a.geo) + en.pair();
+        GeoNode<double> gn;
+#pragma unroll
+        for (int c = 0; c < 5; ++c) gn.v[c] = gp[c * en.pair_stride()];
 #pragma unroll
         for (int d = 0; d < 3; ++d)
 #pragma unroll

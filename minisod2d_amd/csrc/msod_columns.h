@@ -1,0 +1,213 @@
+// Column kernels: shapes, data layout and device helpers (porder 1..kColMaxP).
+//
+// A workgroup takes the EPB elements of one batch.  Thread t < LANES owns the
+// column of the Q nodes (I, J, 0..Q-1) of one element:
+//   t = I + Q*(le + EPB*J),  le the element within the batch
+// and walks it slice by slice (K = 0..Q-1).  The derivative along K stays in
+// the thread's registers; those along I and J read the slice's values from
+// LDS (2Q sources instead of 3Q).  Everything is unrolled over K, so a
+// source costs its FP64 work and its LDS reads with immediate offsets, and no
+// address arithmetic.
+//
+// Against one node per thread (all three directions from LDS, rolled loops)
+// the FP64 kernels issue a quarter to a third fewer VALU instructions and
+// two thirds (convection) or half (diffusion) of the LDS reads per element
+// node: 128^3 order 4 12.6 -> 10.3 ms (convection) and 12.9 -> 10.3 ms
+// (diffusion); 64^3 1.61 -> 1.33 and 1.77 -> 1.50; order 3, 96^3 2.32 -> 2.03 and
+// 2.42 -> 2.19; order 2, 100^3 1.17 -> 0.83 and 0.99 -> 0.99; order 5, 40^3 0.88 -> 0.64
+// and 0.79 -> 0.76.  What bounds them now: two waves per SIMD (220-256
+// VGPRs), whose FP64 work and LDS reads alone take 7.1 ms (convection, 128^3),
+// then the gathers (2.1 ms more) and the atomics (2.8 ms).
+//
+// The launch takes the batches in mesh order, one workgroup each: neighbouring
+// batches run side by side and share lines in L2 (order 4, 128^3 convection:
+// 15.9 ms in colour order).  A workgroup that walked several batches with the
+// next one's gathers in flight was slower (128^3 14.6-15.5 ms): its waits for
+// the gathers wait for the atomics issued after them as well.
+//
+// Lane layout of the element-sized arrays (entry (b, K, t) of batch b):
+//   conn, lidx  [b][K][LANES]
+//   geo         [b][K][5][LANES] pairs (GeoNode's five pairs)
+// so that a wave's loads are contiguous.  I, J, K count the nodes of a line
+// from one end to the other (ascending xi), unlike the reference's 1-D order
+// (both ends first): with it, and with the elements side by side between I
+// and J, consecutive lanes gather consecutive nodes of a mesh numbered along its
+// rows, and the L1 serves four of them with one access.  The last batch is
+// padded with copies of the last element, so that every load is unconditional.
+#pragma once
+
+#include "msod_kernels.h"
+
+namespace msod {
+
+template <int P>
+struct ColShape {
+    static constexpr int Q = P + 1;
+    static constexpr int QQ = Q * Q;
+    static constexpr int NN = Q * QQ;
+    // 256 threads: 10 elements at order 4, whose rows of 41 nodes share more
+    // lines and nodes than two batches of 5 (64^3: convection 1.41 -> 1.31 ms,
+    // diffusion 1.70 -> 1.61; 128^3: 10.65 -> 10.30 and 12.05 -> 11.20).  Order 5
+    // takes 128 threads and three elements (40^3: convection 0.645 ms, diffusion
+    // 0.760; with 256 and seven 0.575 and 0.860).
+    static constexpr int NT = P == 5 ? 128 : 256;
+    static constexpr int EPB = NT / QQ;         // elements of a batch
+    static constexpr int LANES = EPB * QQ;
+    static constexpr int UMAX = EPB * NN;       // element nodes, and most distinct nodes, of a batch
+    static constexpr int UPT = (UMAX + NT - 1) / NT;
+};
+
+// Position m of a line (0..P, ascending xi) in the reference's 1-D order
+// (0: xi = -1, 1: xi = +1, 2..P: the interior), and back.
+template <int P>
+__host__ __device__ constexpr int line_ref(int m) { return m == 0 ? 0 : (m == P ? 1 : m + 1); }
+template <int P>
+__host__ __device__ constexpr int line_pos(int s) { return s == 0 ? 0 : (s == 1 ? P : s - 1); }
+
+// Entry of element node (e, l) in the element-sized arrays of either layout:
+// conn at entry(), geo's pair c at pair() + c*pair_stride().
+template <int P, bool COL = (P <= kColMaxP)>
+struct ElemEntry {
+    static constexpr int Q = P + 1, QQ = Q * Q, NN = Q * QQ;
+    int64_t e;
+    int l;
+    __device__ __forceinline__ int64_t entry() const { return e * NN + l; }
+    __device__ __forceinline__ int64_t pair() const { return e * 5 * NN + l; }
+    static constexpr int pair_stride() { return NN; }
+};
+template <int P>
+struct ElemEntry<P, true> {
+    using S = ColShape<P>;
+    int64_t e;
+    int l;
+    __device__ __forceinline__ int64_t slice() const { return (e / S::EPB) * S::Q + line_pos<P>(l / S::QQ); }
+    __device__ __forceinline__ int lane() const
+    {
+        return line_pos<P>(l % S::Q) + S::Q * ((int)(e % S::EPB) + S::EPB * line_pos<P>(l / S::Q % S::Q));
+    }
+    __device__ __forceinline__ int64_t entry() const { return slice() * S::LANES + lane(); }
+    __device__ __forceinline__ int64_t pair() const { return slice() * 5 * S::LANES + lane(); }
+    static constexpr int pair_stride() { return S::LANES; }
+};
+
+// Uniform read-only data (the derivative table, the batch list): read through
+// the constant address space, so that the loads are scalar (SGPRs, lgkmcnt).
+// Through a plain pointer the compiler must assume that the kernel's atomics
+// change them, loads them into VGPRs and waits for every load in flight.
+template <typename T>
+using Uniform = const __attribute__((address_space(4))) T *;
+template <typename T>
+__device__ __forceinline__ Uniform<T> uniform(const T *p)
+{
+    return (Uniform<T>)p;
+}
+
+// One thread's place in its batch.
+template <int P>
+struct ColThread {
+    int tc, le, I, J;
+    __device__ __forceinline__ ColThread(int t)
+    {
+        using S = ColShape<P>;
+        tc = t < S::LANES ? t : S::LANES - 1;  // idle threads load a real entry
+        I = tc % S::Q;
+        le = tc / S::Q % S::EPB;
+        J = tc / (S::Q * S::EPB);
+    }
+};
+
+// The derivative table in ascending line order: sD[i*Q + n] = l_n'(xi_i).
+template <int P, typename T>
+__device__ __forceinline__ void col_table(const double *D, T *sD)
+{
+    constexpr int Q = P + 1;
+    const int t = threadIdx.x;
+    if (t < Q * Q) sD[t] = (T)D[line_ref<P>(t / Q) * Q + line_ref<P>(t % Q)];
+}
+// Its entry (i, n), i and n compile-time constants (a scalar load).
+template <int P>
+__device__ __forceinline__ double col_D(Uniform<double> D, int i, int n)
+{
+    return D[line_ref<P>(i) * (P + 1) + line_ref<P>(n)];
+}
+
+// GeoNode of entry (b, K, tc).
+template <int P, bool NTL, typename T>
+__device__ __forceinline__ GeoNode<T> col_geo(const T *geo, uint32_t b, int K, int tc)
+{
+    using S = ColShape<P>;
+    const GeoPair<T> *p = reinterpret_cast<const GeoPair<T> *>(geo) + ((int64_t)b * S::Q + K) * 5 * S::LANES + tc;
+    GeoNode<T> g;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) g.v[c] = NTL ? __builtin_nontemporal_load(&p[c * S::LANES]) : p[c * S::LANES];
+    return g;
+}
+
+// Adds one slice's five residual values to the batch's node sums sR[c*US + li].
+// Atomic mode: LDS atomics.  Coloured mode: one element after the other, so
+// that the order of the sums is fixed (barriers: uniform control flow).
+template <int P, bool COLORED>
+__device__ __forceinline__ void col_add(double *sR, int US, bool active, int le, uint32_t li, const double (&v)[5])
+{
+    if constexpr (!COLORED) {
+        if (active) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c)
+                __hip_atomic_fetch_add(&sR[c * US + li], v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    } else {
+#pragma unroll 1
+        for (int k = 0; k < ColShape<P>::EPB; ++k) {
+            if (active && le == k) {
+#pragma unroll
+                for (int c = 0; c < 5; ++c) sR[c * US + li] += v[c];
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// A thread's entries t, t + NT, ... of a batch's node list.
+template <int P>
+__device__ __forceinline__ void col_list(const uint32_t *unode, uint32_t U, uint32_t (&wn)[ColShape<P>::UPT])
+{
+#pragma unroll
+    for (int j = 0; j < ColShape<P>::UPT; ++j) {
+        const uint32_t i = threadIdx.x + j * ColShape<P>::NT;
+        wn[j] = unode[i < U ? i : U - 1];
+    }
+}
+
+// The batch's node sums to the outputs, each distinct node once (atomically
+// onto zeroed outputs; coloured: stored by the node's first writer, added by
+// the others).
+template <int P, bool COLORED, typename TO>
+__device__ __forceinline__ void col_write(double *sR, int US, const uint32_t (&wn)[ColShape<P>::UPT],
+                                          uint32_t U, TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin)
+{
+    uint32_t t = threadIdx.x;
+    asm volatile("" : "+v"(t));  // no index or address of the sums held across the batch
+#pragma unroll
+    for (int j = 0; j < ColShape<P>::UPT; ++j) {
+        const uint32_t i = t + j * ColShape<P>::NT;
+        if (i >= U) break;
+        const uint32_t w = wn[j];
+        const int64_t g = w & 0x7fffffffu;
+        TO *dst[5] = {Rmass + g, Rmom + g, Rmom + npoin + g, Rmom + 2 * npoin + g, Rener + g};
+        TO v[5];
+#pragma unroll
+        for (int c = 0; c < 5; ++c) v[c] = (TO)sR[c * US + i];
+        if constexpr (!COLORED) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) unsafeAtomicAdd(dst[c], v[c]);
+        } else if (w >> 31) {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) *dst[c] = v[c];
+        } else {
+#pragma unroll
+            for (int c = 0; c < 5; ++c) *dst[c] += v[c];
+        }
+    }
+}
+
+}  // namespace msod

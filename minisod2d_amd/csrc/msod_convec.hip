@@ -295,12 +295,8 @@ static hipError_t launch_p(const A &a, hipStream_t s)
 template <class A>
 hipError_t launch_convec(int porder, const A &a, hipStream_t s)
 {
+    if (porder <= kColMaxP) return launch_convec_col<A, double>(porder, a, s);
     switch (porder) {
-    case 1: return launch_p<1, A>(a, s);
-    case 2: return launch_p<2, A>(a, s);
-    case 3: return launch_p<3, A>(a, s);
-    case 4: return launch_p<4, A>(a, s);
-    case 5: return launch_p<5, A>(a, s);
     case 6: return launch_p<6, A>(a, s);
     case 7: return launch_p<7, A>(a, s);
     case 8: return launch_p<8, A>(a, s);
@@ -310,12 +306,8 @@ hipError_t launch_convec(int porder, const A &a, hipStream_t s)
 
 hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s)
 {
+    if (porder <= kColMaxP) return launch_convec_col<ConvecArgs<float, float>, float>(porder, a, s);
     switch (porder) {
-    case 1: return launch_p<1, ConvecArgs<float, float>, float>(a, s);
-    case 2: return launch_p<2, ConvecArgs<float, float>, float>(a, s);
-    case 3: return launch_p<3, ConvecArgs<float, float>, float>(a, s);
-    case 4: return launch_p<4, ConvecArgs<float, float>, float>(a, s);
-    case 5: return launch_p<5, ConvecArgs<float, float>, float>(a, s);
     case 6: return launch_p<6, ConvecArgs<float, float>, float>(a, s);
     case 7: return launch_p<7, ConvecArgs<float, float>, float>(a, s);
     case 8: return launch_p<8, ConvecArgs<float, float>, float>(a, s);

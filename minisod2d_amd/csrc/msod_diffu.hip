@@ -382,12 +382,8 @@ static hipError_t launch_p(const A &a, hipStream_t s, const float *mlp = nullptr
 template <class A>
 hipError_t launch_diffu(int porder, const A &a, hipStream_t s)
 {
+    if (porder <= kColMaxP) return launch_diffu_col<A, false, double>(porder, a, nullptr, s);
     switch (porder) {
-    case 1: return launch_p<1, A>(a, s);
-    case 2: return launch_p<2, A>(a, s);
-    case 3: return launch_p<3, A>(a, s);
-    case 4: return launch_p<4, A>(a, s);
-    case 5: return launch_p<5, A>(a, s);
     case 6: return launch_p<6, A>(a, s);
     case 7: return launch_p<7, A>(a, s);
     case 8: return launch_p<8, A>(a, s);
@@ -397,12 +393,8 @@ hipError_t launch_diffu(int porder, const A &a, hipStream_t s)
 
 hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
 {
+    if (porder <= kColMaxP) return launch_diffu_col<DiffuArgs<float, float>, false, float>(porder, a, nullptr, s);
     switch (porder) {
-    case 1: return launch_p<1, DiffuArgs<float, float>, false, float>(a, s);
-    case 2: return launch_p<2, DiffuArgs<float, float>, false, float>(a, s);
-    case 3: return launch_p<3, DiffuArgs<float, float>, false, float>(a, s);
-    case 4: return launch_p<4, DiffuArgs<float, float>, false, float>(a, s);
-    case 5: return launch_p<5, DiffuArgs<float, float>, false, float>(a, s);
     case 6: return launch_p<6, DiffuArgs<float, float>, false, float>(a, s);
     case 7: return launch_p<7, DiffuArgs<float, float>, false, float>(a, s);
     case 8: return launch_p<8, DiffuArgs<float, float>, false, float>(a, s);
@@ -419,12 +411,8 @@ template hipError_t launch_diffu(int, const DiffuSplitArgs &, hipStream_t);
 hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp,
                                         hipStream_t s)
 {
+    if (porder <= kColMaxP) return launch_diffu_col<DiffuArgs<double, double>, true, double>(porder, a, mlp, s);
     switch (porder) {
-    case 1: return launch_p<1, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 2: return launch_p<2, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 3: return launch_p<3, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 4: return launch_p<4, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 5: return launch_p<5, DiffuArgs<double, double>, true>(a, s, mlp);
     case 6: return launch_p<6, DiffuArgs<double, double>, true>(a, s, mlp);
     case 7: return launch_p<7, DiffuArgs<double, double>, true>(a, s, mlp);
     case 8: return launch_p<8, DiffuArgs<double, double>, true>(a, s, mlp);

@@ -1,9 +1,9 @@
 // Internal interface between the runtime (msod_runtime.hip) and the kernel
 // translation units.  All pointers are device pointers.
 //
-// Element data are element-major, with the element-local node index l
-// lexicographic in the reference's 1-D SOD order: l = I + q*(J + q*K),
-// (I,J,K) = (AtoI,AtoJ,AtoK) - 1.
+// Element data are element-major above kColMaxP, with the element-local node
+// index l lexicographic in the reference's 1-D SOD order: l = I + q*(J + q*K),
+// (I,J,K) = (AtoI,AtoJ,AtoK) - 1 (the column kernels' layout: msod_columns.h).
 //   geo   [nelem][5][nn][2] He(i,k) (component c = i + 3k) and gpvol of each
 //                          element node as five pairs (c = 0,1 | 2,3 | 4,5 |
 //                          6,7 | 8 and gpvol): a node's ten values in five
@@ -14,8 +14,8 @@
 // reference layout (mu_e, mu_sgs).
 //
 // Assembly plan (built once per mesh by the runtime).  Elements are grouped
-// into batches of Shape<P>::BATCH consecutive elements; one workgroup owns a
-// batch, sums the contributions of its elements to every node of the batch in
+// into batches of consecutive elements (ColShape<P>::EPB, Shape<P>::BATCH,
+// CShape<P>::BATCH); one workgroup owns a batch, sums the contributions of its elements to every node of the batch in
 // LDS, and writes each of the batch's distinct nodes once:
 //   conn  [nelem][nn]   0-based global node of each element node
 //   lidx  [nelem][nn]   position of that node in its batch's node list
@@ -42,6 +42,10 @@
 namespace msod {
 
 constexpr int kMaxP = 8;
+// Column kernels (msod_columns.h) up to this order, one node per thread above:
+// a column's values stay in registers (convection 244, diffusion 256 VGPRs at
+// order 5 in FP64) and spill past it.
+constexpr int kColMaxP = 5;
 constexpr int kMaxKpb = 16;           // batches per workgroup, at most (LDS list of the block's batches)
 constexpr int kBatchesPerBlock = 8;   // batches per workgroup (convection: measured best of 1..16 at p=4)
 static_assert(kBatchesPerBlock <= kMaxKpb, "the block's batch list holds kpb entries");
@@ -77,8 +81,9 @@ struct CShape {
     static constexpr int UMAX = BATCH * NN;
 };
 
-// Host-side copies of Shape<P>::BATCH (diffusion and closure kernels) and
-// CShape<P>::BATCH (convection) for run-time porder.
+// Elements per batch of the diffusion's (and closure kernels') and of the
+// convection's plan for run-time porder: ColShape<P>::EPB for both up to
+// kColMaxP, then Shape<P>::BATCH and CShape<P>::BATCH.
 int batch_size(int porder);
 int convec_batch_size(int porder);
 
@@ -96,6 +101,7 @@ struct Plan {
     int64_t nb;
     int mode;
     int kpb;  // consecutive batches of the list per workgroup
+    int ustride;  // column kernels: stride of the node sums, the most nodes of any batch rounded up
 };
 
 // Workgroups of a launch: each takes kpb consecutive batches of the list.
@@ -157,6 +163,13 @@ struct DiffuArgs {
 using ConvecSplitArgs = ConvecArgs<float, float, double, double, double>;
 using DiffuSplitArgs = DiffuArgs<float, float, double, double>;
 
+// Column kernels, porder <= kColMaxP (msod_convec_col.hip, msod_diffu_col.hip);
+// TA: arithmetic type.
+template <class A, typename TA>
+hipError_t launch_convec_col(int porder, const A &a, hipStream_t s);
+template <class A, bool CLOSURE, typename TA>
+hipError_t launch_diffu_col(int porder, const A &a, const float *mlp, hipStream_t s);
+
 // Launchers (return hipError_t of the launch); A is a ConvecArgs or
 // DiffuArgs instantiation.
 template <class A>
@@ -177,10 +190,17 @@ template <typename TO>
 hipError_t launch_zero_nodes(TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin, const uint32_t *nodes,
                              int64_t count, hipStream_t s);
 
-// Element-major geometry from the reference layouts (see top of file).
+// Element-major geometry from the reference layouts (see top of file), of
+// geo_elems(porder, nelem) elements.
 template <typename T>
-hipError_t launch_build_geo(const T *He, const T *gpvol, int64_t nelem, int nn,
-                            const int32_t *l2g, T *geo, hipStream_t s);
+hipError_t launch_build_geo(int porder, const T *He, const T *gpvol, int64_t nelem, const int32_t *l2g, T *geo,
+                            hipStream_t s);
+// conn and lidx of the column kernels' lane layout from the element-major ones.
+hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *lidx, int64_t nelem, uint32_t *lconn,
+                             uint16_t *llidx, hipStream_t s);
+// Elements that geo, conn and lidx hold: nelem, padded to whole batches where
+// the column kernels run.
+int64_t geo_elems(int porder, int64_t nelem);
 
 // He and gpvol of one element node from geo: He(i,k) = he(i + 3k), with the
 // component index a compile-time constant (a register of the loaded pair, no

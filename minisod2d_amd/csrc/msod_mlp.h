@@ -127,23 +127,24 @@ __device__ __forceinline__ void wave_lds_sync()
 }
 
 // z3 of the MLP for this lane's node (mu_sgs = scale*softplus(z3)).
-// scratch: this wave's LDS area of 64*32 shorts (4 KiB), used by this wave
-// only (no block barrier inside).  All 64 lanes of the wave call it
-// (inactive lanes pass any finite features).
+// scratch: this wave's LDS area, four tiles of 16*32 shorts (1 KiB each), TS
+// shorts apart, used by this wave only (no block barrier inside).  All 64
+// lanes of the wave call it (inactive lanes pass any finite features).
+template <int TS = 16 * kMlpH>
 __device__ inline float mlp_forward_z3(const MlpShared &s, const float feat[kMlpIn], short *scratch)
 {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    short *X = scratch;  // [64][16]
+    short *X = scratch;  // [4 tiles][16][16]
 #pragma unroll
     for (int k = 0; k < 16; ++k)
-        X[lane * 16 + k] = k < kMlpIn ? f2bf((feat[k] - s.mean[k]) * s.istd[k]) : (short)0;
+        X[g * TS + r * 16 + k] = k < kMlpIn ? f2bf((feat[k] - s.mean[k]) * s.istd[k]) : (short)0;
     wave_lds_sync();
     f32x4 z1[4][2];
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt) {
         s16x4 a;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = X[(mt * 16 + r) * 16 + 4 * g + i];
+        for (int i = 0; i < 4; ++i) a[i] = X[mt * TS + r * 16 + 4 * g + i];
 #pragma unroll
         for (int nt = 0; nt < 2; ++nt) {
             s16x4 b;
@@ -153,7 +154,7 @@ __device__ inline float mlp_forward_z3(const MlpShared &s, const float feat[kMlp
         }
     }
     wave_lds_sync();
-    short *H = scratch;  // [64][32], over X
+    short *H = scratch;  // [4 tiles][16][32], over X
 #pragma unroll
     for (int mt = 0; mt < 4; ++mt)
 #pragma unroll
@@ -161,7 +162,7 @@ __device__ inline float mlp_forward_z3(const MlpShared &s, const float feat[kMlp
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int n = nt * 16 + r;
-                H[(mt * 16 + 4 * g + i) * kMlpH + n] = f2bf(siluf_(z1[mt][nt][i] + s.b1[n]));
+                H[mt * TS + (4 * g + i) * kMlpH + n] = f2bf(siluf_(z1[mt][nt][i] + s.b1[n]));
             }
     wave_lds_sync();
     float part[4][4];
@@ -170,8 +171,8 @@ __device__ inline float mlp_forward_z3(const MlpShared &s, const float feat[kMlp
         s16x4 a0, a1;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            a0[i] = H[(mt * 16 + r) * kMlpH + 4 * g + i];
-            a1[i] = H[(mt * 16 + r) * kMlpH + 16 + 4 * g + i];
+            a0[i] = H[mt * TS + r * kMlpH + 4 * g + i];
+            a1[i] = H[mt * TS + r * kMlpH + 16 + 4 * g + i];
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) part[mt][i] = 0.f;

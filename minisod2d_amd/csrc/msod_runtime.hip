@@ -8,7 +8,7 @@
 #include "msod_geom.h"
 #include <rocprofiler-sdk-roctx/roctx.h>
 
-#include "msod_kernels.h"
+#include "msod_columns.h"
 #include "msod_mlp.h"
 #include "msod_plan.h"
 #include "msod_tet.h"
@@ -131,29 +131,43 @@ __global__ void k_zero_nodes(TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin,
     }
 }
 
-// geo[e][k][l][0..1]: the pairs (He c = 2k, 2k+1) for k < 4, (He c = 8,
-// gpvol) for k = 4 (GeoNode), from He(3,3,nn,nelem) and gpvol(1,nn,nelem).
-template <typename T>
-__global__ void k_build_geo(const T *He, const T *gpvol, int64_t nelem, int nn, const int32_t *l2g,
-                            T *geo)
+// geo of the element nodes (msod_columns.h: the column kernels' lane layout,
+// element-major above kColMaxP): the pairs (He c = 2k, 2k+1) for k < 4, (He
+// c = 8, gpvol) for k = 4 (GeoNode), from He(3,3,nn,nelem) and
+// gpvol(1,nn,nelem).  Padding entries repeat the last element.
+template <int P, typename T>
+__global__ void k_build_geo(const T *He, const T *gpvol, int64_t nelem, int64_t total, const int32_t *l2g, T *geo)
 {
-    const int64_t total = nelem * nn;
+    constexpr int NN = (P + 1) * (P + 1) * (P + 1);
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const int64_t e = i / nn;
-        const int l = (int)(i - e * nn);
+        const int64_t e = i / NN, ec = e < nelem ? e : nelem - 1;
+        const int l = (int)(i - e * NN);
         const int64_t a = l2g[l];
-        const T *src = He + 9 * (a + (int64_t)nn * e);
+        const T *src = He + 9 * (a + NN * ec);
         T v[10];
 #pragma unroll
         for (int c = 0; c < 9; ++c) v[c] = src[c];
-        v[9] = gpvol[a + (int64_t)nn * e];
-        T *dst = geo + 2 * (e * 5 * nn + l);
+        v[9] = gpvol[a + NN * ec];
+        const ElemEntry<P> en{e, l};
+        GeoPair<T> *dst = reinterpret_cast<GeoPair<T> *>(geo) + en.pair();
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            dst[2 * k * nn] = v[2 * k];
-            dst[2 * k * nn + 1] = v[2 * k + 1];
-        }
+        for (int k = 0; k < 5; ++k) dst[k * en.pair_stride()] = GeoPair<T>{v[2 * k], v[2 * k + 1]};
+    }
+}
+
+template <int P>
+__global__ void k_plan_lanes(const uint32_t *conn, const uint16_t *lidx, int64_t nelem, int64_t total, uint32_t *lconn,
+                             uint16_t *llidx)
+{
+    constexpr int NN = (P + 1) * (P + 1) * (P + 1);
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
+        const int64_t e = i / NN, ec = e < nelem ? e : nelem - 1;
+        const int l = (int)(i - e * NN);
+        const ElemEntry<P> en{e, l};
+        lconn[en.entry()] = conn[ec * NN + l];
+        llidx[en.entry()] = lidx[ec * NN + l];
     }
 }
 
@@ -225,48 +239,73 @@ hipError_t launch_zero_outputs(float *Rmass, float *Rmom, float *Rener, int64_t 
     return hipSuccess;
 }
 
-int batch_size(int porder)
+// Calls f with porder as a compile-time constant (porder in 1..kMaxP).
+template <class F>
+static auto with_porder(int porder, F f)
 {
     switch (porder) {
-    case 1: return Shape<1>::BATCH;
-    case 2: return Shape<2>::BATCH;
-    case 3: return Shape<3>::BATCH;
-    case 4: return Shape<4>::BATCH;
-    case 5: return Shape<5>::BATCH;
-    case 6: return Shape<6>::BATCH;
-    case 7: return Shape<7>::BATCH;
-    case 8: return Shape<8>::BATCH;
-    default: return 1;
+    case 1: return f(std::integral_constant<int, 1>{});
+    case 2: return f(std::integral_constant<int, 2>{});
+    case 3: return f(std::integral_constant<int, 3>{});
+    case 4: return f(std::integral_constant<int, 4>{});
+    case 5: return f(std::integral_constant<int, 5>{});
+    case 6: return f(std::integral_constant<int, 6>{});
+    case 7: return f(std::integral_constant<int, 7>{});
+    default: return f(std::integral_constant<int, 8>{});
     }
+}
+
+int batch_size(int porder)
+{
+    return with_porder(porder, [](auto p) {
+        if constexpr (p() <= kColMaxP) return (int)ColShape<p()>::EPB;
+        else return (int)Shape<p()>::BATCH;
+    });
 }
 
 int convec_batch_size(int porder)
 {
-    switch (porder) {
-    case 1: return CShape<1>::BATCH;
-    case 2: return CShape<2>::BATCH;
-    case 3: return CShape<3>::BATCH;
-    case 4: return CShape<4>::BATCH;
-    case 5: return CShape<5>::BATCH;
-    case 6: return CShape<6>::BATCH;
-    case 7: return CShape<7>::BATCH;
-    case 8: return CShape<8>::BATCH;
-    default: return 1;
-    }
+    return with_porder(porder, [](auto p) {
+        if constexpr (p() <= kColMaxP) return (int)ColShape<p()>::EPB;
+        else return (int)CShape<p()>::BATCH;
+    });
+}
+
+int64_t geo_elems(int porder, int64_t nelem)
+{
+    if (porder > kColMaxP) return nelem;
+    const int64_t B = batch_size(porder);
+    return (nelem + B - 1) / B * B;
 }
 
 template <typename T>
-hipError_t launch_build_geo(const T *He, const T *gpvol, int64_t nelem, int nn,
-                            const int32_t *l2g, T *geo, hipStream_t s)
+hipError_t launch_build_geo(int porder, const T *He, const T *gpvol, int64_t nelem, const int32_t *l2g, T *geo,
+                            hipStream_t s)
 {
-    hipLaunchKernelGGL((k_build_geo<T>), dim3(grid_for(nelem * nn, 256)), dim3(256), 0, s, He,
-                       gpvol, nelem, nn, l2g, geo);
-    return hipGetLastError();
+    return with_porder(porder, [&](auto p) {
+        constexpr int NN = (p() + 1) * (p() + 1) * (p() + 1);
+        const int64_t total = geo_elems(p(), nelem) * NN;
+        hipLaunchKernelGGL((k_build_geo<p(), T>), dim3(grid_for(total, 256)), dim3(256), 0, s, He, gpvol, nelem, total,
+                           l2g, geo);
+        return hipGetLastError();
+    });
 }
-template hipError_t launch_build_geo<double>(const double *, const double *, int64_t, int,
-                                             const int32_t *, double *, hipStream_t);
-template hipError_t launch_build_geo<float>(const float *, const float *, int64_t, int,
-                                            const int32_t *, float *, hipStream_t);
+template hipError_t launch_build_geo<double>(int, const double *, const double *, int64_t, const int32_t *, double *,
+                                             hipStream_t);
+template hipError_t launch_build_geo<float>(int, const float *, const float *, int64_t, const int32_t *, float *,
+                                            hipStream_t);
+
+hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *lidx, int64_t nelem, uint32_t *lconn,
+                             uint16_t *llidx, hipStream_t s)
+{
+    return with_porder(porder, [&](auto p) {
+        constexpr int NN = (p() + 1) * (p() + 1) * (p() + 1);
+        const int64_t total = geo_elems(p(), nelem) * NN;
+        hipLaunchKernelGGL((k_plan_lanes<p()>), dim3(grid_for(total, 256)), dim3(256), 0, s, conn, lidx, nelem, total,
+                           lconn, llidx);
+        return hipGetLastError();
+    });
+}
 
 }  // namespace msod
 
@@ -305,6 +344,7 @@ struct PlanEntry {
     std::vector<int32_t> l2g;
     int B = 1;
     int64_t nbatch = 0;
+    int ustride = 0;  // most distinct nodes of any batch
     uint32_t *conn = nullptr, *uoff = nullptr, *unode = nullptr, *order = nullptr;
     uint16_t *lidx = nullptr;
     std::vector<int64_t> color_off;  // batches of colour c: order[color_off[c] .. color_off[c+1])
@@ -604,9 +644,24 @@ int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet
     P.nbatch = H.nbatch;
     P.color_off = H.color_off;
     P.colored = H.colored;
+    for (int64_t k = 0; k < H.nbatch; ++k) P.ustride = std::max(P.ustride, (int)(H.uoff[k + 1] - H.uoff[k]));
     int st;
     if ((st = upload(H.conn, &P.conn, "plan upload"))) return st;
     if ((st = upload(H.lidx, &P.lidx, "plan upload"))) return st;
+    if (ts->porder <= kColMaxP) {  // element-major to the column kernels' lane layout
+        const int64_t n = geo_elems(ts->porder, nelem) * (int64_t)ts->l2g.size();
+        uint32_t *conn = P.conn;
+        uint16_t *lidx = P.lidx;
+        P.conn = nullptr;
+        P.lidx = nullptr;
+        hipError_t e = hipMalloc((void **)&P.conn, sizeof(uint32_t) * n);
+        if (e == hipSuccess) e = hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n);
+        if (e == hipSuccess) e = launch_plan_lanes(ts->porder, conn, lidx, nelem, P.conn, P.lidx, g.stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
+        (void)hipFree(conn);
+        (void)hipFree(lidx);
+        if (e != hipSuccess) return hipfail(e, "plan layout");
+    }
     if ((st = upload(H.uoff, &P.uoff, "plan upload"))) return st;
     if ((st = upload(H.unode, &P.unode, "plan upload"))) return st;
     if ((st = upload(H.order, &P.order, "plan upload"))) return st;
@@ -682,9 +737,9 @@ int get_geo(const void *dHe, uint64_t vHe, const void *dVol, uint64_t vVol, int6
         }
     const int nn = (int)ts->l2g.size();
     DerivedGeo c{dHe, dVol, vHe, vVol, nelem, ts->porder, sizeof(T), ts->l2g, nullptr};
-    HIPCHK(hipMalloc(&c.geo, sizeof(T) * 10 * nelem * nn), "hipMalloc element-major He and gpvol");
-    hipError_t e = launch_build_geo<T>((const T *)dHe, (const T *)dVol, nelem, nn, ts->dl2g, (T *)c.geo,
-                                       g.stream);
+    HIPCHK(hipMalloc(&c.geo, sizeof(T) * 10 * geo_elems(ts->porder, nelem) * nn),
+           "hipMalloc element-major He and gpvol");
+    hipError_t e = launch_build_geo<T>(ts->porder, (const T *)dHe, (const T *)dVol, nelem, ts->dl2g, (T *)c.geo, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
     if (e != hipSuccess) {
         (void)hipFree(c.geo);
@@ -837,6 +892,7 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     pl.lidx = P.lidx;
     pl.uoff = P.uoff;
     pl.unode = P.unode;
+    pl.ustride = P.ustride;
     pl.mode = g.assembly;
     // batches per workgroup: kpb_max on large meshes, fewer where that would
     // leave the launch short of 2048 workgroups (8 per CU); 8^3 p=3 has 64
@@ -933,7 +989,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
                                 return launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch", kConvecNatural, kConvecKpb)))
+                            "convection kernel launch", porder <= kColMaxP || kConvecNatural, kConvecKpb)))
         return st;
     return finish_call("convection kernel");
 }
