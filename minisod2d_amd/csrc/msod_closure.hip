@@ -156,203 +156,301 @@ __global__ void __launch_bounds__(Shape<P>::NT) k_closure_elem(ClosureElemArgs a
 // ---------------------------------------------------------------------------
 // MLP: inference into mu_sgs (reference layout), and parameter gradients
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_mlp_predict(const float *P, const float *feat, int64_t nelem,
-                                                     int nn, const int32_t *l2g, double *mu_sgs)
+// Four features of a sample, from an address that need not be 16-byte aligned.
+__device__ __forceinline__ f32x4 load_feat4(const float *p, bool aligned)
+{
+    if (aligned) return *reinterpret_cast<const f32x4 *>(p);
+    return f32x4{p[0], p[1], p[2], p[3]};
+}
+
+// mu_sgs(nelem,nn) from the features [nelem*nn][12].  A workgroup takes kPE
+// elements and at most kPL of their nodes: the samples are read in memory
+// order, and the results change lanes in LDS, so that each store fills kPE
+// consecutive elements of one node (the reference layout puts an element's
+// nodes 8*nelem bytes apart; with the sample's lane storing it 82 us at 32^3
+// order 3, now 68, most of it the activations).
+constexpr int kPE = 16, kPL = 64;
+__global__ void __launch_bounds__(256) k_mlp_predict(const float *P, const float *feat, int64_t nelem, int nn,
+                                                     const int32_t *l2g, double *mu_sgs)
 {
     __shared__ MlpShared s;
-    __shared__ short scratch[4][64 * kMlpH];
+    __shared__ double out[kPE][kPL + 1];
     mlp_stage(s, P);
     __syncthreads();
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const bool valid = i < nelem * nn;
-    float f[kMlpIn];
-#pragma unroll
-    for (int k = 0; k < kMlpIn; ++k) f[k] = valid ? feat[i * kMlpIn + k] : s.mean[k];
-    const float z3 = mlp_forward_z3(s, f, scratch[threadIdx.x >> 6]);
-    if (valid) {
-        const int64_t e = i / nn;
-        const int l = (int)(i - e * nn);
-        mu_sgs[e + nelem * (int64_t)l2g[l]] = (double)(s.scale * softplusf_(z3));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int64_t e0 = (int64_t)blockIdx.x * kPE;
+    const int l0 = blockIdx.y * kPL, nl = nn - l0 < kPL ? nn - l0 : kPL;
+    const int ne = (int)(nelem - e0 < kPE ? nelem - e0 : kPE), total = ne * nl;
+    const bool aligned = ((uintptr_t)feat & 15) == 0;
+    const f32x4 mean = *reinterpret_cast<const f32x4 *>(&s.mean[4 * g]);
+    const f32x4 istd = *reinterpret_cast<const f32x4 *>(&s.istd[4 * g]);
+    for (int base = (threadIdx.x >> 6) * 64; base < total; base += 256) {
+        const float z3 = mlp_z3(s, [&](int mt) {
+            const int i = base + 16 * mt + r, ic = i < total ? i : total - 1;
+            const int64_t smp = (e0 + ic / nl) * nn + l0 + ic % nl;
+            // lanes of inputs 12..15 read 0..3, standardised to zero
+            const f32x4 f = load_feat4(feat + smp * kMlpIn + (g < 3 ? 4 * g : 0), aligned);
+            return pack_bf16((f - mean) * istd);
+        });
+        const int i = base + lane;
+        if (i < total) out[i / nl][i % nl] = (double)(s.scale * softplusf_(z3));
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nl * kPE; i += 256) {
+        const int e = i % kPE, l = i / kPE;
+        if (e < ne) mu_sgs[e0 + e + nelem * (int64_t)l2g[l0 + l]] = out[e][l];
     }
 }
 
-// One wave per block; each block accumulates the gradient of its chunks of
-// 64 samples and writes it to partial[blockIdx.x][kMlpTrain].
-__global__ void __launch_bounds__(64) k_mlp_grad(const float *P, const float *feat, const float *gnu,
-                                                 int64_t nsamp, float *partial)
+// Parameter gradient.  A workgroup's four waves take four chunks of 64 samples
+// at a time; its sum, chunk after chunk in a fixed order, goes to
+// partial[blockIdx.x][kMlpTrain].
+//
+// The layers are formed transposed as in the forward pass (lane (r, g): sample
+// r of a tile of 16, hidden units 4g..4g+3), so that forward and backward
+// products chain in registers; one sigmoid per activation serves the value and
+// the derivative.  Through the wave's own LDS go the operands of the weight
+// gradients, which contract over the samples, and the sums over the output
+// layer's 32 units (a lane per sample) and over the samples (a lane per unit),
+// which keep one fixed sequential order.  What bounds it: the activations (64
+// exponentials and reciprocals a sample) and the LDS.  2.1 M samples: 760 us
+// with one wave per workgroup and every operand gathered from LDS in 16-bit
+// pieces, 150 us now.
+constexpr int kGW = 4;     // waves per workgroup
+constexpr int kLH = 68;    // LDS row strides: 64 floats,
+constexpr int kLT = 20;    // 16 floats or shorts, padded
+struct MlpGradWave {
+    float H2[kMlpH][kLH];  // silu(Z2), [unit][sample]
+    float S[kMlpH][kLT];   // silu'(Z2), then dZ1, of one tile
+    short H1[kMlpH][kLT];  // bf16 operands of one tile, [unit][sample]
+    short D[kMlpH][kLT];   // dZ2, then dZ1
+    short X[16][kLT];      // inputs
+    float dz3[64];
+};
+union MlpGradShared {
+    MlpGradWave w[kGW];
+    float sum[kGW][kMlpTrain];  // the waves' chunk sums
+};
+
+__global__ void __launch_bounds__(64 * kGW, 2) k_mlp_grad(const float *P, const float *feat, const float *gnu,
+                                                       int64_t nsamp, float *partial)
 {
-    __shared__ MlpShared s;
-    __shared__ short X[64][16];
-    __shared__ float Z1[64][kMlpH + 1];   // pre-activations of layer 1, then dZ1
-    __shared__ short H1[64][kMlpH];
-    __shared__ float Z2[64][kMlpH + 1];   // pre-activations of layer 2
-    __shared__ short dZ2[64][kMlpH];
-    __shared__ short dZ1[64][kMlpH];
-    __shared__ float dz3s[64];
-    __shared__ float gacc[kMlpTrain];
-    mlp_stage(s, P);
-    for (int j = threadIdx.x; j < kMlpTrain; j += 64) gacc[j] = 0.f;
-    __syncthreads();
-    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+    __shared__ __attribute__((aligned(16))) MlpGradShared sh;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    MlpGradWave &L = sh.w[wave];
+    // left operands: row r, columns 4g..4g+3
+    s16x4 W1t[2], W2t[2][2], W2[2][2];  // W1^T[t]; W2^T[in][out]; W2[in][out]
+    f32x4 b1[2], b2[2], w3[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        f32x4 v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            v[q] = 4 * g + q < kMlpIn ? P[kOW1 + (4 * g + q) * kMlpH + 16 * t + r] : 0.f;
+            b1[t][q] = P[kOb1 + 16 * t + 4 * g + q];
+            b2[t][q] = P[kOb2 + 16 * t + 4 * g + q];
+            w3[t][q] = P[kOw3 + 16 * t + 4 * g + q];
+        }
+        W1t[t] = pack_bf16(v);
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = P[kOW2 + (16 * k + 4 * g + q) * kMlpH + 16 * t + r];
+            W2t[k][t] = pack_bf16(v);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) v[q] = P[kOW2 + (16 * k + r) * kMlpH + 16 * t + 4 * g + q];
+            W2[k][t] = pack_bf16(v);
+        }
+    }
+    const auto Pu = (const __attribute__((address_space(4))) float *)P;
+    const float scale = Pu[kOScale], w3c = P[kOw3 + (lane & 31)];
+    f32x4 mean, istd;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        mean[q] = g < 3 ? P[kOMean + (g < 3 ? 4 * g + q : 0)] : 0.f;
+        istd[q] = g < 3 ? P[kOIstd + (g < 3 ? 4 * g + q : 0)] : 0.f;
+    }
+    const bool aligned = ((uintptr_t)feat & 15) == 0;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    for (int64_t chunk = blockIdx.x; chunk * 64 < nsamp; chunk += gridDim.x) {
-        const int64_t i = chunk * 64 + lane;
-        const bool valid = i < nsamp;
+    constexpr int kPT = (kMlpTrain + 64 * kGW - 1) / (64 * kGW);
+    float run[kPT];  // the workgroup's sum of entries threadIdx.x + 256 j
 #pragma unroll
-        for (int k = 0; k < 16; ++k)
-            X[lane][k] = (valid && k < kMlpIn) ? f2bf((feat[i * kMlpIn + k] - s.mean[k]) * s.istd[k]) : (short)0;
-        const float gv = valid ? gnu[i] : 0.f;
-        __syncthreads();
-        // layer 1
+    for (int j = 0; j < kPT; ++j) run[j] = 0.f;
+
+    const int64_t nchunk = (nsamp + 63) / 64;
+    for (int64_t c0 = blockIdx.x; c0 < nchunk; c0 += (int64_t)gridDim.x * kGW) {
+        const int64_t chunk = c0 + (int64_t)gridDim.x * wave;
+        f32x4 dW1[2] = {zero, zero}, dW2[2][2] = {{zero, zero}, {zero, zero}};
+        float s23 = 0.f, s1 = 0.f, s3 = 0.f;  // lanes 0..31: dw3, db1; 32..63: db2; all: db3
+        if (chunk < nchunk) {
+            s16x4 xb[4], h1[4][2];
+            f32x4 ds1[4][2], ds2[4][2];
+            f32x4 f[4];
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            s16x4 av;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) av[q] = X[mt * 16 + r][4 * g + q];
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                s16x4 bv;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) bv[q] = s.W1[4 * g + q][nt * 16 + r];
-                const f32x4 z = mfma16(av, bv, zero);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int m = mt * 16 + 4 * g + q, n = nt * 16 + r;
-                    const float zz = z[q] + s.b1[n];
-                    Z1[m][n] = zz;
-                    H1[m][n] = f2bf(siluf_(zz));
-                }
+            for (int mt = 0; mt < 4; ++mt) {
+                const int64_t i = chunk * 64 + 16 * mt + r;
+                f[mt] = load_feat4(feat + (i < nsamp ? i : nsamp - 1) * kMlpIn + (g < 3 ? 4 * g : 0), aligned);
             }
-        }
-        __syncthreads();
-        // layer 2
+            const int64_t me = chunk * 64 + lane;
+            const float gv = gnu[me < nsamp ? me : nsamp - 1];
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt) {
-            s16x4 a0, a1;
+            for (int mt = 0; mt < 4; ++mt) {
+                const bool valid = chunk * 64 + 16 * mt + r < nsamp;
+                xb[mt] = pack_bf16((f[mt] - mean) * istd);
+                if (!valid) xb[mt] = s16x4{0, 0, 0, 0};
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                a0[q] = H1[mt * 16 + r][4 * g + q];
-                a1[q] = H1[mt * 16 + r][16 + 4 * g + q];
-            }
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                s16x4 b0, b1;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    b0[q] = s.W2[4 * g + q][nt * 16 + r];
-                    b1[q] = s.W2[16 + 4 * g + q][nt * 16 + r];
-                }
-                f32x4 z = mfma16(a0, b0, zero);
-                z = mfma16(a1, b1, z);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) Z2[mt * 16 + 4 * g + q][nt * 16 + r] = z[q] + s.b2[nt * 16 + r];
-            }
-        }
-        __syncthreads();
-        // output layer and its gradient, per node (lane = node)
-        float z3 = s.b3;
-#pragma unroll 4
-        for (int c = 0; c < kMlpH; ++c) z3 += siluf_(Z2[lane][c]) * s.w3[c];
-        const float dz3 = valid ? gv * s.scale * sigmoidf_(z3) : 0.f;
-        dz3s[lane] = dz3;
-#pragma unroll 4
-        for (int c = 0; c < kMlpH; ++c) dZ2[lane][c] = f2bf(dz3 * s.w3[c] * dsiluf_(Z2[lane][c]));
-        __syncthreads();
-        if (lane < kMlpH) {
-            float sw = 0.f, sb = 0.f;
-            for (int m = 0; m < 64; ++m) {
-                const float d = dz3s[m], z = Z2[m][lane];
-                sw += d * siluf_(z);
-                sb += d * s.w3[lane] * dsiluf_(z);
-            }
-            gacc[kOw3 + lane] += sw;
-            gacc[kOb2 + lane] += sb;
-        } else if (lane == kMlpH) {
-            float sum = 0.f;
-            for (int m = 0; m < 64; ++m) sum += dz3s[m];
-            gacc[kOb3] += sum;
-        }
-        // dW2 = H1^T dZ2   (M = 32 inputs, N = 32 outputs, K = 64 samples)
-#pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                f32x4 acc = zero;
-#pragma unroll
-                for (int kt = 0; kt < 4; ++kt) {
-                    s16x4 av, bv;
+                for (int t = 0; t < 2; ++t) {
+                    f32x4 z = mfma16(W1t[t], xb[mt], zero);
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        av[q] = H1[kt * 16 + 4 * g + q][mt * 16 + r];
-                        bv[q] = dZ2[kt * 16 + 4 * g + q][nt * 16 + r];
+                        const float zz = z[q] + b1[t][q], sg = sigmoidf_(zz);
+                        z[q] = zz * sg;
+                        ds1[mt][t][q] = sg * (1.f + zz * (1.f - sg));
                     }
-                    acc = mfma16(av, bv, acc);
+                    h1[mt][t] = pack_bf16(z);
                 }
 #pragma unroll
-                for (int q = 0; q < 4; ++q) gacc[kOW2 + (mt * 16 + 4 * g + q) * kMlpH + nt * 16 + r] += acc[q];
-            }
-        // dH1 = dZ2 W2^T (M = 64 samples, N = 32, K = 32), then dZ1 = dH1 * silu'(Z1)
-#pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) {
-                f32x4 acc = zero;
-#pragma unroll
-                for (int kt = 0; kt < 2; ++kt) {
-                    s16x4 av, bv;
+                for (int t = 0; t < 2; ++t) {
+                    const f32x4 z = mfma16(W2t[1][t], h1[mt][1], mfma16(W2t[0][t], h1[mt][0], zero));
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        av[q] = dZ2[mt * 16 + r][kt * 16 + 4 * g + q];
-                        bv[q] = s.W2[nt * 16 + r][kt * 16 + 4 * g + q];
+                        const float zz = z[q] + b2[t][q], sg = sigmoidf_(zz);
+                        L.H2[16 * t + 4 * g + q][16 * mt + r] = zz * sg;
+                        ds2[mt][t][q] = sg * (1.f + zz * (1.f - sg));
                     }
-                    acc = mfma16(av, bv, acc);
-                }
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int m = mt * 16 + 4 * g + q, k = nt * 16 + r;
-                    const float d = acc[q] * dsiluf_(Z1[m][k]);
-                    Z1[m][k] = d;
-                    dZ1[m][k] = f2bf(d);
                 }
             }
-        __syncthreads();
-        if (lane < kMlpH) {
-            float sum = 0.f;
-            for (int m = 0; m < 64; ++m) sum += Z1[m][lane];
-            gacc[kOb1 + lane] += sum;
+            wave_lds_sync();
+            float z3 = Pu[kOb3];
+#pragma unroll
+            for (int c = 0; c < kMlpH; ++c) z3 += L.H2[c][lane] * Pu[kOw3 + c];
+            L.dz3[lane] = me < nsamp ? gv * scale * sigmoidf_(z3) : 0.f;
+            wave_lds_sync();
+#pragma unroll
+            for (int mt = 0; mt < 4; ++mt) {
+                const float d = L.dz3[16 * mt + r];
+                s16x4 d2[2];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) L.X[4 * g + q][r] = xb[mt][q];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    f32x4 v;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) v[q] = d * w3[t][q] * ds2[mt][t][q];
+                    d2[t] = pack_bf16(v);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int n = 16 * t + 4 * g + q;
+                        L.S[n][r] = ds2[mt][t][q];
+                        L.H1[n][r] = h1[mt][t][q];
+                        L.D[n][r] = d2[t][q];
+                    }
+                }
+                wave_lds_sync();
+                // dw3 = sum dz3 silu(Z2), db2 = sum dz3 w3 silu'(Z2), db3 = sum dz3
+                {
+                    const float *col = lane < 32 ? &L.H2[lane & 31][16 * mt] : L.S[lane & 31];
+                    const float wl = lane < 32 ? 1.f : w3c;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const f32x4 z = *reinterpret_cast<const f32x4 *>(&L.dz3[16 * mt + 4 * i]);
+                        const f32x4 v = *reinterpret_cast<const f32x4 *>(&col[4 * i]);
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            s23 += z[q] * wl * v[q];
+                            s3 += z[q];
+                        }
+                    }
+                }
+                // dW2 = H1^T dZ2; dZ1^T = (W2 dZ2^T) silu'(Z1)
+                s16x4 av[2], bv[2];
+                f32x4 dz1[2];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    av[t] = *reinterpret_cast<const s16x4 *>(&L.H1[16 * t + r][4 * g]);
+                    bv[t] = *reinterpret_cast<const s16x4 *>(&L.D[16 * t + r][4 * g]);
+                }
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+#pragma unroll
+                    for (int k = 0; k < 2; ++k) dW2[k][t] = mfma16(av[k], bv[t], dW2[k][t]);
+                    dz1[t] = mfma16(W2[t][1], d2[1], mfma16(W2[t][0], d2[0], zero)) * ds1[mt][t];
+                }
+                wave_lds_sync();
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    const s16x4 d1 = pack_bf16(dz1[t]);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int n = 16 * t + 4 * g + q;
+                        L.S[n][r] = dz1[t][q];
+                        L.D[n][r] = d1[q];
+                    }
+                }
+                wave_lds_sync();
+                // db1 = sum dZ1; dW1 = X^T dZ1
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const f32x4 v = *reinterpret_cast<const f32x4 *>(&L.S[lane & 31][4 * i]);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) s1 += v[q];
+                }
+                const s16x4 xt = *reinterpret_cast<const s16x4 *>(&L.X[r][4 * g]);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) {
+                    bv[t] = *reinterpret_cast<const s16x4 *>(&L.D[16 * t + r][4 * g]);
+                    dW1[t] = mfma16(xt, bv[t], dW1[t]);
+                }
+                wave_lds_sync();
+            }
         }
-        // dW1 = X^T dZ1   (M = 16 inputs, N = 32, K = 64 samples)
+        // the chunks' sums, added in the order of the chunks
+        __syncthreads();  // every wave is done with its part of the LDS
+        float *sum = sh.sum[wave];
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) {
-            f32x4 acc = zero;
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                s16x4 av, bv;
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    av[q] = X[kt * 16 + 4 * g + q][r];
-                    bv[q] = dZ1[kt * 16 + 4 * g + q][nt * 16 + r];
-                }
-                acc = mfma16(av, bv, acc);
-            }
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const int k = 4 * g + q;
-                if (k < kMlpIn) gacc[kOW1 + k * kMlpH + nt * 16 + r] += acc[q];
+                if (4 * g + q < kMlpIn) sum[kOW1 + (4 * g + q) * kMlpH + 16 * t + r] = dW1[t][q];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) sum[kOW2 + (16 * k + 4 * g + q) * kMlpH + 16 * t + r] = dW2[k][t][q];
             }
+        sum[(lane < 32 ? kOw3 : kOb2) + (lane & 31)] = s23;
+        if (lane < 32) sum[kOb1 + lane] = s1;
+        if (lane == 0) sum[kOb3] = s3;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < kPT; ++j) {
+            const int i = threadIdx.x + 64 * kGW * j;
+            if (i < kMlpTrain)
+                for (int w = 0; w < kGW && c0 + (int64_t)gridDim.x * w < nchunk; ++w) run[j] += sh.sum[w][i];
         }
         __syncthreads();
     }
-    for (int j = threadIdx.x; j < kMlpTrain; j += 64) partial[(int64_t)blockIdx.x * kMlpTrain + j] = gacc[j];
+#pragma unroll
+    for (int j = 0; j < kPT; ++j) {
+        const int i = threadIdx.x + 64 * kGW * j;
+        if (i < kMlpTrain) partial[(int64_t)blockIdx.x * kMlpTrain + i] = run[j];
+    }
 }
 
-__global__ void k_grad_reduce(const float *partial, int nblocks, float *grad)
+// Sum of the workgroups' rows in FP64: 64 columns per workgroup, 16 lanes of
+// rows each, then a fixed tree (one thread per column over all rows: 248 us
+// for 1024 rows, now 6).
+__global__ void __launch_bounds__(1024) k_grad_reduce(const float *partial, int nblocks, float *grad)
 {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= kMlpTrain) return;
+    __shared__ double red[16][64];
+    const int c = threadIdx.x & 63, k = threadIdx.x >> 6, j = blockIdx.x * 64 + c;
     double s = 0.0;
-    for (int b = 0; b < nblocks; ++b) s += partial[(int64_t)b * kMlpTrain + j];
-    grad[j] = (float)s;
+    if (j < kMlpTrain)
+#pragma unroll 8
+        for (int b = k; b < nblocks; b += 16) s += partial[(int64_t)b * kMlpTrain + j];
+    red[k][c] = s;
+    for (int h = 8; h > 0; h >>= 1) {
+        __syncthreads();
+        if (k < h) red[k][c] += red[k + h][c];
+    }
+    if (k == 0 && j < kMlpTrain) grad[j] = (float)red[0][c];
 }
 
 // Adam (Kingma & Ba 2015, Algorithm 1).  ob1 = 1 - b1, ob2 = 1 - b2 and the
@@ -437,19 +535,18 @@ hipError_t launch_closure_adjoint(int porder, const ClosureElemArgs &a, hipStrea
 hipError_t launch_mlp_predict(const float *P, const float *feat, int64_t nelem, int nn,
                               const int32_t *l2g, double *mu_sgs, hipStream_t s)
 {
-    const int64_t n = nelem * nn;
-    hipLaunchKernelGGL(k_mlp_predict, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, P, feat, nelem, nn,
-                       l2g, mu_sgs);
+    hipLaunchKernelGGL(k_mlp_predict, dim3((unsigned)((nelem + kPE - 1) / kPE), (nn + kPL - 1) / kPL), dim3(256), 0, s,
+                       P, feat, nelem, nn, l2g, mu_sgs);
     return hipGetLastError();
 }
 
 hipError_t launch_mlp_grad(const float *P, const float *feat, const float *gnu, int64_t nsamp,
                            float *partial, int nblocks, float *grad, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mlp_grad, dim3(nblocks), dim3(64), 0, s, P, feat, gnu, nsamp, partial);
+    hipLaunchKernelGGL(k_mlp_grad, dim3(nblocks), dim3(64 * kGW), 0, s, P, feat, gnu, nsamp, partial);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_grad_reduce, dim3((kMlpTrain + 255) / 256), dim3(256), 0, s, partial, nblocks, grad);
+    hipLaunchKernelGGL(k_grad_reduce, dim3((kMlpTrain + 63) / 64), dim3(1024), 0, s, partial, nblocks, grad);
     return hipGetLastError();
 }
 

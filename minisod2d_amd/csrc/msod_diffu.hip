@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(Shape<P>::NT, (diffu_waves<P, typename A::G, T
     // (fluxes of one direction); the MLP scratch of the closure overlays it
     // between the two
     constexpr size_t kRec = sizeof(T) * EPB * 6 * NN;
-    constexpr size_t kScr = CLOSURE ? (size_t)(S::NT / 64) * 64 * kMlpH * sizeof(short) : 0;
+    constexpr size_t kScr = CLOSURE ? (size_t)(S::NT / 64) * 64 * 16 * sizeof(short) : 0;
     constexpr size_t kBuf = kRec > kScr ? kRec : kScr;
     __shared__ T sD[Q * Q];
     __shared__ __attribute__((aligned(16))) unsigned char sbuf[kBuf];
@@ -301,7 +301,7 @@ __global__ void __launch_bounds__(Shape<P>::NT, (diffu_waves<P, typename A::G, T
             } else
 #pragma unroll
                 for (int k = 0; k < kMlpIn; ++k) f[k] = smlp.mean[k];
-            const float z3 = mlp_forward_z3(smlp, f, reinterpret_cast<short *>(sbuf) + (t >> 6) * 64 * kMlpH);
+            const float z3 = mlp_forward_z3(smlp, f, reinterpret_cast<short *>(sbuf) + (t >> 6) * 64 * 16);
             mus = active ? (T)(smlp.scale * softplusf_(z3)) : (T)0;
         }
         if (active) {

@@ -1063,6 +1063,10 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
 // --- learned closure -----------------------------------------------------
 enum { kScrWeights = 0, kScrPartial = 1, kScrLoss = 2 };
 
+// Workgroups of the gradient kernel, one row of partial sums each, taking the
+// chunks of 64 samples in turn.
+int grad_blocks(int64_t nsamples) { return (int)std::min<int64_t>((nsamples + 63) / 64, kNoAllocBlocks); }
+
 // Library-owned device buffer `slot` of at least `bytes` (grow-only).
 int library_buffer(int slot, size_t bytes, void **p)
 {
@@ -2248,7 +2252,7 @@ int msod_closure_gradient(int64_t nsamples, const float *mlp_params, const float
     if ((st = resolve(features, sizeof(float) * kMlpIn * nsamples, "features", &df, &vx))) return st;
     if ((st = resolve(gnu, sizeof(float) * nsamples, "gnu", &dg, &vx))) return st;
     if ((st = resolve(grad, sizeof(float) * kMlpTrain, "grad", &dgr, &vx))) return st;
-    const int nblocks = (int)std::min<int64_t>((nsamples + 63) / 64, 1024);
+    const int nblocks = grad_blocks(nsamples);
     void *part;
     if ((st = library_buffer(kScrPartial, sizeof(float) * kMlpTrain * nblocks, &part))) return st;
     TimedLaunch tk(6);
@@ -2268,10 +2272,7 @@ int msod_closure_gradient_noalloc(int64_t nsamples, const float *mlp_params, con
     if (nsamples <= 0) return fail(MSOD_ERR_ARG, "nsamples=%lld", (long long)nsamples);
     if (g.device >= kMaxDevices || !g_noalloc_scratch[g.device])
         return fail(MSOD_ERR_STATE, "no partial-sum array on device %d", g.device);
-    const int64_t nblocks = std::min<int64_t>((nsamples + 63) / 64, kNoAllocBlocks);
-    if (nblocks > kNoAllocBlocks)  // the workgroups stride over the samples: never taken
-        return fail(MSOD_ERR_ARG, "closure gradient: %lld workgroups exceed the %d rows of the partial-sum array",
-                    (long long)nblocks, kNoAllocBlocks);
+    const int nblocks = grad_blocks(nsamples);  // at most kNoAllocBlocks rows of the partial-sum array
     // the weights must already be on the device: a host block would need a
     // library buffer
     const void *dmlp, *df, *dg, *dgr;
@@ -2294,7 +2295,7 @@ int msod_closure_gradient_noalloc(int64_t nsamples, const float *mlp_params, con
     // every workgroup overwrites its whole row before the reduction reads
     // it, so the rows left by an earlier call need no clearing
     HIPCHK(launch_mlp_grad((const float *)dmlp, (const float *)df, (const float *)dg, nsamples,
-                           g_noalloc_scratch[g.device], (int)nblocks, (float *)dgr, g.stream),
+                           g_noalloc_scratch[g.device], nblocks, (float *)dgr, g.stream),
            "closure gradient launch");
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hipfail(e, "closure gradient");
