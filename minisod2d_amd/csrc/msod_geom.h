@@ -10,12 +10,13 @@ struct GeomArgs {
     const int32_t *connec;   // (nelem,nnode) reference layout, 1-based
     const double *coord;     // (npoin,3)
     const double *wgp;       // [ngaus]
-    // nonzero entries of dNgp(d,:,g): nza/nzw[(g*3 + d)*mz + k], k < nzn[g*3 + d]
+    // nonzero entries k = 0.. of dNgp(d,:,g) at row (k*3 + d)*ngaus + g, in
+    // increasing a; shorter rows are padded with weight 0 and a = nnode, a node
+    // whose coordinates the kernel holds as zeros
     const uint16_t *nza;     // local node a (0-based)
     const double *nzw;       // dNgp(d,a,g)
-    const uint16_t *nzn;     // count
     int64_t nelem, npoin;
-    int mz;
+    int mz;                  // longest row
     double *He;              // He(3,3,ngaus,nelem)
     double *gpvol;           // gpvol(1,ngaus,nelem)
     unsigned long long *counts;  // [0] connec entries outside 1..npoin, [1] det(Je) <= 0

@@ -1481,44 +1481,39 @@ int msod_elem_jacobian(int porder, int nelem, int npoin, const int32_t *connec, 
     if ((st = host_view(dNgp, sizeof(double) * 3 * nn * nn, t0, &pd, "dNgp"))) return st;
     if ((st = host_view(wgp, sizeof(double) * nn, t1, &pw, "wgp"))) return st;
     const double *D = (const double *)pd;
-    std::vector<uint16_t> nzn(nn * 3, 0);
+    std::vector<int> cnt(nn * 3, 0);
     int mz = 1;
     for (int64_t gg = 0; gg < nn; ++gg)
-        for (int d = 0; d < 3; ++d) {
-            int c = 0;
-            for (int64_t a = 0; a < nn; ++a) c += D[d + 3 * (a + nn * gg)] != 0.0;
-            nzn[gg * 3 + d] = (uint16_t)c;
-            mz = std::max(mz, c);
-        }
-    std::vector<uint16_t> nza(nn * 3 * mz, 0);
-    std::vector<double> nzw(nn * 3 * mz, 0.0);
+        for (int64_t a = 0; a < nn; ++a)
+            for (int d = 0; d < 3; ++d)
+                if (D[d + 3 * (a + nn * gg)] != 0.0) mz = std::max(mz, ++cnt[gg * 3 + d]);
+    // one block: counters, weights, dNgp's entries, their nodes
+    const size_t rows = (size_t)nn * 3 * mz;
+    std::vector<char> tab(16 + sizeof(double) * (nn + rows) + sizeof(uint16_t) * rows, 0);
+    double *twg = (double *)(tab.data() + 16), *tzw = twg + nn;
+    uint16_t *tza = (uint16_t *)(tzw + rows);
+    std::memcpy(twg, pw, sizeof(double) * nn);
+    std::fill(tza, tza + rows, (uint16_t)nn);
+    std::fill(cnt.begin(), cnt.end(), 0);
     for (int64_t gg = 0; gg < nn; ++gg)
-        for (int d = 0; d < 3; ++d) {
-            int k = 0;
-            for (int64_t a = 0; a < nn; ++a) {
+        for (int64_t a = 0; a < nn; ++a)
+            for (int d = 0; d < 3; ++d) {
                 const double w = D[d + 3 * (a + nn * gg)];
-                if (w != 0.0) {
-                    nza[(gg * 3 + d) * mz + k] = (uint16_t)a;
-                    nzw[(gg * 3 + d) * mz + k] = w;
-                    ++k;
-                }
+                if (w == 0.0) continue;
+                const size_t row = (size_t)(cnt[gg * 3 + d]++ * 3 + d) * nn + gg;
+                tza[row] = (uint16_t)a;
+                tzw[row] = w;
             }
-        }
-    std::vector<double> w(pw ? (const double *)pw : nullptr, pw ? (const double *)pw + nn : nullptr);
     std::vector<unsigned long long> counts(2, 0ull);
-    DevTemp da, dw, dn, dg, dk;
-    if ((st = dev_temp(nza, da, "geometry tables"))) return st;
-    if ((st = dev_temp(nzw, dw, "geometry tables"))) return st;
-    if ((st = dev_temp(nzn, dn, "geometry tables"))) return st;
-    if ((st = dev_temp(w, dg, "geometry tables"))) return st;
-    if ((st = dev_temp(counts, dk, "geometry counters"))) return st;
+    DevTemp dk;
+    if ((st = dev_temp(tab, dk, "geometry tables"))) return st;
+    char *dt = (char *)dk.p;
     GeomArgs a;
     a.connec = (const int32_t *)dc;
     a.coord = (const double *)dx;
-    a.wgp = (const double *)dg.p;
-    a.nza = (const uint16_t *)da.p;
-    a.nzw = (const double *)dw.p;
-    a.nzn = (const uint16_t *)dn.p;
+    a.wgp = (const double *)(dt + 16);
+    a.nzw = a.wgp + nn;
+    a.nza = (const uint16_t *)(a.nzw + rows);
     a.nelem = NE;
     a.npoin = NP;
     a.mz = mz;
