@@ -16,13 +16,6 @@ pytestmark = pytest.mark.gpu
 EPB = {1: 64, 2: 28, 3: 16, 4: 10, 5: 3}
 
 
-@pytest.fixture(scope="module", autouse=True)
-def gpu():
-    m.init(0)
-    yield
-    m.finalize()
-
-
 def on_gpu(prob, convec, diffu, ins):
     R, D = prob.outputs(), prob.outputs()
     m.copyin(*ins)
@@ -38,7 +31,7 @@ def on_gpu(prob, convec, diffu, ins):
 
 @pytest.mark.parametrize("mode", [m.ASSEMBLY_ATOMIC, m.ASSEMBLY_COLORED])
 @pytest.mark.parametrize("p", [1, 2, 3, 4, 5])
-def test_batch_edges(p, mode):
+def test_batch_edges(gpu, p, mode):
     for n in (1, EPB[p] - 1, EPB[p], EPB[p] + 1, 2 * EPB[p] + 1):
         prob = m.box_problem(n, p, ny=1, nz=1, jitter=0.05)
         print(f"[gpu] p={p} mode={mode} nelem={n}", flush=True)
@@ -54,7 +47,7 @@ def test_batch_edges(p, mode):
 
 
 @pytest.mark.parametrize("p", [2, 4, 5])
-def test_fp32_storage_at_a_batch_edge(p):
+def test_fp32_storage_at_a_batch_edge(gpu, p):
     prob = m.box_problem(EPB[p] + 1, p, ny=2, nz=1, jitter=0.05)
     f, t = prob.fp32(), prob.tables
     idx = (t.dlxigp_ip, t.invAtoIJK, t.AtoI, t.AtoJ, t.AtoK)

@@ -15,13 +15,6 @@ from oracle_lib import Oracle, rel_l2
 pytestmark = pytest.mark.gpu
 
 
-@pytest.fixture(scope="module", autouse=True)
-def gpu():
-    m.init(0)
-    yield
-    m.finalize()
-
-
 def inputs(n, seed, pad):
     rng = np.random.default_rng(seed)
     base = np.zeros(n * 12 + pad, np.float32)
@@ -38,7 +31,7 @@ def inputs(n, seed, pad):
 
 
 @pytest.mark.parametrize("nelem,p,pad", [(1, 1, 0), (15, 2, 0), (17, 2, 1), (16, 3, 0), (33, 4, 0), (5, 7, 3)])
-def test_predict(nelem, p, pad):
+def test_predict(gpu, nelem, p, pad):
     t = m.hex_tables(p)
     base, F, P = inputs(nelem * t.nnode, 10 * p + nelem, pad)
     mu = np.zeros((nelem, t.nnode), order="F")
@@ -57,7 +50,7 @@ def test_predict(nelem, p, pad):
 
 
 @pytest.mark.parametrize("n,pad", [(1, 0), (63, 0), (64, 2), (65, 0), (1024 * 64 + 17, 0), (3 * 1024 * 64 - 1, 0)])
-def test_gradient(n, pad):
+def test_gradient(gpu, n, pad):
     base, F, P = inputs(n, n, pad)
     gnu = np.random.default_rng(3).uniform(0.5, 1.5, n).astype(np.float32)
     grad = np.full(m.CLOSURE_NTRAIN, np.nan, np.float32)
