@@ -1,5 +1,7 @@
 // Assembly plan of a mesh (host code, no HIP): the data the kernels' write
-// phase uses (layout described in msod_kernels.h).  Built once per mesh from
+// phase uses (layout described in msod_kernels.h), for the coloured assembly;
+// the atomic one has its node lists from the device (k_plan_batches in
+// msod_runtime.hip, the same lists).  Built once per mesh from
 // the reference connectivity connec(nelem,nnode) (1-based, Fortran layout):
 //   * batches of B consecutive elements;
 //   * the sorted distinct nodes of every batch (unode, offsets uoff) and the

@@ -171,6 +171,116 @@ __global__ void k_plan_lanes(const uint32_t *conn, const uint16_t *lidx, int64_t
     }
 }
 
+// The batches' node lists from the connectivity, one workgroup per batch: its
+// nodes are sorted in LDS (bitonic) and the distinct ones numbered in
+// ascending order, as build_host_plan does on the host.  FILL = false:
+// count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
+// unode from uoff, conn and lidx in the layout of the order's kernels.
+// A first convection at 64^3, p=4 takes 7 ms in all (193 with the host plan).
+constexpr uint32_t kBadBatch = 0x80000000u;
+template <int P>
+struct PlanShape {
+    static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
+    static constexpr int UMAX = P <= kColMaxP ? ColShape<P <= kColMaxP ? P : 1>::UMAX : CShape<P>::UMAX;
+    static constexpr int NT = 256;
+    static constexpr int SORT = UMAX <= 512 ? 512 : (UMAX <= 1024 ? 1024 : 2048);
+    static constexpr int PER = SORT / NT;
+};
+template <int P, bool FILL>
+__global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int64_t nelem, int64_t npoin, int B,
+                                                      const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
+                                                      uint32_t *unode, uint32_t *conn, uint16_t *lidx)
+{
+    using S = PlanShape<P>;
+    constexpr int NN = S::NN, NT = S::NT, SORT = S::SORT, PER = S::PER;
+    __shared__ uint32_t s[SORT];
+    __shared__ uint32_t su[SORT];
+    __shared__ uint32_t sw[NT / 64], sbad;
+    const int t = threadIdx.x;
+    const int64_t b = xcd_slot(blockIdx.x, gridDim.x), e0 = b * B;
+    const int ne = (int)(nelem - e0 < B ? nelem - e0 : B);
+    // the column kernels' layout is padded with copies of the last element
+    const int nf = P <= kColMaxP ? B : ne, n = nf * NN;
+    if (t == 0) sbad = 0;
+    __syncthreads();
+    uint32_t v[PER];
+    unsigned bad = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = t + j * NT;
+        v[j] = 0xffffffffu;
+        if (i < n) {
+            const int le = i % nf, l = i / nf;  // neighbouring lanes: neighbouring elements
+            const int32_t c = connec[e0 + (le < ne ? le : ne - 1) + nelem * (int64_t)l2g[l]];
+            const bool ok = c >= 1 && c <= npoin;
+            bad += !ok && le < ne;
+            v[j] = ok ? (uint32_t)(c - 1) : 0u;
+        }
+        s[i] = v[j];
+    }
+    if (bad) atomicAdd(&sbad, bad);
+    __syncthreads();
+    for (int k = 2; k <= SORT; k *= 2)
+        for (int d = k / 2; d > 0; d /= 2) {
+#pragma unroll
+            for (int j = 0; j < PER / 2; ++j) {
+                const int i = t + j * NT;
+                const int lo = 2 * i - (i & (d - 1)), hi = lo + d;
+                const uint32_t x = s[lo], y = s[hi];
+                if ((x > y) == ((lo & k) == 0)) {
+                    s[lo] = y;
+                    s[hi] = x;
+                }
+            }
+            __syncthreads();
+        }
+    // PER consecutive places per thread: the distinct nodes among them, then
+    // their places by a scan over the workgroup
+    uint32_t first[PER], c = 0;
+#pragma unroll
+    for (int j = 0; j < PER; ++j) {
+        const int i = t * PER + j;
+        first[j] = s[i] != 0xffffffffu && (i == 0 || s[i] != s[i - 1]);
+        c += first[j];
+    }
+    uint32_t sum = c;
+#pragma unroll
+    for (int d = 1; d < 64; d *= 2) {
+        const uint32_t o = __shfl_up(sum, d);
+        if ((t & 63) >= d) sum += o;
+    }
+    if ((t & 63) == 63) sw[t / 64] = sum;
+    __syncthreads();
+    uint32_t at = sum - c, U = 0;
+    for (int w = 0; w < NT / 64; ++w) {
+        at += w < t / 64 ? sw[w] : 0u;
+        U += sw[w];
+    }
+    if constexpr (!FILL) {
+        if (t == 0) count[b] = sbad ? kBadBatch + sbad : U;
+    } else {
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (first[j]) su[at++] = s[t * PER + j];
+        __syncthreads();
+        const uint32_t o = uoff[b];
+        for (uint32_t i = t; i < U; i += NT) unode[o + i] = su[i];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = t + j * NT;
+            if (i >= n) break;
+            uint32_t lo = 0, hi = U;  // su[lo] <= v[j] < su[hi]
+            while (hi - lo > 1) {
+                const uint32_t m = (lo + hi) / 2;
+                (su[m] <= v[j] ? lo : hi) = m;
+            }
+            const ElemEntry<P> en{e0 + i % nf, i / nf};
+            conn[en.entry()] = v[j];
+            lidx[en.entry()] = (uint16_t)lo;
+        }
+    }
+}
+
 static unsigned grid_for(int64_t n, int bs)
 {
     int64_t g = (n + bs - 1) / bs;
@@ -307,6 +417,24 @@ hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *l
     });
 }
 
+// k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
+hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
+                               const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
+                               uint32_t *conn, uint16_t *lidx, hipStream_t s)
+{
+    return with_porder(porder, [&](auto p) {
+        if (B > PlanShape<p()>::UMAX / PlanShape<p()>::NN) return hipErrorInvalidValue;
+        const dim3 grid((unsigned)((nelem + B - 1) / B)), block(PlanShape<p()>::NT);
+        if (fill)
+            hipLaunchKernelGGL((k_plan_batches<p(), true>), grid, block, 0, s, connec, nelem, npoin, B, l2g, uoff, count,
+                               unode, conn, lidx);
+        else
+            hipLaunchKernelGGL((k_plan_batches<p(), false>), grid, block, 0, s, connec, nelem, npoin, B, l2g, uoff,
+                               count, unode, conn, lidx);
+        return hipGetLastError();
+    });
+}
+
 }  // namespace msod
 
 // ---------------------------------------------------------------------------
@@ -350,7 +478,8 @@ struct PlanEntry {
     std::vector<int64_t> color_off;  // batches of colour c: order[color_off[c] .. color_off[c+1])
     uint32_t *unref = nullptr;       // nodes no element references (zeroed per call)
     int64_t nunref = 0;
-    bool colored = false;            // batch colouring built (the coloured assembly needs it)
+    bool host = false;               // built on the host: colours, first writers and unref are there
+    bool colored = false;            // batch colouring found (the coloured assembly needs it)
     void release()
     {
         for (void *p : {(void *)conn, (void *)uoff, (void *)unode, (void *)order, (void *)lidx,
@@ -627,8 +756,53 @@ int upload(const std::vector<V> &h, V **d, const char *what)
     return MSOD_OK;
 }
 
-// Builds the assembly plan of a mesh (msod_plan.h) from its connectivity,
-// a device array in the reference layout, and uploads it.
+// Builds the node lists of a mesh's batches on the device: all that the atomic
+// assembly reads of the plan.
+int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
+{
+    const int64_t nn = (int64_t)ts->l2g.size(), nb = (nelem + B - 1) / B;
+    if (npoin > 0x7fffffff || nelem * nn > 0xffffffffLL)
+        return fail(MSOD_ERR_MESH, "mesh too large for 32-bit node indices");
+    P.B = B;
+    P.nbatch = nb;
+    // connec may come from work on the default stream, which the copy that
+    // feeds the host plan waits for
+    HIPCHK(hipStreamSynchronize(nullptr), "plan");
+    HIPCHK(hipMalloc((void **)&P.uoff, sizeof(uint32_t) * (nb + 1)), "plan");
+    HIPCHK(launch_plan_batches(ts->porder, false, dconnec, nelem, npoin, B, ts->dl2g, nullptr, P.uoff, nullptr, nullptr,
+                               nullptr, g.stream),
+           "batch counts");
+    std::vector<uint32_t> uoff(nb + 1);
+    HIPCHK(hipMemcpyAsync(uoff.data() + 1, P.uoff, sizeof(uint32_t) * nb, hipMemcpyDeviceToHost, g.stream),
+           "batch counts");
+    HIPCHK(hipStreamSynchronize(g.stream), "batch counts");
+    int64_t bad = 0;
+    for (int64_t b = 1; b <= nb; ++b) {
+        if (uoff[b] & kBadBatch) {
+            bad += uoff[b] - kBadBatch;
+            uoff[b] = 0;
+        }
+        P.ustride = std::max(P.ustride, (int)uoff[b]);
+        uoff[b] += uoff[b - 1];
+    }
+    if (bad)
+        return fail(MSOD_ERR_MESH, "connec holds %lld node numbers outside 1..npoin (npoin=%lld)", (long long)bad,
+                    (long long)npoin);
+    const int64_t n = geo_elems(ts->porder, nelem) * nn;
+    HIPCHK(hipMalloc((void **)&P.conn, sizeof(uint32_t) * n), "plan");
+    HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
+    HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * uoff[nb]), "plan");
+    HIPCHK(hipMemcpyAsync(P.uoff, uoff.data(), sizeof(uint32_t) * (nb + 1), hipMemcpyHostToDevice, g.stream), "plan");
+    HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
+                               P.lidx, g.stream),
+           "batch lists");
+    HIPCHK(hipStreamSynchronize(g.stream), "batch lists");
+    return MSOD_OK;
+}
+
+// Builds the whole plan of a mesh (msod_plan.h), with the colouring, on the
+// host from its connectivity, a device array in the reference layout, and
+// uploads it.
 int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
 {
     const int64_t E = nelem * (int64_t)ts->l2g.size();
@@ -667,6 +841,7 @@ int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet
     if ((st = upload(H.order, &P.order, "plan upload"))) return st;
     if ((st = upload(H.unref, &P.unref, "plan upload"))) return st;
     P.nunref = (int64_t)H.unref.size();
+    P.host = true;
     return MSOD_OK;
 }
 
@@ -696,12 +871,20 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
              const PlanEntry **out)
 {
     if (ver == 0) drop_unversioned(dconnec);
-    for (auto &c : g.plans)
-        if (c.src == dconnec && c.ver == ver && c.nelem == nelem && c.npoin == npoin &&
-            c.porder == ts->porder && c.l2g == ts->l2g && c.B == B) {
+    const bool host = g.assembly == kColored;  // the atomic assembly takes either plan
+    for (size_t i = 0; i < g.plans.size(); ++i) {
+        PlanEntry &c = g.plans[i];
+        if (c.src != dconnec || c.ver != ver || c.nelem != nelem || c.npoin != npoin || c.porder != ts->porder ||
+            c.l2g != ts->l2g || c.B != B)
+            continue;
+        if (c.host || !host) {
             *out = &c;
             return MSOD_OK;
         }
+        c.release();  // hipFree waits for the work queued
+        g.plans.erase(g.plans.begin() + i);
+        break;
+    }
     PlanEntry P;
     P.src = dconnec;
     P.ver = ver;
@@ -709,7 +892,8 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
     P.npoin = npoin;
     P.porder = ts->porder;
     P.l2g = ts->l2g;
-    int st = build_plan(dconnec, nelem, npoin, ts, B, P);
+    int st = host ? build_plan(dconnec, nelem, npoin, ts, B, P)
+                  : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, P);
     if (st) {
         P.release();
         return st;
@@ -867,12 +1051,6 @@ int check_sizes(int porder, int nelem, int npoin)
     return MSOD_OK;
 }
 
-// Batch order of the atomic mode, per kernel (measured at 128^3 porder 4):
-// mesh order lets neighbouring batches meet in L2, which pays in the
-// diffusion; the convection ran faster in colour order (12.81 against 13.30
-// ms; colour order within chunks of 256..16384 batches: 13.07..19.90 ms).
-constexpr bool kConvecNatural = false;
-constexpr bool kDiffuNatural = true;
 // Batches per workgroup, at most, per kernel.  The diffusion takes one: a
 // form that ran kpb batches per workgroup with every load one pass ahead
 // needed 148-152 VGPRs against 120 (3 waves per SIMD against 4) and ran
@@ -882,10 +1060,10 @@ constexpr int kConvecKpb = kBatchesPerBlock;
 constexpr int kDiffuKpb = 1;
 
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
-// the kernel: one launch per colour, or one launch over all batches, taken
-// in mesh order (natural) or grouped by colour.
+// the kernel: one launch per colour, or one launch over all batches in mesh
+// order, where neighbouring batches meet in L2.
 template <class A, class L>
-int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what, bool natural, int kpb_max)
+int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what, int kpb_max)
 {
     Plan pl;
     pl.conn = P.conn;
@@ -916,7 +1094,7 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     }
     TimedLaunch tk(timer);
     if (g.assembly == kAtomic) {
-        pl.batches = natural ? nullptr : P.order;  // null: mesh order, no list
+        pl.batches = nullptr;  // mesh order, no list
         pl.nb = P.nbatch;
         pl.kpb = kpb_for(pl.nb);
         a.plan = pl;
@@ -989,7 +1167,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
                                 return launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch", porder <= kColMaxP || kConvecNatural, kConvecKpb)))
+                            "convection kernel launch", kConvecKpb)))
         return st;
     return finish_call("convection kernel");
 }
@@ -1055,7 +1233,7 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
                                     if (fp32_arith) return launch_diffu_fp32(porder, x, g.stream);
                                 return launch_diffu(porder, x, g.stream);
                             },
-                            "diffusion kernel launch", kDiffuNatural, kDiffuKpb)))
+                            "diffusion kernel launch", kDiffuKpb)))
         return st;
     return finish_call("diffusion kernel");
 }
