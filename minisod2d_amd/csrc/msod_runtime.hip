@@ -459,6 +459,7 @@ struct TableSet {
     int porder;
     std::vector<double> D;       // q*q
     std::vector<int32_t> l2g;    // nn
+    std::vector<char> raw[2];    // the checked arguments' bytes (get_tables), dlxigp_ip in FP64, FP32
     double *dD = nullptr;
     int32_t *dl2g = nullptr;
 };
@@ -668,7 +669,8 @@ int host_view(const void *p, size_t bytes, std::vector<char> &tmp, const char **
 
 // Checks invAtoIJK/AtoI/J/K/dlxigp_ip and returns the cached device table set.
 // dl32: dlxigp_ip holds float (a caller built at rp = 4); its values are
-// widened to double exactly.
+// widened to double exactly.  Arguments equal in every byte to a set's checked
+// ones need no second check, which takes longer than the comparison.
 int get_tables(int porder, const int32_t *invAtoIJK, const int32_t *AtoI, const int32_t *AtoJ,
                const int32_t *AtoK, const void *dlxigp_ip, TableSet **out, bool dl32 = false)
 {
@@ -685,6 +687,29 @@ int get_tables(int porder, const int32_t *invAtoIJK, const int32_t *AtoI, const 
         return st;
     const int32_t *inv = (const int32_t *)pinv, *ai = (const int32_t *)pi,
                   *aj = (const int32_t *)pj, *ak = (const int32_t *)pk;
+    const std::pair<const char *, size_t> arg[5] = {{pinv, sizeof(int32_t) * nn},
+                                                    {pi, sizeof(int32_t) * nn},
+                                                    {pj, sizeof(int32_t) * nn},
+                                                    {pk, sizeof(int32_t) * nn},
+                                                    {pdl, (dl32 ? sizeof(float) : sizeof(double)) * nn * 3 * q}};
+    for (TableSet *ts : g.tables) {
+        if (ts->porder != porder || ts->raw[dl32].empty()) continue;
+        const char *r = ts->raw[dl32].data();
+        bool same = true;
+        for (const auto &x : arg) {
+            same = same && std::memcmp(r, x.first, x.second) == 0;
+            r += x.second;
+        }
+        if (same) {
+            *out = ts;
+            return MSOD_OK;
+        }
+    }
+    auto keep = [&](TableSet *ts) {
+        ts->raw[dl32].clear();
+        for (const auto &x : arg) ts->raw[dl32].insert(ts->raw[dl32].end(), x.first, x.first + x.second);
+        *out = ts;
+    };
     std::vector<double> dlw;
     if (dl32) {
         dlw.resize((size_t)nn * 3 * q);
@@ -726,7 +751,7 @@ int get_tables(int porder, const int32_t *invAtoIJK, const int32_t *AtoI, const 
     for (TableSet *ts : g.tables)
         if (ts->porder == porder && ts->l2g == l2g && ts->D.size() == D.size() &&
             std::memcmp(ts->D.data(), D.data(), sizeof(double) * q * q) == 0) {
-            *out = ts;
+            keep(ts);
             return MSOD_OK;
         }
     TableSet *ts = new TableSet;
@@ -738,7 +763,7 @@ int get_tables(int porder, const int32_t *invAtoIJK, const int32_t *AtoI, const 
     HIPCHK(hipMemcpy(ts->dD, D.data(), sizeof(double) * q * q, hipMemcpyHostToDevice), "upload D");
     HIPCHK(hipMemcpy(ts->dl2g, l2g.data(), sizeof(int32_t) * nn, hipMemcpyHostToDevice), "upload l2g");
     g.tables.push_back(ts);
-    *out = ts;
+    keep(ts);
     return MSOD_OK;
 }
 
