@@ -24,10 +24,19 @@ namespace msod {
 // ---------------------------------------------------------------------------
 // element kernels: features (MODE 0) and mu_sgs gradients (MODE 1)
 // ---------------------------------------------------------------------------
+// One node per thread; several elements per workgroup while they fit 256 threads.
+template <int P>
+struct ElemShape {
+    static constexpr int Q = P + 1;
+    static constexpr int NN = Q * Q * Q;
+    static constexpr int EPB = NN <= 128 ? 256 / NN : 1;
+    static constexpr int NT = NN <= 128 ? 256 : ((NN + 63) / 64) * 64;
+};
+
 template <int P, int MODE>
-__global__ void __launch_bounds__(Shape<P>::NT) k_closure_elem(ClosureElemArgs a)
+__global__ void __launch_bounds__(ElemShape<P>::NT) k_closure_elem(ClosureElemArgs a)
 {
-    using S = Shape<P>;
+    using S = ElemShape<P>;
     constexpr int Q = S::Q, NN = S::NN, EPB = S::EPB;
     __shared__ double sD[Q * Q];
     __shared__ double sA[EPB][5][NN];                  // rho, T, u0, u1, u2
@@ -500,7 +509,7 @@ __global__ void k_residual_error(const double *Rmom, const double *Rener, const 
 template <int P, int MODE>
 static hipError_t launch_elem_p(const ClosureElemArgs &a, hipStream_t s)
 {
-    using S = Shape<P>;
+    using S = ElemShape<P>;
     const int64_t groups = (a.nelem + S::EPB - 1) / S::EPB;
     hipLaunchKernelGGL((k_closure_elem<P, MODE>), dim3((unsigned)groups), dim3(S::NT), 0, s, a);
     return hipGetLastError();

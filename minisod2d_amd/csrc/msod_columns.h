@@ -1,4 +1,4 @@
-// Column kernels: shapes, data layout and device helpers (porder 1..kColMaxP).
+// Column kernels: shapes, data layout and device helpers (porder 1..kMaxP).
 //
 // A workgroup takes the EPB elements of one batch.  Thread t < LANES owns the
 // column of the Q nodes (I, J, 0..Q-1) of one element:
@@ -36,6 +36,8 @@
 // padded with copies of the last element, so that every load is unconditional.
 #pragma once
 
+#include <type_traits>
+
 #include "msod_kernels.h"
 
 namespace msod {
@@ -47,10 +49,11 @@ struct ColShape {
     static constexpr int NN = Q * QQ;
     // 256 threads: 10 elements at order 4, whose rows of 41 nodes share more
     // lines and nodes than two batches of 5 (64^3: convection 1.41 -> 1.31 ms,
-    // diffusion 1.70 -> 1.61; 128^3: 10.65 -> 10.30 and 12.05 -> 11.20).  Order 5
-    // takes 128 threads and three elements (40^3: convection 0.645 ms, diffusion
-    // 0.760; with 256 and seven 0.575 and 0.860).
-    static constexpr int NT = P == 5 ? 128 : 256;
+    // diffusion 1.70 -> 1.61; 128^3: 10.65 -> 10.30 and 12.05 -> 11.20).  Above
+    // kNarrowP the rows matter most, as they merge the neighbours' nodes
+    // (convection 40^3 order 6: one element 1.29 ms, two 1.16, five 1.03; 48^3
+    // order 7: one 3.07, two 2.67, four 2.56).
+    static constexpr int NT = 256;
     static constexpr int EPB = NT / QQ;         // elements of a batch
     static constexpr int LANES = EPB * QQ;
     static constexpr int UMAX = EPB * NN;       // element nodes, and most distinct nodes, of a batch
@@ -64,19 +67,10 @@ __host__ __device__ constexpr int line_ref(int m) { return m == 0 ? 0 : (m == P 
 template <int P>
 __host__ __device__ constexpr int line_pos(int s) { return s == 0 ? 0 : (s == 1 ? P : s - 1); }
 
-// Entry of element node (e, l) in the element-sized arrays of either layout:
-// conn at entry(), geo's pair c at pair() + c*pair_stride().
-template <int P, bool COL = (P <= kColMaxP)>
-struct ElemEntry {
-    static constexpr int Q = P + 1, QQ = Q * Q, NN = Q * QQ;
-    int64_t e;
-    int l;
-    __device__ __forceinline__ int64_t entry() const { return e * NN + l; }
-    __device__ __forceinline__ int64_t pair() const { return e * 5 * NN + l; }
-    static constexpr int pair_stride() { return NN; }
-};
+// Entry of element node (e, l) in the element-sized arrays: conn at entry(),
+// geo's pair c at pair() + c*pair_stride().
 template <int P>
-struct ElemEntry<P, true> {
+struct ElemEntry {
     using S = ColShape<P>;
     int64_t e;
     int l;
@@ -131,6 +125,14 @@ __device__ __forceinline__ double col_D(Uniform<double> D, int i, int n)
     return D[line_ref<P>(i) * (P + 1) + line_ref<P>(n)];
 }
 
+// Pair c of entry (b, K, tc).
+template <int P, bool NTL, typename T>
+__device__ __forceinline__ GeoPair<T> col_geo_pair(const T *geo, uint32_t b, int K, int tc, int c)
+{
+    using S = ColShape<P>;
+    const GeoPair<T> *p = reinterpret_cast<const GeoPair<T> *>(geo) + ((int64_t)b * S::Q + K) * 5 * S::LANES + tc;
+    return NTL ? __builtin_nontemporal_load(&p[c * S::LANES]) : p[c * S::LANES];
+}
 // GeoNode of entry (b, K, tc).
 template <int P, bool NTL, typename T>
 __device__ __forceinline__ GeoNode<T> col_geo(const T *geo, uint32_t b, int K, int tc)
@@ -165,6 +167,44 @@ __device__ __forceinline__ void col_add(double *sR, int US, bool active, int le,
             __syncthreads();
         }
     }
+}
+
+// f(0), f(1), .. f(Q - 1) with compile-time arguments: a loop that is unrolled
+// whatever its size (order 8's slices pass the compiler's limit).
+template <int Q, class F, int K = 0>
+__device__ __forceinline__ void col_slices(const F &f)
+{
+    if constexpr (K < Q) {
+        f(std::integral_constant<int, K>{});
+        col_slices<Q, F, K + 1>(f);
+    }
+}
+
+// The last node of an element's I line and the first of its right neighbour's
+// sit in neighbouring lanes: where they are one node of the mesh, its values
+// are summed in the right lane (both active), and the left one has nothing to
+// write (false).
+template <int P, int EPB = ColShape<P>::EPB>
+__device__ __forceinline__ bool col_merge(uint32_t node, int I, int le, bool both, double (&v)[5])
+{
+    const uint32_t next = __shfl_down(node, 1);  // by every lane
+    const bool give = both && I == P && le + 1 < EPB && (threadIdx.x & 63) != 63 &&
+                      next == node;
+#pragma unroll
+    for (int c = 0; c < 5; ++c) v[c] += __shfl_up(give ? v[c] : 0.0, 1);
+    return !give;
+}
+
+// One element node's values to the outputs (atomic mode).
+template <typename TO>
+__device__ __forceinline__ void col_scatter(uint32_t node, const double (&v)[5], TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin)
+{
+    const int64_t g = node;
+    unsafeAtomicAdd(Rmass + g, (TO)v[0]);
+    unsafeAtomicAdd(Rmom + g, (TO)v[1]);
+    unsafeAtomicAdd(Rmom + npoin + g, (TO)v[2]);
+    unsafeAtomicAdd(Rmom + 2 * npoin + g, (TO)v[3]);
+    unsafeAtomicAdd(Rener + g, (TO)v[4]);
 }
 
 // A thread's entries t, t + NT, ... of a batch's node list.

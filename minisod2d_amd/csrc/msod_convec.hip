@@ -1,318 +1,431 @@
-// Convective residual kernel (counterpart of full_convec_ijk,
+// Convective residual (counterpart of full_convec_ijk,
 // src/kernels/sources/elem_convec.f90:198-431, with the energy fluxes of
-// full_convec_ijk_split, :674-832).
+// full_convec_ijk_split, :674-832); see msod_columns.h for the thread layout.
 //
-// One workgroup per batch of CShape<P>::BATCH elements, processed in passes of
-// CShape<P>::EPB elements with one thread per element node.  Per pass:
-//  1. gather: each thread reads its global node (conn, element-major) and
-//     writes 10 nodal values to LDS:
-//       rho, p, H = E + k, rhoH = rho E + rho k, u(3), q(3)     (k = |u|^2/2)
-//  2. sweeps: for each reference direction d the thread runs the 1-D
-//     derivative D[I_d][n] along its grid line.  Rather than differentiating
-//     the 39 flux components the reference forms, the He column of the
-//     TARGET node is folded into the fluxes at the source nodes:
-//     U_d(s) = sum_i He(i,d)u_i(s).  Since He is taken at the target node,
-//       div(q (x) u)_i = sum_d D_d[ q_i U_d ],  div u = sum_d He(:,d).D_d[u], ...
-//     Per line the thread forms the plain 1-D derivatives of r, p, H, rH, u, q and the
-//     derivatives of the products with U_d; the node's own r, u, q, H and He
-//     column then contract them (eleven accumulators over the three
-//     directions; the sweep code is shared by the directions).  LDS holds the
-//     ten values of a node contiguously, so a source costs one address and
-//     five 16-byte reads (nine values, rH formed in the sweep, where that
-//     fits another workgroup per CU: convec_drop_rh).
-//     The result equals the reference's algebra exactly in real arithmetic;
-//     rounding differs at the 1e-16 level.
-//  3. residual x gpvol, added into the batch's per-node sums in LDS in a
-//     fixed order (add_pass).
-// After the passes the batch's distinct nodes are written once each
-// (write_batch_nodes: plain store / read-add-store per colour, or FP64 atomics).
+// With He(:,d) of the TARGET node a folded into the source values,
+//   U_n = sum_i He(i,d) u_i(n),  Q_n = sum_i He(i,d) q_i(n),
+// every term of the split form is, over the three directions d and the
+// sources n of a line (D = D[I_d(a)][n]),
+//   S3 = sum D (Q_n + U_a r_n)          (div q + u.grad r)
+//   S4 = sum D U_n                      (div u)
+//   M_i = sum D [(U_n + U_a) q_i(n) + (r_a U_n + Q_a) u_i(n) + 4 He(i,d) p(n)]
+//   X = sum D [(U_n + U_a) rH(n) + (r_a U_n + Q_a) H(n)]
+//   Rmass = (S3 + r_a S4)/2,  Rmom_i = (M_i + u_i S3 + q_i S4)/4,
+//   Rener = (X + H_a S3 + rH_a S4)/4
+// with H = E + |u|^2/2 and rH = r H: the terms of elem_convec.f90:228-428 and
+// :694-697, collected by the factors they share.  The result equals the
+// reference's algebra exactly in real arithmetic; rounding differs at the
+// 1e-16 level.
 //
 // Storage types TG (geometry) and TF (nodal fields), FP64 arithmetic
-// throughout (msod_kernels.h).  Without a pressure array the pressure is
-// recovered as p = (gamma-1)(E - rho|u|^2/2) from the stored state.
-#include "msod_kernels.h"
+// (msod_kernels.h), or TA = float for the FP32-arithmetic form.  Without a
+// pressure array the pressure is recovered as p = (gamma-1)(E - rho|u|^2/2)
+// from the stored state.
+#include "msod_columns.h"
 
 namespace msod {
 
-// Inputs of one element node, loaded one pass ahead of their use so that
-// the gathers of the next pass are in flight while this pass computes.
-template <class A>
-struct ConvecNode {
-    typename A::F r, E, q[3];
-    typename A::U u[3];
-    typename A::Pt p;
-    uint32_t li;
+// One direction's factors of the target node.
+template <typename T>
+struct ConvecDir { T h0, h1, h2, Ua, Qa, dp; };
+
+// The sums of one target node; ra, u, q: its own values.
+template <typename T>
+struct ConvecSums {
+    T S3 = 0, S4 = 0, X = 0, M[3] = {0, 0, 0};
+    template <class G>
+    __device__ __forceinline__ ConvecDir<T> direction(const G &g, int d, const T (&u)[3], const T (&q)[3]) const
+    {
+        const T h0 = (T)g.he(3 * d), h1 = (T)g.he(3 * d + 1), h2 = (T)g.he(3 * d + 2);
+        return ConvecDir<T>{h0, h1, h2, h0 * u[0] + h1 * u[1] + h2 * u[2], h0 * q[0] + h1 * q[1] + h2 * q[2], (T)0};
+    }
+    __device__ __forceinline__ void source(ConvecDir<T> &x, T ra, T Dv, T rs, T ps, T Hs, T us0, T us1, T us2, T qs0, T qs1, T qs2)
+    {
+        const T Un = x.h0 * us0 + x.h1 * us1 + x.h2 * us2;
+        const T Qn = x.h0 * qs0 + x.h1 * qs1 + x.h2 * qs2;
+        S3 += Dv * (Qn + x.Ua * rs);
+        S4 += Dv * Un;
+        x.dp += Dv * ps;
+        const T S1 = Dv * (Un + x.Ua), S2 = Dv * (ra * Un + x.Qa);
+        M[0] += S1 * qs0 + S2 * us0;
+        M[1] += S1 * qs1 + S2 * us1;
+        M[2] += S1 * qs2 + S2 * us2;
+        X += (S1 * rs + S2) * Hs;  // S1 rH + S2 H
+        // summed here: left to the compiler the sums sink to the
+        // end of the slice and every source's values stay live
+        asm volatile("" : "+v"(S3), "+v"(S4), "+v"(x.dp), "+v"(M[0]), "+v"(M[1]), "+v"(M[2]), "+v"(X));
+    }
+    __device__ __forceinline__ void finish(const ConvecDir<T> &x)
+    {
+        const T dp4 = (T)4 * x.dp;
+        M[0] += x.h0 * dp4;
+        M[1] += x.h1 * dp4;
+        M[2] += x.h2 * dp4;
+        asm volatile("" : "+v"(M[0]), "+v"(M[1]), "+v"(M[2]));
+    }
+    __device__ __forceinline__ void values(T gv, T ra, T Ha, const T (&u)[3], const T (&q)[3], double (&v)[5]) const
+    {
+        v[0] = (double)(gv * ((T)0.5 * (S3 + ra * S4)));
+#pragma unroll
+        for (int i = 0; i < 3; ++i) v[1 + i] = (double)(gv * ((T)0.25 * (M[i] + u[i] * S3 + q[i] * S4)));
+        v[4] = (double)(gv * ((T)0.25 * (X + Ha * S3 + ra * Ha * S4)));
+    }
 };
 
-template <int NN, class A>
-__device__ __forceinline__ void convec_fetch(const A &a, int64_t e, int l, uint32_t gnode, ConvecNode<A> &x)
+template <int P, bool COLORED, class A, typename TA>
+__global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
 {
-    const int64_t g = gnode;
-    const int64_t np = a.npoin;
-    x.r = a.rho[g];
-    x.E = a.E[g];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-        x.u[d] = a.u[g + d * np];
-        x.q[d] = a.q[g + d * np];
-    }
-    x.p = a.pr ? a.pr[g] : (typename A::Pt)0;
-    x.li = __builtin_nontemporal_load(&a.plan.lidx[e * NN + l]);
-}
-
-// LDS bytes of a workgroup with NF values per node record.
-template <int P, typename TA>
-constexpr size_t convec_lds(int nf)
-{
-    using S = CShape<P>;
-    return sizeof(TA) * (S::Q * S::Q + (size_t)S::EPB * S::NN * nf) + sizeof(double) * 5 * S::UMAX +
-           3 * sizeof(uint32_t) * kMaxKpb;
-}
-// rH = rho E + rho k is left out of the records (formed as r H in the sweep)
-// where that fits one more workgroup per CU, for FP32 element arrays with
-// FP64 arithmetic at porder 6 and 7 (p=7: 82.6 -> 78.5 KB, two 512-thread
-// workgroups instead of one, at most 128 VGPRs: 44 B of spills per lane;
-// 48^3 p=7: 3.66 -> 3.35 ms for the FP32 split, 3.51 -> 3.21 ms with every
-// input in FP32).  With FP64 element arrays the 128-VGPR bound spills 108 B
-// per lane and ran slower (3.98 -> 4.18 ms): one workgroup there.
-template <int P, typename TA, typename TG>
-constexpr bool convec_drop_rh()
-{
-    return sizeof(TG) < sizeof(TA) && 163840 / convec_lds<P, TA>(9) > 163840 / convec_lds<P, TA>(10);
-}
-// Launch bound in waves per SIMD: 3 (up to 168 VGPRs, room for the loads in
-// flight; 4 would force spills at p=4); 4 for 512-thread workgroups whose
-// LDS lets two share a CU.
-template <int P, typename TA, typename TG>
-constexpr int convec_waves()
-{
-    return CShape<P>::NT == 512 && convec_drop_rh<P, TA, TG>() ? 4 : 3;
-}
-
-// TA: arithmetic type of the gathers, fluxes and sweeps (FP64, or FP32 for
-// the FP32-arithmetic form); the node sums and the assembly stay FP64.
-template <int P, class A, typename TA = double>
-__global__ void __launch_bounds__(CShape<P>::NT, (convec_waves<P, TA, typename A::G>())) k_convec(A a)
-{
+    using S = ColShape<P>;
+    using T = TA;
     using TG = typename A::G;
-    using S = CShape<P>;
-    using T = TA;  // arithmetic
-    constexpr int Q = S::Q, NN = S::NN, EPB = S::EPB, UMAX = S::UMAX, NPASS = S::NPASS;
-    // record: r, p, H, [rH,] u(3), q(3)
-    constexpr bool kRH = !convec_drop_rh<P, TA, TG>();
-    constexpr int NF = kRH ? 10 : 9, iU = kRH ? 4 : 3, iQ = iU + 3;
+    constexpr int Q = S::Q, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
+    struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
-    __shared__ __attribute__((aligned(16))) T sF[EPB][NN][NF];  // node-major: one base address per source
-    __shared__ double sR[5][UMAX];
-    __shared__ uint32_t sB[kMaxKpb], sU0[kMaxKpb], sU1[kMaxKpb];
-    constexpr int NT = S::NT, UPT = (UMAX + NT - 1) / NT;
+    __shared__ V2 sP[4][NT];  // one slice: (r,p) (u0,u1) (u2,q0) (q1,q2)
+    __shared__ T sH[NT];      // and H
+    extern __shared__ __attribute__((aligned(16))) double sR[];  // node sums [5][US]
 
     const Plan &pl = a.plan;
-    const int64_t first = (int64_t)xcd_slot(blockIdx.x, gridDim.x) * pl.kpb;
-    const int nbat = (int)(pl.nb - first < pl.kpb ? pl.nb - first : pl.kpb);
-    const int npass = nbat * NPASS;  // passes of this block, over its batches
-    const int t = threadIdx.x;
-    const int le = t / NN;  // >= EPB for the few idle threads
-    const int l = t - le * NN;
-    const int I = l % Q, J = (l / Q) % Q, K = l / (Q * Q);
-    // Loads are unconditional, so that the compiler can count them exactly
-    // and wait for each one only where it is used: idle threads and the
-    // elements past the end of the mesh load a real element, and the result
-    // is not used.
-    const int lec = le < EPB ? le : EPB - 1;
-    auto elem = [&](int64_t bb, int p) -> int64_t {
-        const int64_t e = bb * S::BATCH + p * EPB + lec;
-        return e < a.nelem ? e : a.nelem - 1;
-    };
-    // element of pass g of this block (g clamped to the last pass)
-    auto elem_of = [&](int g) -> int64_t {
-        const int gc = g < npass ? g : npass - 1;
-        return elem((int64_t)sB[gc / NPASS], gc % NPASS);
-    };
+    const int US = pl.ustride, t = threadIdx.x;
+    const ColThread<P> th(t);
+    const int tc = th.tc, le = th.le, I = th.I, J = th.J;
+    const int64_t np = a.npoin;
+    const auto D = uniform(a.tab.D);
+    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
+    const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+    const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
+    // FP32 state with FP64 outputs comes without a pressure array
+    constexpr bool kRecover = sizeof(typename A::F) == 4 && sizeof(typename A::Pt) == 4 && sizeof(typename A::O) == 8;
 
-    for (int i = t; i < nbat; i += blockDim.x) {
-        const uint32_t bi = plan_batch(pl.batches, first + i);
-        sB[i] = bi;
-        sU0[i] = pl.uoff[bi];
-        sU1[i] = pl.uoff[bi + 1];
+    uint32_t gn[Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) gn[k] = __builtin_nontemporal_load(&pl.conn[((int64_t)b * Q + k) * LANES + tc]);
+    GeoNode<TG> geo[2];
+    geo[0] = col_geo<P, true>(a.geo, b, 0, tc);
+    typename A::F fr[Q], fE[Q], fq[Q][3];
+    typename A::U fu[Q][3];
+    typename A::Pt fp[Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        const int64_t g = gn[k];
+        fr[k] = a.rho[g];
+        fE[k] = a.E[g];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            fu[k][d] = a.u[g + d * np];
+            fq[k][d] = a.q[g + d * np];
+        }
+        if constexpr (!kRecover) fp[k] = a.pr[g];
     }
-    for (int i = t; i < Q * Q; i += blockDim.x) sD[i] = (T)a.tab.D[i];
+    col_table<P>(a.tab.D, sD);
+    for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
 
-    // prologue: nodal values of pass 0, connectivity of pass 1
-    ConvecNode<A> nd[2];
-    uint32_t gnext;  // global node of the next pass's element node
+    T r[Q], p[Q], H[Q], u[Q][3], q[Q][3];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        r[k] = (T)fr[k];
+        const T E = (T)fE[k];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            u[k][d] = (T)fu[k][d];
+            q[k][d] = (T)fq[k][d];
+        }
+        const T ke = u[k][0] * u[k][0] * (T)0.5 + u[k][1] * u[k][1] * (T)0.5 + u[k][2] * u[k][2] * (T)0.5;
+        if constexpr (kRecover)
+            // p = (gamma-1)(E - rho|u|^2/2), in FP64 whatever T: the difference cancels
+            p[k] = (T)(a.gamma_m1 * ((double)E - (double)r[k] * 0.5 *
+                                                     ((double)u[k][0] * u[k][0] + (double)u[k][1] * u[k][1] +
+                                                      (double)u[k][2] * u[k][2])));
+        else
+            p[k] = (T)fp[k];
+        H[k] = E + ke;
+    }
+    uint32_t wn[S::UPT];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        const T ra = r[k], Ha = H[k];
+        if (k > 0) __syncthreads();  // the previous slice is read
+        sP[0][t] = V2{ra, p[k]};
+        sP[1][t] = V2{u[k][0], u[k][1]};
+        sP[2][t] = V2{u[k][2], q[k][0]};
+        sP[3][t] = V2{q[k][1], q[k][2]};
+        sH[t] = Ha;
+        const uint32_t li = __builtin_nontemporal_load(&pl.lidx[((int64_t)b * Q + k) * LANES + tc]);
+        if (k + 1 < Q)
+            geo[(k + 1) & 1] = col_geo<P, true>(a.geo, b, k + 1, tc);
+        else
+            col_list<P>(pl.unode + u0, U, wn);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        const GeoNode<TG> &gk = geo[k & 1];
+        ConvecSums<T> sum;
+        // Steps 0..2Q-1: the sources along I, then J, from LDS; a source's
+        // record is read while the one before it is used, and every other
+        // step a source along K, which needs no LDS, is used as well, so that
+        // the LDS reads spread over all of the slice's arithmetic.  The
+        // scheduling barriers keep the order (and the registers).
+        ConvecDir<T> dz = sum.direction(gk, 2, u[k], q[k]), dl = sum.direction(gk, 0, u[k], q[k]);
+        const int sI = tc - I, sJ = tc - J * EPB * Q;
+        auto slot = [&](int s) { return s < Q ? sI + s : sJ + (s - Q) * EPB * Q; };
+        V2 c0 = sP[0][sI], c1 = sP[1][sI], c2 = sP[2][sI], c3 = sP[3][sI];
+        T cH = sH[sI], cD = sD[I * Q];
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            const int m = slot(s + 1 < 2 * Q ? s + 1 : s);
+            const V2 n0 = sP[0][m], n1 = sP[1][m], n2 = sP[2][m], n3 = sP[3][m];
+            const T nH = sH[m], nD = s + 1 < Q ? sD[I * Q + s + 1] : sD[J * Q + (s + 1 < 2 * Q ? s + 1 - Q : 0)];
+            __builtin_amdgcn_sched_barrier(0);
+            if (s % 2 == 0) {
+                const int n = s / 2;
+                sum.source(dz, ra, (T)col_D<P>(D, k, n), r[n], p[n], H[n], u[n][0], u[n][1], u[n][2], q[n][0], q[n][1], q[n][2]);
+            }
+            sum.source(dl, ra, cD, c0.x, c0.y, cH, c1.x, c1.y, c2.x, c2.y, c3.x, c3.y);
+            if (s == Q - 1) {
+                sum.finish(dl);
+                dl = sum.direction(gk, 1, u[k], q[k]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            c0 = n0;
+            c1 = n1;
+            c2 = n2;
+            c3 = n3;
+            cH = nH;
+            cD = nD;
+        }
+        sum.finish(dl);
+        sum.finish(dz);
+        double v[5];
+        sum.values((T)gk.gvol(), ra, Ha, u[k], q[k], v);
+        col_add<P, COLORED>(sR, US, active, le, li, v);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();  // every node sum of the batch done
+    col_write<P, COLORED>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
+}
+
+// Orders above kNarrowP: the same walk within 256 VGPRs, of which the column
+// takes up to 162.  The directions follow one another (one set of factors live)
+// and the geometry has one buffer, whose pairs are loaded anew for the next
+// slice as soon as a direction is done with them.  The atomic mode adds to the
+// outputs from the registers (col_merge, col_scatter).  Against one node per
+// thread with everything read from LDS: 48^3 order 7 4.05 -> 2.56 ms, FP32
+// split 3.21 -> 2.18; 40^3 order 6 1.96 -> 1.03; 32^3 order 8 1.96 -> 1.49; order 5,
+// against the kernel above with LDS sums, 64^3 2.60 -> 2.38.  Of order 7's 2.56
+// ms, outputs take about a third (2.0 ms of 3.07 without any, 2.4 with plain
+// stores, before neighbours' nodes were merged); the rest is the FP64 work and
+// LDS reads of two waves per SIMD.
+template <int P, bool COLORED, class A, typename TA>
+__global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
+{
+    using S = ColShape<P>;
+    using T = TA;
+    using TG = typename A::G;
+    constexpr int Q = S::Q, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
+    struct alignas(2 * sizeof(T)) V2 { T x, y; };
+    __shared__ T sD[Q * Q];
+    __shared__ V2 sP[4][NT];  // one slice: (r,p) (u0,u1) (u2,q0) (q1,q2)
+    __shared__ T sH[NT];      // and H
+    extern __shared__ __attribute__((aligned(16))) double sR[];  // coloured mode: node sums [5][US]
+
+    const Plan &pl = a.plan;
+    const int US = pl.ustride, t = threadIdx.x;
+    const ColThread<P> th(t);
+    const int tc = th.tc, le = th.le, I = th.I, J = th.J;
+    const int64_t np = a.npoin;
+    const auto D = uniform(a.tab.D);
+    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
+    const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
+    constexpr bool kRecover = sizeof(typename A::F) == 4 && sizeof(typename A::Pt) == 4 && sizeof(typename A::O) == 8;
+
+    T r[Q], p[Q], H[Q], u[Q][3], q[Q][3];
+    GeoNode<TG> geo;
     {
-        const int64_t b0 = plan_batch(pl.batches, first);
-        const int64_t e0 = elem(b0, 0);
-        convec_fetch<NN>(a, e0, l, __builtin_nontemporal_load(&pl.conn[e0 * NN + l]), nd[0]);
-        const int64_t b1 = npass > 1 ? (int64_t)plan_batch(pl.batches, first + 1 / NPASS) : b0;
-        const int64_t e1 = npass > 1 ? elem(b1, 1 % NPASS) : e0;
-        gnext = __builtin_nontemporal_load(&pl.conn[e1 * NN + l]);
+        uint32_t gn[Q];
+#pragma unroll
+        for (int k = 0; k < Q; ++k) gn[k] = pl.conn[((int64_t)b * Q + k) * LANES + tc];
+        typename A::F fr[Q], fE[Q], fq[Q][3];
+        typename A::U fu[Q][3];
+        typename A::Pt fp[Q];
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            const int64_t g = gn[k];
+            fr[k] = a.rho[g];
+            fE[k] = a.E[g];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                fu[k][d] = a.u[g + d * np];
+                fq[k][d] = a.q[g + d * np];
+            }
+            if constexpr (!kRecover) fp[k] = a.pr[g];
+        }
+        geo = col_geo<P, true>(a.geo, b, 0, tc);
+        col_table<P>(a.tab.D, sD);
+        if constexpr (COLORED)
+            for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            r[k] = (T)fr[k];
+            const T E = (T)fE[k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                u[k][d] = (T)fu[k][d];
+                q[k][d] = (T)fq[k][d];
+            }
+            const T ke = u[k][0] * u[k][0] * (T)0.5 + u[k][1] * u[k][1] * (T)0.5 + u[k][2] * u[k][2] * (T)0.5;
+            if constexpr (kRecover)
+                p[k] = (T)(a.gamma_m1 * ((double)E - (double)r[k] * 0.5 *
+                                                         ((double)u[k][0] * u[k][0] + (double)u[k][1] * u[k][1] +
+                                                          (double)u[k][2] * u[k][2])));
+            else
+                p[k] = (T)fp[k];
+            H[k] = E + ke;
+        }
     }
-
-    for (int kb = 0; kb < nbat; ++kb) {
-        __syncthreads();  // sB, sD visible; the previous batch's write phase is done with sR
-        const int64_t b = sB[kb];
-        const uint32_t u0 = sU0[kb], U = sU1[kb] - u0;
-        uint32_t wn[UPT];  // this thread's entries of the batch's node list, for the write phase
+    // the next slice's place in the outputs: its node, or (coloured) its
+    // position in the batch's list
+    uint32_t at = COLORED ? pl.lidx[(int64_t)b * Q * LANES + tc] : pl.conn[(int64_t)b * Q * LANES + tc];
+    const int sI = tc - I, sJ = tc - J * EPB * Q;
+    col_slices<Q>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = kc();
+        const T ra = r[k], Ha = H[k];
+        if (k > 0) __syncthreads();  // the previous slice is read
+        sP[0][t] = V2{ra, p[k]};
+        sP[1][t] = V2{u[k][0], u[k][1]};
+        sP[2][t] = V2{u[k][2], q[k][0]};
+        sP[3][t] = V2{q[k][1], q[k][2]};
+        sH[t] = Ha;
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        ConvecSums<T> sum;
+        auto next_geo = [&](int c) {
+            if (k + 1 < Q) geo.v[c] = col_geo_pair<P, true>(a.geo, b, k + 1, tc, c);
+        };
+        // the sources along I, then J; each read one ahead of its use
+        struct Rec { V2 a, b, c, d; T H, D; };
+        auto read = [&](int m, const T *Dv) { return Rec{sP[0][m], sP[1][m], sP[2][m], sP[3][m], sH[m], *Dv}; };
+        Rec ra0 = read(sI, sD + I * Q), rb0;
+        ConvecDir<T> x = sum.direction(geo, 2, u[k], q[k]);
 #pragma unroll
-        for (int j = 0; j < UPT; ++j) {
-            const uint32_t i = t + j * NT;
-            wn[j] = pl.unode[u0 + (i < U ? i : U - 1)];
+        for (int n = 0; n < Q; ++n) {
+            sum.source(x, ra, (T)col_D<P>(D, k, n), r[n], p[n], H[n], u[n][0], u[n][1], u[n][2], q[n][0], q[n][1], q[n][2]);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        for (uint32_t i = t; i < U; i += blockDim.x)
+        sum.finish(x);
+        T gv = (T)geo.gvol();
+        asm volatile("" : "+v"(gv));
+        next_geo(3);
+        next_geo(4);
+        auto use = [&](const Rec &c) {
+            __builtin_amdgcn_sched_barrier(0);
+            sum.source(x, ra, c.D, c.a.x, c.a.y, c.H, c.b.x, c.b.y, c.c.x, c.c.y, c.d.x, c.d.y);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        // a line's q sources, the first of them in ra0; ends with the record at
+        // `then` in ra0
+        auto line = [&](int m, int step, const T *Dv, int then, const T *Dthen) {
+            if constexpr (Q % 2) {
 #pragma unroll
-            for (int c = 0; c < 5; ++c) sR[c][i] = 0.0;
-#pragma unroll
-        for (int p = 0; p < NPASS; ++p) {
-            ConvecNode<A> &cur = nd[p & 1];
-            ConvecNode<A> &nxt = nd[(p + 1) & 1];
-            const int g = kb * NPASS + p;
-            const int64_t e = b * S::BATCH + p * EPB + le;
-            const bool active = (le < EPB) && (e < a.nelem);
-            if (p > 0) __syncthreads();  // the previous pass is done with sF
-            if (active) {
-                const T r = cur.r, Ev = cur.E;
-                const T ux = cur.u[0], uy = cur.u[1], uz = cur.u[2];
-                const T k = ux * ux * (T)0.5 + uy * uy * (T)0.5 + uz * uz * (T)0.5;
-                // p = (gamma-1)(E - rho|u|^2/2) when no pressure array is given, in
-                // FP64 whatever T: the difference cancels
-                const double p64 = a.gamma_m1 * ((double)Ev - (double)r * 0.5 *
-                                                     ((double)ux * ux + (double)uy * uy + (double)uz * uz));
-                const T pv = a.pr ? (T)cur.p : (T)p64;
-                const T H = Ev + k;
-                const T rH = r * Ev + r * k;
-                sF[le][l][0] = r;
-                sF[le][l][1] = pv;
-                sF[le][l][2] = H;
-                if constexpr (kRH) sF[le][l][3] = rH;
-                sF[le][l][iU] = ux;
-                sF[le][l][iU + 1] = uy;
-                sF[le][l][iU + 2] = uz;
-                sF[le][l][iQ] = cur.q[0];
-                sF[le][l][iQ + 1] = cur.q[1];
-                sF[le][l][iQ + 2] = cur.q[2];
-            }
-            const uint32_t li = cur.li;
-            // issued now, used later: He and gpvol of this pass (after the
-            // barrier), the next pass's nodal values (next pass), the
-            // connectivity of the pass after it.  The element arrays are read
-            // once: non-temporal loads keep them from evicting the gathered
-            // nodal lines, which neighbouring elements read again, from L2.
-            const int64_t ec = elem(b, p);
-            // kept in the storage type until used: a conversion here would
-            // wait for the load before the barrier
-            const GeoNode<TG> gn = load_geo<NN, true>(a.geo, ec, l);  // He(i,d) = gn.he(i + 3d)
-            convec_fetch<NN>(a, elem_of(g + 1), l, gnext, nxt);
-            gnext = __builtin_nontemporal_load(&pl.conn[elem_of(g + 2) * NN + l]);
-            __syncthreads();
-            double v[5] = {0, 0, 0, 0, 0};
-            if (active) {
-                // Accumulators, each a sum over the three directions and the
-                // q sources of one line (r, H, rH, u, q: the node's own values):
-                //   aU = div u, aQ = div q                       (from the line derivatives)
-                //   aE = sum D[(U.)(rH + r H)],  aM_i = sum D[(U.)(q_i + r u_i)]
-                //   sRho = sum U_d D_d[r],  sE = sum Q_d D_d[H] + U_d D_d[rH]
-                //   mM_i = sum Q_d D_d[u_i] + U_d D_d[q_i] + 4 He(i,d) D_d[p]
-                const T r = (T)cur.r;
-                T aQ = 0, aU = 0, aE = 0, aM[3] = {0, 0, 0};
-                T sRho = 0, sE = 0, mM[3] = {0, 0, 0};
-#pragma unroll 1
-                for (int d = 0; d < 3; ++d) {
-                    // one copy of the sweep code for the three directions
-                    const T h0 = (T)(d == 0 ? gn.he(0) : (d == 1 ? gn.he(3) : gn.he(6)));
-                    const T h1 = (T)(d == 0 ? gn.he(1) : (d == 1 ? gn.he(4) : gn.he(7)));
-                    const T h2 = (T)(d == 0 ? gn.he(2) : (d == 1 ? gn.he(5) : gn.he(8)));
-                    const int Id = d == 0 ? I : (d == 1 ? J : K);
-                    const int stride = d == 0 ? 1 : (d == 1 ? Q : Q * Q);
-                    const int base = l - Id * stride;
-                    const T Ua = h0 * sF[le][l][iU] + h1 * sF[le][l][iU + 1] + h2 * sF[le][l][iU + 2];
-                    const T Qa = h0 * sF[le][l][iQ] + h1 * sF[le][l][iQ + 1] + h2 * sF[le][l][iQ + 2];
-                    // 1-D derivatives along this line of the stored values
-                    T dp = 0, du[3] = {0, 0, 0}, dq[3] = {0, 0, 0}, dr = 0, dH = 0, drH = 0;
-#pragma unroll 1
-                    for (int n = 0; n < Q; ++n) {
-                        const int s = base + n * stride;
-                        const T Dv = sD[Id * Q + n];
-                        const T rs = sF[le][s][0], ps = sF[le][s][1], Hs = sF[le][s][2];
-                        const T rHs = kRH ? sF[le][s][kRH ? 3 : 0] : rs * Hs;
-                        const T us0 = sF[le][s][iU], us1 = sF[le][s][iU + 1], us2 = sF[le][s][iU + 2];
-                        const T qs0 = sF[le][s][iQ], qs1 = sF[le][s][iQ + 1], qs2 = sF[le][s][iQ + 2];
-                        dr += Dv * rs;
-                        dH += Dv * Hs;
-                        drH += Dv * rHs;
-                        dp += Dv * ps;
-                        du[0] += Dv * us0; du[1] += Dv * us1; du[2] += Dv * us2;
-                        dq[0] += Dv * qs0; dq[1] += Dv * qs1; dq[2] += Dv * qs2;
-                        // products with the target's contravariant velocity
-                        const T DU = Dv * (h0 * us0 + h1 * us1 + h2 * us2);
-                        aE += DU * (rHs + r * Hs);
-                        aM[0] += DU * (qs0 + r * us0);
-                        aM[1] += DU * (qs1 + r * us1);
-                        aM[2] += DU * (qs2 + r * us2);
-                    }
-                    sRho += Ua * dr;
-                    sE += Qa * dH + Ua * drH;
-                    const T dp4 = (T)4 * dp;
-                    mM[0] += Qa * du[0] + Ua * dq[0] + h0 * dp4;
-                    mM[1] += Qa * du[1] + Ua * dq[1] + h1 * dp4;
-                    mM[2] += Qa * du[2] + Ua * dq[2] + h2 * dp4;
-                    aU += h0 * du[0] + h1 * du[1] + h2 * du[2];
-                    aQ += h0 * dq[0] + h1 * dq[1] + h2 * dq[2];
+                for (int n = 0; n < Q - 1; n += 2) {
+                    m += step;
+                    rb0 = read(m, ++Dv);
+                    use(ra0);
+                    m += step;
+                    ra0 = read(m, ++Dv);
+                    use(rb0);
                 }
-                const T H = sF[le][l][2], rH = kRH ? sF[le][l][kRH ? 3 : 0] : r * H;
-                const T uu[3] = {sF[le][l][iU], sF[le][l][iU + 1], sF[le][l][iU + 2]};
-                const T qq[3] = {sF[le][l][iQ], sF[le][l][iQ + 1], sF[le][l][iQ + 2]};
-                const T Rm = (T)0.5 * (aQ + r * aU) + (T)0.5 * sRho;
-                const T Re = (T)0.25 * (aE + H * aQ + rH * aU) + (T)0.25 * (sE + H * sRho);
-                T Rmo[3];
+                rb0 = read(then, Dthen);
+                use(ra0);
+                ra0 = rb0;
+            } else {
 #pragma unroll
-                for (int i = 0; i < 3; ++i)
-                    Rmo[i] = (T)0.25 * (aM[i] + uu[i] * aQ + qq[i] * aU + uu[i] * sRho + mM[i]);
-                const T gv = (T)gn.gvol();
-                v[0] = (double)(gv * Rm);
-                v[1] = (double)(gv * Rmo[0]);
-                v[2] = (double)(gv * Rmo[1]);
-                v[3] = (double)(gv * Rmo[2]);
-                v[4] = (double)(gv * Re);
+                for (int n = 0; n < Q - 2; n += 2) {
+                    m += step;
+                    rb0 = read(m, ++Dv);
+                    use(ra0);
+                    m += step;
+                    ra0 = read(m, ++Dv);
+                    use(rb0);
+                }
+                rb0 = read(m + step, Dv + 1);
+                use(ra0);
+                ra0 = read(then, Dthen);
+                use(rb0);
             }
-            add_pass<UMAX, EPB>(sR, pl.mode, le, active, li, v);
+        };
+        x = sum.direction(geo, 0, u[k], q[k]);
+        line(sI, 1, sD + I * Q, sJ, sD + J * Q);
+        sum.finish(x);
+        next_geo(0);
+        x = sum.direction(geo, 1, u[k], q[k]);
+        line(sJ, EPB * Q, sD + J * Q, sJ, sD + J * Q);
+        sum.finish(x);
+        next_geo(1);
+        next_geo(2);
+        double v[5];
+        sum.values(gv, ra, Ha, u[k], q[k], v);
+        const uint32_t here = at;
+        if (k + 1 < Q) {
+            const int64_t i = ((int64_t)b * Q + k + 1) * LANES + tc;
+            at = COLORED ? pl.lidx[i] : pl.conn[i];
         }
-        if (pl.mode == kAtomic) __syncthreads();  // every LDS atomic of the batch done
-        write_batch_nodes<UMAX, NT>(pl.mode, wn, U, sR, a.Rmass, a.Rmom, a.Rener, a.npoin);
-        if (NPASS & 1) nd[0] = nd[1];  // odd pass count: the next batch starts from slot 0
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (COLORED)
+            col_add<P, true>(sR, US, active, le, here, v);
+        else if (col_merge<P>(here, I, le, active && (int64_t)b * EPB + le + 1 < a.nelem, v) && active)
+            col_scatter(here, v, a.Rmass, a.Rmom, a.Rener, np);
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (COLORED) {
+        const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+        uint32_t wn[S::UPT];
+        col_list<P>(pl.unode + u0, U, wn);
+        __syncthreads();
+        col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
     }
 }
 
-template <int P, class A, typename TA = double>
+template <int P, class A, typename TA>
 static hipError_t launch_p(const A &a, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_convec<P, A, TA>), dim3(plan_blocks(a.plan)), dim3(CShape<P>::NT), 0, s, a);
+    const bool atomic = a.plan.mode == kAtomic;
+    const size_t sums = P > kNarrowP && atomic ? 0 : sizeof(double) * 5 * a.plan.ustride;
+    if constexpr (P > kNarrowP)
+        hipLaunchKernelGGL((atomic ? k_convec_wide<P, false, A, TA> : k_convec_wide<P, true, A, TA>),
+                           dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
+    else
+        hipLaunchKernelGGL((atomic ? k_convec_col<P, false, A, TA> : k_convec_col<P, true, A, TA>),
+                           dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
     return hipGetLastError();
+}
+
+template <class A, typename TA>
+static hipError_t launch_order(int porder, const A &a, hipStream_t s)
+{
+    switch (porder) {
+    case 1: return launch_p<1, A, TA>(a, s);
+    case 2: return launch_p<2, A, TA>(a, s);
+    case 3: return launch_p<3, A, TA>(a, s);
+    case 4: return launch_p<4, A, TA>(a, s);
+    case 5: return launch_p<5, A, TA>(a, s);
+    case 6: return launch_p<6, A, TA>(a, s);
+    case 7: return launch_p<7, A, TA>(a, s);
+    case 8: return launch_p<8, A, TA>(a, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 template <class A>
 hipError_t launch_convec(int porder, const A &a, hipStream_t s)
 {
-    if (porder <= kColMaxP) return launch_convec_col<A, double>(porder, a, s);
-    switch (porder) {
-    case 6: return launch_p<6, A>(a, s);
-    case 7: return launch_p<7, A>(a, s);
-    case 8: return launch_p<8, A>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    return launch_order<A, double>(porder, a, s);
 }
 
 hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s)
 {
-    if (porder <= kColMaxP) return launch_convec_col<ConvecArgs<float, float>, float>(porder, a, s);
-    switch (porder) {
-    case 6: return launch_p<6, ConvecArgs<float, float>, float>(a, s);
-    case 7: return launch_p<7, ConvecArgs<float, float>, float>(a, s);
-    case 8: return launch_p<8, ConvecArgs<float, float>, float>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    return launch_order<ConvecArgs<float, float>, float>(porder, a, s);
 }
 
 template hipError_t launch_convec(int, const ConvecArgs<double, double> &, hipStream_t);

@@ -1,405 +1,914 @@
-// Diffusive residual kernel (counterpart of full_diffusion_ijk,
-// src/kernels/sources/elem_diffu.f90:10-197).
+// Diffusive residual (counterpart of full_diffusion_ijk,
+// src/kernels/sources/elem_diffu.f90:10-197); see msod_columns.h for the thread
+// layout.
 //
-// One workgroup per batch of Shape<P>::BATCH elements, passes of
-// Shape<P>::EPB elements with one thread per element node.  Per pass:
-//  pass 1 (elem_diffu.f90:67-139): sweeps of rho, T, u along the node's three
-//    grid lines; He of the node gives grad rho, grad T and G = grad u; then
-//    the viscous stress tau and tau.u, kept in registers.
-//  pass 2 (elem_diffu.f90:141-193): the reference re-reads He, gpvol and the
-//    six flux vectors Phi (grad rho, tau.u, grad T, tau rows) at every source
-//    node of the target's three lines.  Here each thread publishes, one
-//    reference direction d at a time, the contravariant components
-//        F_d = gpvol * sum_i He(i,d) Phi_i        (6 values per node)
-//    and the target accumulates the transposed sweep
-//        W[Phi](a) += sum_n D[n][I_d(a)] F_d(s_d(n))
-//    (LDS holds 6 values per node instead of 18, node-major, in the buffer
-//    pass 1 used for rho, T, u).  Then
-//    Rmass += nu_e W[grad rho], Rener += W[tau.u] + kappa_e W[grad T],
-//    Rmom_r += W[tau_r], with nu_e and kappa_e of the target node (the
-//    reference multiplies kappa_e inside the sum; same value, other rounding).
-// Each element node's five values are added into the batch's per-node sums
-// in LDS in a fixed order (add_pass); the batch's distinct nodes are then
-// written once (write_batch_nodes).
+// Per slice K of the element's nodes:
+//  1. rho, T, u of the slice in LDS; gradients along I and J from there, along
+//     K from the thread's column; He gives grad rho, grad T, G = grad u, then
+//     the stress tau and tau.u.
+//  2. the contravariant fluxes F_d = gpvol sum_i He(i,d) Phi_i of the six flux
+//     vectors Phi (grad rho, tau.u, grad T, the rows of tau): those of d = I, J
+//     go to LDS, those of d = K are added at once into the column's six sums
+//     W[K'] with D[K][K'].
+//  3. the transposed sweeps along I and J from LDS into W[K].
+// After the last slice Rmass = nu_e W0, Rmom = W3..W5, Rener = W1 + kappa_e W2,
+// with nu_e and kappa_e of the target node (the reference multiplies kappa_e
+// inside the sum; same value, other rounding).  It also re-reads He, gpvol and
+// the six flux vectors at every source of the target's lines (:141-193), where
+// step 2 publishes one component per direction.
 //
 // Storage types TG (geometry, mu_e, mu_sgs) and TF (nodal fields), FP64
-// arithmetic throughout (msod_kernels.h).  CLOSURE (FP64 storage only):
-// mu_sgs is not read but predicted per
-// element node by the learned closure (msod_mlp.h) from the pass-1 velocity
-// gradient, evaluated with bf16 MFMA inside the kernel before the stress is
-// formed; its LDS scratch overlays the field buffers between the passes.
+// arithmetic (msod_kernels.h) or TA = float.  CLOSURE (FP64 storage): mu_sgs is not read but predicted by the learned
+// closure (msod_mlp.h) from the velocity gradient before the stress is
+// formed; its per-wave LDS scratch is the wave's own part of the flux buffer,
+// free between the slice's first barrier and the fluxes.
+#include <algorithm>
 #include <type_traits>
 
-#include "msod_kernels.h"
+#include "msod_columns.h"
 #include "msod_mlp.h"
 #include "msod_closure.h"
 
 namespace msod {
 
-// Inputs of one element node, loaded one pass ahead of their use so that
-// the gathers of the next pass are in flight while this pass computes.
-template <class A>
-struct DiffuNode {
-    typename A::F r, T_, muf;
-    typename A::U u[3];
-};
-
-template <class A>
-__device__ __forceinline__ void diffu_fetch(const A &a, uint32_t gnode, DiffuNode<A> &x)
+template <int P, bool COLORED, class A, bool CLOSURE, typename TA>
+__global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const float *mlp)
 {
-    const int64_t g = gnode;
-    const int64_t np = a.npoin;
-    x.r = a.rho[g];
-    x.T_ = a.Tem[g];
-    x.muf = a.mu_fluid[g];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) x.u[d] = a.u[g + d * np];
-}
-
-// mu_e and mu_sgs of ME consecutive elements from e0 on into LDS.  Their
-// reference layout (nelem,ngaus) puts the values of one element node
-// 8*nelem bytes apart, so a wave reading one element's nodes would touch 64
-// lines (and pages) per load; here ME neighbouring lanes read ME
-// consecutive elements of one node, and the batches that follow in mesh
-// order reuse the lines.
-template <int NN, int ME, int NT, bool CLOSURE, class A, typename TG = typename A::G>
-__device__ __forceinline__ void diffu_stage_mu(const A &a, int64_t e0, TG (*sMu)[ME][NN])
-{
-    // every load unconditional and issued before any LDS write (entries past
-    // the table or the mesh re-read a valid entry and are not written or not
-    // used), so that the loads of one thread are in flight together
-    constexpr int IT = (ME * NN + NT - 1) / NT;
-    int32_t gl[IT];
-    TG v0[IT], v1[IT];
-#pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = (int)threadIdx.x + k * NT < ME * NN ? (int)threadIdx.x + k * NT : ME * NN - 1;
-        gl[k] = a.tab.l2g[i / ME];
-    }
-#pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = (int)threadIdx.x + k * NT < ME * NN ? (int)threadIdx.x + k * NT : ME * NN - 1;
-        const int64_t e = e0 + i % ME < a.nelem ? e0 + i % ME : a.nelem - 1;
-        const int64_t ge = e + a.nelem * (int64_t)gl[k];  // reference layout (nelem,ngaus)
-        v0[k] = a.mu_e[ge];
-        v1[k] = (!CLOSURE && a.mu_sgs) ? a.mu_sgs[ge] : (TG)0;  // NULL: closure fallback
-    }
-#pragma unroll
-    for (int k = 0; k < IT; ++k) {
-        const int i = (int)threadIdx.x + k * NT;
-        if (i < ME * NN) {
-            sMu[0][i % ME][i / ME] = v0[k];
-            sMu[1][i % ME][i / ME] = v1[k];
-        }
-    }
-}
-
-// Launch bound in waves per SIMD.  The closure form is bounded to 3
-// workgroups per CU: the compiler then keeps the MFMA accumulators in VGPRs
-// (about 148 in all) instead of 188 VGPRs and 32 AGPRs, 3 waves per SIMD
-// instead of 2 (4.7 against 6.2 ms at 96^3 p=3).  512-thread workgroups with
-// FP32 element arrays and FP64 arithmetic: 6, three workgroups per CU (their
-// LDS fits three), at 80 VGPRs with 20 B of spills per lane (48^3 p=7: FP32
-// split 3.96 -> 3.45 ms, every input in FP32 4.21 -> 3.41 ms); the FP64 form
-// spilled 28 B there and ran slower (3.61 -> 3.90 ms), so it keeps two.
-template <int P, typename TG, typename TA, bool CLOSURE>
-constexpr int diffu_waves()
-{
-    return CLOSURE ? (Shape<P>::NT == 256 ? 3 : 1)
-                   : (Shape<P>::NT == 512 && sizeof(TG) < sizeof(TA) ? 6 : 1);
-}
-
-template <int P, class A, bool CLOSURE, typename TA = double>
-__global__ void __launch_bounds__(Shape<P>::NT, (diffu_waves<P, typename A::G, TA, CLOSURE>())) k_diffu(A a, const float *mlp)
-{
+    using S = ColShape<P>;
+    using T = TA;
     using TG = typename A::G;
-    using S = Shape<P>;
-    using T = TA;  // arithmetic: FP64, or FP32 for the FP32-arithmetic form (node sums stay FP64)
-    constexpr int Q = S::Q, NN = S::NN, EPB = S::EPB, UMAX = S::UMAX;
-    // one buffer of node records (sN) serves pass 1 (rho, T, u) and pass 2
-    // (fluxes of one direction); the MLP scratch of the closure overlays it
-    // between the two
-    constexpr size_t kRec = sizeof(T) * EPB * 6 * NN;
-    constexpr size_t kScr = CLOSURE ? (size_t)(S::NT / 64) * 64 * 16 * sizeof(short) : 0;
-    constexpr size_t kBuf = kRec > kScr ? kRec : kScr;
-    __shared__ T sD[Q * Q];
-    __shared__ __attribute__((aligned(16))) unsigned char sbuf[kBuf];
-    __shared__ double sR[5][UMAX];
-    // mu_e, mu_sgs of the batch, staged once; of the pass, staged per pass,
-    // where the batch's would cost a workgroup per CU (four fit 160 KB of LDS)
-    constexpr size_t kLdsRest = sizeof(T) * Q * Q + kBuf + sizeof(double) * 5 * UMAX +
-                                (CLOSURE ? sizeof(MlpShared) : 0);
-    constexpr size_t kLdsCu = 160 * 1024 / 4;
-    constexpr bool kMuPerPass = kLdsRest + 2 * sizeof(TG) * S::BATCH * NN > kLdsCu &&
-                                kLdsRest + 2 * sizeof(TG) * EPB * NN <= kLdsCu;
-    constexpr int ME = kMuPerPass ? EPB : S::BATCH;
-    __shared__ TG sMu[2][ME][NN];
-    __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
-    // node-major records of 6 values (pass 1: rho, T, u0, u1, u2, unused;
-    // pass 2: the contravariant fluxes of one direction), read in pairs: in
-    // FP64 three ds_read_b128 per source instead of ds_read2_b64 pairs
-    // (diffusion 13.71 -> 13.51 ms at 128^3 p=4, 3.81 -> 3.67 ms at 48^3 p=7)
+    constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
+    constexpr int LA = 2;  // line sources read ahead of their use (3 and 4: no faster; order 5 spills)
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
-    auto sN = reinterpret_cast<V2 (*)[NN][3]>(sbuf);
+    __shared__ T sD[Q * Q];
+    __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
+    __shared__ T sU2[NT];     // and u2
+    __shared__ __attribute__((aligned(16))) V2 sF[6][NT];  // its fluxes along I (0..2) and J (3..5)
+    __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
+    __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
+    extern __shared__ __attribute__((aligned(16))) double sR[];  // node sums [5][US]
 
     const Plan &pl = a.plan;
-    constexpr int NT = S::NT, UPT = (UMAX + NT - 1) / NT;
-    const int64_t b = plan_batch(pl.batches, xcd_slot(blockIdx.x, gridDim.x));
-    const uint32_t u0 = pl.uoff[b], U = pl.uoff[b + 1] - u0;
-    const int t = threadIdx.x;
-    uint32_t wn[UPT];  // this thread's entries of the batch's node list, for the write phase
+    const int US = pl.ustride, t = threadIdx.x;
+    const ColThread<P> th(t);
+    const int tc = th.tc, le = th.le, I = th.I, J = th.J;
+    const int64_t np = a.npoin;
+    const auto D = uniform(a.tab.D);
+    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
+    const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+    const int64_t e0 = (int64_t)b * EPB;
+    const bool active = t < LANES && e0 + le < a.nelem;
+
+    uint32_t gn[Q];
 #pragma unroll
-    for (int j = 0; j < UPT; ++j) {
-        const uint32_t i = t + j * NT;
-        wn[j] = pl.unode[u0 + (i < U ? i : U - 1)];
+    for (int k = 0; k < Q; ++k) gn[k] = __builtin_nontemporal_load(&pl.conn[((int64_t)b * Q + k) * LANES + tc]);
+    // mu_e and mu_sgs in the reference layout (nelem,ngaus) put one element's
+    // values 8*nelem bytes apart and neighbouring elements side by side: they are
+    // loaded with the element as the fastest lane index and change lanes in LDS
+    const int lem = tc % EPB, Im = tc / EPB % Q, Jm = tc / (EPB * Q);
+    const int lm = line_ref<P>(Im) + Q * line_ref<P>(Jm), tm = t < LANES ? Im + Q * (lem + EPB * Jm) : t;
+    const int64_t em = e0 + lem < a.nelem ? e0 + lem : a.nelem - 1;
+    int32_t gl[Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) gl[k] = a.tab.l2g[lm + QQ * line_ref<P>(k)];
+    const bool has_sgs = !CLOSURE && a.mu_sgs;  // NULL: closure fallback
+    const TG *mu_sgs = has_sgs ? a.mu_sgs : a.mu_e;
+    TG mue, mus = (TG)0;
+    auto load_mu = [&](int k) {
+        const int64_t ge = em + a.nelem * (int64_t)gl[k];
+        mue = a.mu_e[ge];
+        if constexpr (!CLOSURE) mus = mu_sgs[ge];
+    };
+    typename A::F fr[Q], fT[Q], fmu[Q];
+    typename A::U fu[Q][3];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        const int64_t g = gn[k];
+        fr[k] = a.rho[g];
+        fT[k] = a.Tem[g];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) fu[k][d] = a.u[g + d * np];
+        fmu[k] = a.mu_fluid[g];
     }
-    const int le = t / NN;
-    const int l = t - le * NN;
-    const int I = l % Q, J = (l / Q) % Q, K = l / (Q * Q);
+    load_mu(0);
+    GeoNode<TG> gk = col_geo<P, false>(a.geo, b, 0, tc);
+    col_table<P>(a.tab.D, sD);
+    if constexpr (CLOSURE) mlp_stage(smlp, mlp);
+    for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
     const T Cp = (T)a.Cp, Pr = (T)a.Pr;
 
-    DiffuNode<A> cur, nxt;
-    // the connectivity is read a pass ahead of the gathers that use it, so
-    // that the next pass's gathers issue without a trip to memory (idle
-    // threads and elements past the mesh read a real entry)
-    uint32_t gnext = 0;
-    auto conn_of = [&](int p) -> uint32_t {
-        const int64_t ep = b * S::BATCH + p * EPB + (le < EPB ? le : 0);
-        return __builtin_nontemporal_load(&pl.conn[(ep < a.nelem ? ep : a.nelem - 1) * NN + l]);
-    };
-    static_assert(Q * Q <= S::NT, "one derivative-table entry per thread");
-    {
-        // prologue: the tables and the connectivity first, then the values
-        // that depend on them, then the LDS writes; every load unconditional
-        // (idle threads read a real entry), so that each group is in flight
-        // together
-        const T dv = (T)a.tab.D[t < Q * Q ? t : Q * Q - 1];
-        constexpr int IT = (ME * NN + NT - 1) / NT;
-        int32_t gl[IT];
-        TG v0[IT], v1[IT];
-        auto mu_i = [&](int k) {
-            return (int)t + k * NT < ME * NN ? (int)t + k * NT : ME * NN - 1;
-        };
-        if (!kMuPerPass) {
+    T r[Q], Te[Q], muf[Q], u[Q][3], W[Q][6], nu[Q], kappa[Q];
+    uint32_t li[Q], wn[S::UPT];
 #pragma unroll
-            for (int k = 0; k < IT; ++k) gl[k] = a.tab.l2g[mu_i(k) / ME];
-        }
-        const int64_t e = b * S::BATCH + le;
-        const int64_t ec = e < a.nelem ? e : a.nelem - 1;
-        const uint32_t gcur = __builtin_nontemporal_load(&pl.conn[ec * NN + l]);
-        if (S::NPASS > 1) gnext = conn_of(1);
-        diffu_fetch(a, gcur, cur);
-        if (!kMuPerPass) {
+    for (int k = 0; k < Q; ++k) {
+        r[k] = (T)fr[k];
+        Te[k] = (T)fT[k];
+        muf[k] = (T)fmu[k];
 #pragma unroll
-            for (int k = 0; k < IT; ++k) {
-                const int i = mu_i(k);
-                const int64_t em = b * S::BATCH + i % ME < a.nelem ? b * S::BATCH + i % ME : a.nelem - 1;
-                const int64_t ge = em + a.nelem * (int64_t)gl[k];
-                v0[k] = a.mu_e[ge];
-                v1[k] = (!CLOSURE && a.mu_sgs) ? a.mu_sgs[ge] : (TG)0;
-            }
-        }
-        for (uint32_t i = t; i < U; i += blockDim.x)
+        for (int d = 0; d < 3; ++d) u[k][d] = (T)fu[k][d];
 #pragma unroll
-            for (int c = 0; c < 5; ++c) sR[c][i] = 0.0;
-        if (t < Q * Q) sD[t] = dv;
-        if (!kMuPerPass) {
-#pragma unroll
-            for (int k = 0; k < IT; ++k) {
-                const int i = (int)t + k * NT;
-                if (i < ME * NN) {
-                    sMu[0][i % ME][i / ME] = v0[k];
-                    sMu[1][i % ME][i / ME] = v1[k];
-                }
-            }
-        }
+        for (int f = 0; f < 6; ++f) W[k][f] = 0;
     }
-    if constexpr (CLOSURE) mlp_stage(smlp, mlp);
+    const int sI = tc - I, sJ = tc - J * EPB * Q;  // a line's source n: sI + n, sJ + n*EPB*Q
 
 #pragma unroll
-    for (int pass = 0; pass < S::NPASS; ++pass) {
-        const int64_t e = b * S::BATCH + pass * EPB + le;
-        const bool active = (le < EPB) && (e < a.nelem);
-        T r = 0, muf = 0, mue = 0, mus = 0, uu[3] = {0, 0, 0};
-        // the previous pass read its sMu entries before its pass-2 barriers
-        if (kMuPerPass) diffu_stage_mu<NN, ME, NT, CLOSURE>(a, b * S::BATCH + pass * EPB, sMu);
-        __syncthreads();  // previous pass done with sN (and sR zeroed, sMu staged)
-        if (active) {
-            r = cur.r;
-            muf = cur.muf;
-            mue = (T)sMu[0][kMuPerPass ? le : pass * EPB + le][l];
-            mus = (T)sMu[1][kMuPerPass ? le : pass * EPB + le][l];
-            for (int d = 0; d < 3; ++d) uu[d] = cur.u[d];
-            sN[le][l][0] = V2{r, (T)cur.T_};
-            sN[le][l][1] = V2{uu[0], uu[1]};
-            sN[le][l][2] = V2{uu[2], (T)0};
-        }
-        if (pass + 1 < S::NPASS) {  // next pass's inputs: in flight during this pass
-            const int64_t en = e + EPB;
-            if (le < EPB && en < a.nelem) diffu_fetch(a, gnext, nxt);
-            if (pass + 2 < S::NPASS) gnext = conn_of(pass + 2);
-        }
-        // this pass's element arrays, issued before the barrier;
-        // unconditional, idle threads read a real element; kept in the
-        // storage type until used.  Plain loads: with the non-temporal hint
-        // the 128^3 p=4 diffusion ran 4% slower in FP64 and 5-7% with FP32
-        // element arrays (the hint still pays in the convection)
-        GeoNode<TG> gn;  // He(i,d) = gn.he(i + 3d), gpvol = gn.gvol()
-        uint32_t li;
-        {
-            const int64_t ec = e < a.nelem ? (le < EPB ? e : b * S::BATCH + pass * EPB) : a.nelem - 1;
-            gn = load_geo<NN, false>(a.geo, ec, l);
-            li = pl.lidx[ec * NN + l];
-        }
+    for (int k = 0; k < Q; ++k) {
+        // the previous slice's values were read before its second barrier
+        sP[0][t] = V2{r[k], Te[k]};
+        sP[1][t] = V2{u[k][0], u[k][1]};
+        sU2[t] = u[k][2];
+        sMu[0][tm] = mue;
+        sMu[1][tm] = mus;
+        if (k + 1 < Q) load_mu(k + 1);
         __syncthreads();
-
-        // ---- pass 1: gradients, stress ------------------------------------
-        // He(i,d) = gn.he(i + 3d), converted where used: a conversion placed
-        // ahead of the sweeps would wait for every load there
-        T gR[3] = {0, 0, 0}, gT[3] = {0, 0, 0}, tau[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-        T tauU[3] = {0, 0, 0}, gv = 0, G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-        if (active) {
+        __builtin_amdgcn_sched_barrier(0);
+        // line derivatives x[d] of rho, T, u; the slice's geometry is still in
+        // flight.  The line sources, first along I, then J, are read LA ahead of
+        // their use.
+        T x[3][5];
 #pragma unroll
-            for (int d = 0; d < 3; ++d) {
-                const int Id = d == 0 ? I : (d == 1 ? J : K);
-                const int stride = d == 0 ? 1 : (d == 1 ? Q : Q * Q);
-                const int base = l - Id * stride;
-                T aR = 0, aT = 0, aU0 = 0, aU1 = 0, aU2 = 0;
-#pragma unroll 1
-                for (int n = 0; n < Q; ++n) {
-                    const int s = base + n * stride;
-                    const T Dv = sD[Id * Q + n];
-                    const V2 p0 = sN[le][s][0], p1 = sN[le][s][1], p2 = sN[le][s][2];
-                    aR += Dv * p0.x;
-                    aT += Dv * p0.y;
-                    aU0 += Dv * p1.x;
-                    aU1 += Dv * p1.y;
-                    aU2 += Dv * p2.x;
-                }
+        for (int d = 0; d < 3; ++d)
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const T hid = (T)gn.he(i + 3 * d);
-                    gR[i] += hid * aR;
-                    gT[i] += hid * aT;
-                    // G[i][j] = d u_i / d x_j = sum_d He(j,d) D_d[u_i]
-                    G[0][i] += hid * aU0;
-                    G[1][i] += hid * aU1;
-                    G[2][i] += hid * aU2;
-                }
-            }
+            for (int f = 0; f < 5; ++f) x[d][f] = 0;
+        V2 s0[LA], s1[LA];
+        T s2[LA], Dv[LA];
+        auto read_source = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * EPB * Q;
+            s0[s % LA] = sP[0][m];
+            s1[s % LA] = sP[1][m];
+            s2[s % LA] = sU2[m];
+            Dv[s % LA] = s < Q ? sD[I * Q + s] : sD[J * Q + s - Q];
+        };
+#pragma unroll
+        for (int s = 0; s < LA; ++s) read_source(s);
+#pragma unroll
+        for (int n = 0; n < Q; ++n) {
+            const T Dk = (T)col_D<P>(D, k, n);
+            x[2][0] += Dk * r[n];
+            x[2][1] += Dk * Te[n];
+            x[2][2] += Dk * u[n][0];
+            x[2][3] += Dk * u[n][1];
+            x[2][4] += Dk * u[n][2];
         }
+#pragma unroll
+        for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(x[2][f]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            const int d = s < Q ? 0 : 1, n = s % LA;
+            x[d][0] += Dv[n] * s0[n].x;
+            x[d][1] += Dv[n] * s0[n].y;
+            x[d][2] += Dv[n] * s1[n].x;
+            x[d][3] += Dv[n] * s1[n].y;
+            x[d][4] += Dv[n] * s2[n];
+            asm volatile("" : "+v"(x[d][0]), "+v"(x[d][1]), "+v"(x[d][2]), "+v"(x[d][3]), "+v"(x[d][4]));
+            if (s + LA < 2 * Q) read_source(s + LA);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        // grad rho, grad T, G[i][j] = d u_i / d x_j = sum_d He(j,d) D_d[u_i]
+        T gR[3], gT[3], G[3][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const T h0 = (T)gk.he(i), h1 = (T)gk.he(3 + i), h2 = (T)gk.he(6 + i);
+            gR[i] = h0 * x[0][0] + h1 * x[1][0] + h2 * x[2][0];
+            gT[i] = h0 * x[0][1] + h1 * x[1][1] + h2 * x[2][1];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) G[c][i] = h0 * x[0][2 + c] + h1 * x[1][2 + c] + h2 * x[2][2 + c];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            asm volatile("" : "+v"(gR[i]), "+v"(gT[i]), "+v"(G[0][i]), "+v"(G[1][i]), "+v"(G[2][i]));
+        __builtin_amdgcn_sched_barrier(0);
+        const T me = (T)sMu[0][tc], gv = (T)gk.gvol();
+        T ms = has_sgs ? (T)sMu[1][tc] : (T)0;
         if constexpr (CLOSURE) {
-            __syncthreads();  // every pass-1 sweep over sN done: the MLP scratch overlays it
             float f[kMlpIn];
-            if (active) {
-                T hinv[3][3];
+            T hinv[3][3];
 #pragma unroll
-                for (int i = 0; i < 3; ++i)
+            for (int i = 0; i < 3; ++i)
 #pragma unroll
-                    for (int d = 0; d < 3; ++d) hinv[i][d] = (T)gn.he(i + 3 * d);
-                mlp_features<T>(G, r, uu, hinv, f);
-            } else
-#pragma unroll
-                for (int k = 0; k < kMlpIn; ++k) f[k] = smlp.mean[k];
-            const float z3 = mlp_forward_z3(smlp, f, reinterpret_cast<short *>(sbuf) + (t >> 6) * 64 * 16);
-            mus = active ? (T)(smlp.scale * softplusf_(z3)) : (T)0;
+                for (int d = 0; d < 3; ++d) hinv[i][d] = (T)gk.he(i + 3 * d);
+            mlp_features<T>(G, r[k], u[k], hinv, f);
+            // idle lanes hold a real element node (finite features)
+            const float z3 =
+                mlp_forward_z3<NT * (int)sizeof(V2) / 2>(smlp, f, reinterpret_cast<short *>(&sF[0][t & ~63]));
+            ms = (T)(smlp.scale * softplusf_(z3));
         }
-        if (active) {
-            const T divU = G[0][0] + G[1][1] + G[2][2];
-            const T mu_f = muf + r * mus;
-            const T mu_t = mu_f + mue;
-            const T lam = mu_f * (T)(2.0 / 3.0) * divU;
+        nu[k] = (T)a.c_rho * me / r[k];
+        kappa[k] = muf[k] * Cp / Pr + (T)a.c_ener * me * Cp / Pr + Cp * r[k] * ms / (T)0.9;
+        asm volatile("" : "+v"(nu[k]), "+v"(kappa[k]));
+        __builtin_amdgcn_sched_barrier(0);
+        const T mu_f = muf[k] + r[k] * ms, mu_t = mu_f + me;
+        const T lam = mu_f * (T)(2.0 / 3.0) * (G[0][0] + G[1][1] + G[2][2]);
+        T tau[3][3], tauU[3];
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                T acc = 0;
+        for (int i = 0; i < 3; ++i) {
+            T acc = 0;
 #pragma unroll
-                for (int j = 0; j < 3; ++j) {
-                    tau[i][j] = mu_t * (G[i][j] + G[j][i]);
-                    acc += tau[i][j] * uu[j];
-                }
-                tauU[i] = acc - lam * uu[i];
-                tau[i][i] -= lam;
+            for (int j = 0; j < 3; ++j) {
+                tau[i][j] = mu_t * (G[i][j] + G[j][i]);
+                acc += tau[i][j] * u[k][j];
             }
-            gv = (T)gn.gvol();
+            tauU[i] = acc - lam * u[k][i];
         }
-
-        // ---- pass 2: transposed sweeps, one reference direction at a time -
-        __syncthreads();  // every pass-1 sweep over sN done: the fluxes overwrite it
-        T W[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int i = 0; i < 3; ++i) tau[i][i] -= lam;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            if (active) {
-                const T c0 = gv * (T)gn.he(3 * d), c1 = gv * (T)gn.he(1 + 3 * d), c2 = gv * (T)gn.he(2 + 3 * d);
-                sN[le][l][0] = V2{c0 * gR[0] + c1 * gR[1] + c2 * gR[2], c0 * tauU[0] + c1 * tauU[1] + c2 * tauU[2]};
-                sN[le][l][1] = V2{c0 * gT[0] + c1 * gT[1] + c2 * gT[2], c0 * tau[0][0] + c1 * tau[0][1] + c2 * tau[0][2]};
-                sN[le][l][2] = V2{c0 * tau[1][0] + c1 * tau[1][1] + c2 * tau[1][2], c0 * tau[2][0] + c1 * tau[2][1] + c2 * tau[2][2]};
-            }
-            __syncthreads();
-            if (active) {
-                const int Id = d == 0 ? I : (d == 1 ? J : K);
-                const int stride = d == 0 ? 1 : (d == 1 ? Q : Q * Q);
-                const int base = l - Id * stride;
-#pragma unroll 1
-                for (int n = 0; n < Q; ++n) {
-                    const int s = base + n * stride;
-                    const T Dv = sD[n * Q + Id];  // transposed: l_{I_d(a)}'(xi_n)
+            const T c0 = gv * (T)gk.he(3 * d), c1 = gv * (T)gk.he(3 * d + 1), c2 = gv * (T)gk.he(3 * d + 2);
+            T F[6];
+            F[0] = c0 * gR[0] + c1 * gR[1] + c2 * gR[2];
+            F[1] = c0 * tauU[0] + c1 * tauU[1] + c2 * tauU[2];
+            F[2] = c0 * gT[0] + c1 * gT[1] + c2 * gT[2];
 #pragma unroll
-                    for (int f = 0; f < 3; ++f) {
-                        const V2 pf = sN[le][s][f];
-                        W[2 * f] += Dv * pf.x;
-                        W[2 * f + 1] += Dv * pf.y;
+            for (int i = 0; i < 3; ++i) F[3 + i] = c0 * tau[i][0] + c1 * tau[i][1] + c2 * tau[i][2];
+            if (d < 2) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) sF[3 * (d < 2 ? d : 0) + c][t] = V2{F[2 * c], F[2 * c + 1]};
+            } else {
+#pragma unroll
+                for (int n = 0; n < Q; ++n) {
+                    const T Dk = (T)col_D<P>(D, k, n);  // transposed: l_n'(xi_k)
+#pragma unroll
+                    for (int f = 0; f < 6; ++f) {
+                        W[n][f] += Dk * F[f];
+                        // added now: sunk to its use, every F would stay live
+                        asm volatile("" : "+v"(W[n][f]));
                     }
                 }
             }
-            __syncthreads();  // sweep done before sN is overwritten
+            __builtin_amdgcn_sched_barrier(0);
         }
-        double v[5] = {0, 0, 0, 0, 0};
-        if (active) {
-            const T nu_e = (T)a.c_rho * mue / r;
-            const T kappa = muf * Cp / Pr + (T)a.c_ener * mue * Cp / Pr + Cp * r * mus / (T)0.9;
-            v[0] = (double)(nu_e * W[0]);
-            v[1] = (double)W[3];
-            v[2] = (double)W[4];
-            v[3] = (double)W[5];
-            v[4] = (double)(W[1] + kappa * W[2]);
+        if (k + 1 < Q) {
+            gk = col_geo<P, false>(a.geo, b, k + 1, tc);
+        } else {
+            col_list<P>(pl.unode + u0, U, wn);
+#pragma unroll
+            for (int n = 0; n < Q; ++n) li[n] = pl.lidx[((int64_t)b * Q + n) * LANES + tc];
         }
-        add_pass<UMAX, EPB>(sR, pl.mode, le, active, li, v);
-        if (pass + 1 < S::NPASS) cur = nxt;
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        V2 f0[LA], f1[LA], f2[LA];
+        auto read_flux = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * EPB * Q, c = s < Q ? 0 : 3;
+            f0[s % LA] = sF[c][m];
+            f1[s % LA] = sF[c + 1][m];
+            f2[s % LA] = sF[c + 2][m];
+            Dv[s % LA] = s < Q ? sD[s * Q + I] : sD[(s - Q) * Q + J];  // transposed: l_I'(xi_n)
+        };
+#pragma unroll
+        for (int s = 0; s < LA; ++s) read_flux(s);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            const int n = s % LA;
+            W[k][0] += Dv[n] * f0[n].x;
+            W[k][1] += Dv[n] * f0[n].y;
+            W[k][2] += Dv[n] * f1[n].x;
+            W[k][3] += Dv[n] * f1[n].y;
+            W[k][4] += Dv[n] * f2[n].x;
+            W[k][5] += Dv[n] * f2[n].y;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) asm volatile("" : "+v"(W[k][f]));
+            if (s + LA < 2 * Q) read_flux(s + LA);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        const double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
+                             (double)(W[k][1] + kappa[k] * W[k][2])};
+        col_add<P, COLORED>(sR, US, active, le, li[k], v);
     }
     __syncthreads();  // every node sum of the batch done
-    write_batch_nodes<UMAX, NT>(pl.mode, wn, U, sR, a.Rmass, a.Rmom, a.Rener, a.npoin);
+    col_write<P, COLORED>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
 }
 
-template <int P, class A, bool CLOSURE = false, typename TA = double>
-static hipError_t launch_p(const A &a, hipStream_t s, const float *mlp = nullptr)
+// Orders above kNarrowP: the same walk, whose columns (r, T, u and the six sums)
+// take up to 198 VGPRs.  nu and kappa wait in LDS for the end, mu_fluid is
+// gathered a slice ahead, and the gradients replace the line derivatives one
+// field at a time.  The atomic mode adds to the outputs from the registers
+// (col_merge, col_scatter).  Against one node per thread: 40^3 order 6 1.86 ->
+// 1.21 ms (1.32 with the line sources read one ahead: spills); 32^3 order 8,
+// with one wave per SIMD, 2.40 -> 1.88 (two waves and 80 spilled VGPRs: 2.61);
+// order 5, against the kernel above with LDS sums, 64^3 3.08 -> 2.64.
+template <int P, typename TA>
+constexpr int kWideWaves = P == 8 && sizeof(TA) == 8 ? 1 : 2;  // per SIMD
+
+template <int P, bool COLORED, class A, bool CLOSURE, typename TA>
+__global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_wide(A a, const float *mlp)
+{
+    using S = ColShape<P>;
+    using T = TA;
+    using TG = typename A::G;
+    constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
+    constexpr bool AHEAD = kWideWaves<P, TA> == 1;  // read line sources one ahead of their use
+    struct alignas(2 * sizeof(T)) V2 { T x, y; };
+    __shared__ T sD[Q * Q];
+    __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
+    __shared__ T sU2[NT];     // and u2
+    __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
+    __shared__ V2 sN[Q][NT];                               // nu, kappa of the thread's nodes
+    __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
+    // its fluxes along I (0..2) and J (3..5); in the coloured mode, at the end,
+    // the node sums [5][US]
+    extern __shared__ __attribute__((aligned(16))) double sR[];
+    V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
+
+    const Plan &pl = a.plan;
+    const int US = pl.ustride, t = threadIdx.x;
+    const ColThread<P> th(t);
+    const int tc = th.tc, le = th.le, I = th.I, J = th.J;
+    const int64_t np = a.npoin;
+    const auto D = uniform(a.tab.D);
+    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
+    const int64_t e0 = (int64_t)b * EPB;
+    const bool active = t < LANES && e0 + le < a.nelem;
+    const uint32_t *conn = pl.conn + (int64_t)b * Q * LANES + tc;
+
+    // mu_e and mu_sgs change lanes in LDS (k_diffu_col)
+    const int lem = tc % EPB, Im = tc / EPB % Q, Jm = tc / (EPB * Q);
+    const int lm = line_ref<P>(Im) + Q * line_ref<P>(Jm), tm = t < LANES ? Im + Q * (lem + EPB * Jm) : t;
+    const int64_t em = e0 + lem < a.nelem ? e0 + lem : a.nelem - 1;
+    const bool has_sgs = !CLOSURE && a.mu_sgs;  // NULL: closure fallback
+    const TG *mu_sgs = has_sgs ? a.mu_sgs : a.mu_e;
+    TG mue, mus = (TG)0;
+    typename A::F fmu;
+    auto load_mu = [&](int k) {
+        const int64_t ge = em + a.nelem * (int64_t)a.tab.l2g[lm + QQ * line_ref<P>(k)];
+        mue = a.mu_e[ge];
+        if constexpr (!CLOSURE) mus = mu_sgs[ge];
+        fmu = a.mu_fluid[conn[k * LANES]];
+    };
+    const T Cp = (T)a.Cp, Pr = (T)a.Pr;
+    T r[Q], Te[Q], u[Q][3], W[Q][6];
+    {
+        uint32_t gn[Q];
+#pragma unroll
+        for (int k = 0; k < Q; ++k) gn[k] = conn[k * LANES];
+        typename A::F fr[Q], fT[Q];
+        typename A::U fu[Q][3];
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            const int64_t g = gn[k];
+            fr[k] = a.rho[g];
+            fT[k] = a.Tem[g];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) fu[k][d] = a.u[g + d * np];
+        }
+        load_mu(0);
+        col_table<P>(a.tab.D, sD);
+        if constexpr (CLOSURE) mlp_stage(smlp, mlp);
+#pragma unroll
+        for (int k = 0; k < Q; ++k) {
+            r[k] = (T)fr[k];
+            Te[k] = (T)fT[k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) u[k][d] = (T)fu[k][d];
+        }
+    }
+    GeoNode<TG> gk = col_geo<P, false>(a.geo, b, 0, tc);
+    const int sI = tc - I, sJ = tc - J * EPB * Q;  // a line's source n: sI + n, sJ + n*EPB*Q
+
+    col_slices<Q>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = kc();
+        // the previous slice's values were read before its second barrier
+        sP[0][t] = V2{r[k], Te[k]};
+        sP[1][t] = V2{u[k][0], u[k][1]};
+        sU2[t] = u[k][2];
+        sMu[0][tm] = mue;
+        sMu[1][tm] = mus;
+        const T muf = (T)fmu;
+        if constexpr (k + 1 < Q) load_mu(k + 1);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        // line derivatives x[d] of rho, T, u; the slice's geometry is still in flight
+        T x[3][5];
+#pragma unroll
+        for (int f = 0; f < 5; ++f) x[0][f] = x[1][f] = x[2][f] = 0;
+        struct Src { V2 a, b; T c, D; };
+        auto read_source = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * EPB * Q;
+            return Src{sP[0][m], sP[1][m], sU2[m], s < Q ? sD[I * Q + s] : sD[J * Q + s - Q]};
+        };
+        Src cur = read_source(0), nxt = cur;
+#pragma unroll
+        for (int n = 0; n < Q; ++n) {
+            const T Dk = (T)col_D<P>(D, k, n);
+            x[2][0] += Dk * r[n];
+            x[2][1] += Dk * Te[n];
+            x[2][2] += Dk * u[n][0];
+            x[2][3] += Dk * u[n][1];
+            x[2][4] += Dk * u[n][2];
+        }
+#pragma unroll
+        for (int f = 0; f < 5; ++f) asm volatile("" : "+v"(x[2][f]));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            const int d = s < Q ? 0 : 1;
+            if (AHEAD && s + 1 < 2 * Q) nxt = read_source(s + 1);
+            if (!AHEAD && s > 0) cur = read_source(s);
+            x[d][0] += cur.D * cur.a.x;
+            x[d][1] += cur.D * cur.a.y;
+            x[d][2] += cur.D * cur.b.x;
+            x[d][3] += cur.D * cur.b.y;
+            x[d][4] += cur.D * cur.c;
+            asm volatile("" : "+v"(x[d][0]), "+v"(x[d][1]), "+v"(x[d][2]), "+v"(x[d][3]), "+v"(x[d][4]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD) cur = nxt;
+        }
+        // x[.][f] becomes the gradient: grad rho, grad T, G[c][i] = x[i][2 + c]
+#pragma unroll
+        for (int f = 0; f < 5; ++f) {
+            T g[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                g[i] = (T)gk.he(i) * x[0][f] + (T)gk.he(3 + i) * x[1][f] + (T)gk.he(6 + i) * x[2][f];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                x[i][f] = g[i];
+                asm volatile("" : "+v"(x[i][f]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const T me = (T)sMu[0][tc];
+        T ms = has_sgs ? (T)sMu[1][tc] : (T)0;
+        if constexpr (CLOSURE) {
+            float f[kMlpIn];
+            T hinv[3][3], G[3][3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    hinv[i][d] = (T)gk.he(i + 3 * d);
+                    G[i][d] = x[d][2 + i];
+                }
+            mlp_features<T>(G, r[k], u[k], hinv, f);
+            // idle lanes hold a real element node (finite features)
+            const float z3 =
+                mlp_forward_z3<NT * (int)sizeof(V2) / 2>(smlp, f, reinterpret_cast<short *>(&sF[0][t & ~63]));
+            ms = (T)(smlp.scale * softplusf_(z3));
+        }
+        sN[k][t] = V2{(T)a.c_rho * me / r[k], muf * Cp / Pr + (T)a.c_ener * me * Cp / Pr + Cp * r[k] * ms / (T)0.9};
+        const T mu_f = muf + r[k] * ms, mu_t = mu_f + me;
+        const T lam = mu_f * (T)(2.0 / 3.0) * (x[0][2] + x[1][3] + x[2][4]);
+        // tau (symmetric): xx, yy, zz, xy, xz, yz; tau.u
+        T tau[6] = {mu_t * (x[0][2] + x[0][2]), mu_t * (x[1][3] + x[1][3]), mu_t * (x[2][4] + x[2][4]),
+                    mu_t * (x[1][2] + x[0][3]), mu_t * (x[2][2] + x[0][4]), mu_t * (x[2][3] + x[1][4])};
+        constexpr int at[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
+        T tauU[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            tauU[i] = tau[at[i][0]] * u[k][0] + tau[at[i][1]] * u[k][1] + tau[at[i][2]] * u[k][2] - lam * u[k][i];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            tau[i] -= lam;
+            asm volatile("" : "+v"(tau[i]), "+v"(tau[3 + i]), "+v"(tauU[i]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const T gv = (T)gk.gvol();
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const T c0 = gv * (T)gk.he(3 * d), c1 = gv * (T)gk.he(3 * d + 1), c2 = gv * (T)gk.he(3 * d + 2);
+            T F[6];
+            F[0] = c0 * x[0][0] + c1 * x[1][0] + c2 * x[2][0];
+            F[1] = c0 * tauU[0] + c1 * tauU[1] + c2 * tauU[2];
+            F[2] = c0 * x[0][1] + c1 * x[1][1] + c2 * x[2][1];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) F[3 + i] = c0 * tau[at[i][0]] + c1 * tau[at[i][1]] + c2 * tau[at[i][2]];
+            if (d < 2) {
+#pragma unroll
+                for (int c = 0; c < 3; ++c) sF[3 * (d < 2 ? d : 0) + c][t] = V2{F[2 * c], F[2 * c + 1]};
+            } else {
+#pragma unroll
+                for (int n = 0; n < Q; ++n) {
+                    const T Dk = (T)col_D<P>(D, k, n);  // transposed: l_n'(xi_k)
+#pragma unroll
+                    for (int f = 0; f < 6; ++f) {
+                        if constexpr (k == 0) W[n][f] = Dk * F[f];
+                        else W[n][f] += Dk * F[f];
+                        // added now: sunk to its use, every F would stay live
+                        asm volatile("" : "+v"(W[n][f]));
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (k + 1 < Q) gk = col_geo<P, false>(a.geo, b, k + 1, tc);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        struct Flux { V2 a, b, c; T D; };
+        auto read_flux = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * EPB * Q, c = s < Q ? 0 : 3;
+            // transposed: l_I'(xi_n)
+            return Flux{sF[c][m], sF[c + 1][m], sF[c + 2][m], s < Q ? sD[s * Q + I] : sD[(s - Q) * Q + J]};
+        };
+        Flux fc = read_flux(0), fn = fc;
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            if (AHEAD && s + 1 < 2 * Q) fn = read_flux(s + 1);
+            if (!AHEAD && s > 0) fc = read_flux(s);
+            W[k][0] += fc.D * fc.a.x;
+            W[k][1] += fc.D * fc.a.y;
+            W[k][2] += fc.D * fc.b.x;
+            W[k][3] += fc.D * fc.b.y;
+            W[k][4] += fc.D * fc.c.x;
+            W[k][5] += fc.D * fc.c.y;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) asm volatile("" : "+v"(W[k][f]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD) fc = fn;
+        }
+    });
+    if constexpr (COLORED) {
+        __syncthreads();  // the last slice's fluxes are read
+        for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
+        __syncthreads();
+    }
+    uint32_t at[Q];
+#pragma unroll
+    for (int k = 0; k < Q; ++k)
+        at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k) * LANES + tc] : conn[k * LANES];
+#pragma unroll
+    for (int k = 0; k < Q; ++k) {
+        const V2 c = sN[k][t];
+        double v[5] = {(double)(c.x * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
+                       (double)(W[k][1] + c.y * W[k][2])};
+        if constexpr (COLORED)
+            col_add<P, true>(sR, US, active, le, at[k], v);
+        else if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+            col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
+    }
+    if constexpr (COLORED) {
+        const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+        uint32_t wn[S::UPT];
+        col_list<P>(pl.unode + u0, U, wn);
+        __syncthreads();
+        col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
+    }
+}
+
+// Order 7: a column is shared by two threads (t and its mate HL threads on, in
+// other waves), four nodes each: k_diffu_wide spills 48 to 83 registers there
+// and takes 4.4-4.7 ms at 48^3 (3.7 with one wave per SIMD and no spills).
+// Derivatives along K take the mate's half of the column through LDS once;
+// each slice's K fluxes go to the own nodes and, through LDS, to the mate's.  E2
+// elements of a batch per workgroup (coloured mode: all of them).  48^3: 3.09
+// ms, one node per thread 3.49; with all four elements in a workgroup, alone on
+// its CU, 3.56.
+template <int P, int E2, bool COLORED, class A, bool CLOSURE, typename TA>
+__global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a, const float *mlp)
+{
+    using S = ColShape<P>;
+    using T = TA;
+    using TG = typename A::G;
+    constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES;
+    constexpr int H = Q / 2, HL = E2 * QQ, NT = 2 * HL, PARTS = EPB / E2;
+    static_assert(Q % 2 == 0 && HL % 64 == 0 && LANES == EPB * QQ, "whole waves per half");
+    constexpr bool AHEAD = true;  // read line sources one ahead of their use
+    struct alignas(2 * sizeof(T)) V2 { T x, y; };
+    __shared__ T sD[Q * Q];
+    __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
+    __shared__ T sU2[NT];     // and u2
+    __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
+    __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
+    // its fluxes along I (0..2), J (3..5) and K (6..8); at the start the columns'
+    // values; in the coloured mode, at the end, the node sums [5][US]
+    extern __shared__ __attribute__((aligned(16))) double sR[];
+    V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
+
+    const Plan &pl = a.plan;
+    const int US = pl.ustride, t = threadIdx.x;
+    const int half = __builtin_amdgcn_readfirstlane(t / HL), tl = t - half * HL, mate = half ? t - HL : t + HL;
+    const int I = tl % Q, le = tl / Q % E2, J = tl / (Q * E2);
+    const int64_t np = a.npoin;
+    const auto D = uniform(a.tab.D);
+    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x), bs = slot / PARTS, part = slot % PARTS;
+    const uint32_t b = pl.batches ? uniform(pl.batches)[bs] : bs;
+    const int64_t e0 = (int64_t)b * EPB + part * E2;
+    const bool active = e0 + le < a.nelem;
+    const int tc = I + Q * ((int)part * E2 + le + EPB * J), k0 = half * H;
+    const uint32_t *conn = pl.conn + ((int64_t)b * Q + k0) * LANES + tc;
+    // line_ref of slice j of half h (j a compile-time constant)
+    auto ref = [](int h, int j) { return h ? (j == H - 1 ? 1 : H + j + 1) : (j == 0 ? 0 : j + 1); };
+
+    // mu_e and mu_sgs change lanes in LDS (k_diffu_col)
+    const int lem = tl % E2, Im = tl / E2 % Q, Jm = tl / (E2 * Q);
+    const int lm = line_ref<P>(Im) + Q * line_ref<P>(Jm), tm = half * HL + Im + Q * (lem + E2 * Jm);
+    const int64_t em = e0 + lem < a.nelem ? e0 + lem : a.nelem - 1;
+    const bool has_sgs = !CLOSURE && a.mu_sgs;  // NULL: closure fallback
+    const TG *mu_sgs = has_sgs ? a.mu_sgs : a.mu_e;
+    TG mue, mus = (TG)0;
+    typename A::F fmu;
+    auto load_mu = [&](int k) {
+        const int64_t ge = em + a.nelem * (int64_t)a.tab.l2g[lm + QQ * ref(half, k)];
+        mue = a.mu_e[ge];
+        if constexpr (!CLOSURE) mus = mu_sgs[ge];
+        fmu = a.mu_fluid[conn[k * LANES]];
+    };
+    const T Cp = (T)a.Cp, Pr = (T)a.Pr;
+    T r[H], Te[H], u[H][3], dz[H][5], W[H][6], nu[H], kappa[H];
+    {
+        uint32_t gn[H];
+#pragma unroll
+        for (int k = 0; k < H; ++k) gn[k] = conn[k * LANES];
+        typename A::F fr[H], fT[H];
+        typename A::U fu[H][3];
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            const int64_t g = gn[k];
+            fr[k] = a.rho[g];
+            fT[k] = a.Tem[g];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) fu[k][d] = a.u[g + d * np];
+        }
+        load_mu(0);
+        col_table<P>(a.tab.D, sD);
+        if constexpr (CLOSURE) mlp_stage(smlp, mlp);
+#pragma unroll
+        for (int k = 0; k < H; ++k) {
+            r[k] = (T)fr[k];
+            Te[k] = (T)fT[k];
+#pragma unroll
+            for (int d = 0; d < 3; ++d) u[k][d] = (T)fu[k][d];
+        }
+    }
+    GeoNode<TG> gk = col_geo<P, false>(a.geo, b, k0, tc);
+    // derivatives along K: the mate's half of the column comes through LDS, two
+    // fields at a time
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+        auto field = [&](int k, int f) -> T { return f == 0 ? r[k] : (f == 1 ? Te[k] : u[k][f - 2]); };
+        const int f0 = 2 * c, f1 = c < 2 ? 2 * c + 1 : f0;
+        V2(*buf)[NT] = sF + (c == 1 ? H : 0);
+        if (c == 2) __syncthreads();  // the first buffer is read
+#pragma unroll
+        for (int k = 0; k < H; ++k) buf[k][t] = V2{field(k, f0), field(k, f1)};
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < H; ++j) dz[j][f0] = dz[j][f1] = 0;
+#pragma unroll
+        for (int n = 0; n < H; ++n) {
+            const V2 o = buf[n][mate];
+#pragma unroll
+            for (int j = 0; j < H; ++j) {
+                const T Do = (T)D[ref(half, j) * Q + ref(half, n)], Dm = (T)D[ref(half, j) * Q + ref(1 - half, n)];
+                dz[j][f0] += Do * field(n, f0) + Dm * o.x;
+                if (c < 2) dz[j][f1] += Do * field(n, f1) + Dm * o.y;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < H; ++j) asm volatile("" : "+v"(dz[j][f0]), "+v"(dz[j][f1]));
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // a line's source n: sI + n, sJ + n*E2*Q
+    const int sI = t - I, sJ = t - J * E2 * Q;
+
+    col_slices<H>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int k = kc();
+        // the previous slice's values were read before its second barrier
+        sP[0][t] = V2{r[k], Te[k]};
+        sP[1][t] = V2{u[k][0], u[k][1]};
+        sU2[t] = u[k][2];
+        sMu[0][tm] = mue;
+        sMu[1][tm] = mus;
+        const T muf = (T)fmu;
+        if constexpr (k + 1 < H) load_mu(k + 1);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        // line derivatives x[d] of rho, T, u; the slice's geometry is still in flight
+        T x[3][5];
+#pragma unroll
+        for (int f = 0; f < 5; ++f) {
+            x[0][f] = x[1][f] = 0;
+            x[2][f] = dz[k][f];
+        }
+        struct Src { V2 a, b; T c, D; };
+        auto read_source = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * E2 * Q;
+            return Src{sP[0][m], sP[1][m], sU2[m], s < Q ? sD[I * Q + s] : sD[J * Q + s - Q]};
+        };
+        Src cur = read_source(0), nxt = cur;
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            const int d = s < Q ? 0 : 1;
+            if (AHEAD && s + 1 < 2 * Q) nxt = read_source(s + 1);
+            if (!AHEAD && s > 0) cur = read_source(s);
+            x[d][0] += cur.D * cur.a.x;
+            x[d][1] += cur.D * cur.a.y;
+            x[d][2] += cur.D * cur.b.x;
+            x[d][3] += cur.D * cur.b.y;
+            x[d][4] += cur.D * cur.c;
+            asm volatile("" : "+v"(x[d][0]), "+v"(x[d][1]), "+v"(x[d][2]), "+v"(x[d][3]), "+v"(x[d][4]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD) cur = nxt;
+        }
+        // x[.][f] becomes the gradient: grad rho, grad T, G[c][i] = x[i][2 + c]
+#pragma unroll
+        for (int f = 0; f < 5; ++f) {
+            T g[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+                g[i] = (T)gk.he(i) * x[0][f] + (T)gk.he(3 + i) * x[1][f] + (T)gk.he(6 + i) * x[2][f];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                x[i][f] = g[i];
+                asm volatile("" : "+v"(x[i][f]));
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const T me = (T)sMu[0][t];
+        T ms = has_sgs ? (T)sMu[1][t] : (T)0;
+        if constexpr (CLOSURE) {
+            float f[kMlpIn];
+            T hinv[3][3], G[3][3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    hinv[i][d] = (T)gk.he(i + 3 * d);
+                    G[i][d] = x[d][2 + i];
+                }
+            mlp_features<T>(G, r[k], u[k], hinv, f);
+            // idle lanes hold a real element node (finite features)
+            const float z3 =
+                mlp_forward_z3<NT * (int)sizeof(V2) / 2>(smlp, f, reinterpret_cast<short *>(&sF[0][t & ~63]));
+            ms = (T)(smlp.scale * softplusf_(z3));
+        }
+        nu[k] = (T)a.c_rho * me / r[k];
+        kappa[k] = muf * Cp / Pr + (T)a.c_ener * me * Cp / Pr + Cp * r[k] * ms / (T)0.9;
+        asm volatile("" : "+v"(nu[k]), "+v"(kappa[k]));
+        const T mu_f = muf + r[k] * ms, mu_t = mu_f + me;
+        const T lam = mu_f * (T)(2.0 / 3.0) * (x[0][2] + x[1][3] + x[2][4]);
+        // tau (symmetric): xx, yy, zz, xy, xz, yz; tau.u
+        T tau[6] = {mu_t * (x[0][2] + x[0][2]), mu_t * (x[1][3] + x[1][3]), mu_t * (x[2][4] + x[2][4]),
+                    mu_t * (x[1][2] + x[0][3]), mu_t * (x[2][2] + x[0][4]), mu_t * (x[2][3] + x[1][4])};
+        constexpr int at[3][3] = {{0, 3, 4}, {3, 1, 5}, {4, 5, 2}};
+        T tauU[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+            tauU[i] = tau[at[i][0]] * u[k][0] + tau[at[i][1]] * u[k][1] + tau[at[i][2]] * u[k][2] - lam * u[k][i];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            tau[i] -= lam;
+            asm volatile("" : "+v"(tau[i]), "+v"(tau[3 + i]), "+v"(tauU[i]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const T gv = (T)gk.gvol();
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            const T c0 = gv * (T)gk.he(3 * d), c1 = gv * (T)gk.he(3 * d + 1), c2 = gv * (T)gk.he(3 * d + 2);
+            T F[6];
+            F[0] = c0 * x[0][0] + c1 * x[1][0] + c2 * x[2][0];
+            F[1] = c0 * tauU[0] + c1 * tauU[1] + c2 * tauU[2];
+            F[2] = c0 * x[0][1] + c1 * x[1][1] + c2 * x[2][1];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) F[3 + i] = c0 * tau[at[i][0]] + c1 * tau[at[i][1]] + c2 * tau[at[i][2]];
+#pragma unroll
+            for (int c = 0; c < 3; ++c) sF[3 * d + c][t] = V2{F[2 * c], F[2 * c + 1]};
+            if (d == 2) {
+#pragma unroll
+                for (int n = 0; n < H; ++n) {
+                    const T Dk = (T)D[ref(half, k) * Q + ref(half, n)];  // transposed: l_n'(xi_k)
+#pragma unroll
+                    for (int f = 0; f < 6; ++f) {
+                        if constexpr (k == 0) W[n][f] = Dk * F[f];
+                        else W[n][f] += Dk * F[f];
+                        // added now: sunk to its use, every F would stay live
+                        asm volatile("" : "+v"(W[n][f]));
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (k + 1 < H) gk = col_geo<P, false>(a.geo, b, k0 + k + 1, tc);
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);
+        struct Flux { V2 a, b, c; T D; };
+        auto read_flux = [&](int s) {
+            const int m = s < Q ? sI + s : sJ + (s - Q) * E2 * Q, c = s < Q ? 0 : 3;
+            // transposed: l_I'(xi_n)
+            return Flux{sF[c][m], sF[c + 1][m], sF[c + 2][m], s < Q ? sD[s * Q + I] : sD[(s - Q) * Q + J]};
+        };
+        Flux fc = read_flux(0), fn = fc;
+#pragma unroll
+        for (int s = 0; s < 2 * Q; ++s) {
+            if (AHEAD && s + 1 < 2 * Q) fn = read_flux(s + 1);
+            if (!AHEAD && s > 0) fc = read_flux(s);
+            W[k][0] += fc.D * fc.a.x;
+            W[k][1] += fc.D * fc.a.y;
+            W[k][2] += fc.D * fc.b.x;
+            W[k][3] += fc.D * fc.b.y;
+            W[k][4] += fc.D * fc.c.x;
+            W[k][5] += fc.D * fc.c.y;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) asm volatile("" : "+v"(W[k][f]));
+            __builtin_amdgcn_sched_barrier(0);
+            if (AHEAD) fc = fn;
+        }
+        // the mate's slice
+        const V2 m0 = sF[6][mate], m1 = sF[7][mate], m2 = sF[8][mate];
+#pragma unroll
+        for (int n = 0; n < H; ++n) {
+            const T Dk = (T)D[ref(1 - half, k) * Q + ref(half, n)];
+            W[n][0] += Dk * m0.x;
+            W[n][1] += Dk * m0.y;
+            W[n][2] += Dk * m1.x;
+            W[n][3] += Dk * m1.y;
+            W[n][4] += Dk * m2.x;
+            W[n][5] += Dk * m2.y;
+#pragma unroll
+            for (int f = 0; f < 6; ++f) asm volatile("" : "+v"(W[n][f]));
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    });
+    if constexpr (COLORED) {
+        __syncthreads();  // the last slice's fluxes are read
+        for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
+        __syncthreads();
+    }
+    uint32_t at[H];
+#pragma unroll
+    for (int k = 0; k < H; ++k)
+        at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k0 + k) * LANES + tc] : conn[k * LANES];
+#pragma unroll
+    for (int k = 0; k < H; ++k) {
+        double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
+                       (double)(W[k][1] + kappa[k] * W[k][2])};
+        if constexpr (COLORED)
+            col_add<P, true>(sR, US, active, le, at[k], v);
+        else if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+            col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
+    }
+    if constexpr (COLORED) {
+        const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+        __syncthreads();
+        if (t < S::NT) {
+            uint32_t wn[S::UPT];
+            col_list<P>(pl.unode + u0, U, wn);
+            col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
+        }
+    }
+}
+
+template <int P, class A, bool CLOSURE, typename TA>
+static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_diffu<P, A, CLOSURE, TA>), dim3((unsigned)a.plan.nb), dim3(Shape<P>::NT), 0, s,
-                       a, mlp);
+    const bool atomic = a.plan.mode == kAtomic;
+    const size_t sums = sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(TA) * 12 * ColShape<P>::NT;
+    const dim3 grid((unsigned)a.plan.nb), block(ColShape<P>::NT);
+    if constexpr (P == 7) {
+        constexpr int E2 = 2, EPB = ColShape<P>::EPB, QQ = ColShape<P>::QQ;
+        const size_t part = sizeof(TA) * 2 * 9 * 2 * QQ;  // fluxes per element
+        if (atomic)
+            hipLaunchKernelGGL((k_diffu_split<P, E2, false, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))),
+                               dim3(2 * E2 * QQ), E2 * part, s, a, mlp);
+        else
+            hipLaunchKernelGGL((k_diffu_split<P, EPB, true, A, CLOSURE, TA>), grid, dim3(2 * EPB * QQ),
+                               std::max(EPB * part, sums), s, a, mlp);
+    } else if constexpr (P > kNarrowP)
+        hipLaunchKernelGGL((atomic ? k_diffu_wide<P, false, A, CLOSURE, TA> : k_diffu_wide<P, true, A, CLOSURE, TA>), grid,
+                           block, atomic ? fluxes : std::max(fluxes, sums), s, a, mlp);
+    else
+        hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE, TA> : k_diffu_col<P, true, A, CLOSURE, TA>), grid,
+                           block, sums, s, a, mlp);
     return hipGetLastError();
+}
+
+template <class A, bool CLOSURE, typename TA>
+static hipError_t launch_order(int porder, const A &a, const float *mlp, hipStream_t s)
+{
+    switch (porder) {
+    case 1: return launch_p<1, A, CLOSURE, TA>(a, mlp, s);
+    case 2: return launch_p<2, A, CLOSURE, TA>(a, mlp, s);
+    case 3: return launch_p<3, A, CLOSURE, TA>(a, mlp, s);
+    case 4: return launch_p<4, A, CLOSURE, TA>(a, mlp, s);
+    case 5: return launch_p<5, A, CLOSURE, TA>(a, mlp, s);
+    case 6: return launch_p<6, A, CLOSURE, TA>(a, mlp, s);
+    case 7: return launch_p<7, A, CLOSURE, TA>(a, mlp, s);
+    case 8: return launch_p<8, A, CLOSURE, TA>(a, mlp, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 template <class A>
 hipError_t launch_diffu(int porder, const A &a, hipStream_t s)
 {
-    if (porder <= kColMaxP) return launch_diffu_col<A, false, double>(porder, a, nullptr, s);
-    switch (porder) {
-    case 6: return launch_p<6, A>(a, s);
-    case 7: return launch_p<7, A>(a, s);
-    case 8: return launch_p<8, A>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    return launch_order<A, false, double>(porder, a, nullptr, s);
 }
 
 hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
 {
-    if (porder <= kColMaxP) return launch_diffu_col<DiffuArgs<float, float>, false, float>(porder, a, nullptr, s);
-    switch (porder) {
-    case 6: return launch_p<6, DiffuArgs<float, float>, false, float>(a, s);
-    case 7: return launch_p<7, DiffuArgs<float, float>, false, float>(a, s);
-    case 8: return launch_p<8, DiffuArgs<float, float>, false, float>(a, s);
-    default: return hipErrorInvalidValue;
-    }
+    return launch_order<DiffuArgs<float, float>, false, float>(porder, a, nullptr, s);
+}
+
+hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp, hipStream_t s)
+{
+    return launch_order<DiffuArgs<double, double>, true, double>(porder, a, mlp, s);
 }
 
 template hipError_t launch_diffu(int, const DiffuArgs<double, double> &, hipStream_t);
@@ -407,17 +916,5 @@ template hipError_t launch_diffu(int, const DiffuArgs<float, float> &, hipStream
 template hipError_t launch_diffu(int, const DiffuArgs<float, double> &, hipStream_t);
 template hipError_t launch_diffu(int, const DiffuArgs<float, float, float> &, hipStream_t);
 template hipError_t launch_diffu(int, const DiffuSplitArgs &, hipStream_t);
-
-hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp,
-                                        hipStream_t s)
-{
-    if (porder <= kColMaxP) return launch_diffu_col<DiffuArgs<double, double>, true, double>(porder, a, mlp, s);
-    switch (porder) {
-    case 6: return launch_p<6, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 7: return launch_p<7, DiffuArgs<double, double>, true>(a, s, mlp);
-    case 8: return launch_p<8, DiffuArgs<double, double>, true>(a, s, mlp);
-    default: return hipErrorInvalidValue;
-    }
-}
 
 }  // namespace msod

@@ -1,34 +1,31 @@
 // Internal interface between the runtime (msod_runtime.hip) and the kernel
 // translation units.  All pointers are device pointers.
 //
-// Element data are element-major above kColMaxP, with the element-local node
-// index l lexicographic in the reference's 1-D SOD order: l = I + q*(J + q*K),
-// (I,J,K) = (AtoI,AtoJ,AtoK) - 1 (the column kernels' layout: msod_columns.h).
-//   geo   [nelem][5][nn][2] He(i,k) (component c = i + 3k) and gpvol of each
-//                          element node as five pairs (c = 0,1 | 2,3 | 4,5 |
-//                          6,7 | 8 and gpvol): a node's ten values in five
-//                          16-byte (FP64) or 8-byte (FP32) loads, each wave's
-//                          load contiguous (GeoNode)
+// Element data are in the lane layout of msod_columns.h, which orders the nodes
+// of an element by (I,J,K); l = I + q*(J + q*K) is the lexicographic index in the
+// reference's 1-D SOD order, (I,J,K) = (AtoI,AtoJ,AtoK) - 1.
+//   geo    He(i,k) (component c = i + 3k) and gpvol of each element node as five
+//          pairs (c = 0,1 | 2,3 | 4,5 | 6,7 | 8 and gpvol): a node's ten values
+//          in five 16-byte (FP64) or 8-byte (FP32) loads, each wave's load
+//          contiguous (GeoNode)
 // tab.D[q*q] is the 1-D derivative D[i*q+n] = l_n'(xi_i); tab.l2g[nn] maps l
 // to the 0-based reference (Gmsh) node number, used for arrays kept in the
 // reference layout (mu_e, mu_sgs).
 //
 // Assembly plan (built once per mesh by the runtime).  Elements are grouped
-// into batches of consecutive elements (ColShape<P>::EPB, Shape<P>::BATCH,
-// CShape<P>::BATCH); one workgroup owns a batch, sums the contributions of its elements to every node of the batch in
-// LDS, and writes each of the batch's distinct nodes once:
-//   conn  [nelem][nn]   0-based global node of each element node
-//   lidx  [nelem][nn]   position of that node in its batch's node list
-//   uoff  [nbatch+1]    node list of batch b: unode[uoff[b] .. uoff[b+1])
-//   unode [..]          sorted distinct global nodes of each batch; bit 31 set
-//                       when this batch is the first writer of the node
-//   batches[nb]         the batches processed by one launch; a workgroup takes
-//                       kpb consecutive ones, one after the other, with the
-//                       loads of the next pass always in flight.  Null: the
-//                       batches 0 .. nb-1 in mesh order, with no list to load
-// Within a batch the element-node values are summed in a fixed order
-// (add_pass).  Two ways to combine the batches' partial sums at nodes shared
-// between batches (mode):
+// into batches of ColShape<P>::EPB consecutive elements, one workgroup each,
+// which sums its elements' contributions to every node of the batch in LDS and
+// writes each of the batch's distinct nodes once (above kNarrowP, in the atomic
+// mode, it adds from registers and needs conn alone):
+//   conn          0-based global node of each element node
+//   lidx          position of that node in its batch's node list
+//   uoff [nbatch+1]  node list of batch b: unode[uoff[b] .. uoff[b+1])
+//   unode [..]    sorted distinct global nodes of each batch; bit 31 set when
+//                 this batch is the first writer of the node (host plan)
+//   batches[nb]   the batches processed by one launch.  Null: 0 .. nb-1 in mesh
+//                 order
+// Two ways to combine the batches' partial sums at nodes shared between batches
+// (mode):
 //   kColored: batches are coloured so that batches of one colour share no
 //     node; one launch per colour, each node written with a plain store by its
 //     first batch and read-add-stored by later ones.  No atomics, no zero-fill,
@@ -42,50 +39,17 @@
 namespace msod {
 
 constexpr int kMaxP = 8;
-// Column kernels (msod_columns.h) up to this order, one node per thread above:
-// a column's values stay in registers (convection 244, diffusion 256 VGPRs at
-// order 5 in FP64) and spill past it.
-constexpr int kColMaxP = 5;
-constexpr int kMaxKpb = 16;           // batches per workgroup, at most (LDS list of the block's batches)
-constexpr int kBatchesPerBlock = 8;   // batches per workgroup (convection: measured best of 1..16 at p=4)
-static_assert(kBatchesPerBlock <= kMaxKpb, "the block's batch list holds kpb entries");
+// Orders whose batches sum in LDS.  Above, an element's share of the nodes that
+// meet in a batch is small and the sums cost occupancy: order 5, 64^3, 5.68 ms
+// for the pair with them and 5.01 without; order 4 gains 1 to 3% without
+// (convection 128^3 10.44 -> 10.07 ms), but only where a batch's elements follow
+// each other along I: otherwise it loses 15% (64^3 1.95 -> 2.24 ms, order 2, 100^3
+// 1.84 -> 2.65), order 5 7%.
+constexpr int kNarrowP = 4;
 enum AssemblyMode { kColored = 0, kAtomic = 1 };
 
-template <int P>
-struct Shape {
-    static constexpr int Q = P + 1;
-    static constexpr int NN = Q * Q * Q;
-    // one node per thread; several elements per pass while they fit 256 threads
-    static constexpr int EPB = NN <= 128 ? 256 / NN : 1;
-    static constexpr int NT = NN <= 128 ? 256 : ((NN + 63) / 64) * 64;
-    // elements per batch: about 512 element nodes, a whole number of passes
-    static constexpr int BATCH_RAW = 512 / NN < 1 ? 1 : (512 / NN > 64 ? 64 : 512 / NN);
-    static constexpr int BATCH = BATCH_RAW < EPB ? EPB : (BATCH_RAW / EPB) * EPB;
-    static constexpr int NPASS = BATCH / EPB;
-    static constexpr int UMAX = BATCH * NN;
-};
-
-// The convection's batches: Shape<P>'s, except from porder 6 on, where one
-// element fills a workgroup; there two elements per batch (two passes) share
-// a face in the node sums and halve the write phases per element (48^3 p=7:
-// 4.75 -> 4.01 ms).  The diffusion measured slower with two (3.58 -> 3.81 ms):
-// each kernel has its own plan where the sizes differ.
-template <int P>
-struct CShape {
-    static constexpr int Q = Shape<P>::Q;
-    static constexpr int NN = Shape<P>::NN;
-    static constexpr int EPB = Shape<P>::EPB;
-    static constexpr int NT = Shape<P>::NT;
-    static constexpr int BATCH = NN >= 343 ? 2 * EPB : Shape<P>::BATCH;
-    static constexpr int NPASS = BATCH / EPB;
-    static constexpr int UMAX = BATCH * NN;
-};
-
-// Elements per batch of the diffusion's (and closure kernels') and of the
-// convection's plan for run-time porder: ColShape<P>::EPB for both up to
-// kColMaxP, then Shape<P>::BATCH and CShape<P>::BATCH.
+// Elements per batch: ColShape<P>::EPB for run-time porder.
 int batch_size(int porder);
-int convec_batch_size(int porder);
 
 struct Tables {
     const double *D;      // [q*q]
@@ -100,12 +64,8 @@ struct Plan {
     const uint32_t *batches;
     int64_t nb;
     int mode;
-    int kpb;  // consecutive batches of the list per workgroup
-    int ustride;  // column kernels: stride of the node sums, the most nodes of any batch rounded up
+    int ustride;  // stride of the node sums: the most nodes of any batch
 };
-
-// Workgroups of a launch: each takes kpb consecutive batches of the list.
-inline unsigned plan_blocks(const Plan &p) { return (unsigned)((p.nb + p.kpb - 1) / p.kpb); }
 
 // Kernel arguments.  Storage types: TG for the element-sized arrays (geo;
 // in the diffusion also mu_e, mu_sgs), TF for the nodal fields.  The
@@ -163,13 +123,6 @@ struct DiffuArgs {
 using ConvecSplitArgs = ConvecArgs<float, float, double, double, double>;
 using DiffuSplitArgs = DiffuArgs<float, float, double, double>;
 
-// Column kernels, porder <= kColMaxP (msod_convec_col.hip, msod_diffu_col.hip);
-// TA: arithmetic type.
-template <class A, typename TA>
-hipError_t launch_convec_col(int porder, const A &a, hipStream_t s);
-template <class A, bool CLOSURE, typename TA>
-hipError_t launch_diffu_col(int porder, const A &a, const float *mlp, hipStream_t s);
-
 // Launchers (return hipError_t of the launch); A is a ConvecArgs or
 // DiffuArgs instantiation.
 template <class A>
@@ -190,16 +143,15 @@ template <typename TO>
 hipError_t launch_zero_nodes(TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin, const uint32_t *nodes,
                              int64_t count, hipStream_t s);
 
-// Element-major geometry from the reference layouts (see top of file), of
-// geo_elems(porder, nelem) elements.
+// Lane-layout geometry from the reference layouts, of geo_elems(porder, nelem)
+// elements.
 template <typename T>
 hipError_t launch_build_geo(int porder, const T *He, const T *gpvol, int64_t nelem, const int32_t *l2g, T *geo,
                             hipStream_t s);
-// conn and lidx of the column kernels' lane layout from the element-major ones.
+// conn and lidx of the lane layout from element-major ones.
 hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *lidx, int64_t nelem, uint32_t *lconn,
                              uint16_t *llidx, hipStream_t s);
-// Elements that geo, conn and lidx hold: nelem, padded to whole batches where
-// the column kernels run.
+// Elements that geo, conn and lidx hold: nelem, padded to whole batches.
 int64_t geo_elems(int porder, int64_t nelem);
 
 // He and gpvol of one element node from geo: He(i,k) = he(i + 3k), with the
@@ -215,23 +167,6 @@ struct GeoNode {
     __device__ __forceinline__ T gvol() const { return v[4].y; }
 };
 
-// NT: non-temporal loads (the geometry is read once per call).
-template <int NN, bool NT, typename T>
-__device__ __forceinline__ GeoNode<T> load_geo(const T *geo, int64_t e, int l)
-{
-    const GeoPair<T> *p = reinterpret_cast<const GeoPair<T> *>(geo) + e * 5 * NN + l;
-    GeoNode<T> g;
-#pragma unroll
-    for (int k = 0; k < 5; ++k) g.v[k] = NT ? __builtin_nontemporal_load(&p[k * NN]) : p[k * NN];
-    return g;
-}
-
-// Entry i of a launch's batch list (Plan::batches); a null list is mesh order.
-__device__ __forceinline__ uint32_t plan_batch(const uint32_t *batches, uint32_t i)
-{
-    return batches ? batches[i] : i;
-}
-
 // Blocks of a launch are dealt to the chip's 8 XCDs round robin (block i to
 // XCD i % 8), each XCD with its own L2.  xcd_slot gives every XCD a
 // contiguous range of the launch's batch list, so that batches adjacent in
@@ -242,69 +177,6 @@ __device__ __forceinline__ uint32_t xcd_slot(uint32_t i, uint32_t n)
     constexpr uint32_t kXcd = 8;
     const uint32_t x = i % kXcd, k = i / kXcd, q = n / kXcd, r = n % kXcd;
     return x * q + (x < r ? x : r) + k;
-}
-
-// Write phase shared by the kernels: the batch's node sums sR[c][i]
-// (c = Rmass, Rmom x3, Rener) go to the outputs.  Thread t holds entries t,
-// t + NT, ... of the batch's node list in registers (wn), loaded when the
-// batch started.  Atomic mode: every entry is added atomically onto the
-// zero-filled outputs (agent-scope FP64 atomics, performed past the L2; a
-// plain store of the nodes no other batch holds was tried and is much
-// slower, since those lines also take atomics).  Coloured mode: the first
-// writer stores, the others add.
-template <int UMAX, int NT, typename TO>
-__device__ __forceinline__ void write_batch_nodes(int mode, const uint32_t (&wn)[(UMAX + NT - 1) / NT],
-                                                  uint32_t U, const double (*sR)[UMAX], TO *Rmass,
-                                                  TO *Rmom, TO *Rener, int64_t npoin)
-{
-#pragma unroll
-    for (int j = 0; j < (UMAX + NT - 1) / NT; ++j) {
-        const uint32_t i = threadIdx.x + j * NT;
-        if (i >= U) break;
-        const uint32_t w = wn[j];
-        const int64_t g = w & 0x7fffffffu;
-        TO *dst[5] = {Rmass + g, Rmom + g, Rmom + npoin + g, Rmom + 2 * npoin + g, Rener + g};
-        if (mode == kAtomic) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) unsafeAtomicAdd(dst[c], (TO)sR[c][i]);
-        } else if (w >> 31) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) *dst[c] = (TO)sR[c][i];
-        } else {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) *dst[c] += (TO)sR[c][i];
-        }
-    }
-}
-
-// Adds the five residual values of every element node of a pass into the
-// batch's node sums, one element of the pass after the other: the nodes of
-// one element are distinct, so no two threads of a round touch the same sum,
-// and the summation order (pass, then element, within the batch) is fixed.
-// Every thread of the block calls it (uniform control flow, barriers).
-// In the atomic mode, whose global sums have no fixed order anyway, the
-// batch sums use LDS atomics instead (no rounds); the caller synchronises
-// before the batch is written.
-template <int UMAX, int EPB>
-__device__ __forceinline__ void add_pass(double (*sR)[UMAX], int mode, int le, bool active, uint32_t li,
-                                         const double (&v)[5])
-{
-    if (mode == kAtomic) {
-        if (active) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c)
-                __hip_atomic_fetch_add(&sR[c][li], v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-        return;
-    }
-#pragma unroll 1
-    for (int k = 0; k < EPB; ++k) {
-        if (active && le == k) {
-#pragma unroll
-            for (int c = 0; c < 5; ++c) sR[c][li] += v[c];
-        }
-        __syncthreads();
-    }
 }
 
 }  // namespace msod

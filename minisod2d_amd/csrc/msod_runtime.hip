@@ -131,8 +131,7 @@ __global__ void k_zero_nodes(TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin,
     }
 }
 
-// geo of the element nodes (msod_columns.h: the column kernels' lane layout,
-// element-major above kColMaxP): the pairs (He c = 2k, 2k+1) for k < 4, (He
+// geo of the element nodes (msod_columns.h: the lane layout): the pairs (He c = 2k, 2k+1) for k < 4, (He
 // c = 8, gpvol) for k = 4 (GeoNode), from He(3,3,nn,nelem) and
 // gpvol(1,nn,nelem).  Padding entries repeat the last element.
 template <int P, typename T>
@@ -175,15 +174,17 @@ __global__ void k_plan_lanes(const uint32_t *conn, const uint16_t *lidx, int64_t
 // nodes are sorted in LDS (bitonic) and the distinct ones numbered in
 // ascending order, as build_host_plan does on the host.  FILL = false:
 // count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
-// unode from uoff, conn and lidx in the layout of the order's kernels.
+// unode from uoff, conn and lidx in the lane layout.  Above kNarrowP the atomic
+// kernels read conn alone: no lists (count[b] = 0, the rest null).
 // A first convection at 64^3, p=4 takes 7 ms in all (193 with the host plan).
 constexpr uint32_t kBadBatch = 0x80000000u;
 template <int P>
 struct PlanShape {
     static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
-    static constexpr int UMAX = P <= kColMaxP ? ColShape<P <= kColMaxP ? P : 1>::UMAX : CShape<P>::UMAX;
+    static constexpr int UMAX = ColShape<P>::UMAX;
     static constexpr int NT = 256;
-    static constexpr int SORT = UMAX <= 512 ? 512 : (UMAX <= 1024 ? 1024 : 2048);
+    static constexpr bool LISTS = P <= kNarrowP;
+    static constexpr int SORT = UMAX <= 512 ? 512 : (UMAX <= 1024 ? 1024 : (UMAX <= 2048 ? 2048 : 4096));
     static constexpr int PER = SORT / NT;
 };
 template <int P, bool FILL>
@@ -199,8 +200,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     const int t = threadIdx.x;
     const int64_t b = xcd_slot(blockIdx.x, gridDim.x), e0 = b * B;
     const int ne = (int)(nelem - e0 < B ? nelem - e0 : B);
-    // the column kernels' layout is padded with copies of the last element
-    const int nf = P <= kColMaxP ? B : ne, n = nf * NN;
+    const int n = B * NN;  // the layout is padded with copies of the last element
     if (t == 0) sbad = 0;
     __syncthreads();
     uint32_t v[PER];
@@ -210,7 +210,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
         const int i = t + j * NT;
         v[j] = 0xffffffffu;
         if (i < n) {
-            const int le = i % nf, l = i / nf;  // neighbouring lanes: neighbouring elements
+            const int le = i % B, l = i / B;  // neighbouring lanes: neighbouring elements
             const int32_t c = connec[e0 + (le < ne ? le : ne - 1) + nelem * (int64_t)l2g[l]];
             const bool ok = c >= 1 && c <= npoin;
             bad += !ok && le < ne;
@@ -220,6 +220,18 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     }
     if (bad) atomicAdd(&sbad, bad);
     __syncthreads();
+    if constexpr (!S::LISTS) {
+        if constexpr (!FILL) {
+            if (t == 0) count[b] = sbad ? kBadBatch + sbad : 0u;
+        } else {
+#pragma unroll
+            for (int j = 0; j < PER; ++j) {
+                const int i = t + j * NT;
+                if (i < n) conn[ElemEntry<P>{e0 + i % B, i / B}.entry()] = v[j];
+            }
+        }
+        return;
+    }
     for (int k = 2; k <= SORT; k *= 2)
         for (int d = k / 2; d > 0; d /= 2) {
 #pragma unroll
@@ -274,7 +286,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
                 const uint32_t m = (lo + hi) / 2;
                 (su[m] <= v[j] ? lo : hi) = m;
             }
-            const ElemEntry<P> en{e0 + i % nf, i / nf};
+            const ElemEntry<P> en{e0 + i % B, i / B};
             conn[en.entry()] = v[j];
             lidx[en.entry()] = (uint16_t)lo;
         }
@@ -367,23 +379,11 @@ static auto with_porder(int porder, F f)
 
 int batch_size(int porder)
 {
-    return with_porder(porder, [](auto p) {
-        if constexpr (p() <= kColMaxP) return (int)ColShape<p()>::EPB;
-        else return (int)Shape<p()>::BATCH;
-    });
-}
-
-int convec_batch_size(int porder)
-{
-    return with_porder(porder, [](auto p) {
-        if constexpr (p() <= kColMaxP) return (int)ColShape<p()>::EPB;
-        else return (int)CShape<p()>::BATCH;
-    });
+    return with_porder(porder, [](auto p) { return (int)ColShape<p()>::EPB; });
 }
 
 int64_t geo_elems(int porder, int64_t nelem)
 {
-    if (porder > kColMaxP) return nelem;
     const int64_t B = batch_size(porder);
     return (nelem + B - 1) / B * B;
 }
@@ -815,8 +815,10 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
                     (long long)npoin);
     const int64_t n = geo_elems(ts->porder, nelem) * nn;
     HIPCHK(hipMalloc((void **)&P.conn, sizeof(uint32_t) * n), "plan");
-    HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
-    HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * uoff[nb]), "plan");
+    if (ts->porder <= kNarrowP) {
+        HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
+        HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * uoff[nb]), "plan");
+    }
     HIPCHK(hipMemcpyAsync(P.uoff, uoff.data(), sizeof(uint32_t) * (nb + 1), hipMemcpyHostToDevice, g.stream), "plan");
     HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
                                P.lidx, g.stream),
@@ -847,7 +849,7 @@ int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet
     int st;
     if ((st = upload(H.conn, &P.conn, "plan upload"))) return st;
     if ((st = upload(H.lidx, &P.lidx, "plan upload"))) return st;
-    if (ts->porder <= kColMaxP) {  // element-major to the column kernels' lane layout
+    {  // element-major to the lane layout
         const int64_t n = geo_elems(ts->porder, nelem) * (int64_t)ts->l2g.size();
         uint32_t *conn = P.conn;
         uint16_t *lidx = P.lidx;
@@ -1076,19 +1078,11 @@ int check_sizes(int porder, int nelem, int npoin)
     return MSOD_OK;
 }
 
-// Batches per workgroup, at most, per kernel.  The diffusion takes one: a
-// form that ran kpb batches per workgroup with every load one pass ahead
-// needed 148-152 VGPRs against 120 (3 waves per SIMD against 4) and ran
-// slower (128^3 p=4: 14.4-14.9 against 13.4 ms for kpb 2..16; 48^3 p=7: 5.2
-// against 3.7 ms).
-constexpr int kConvecKpb = kBatchesPerBlock;
-constexpr int kDiffuKpb = 1;
-
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
 // the kernel: one launch per colour, or one launch over all batches in mesh
 // order, where neighbouring batches meet in L2.
 template <class A, class L>
-int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what, int kpb_max)
+int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what)
 {
     Plan pl;
     pl.conn = P.conn;
@@ -1097,12 +1091,6 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     pl.unode = P.unode;
     pl.ustride = P.ustride;
     pl.mode = g.assembly;
-    // batches per workgroup: kpb_max on large meshes, fewer where that would
-    // leave the launch short of 2048 workgroups (8 per CU); 8^3 p=3 has 64
-    // batches, which 8 per workgroup put on 8 CUs
-    auto kpb_for = [kpb_max](int64_t nb) {
-        return (int)std::max<int64_t>(1, std::min<int64_t>(kpb_max, nb / 2048));
-    };
     const int64_t NP = a.npoin;
     if (g.assembly == kColored && !P.colored)
         return fail(MSOD_ERR_MESH, "%s: the batches of this mesh need more than 32 colours (elements in no "
@@ -1121,14 +1109,12 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     if (g.assembly == kAtomic) {
         pl.batches = nullptr;  // mesh order, no list
         pl.nb = P.nbatch;
-        pl.kpb = kpb_for(pl.nb);
         a.plan = pl;
         HIPCHK(launch(a), what);
     } else {
         for (size_t c = 0; c + 1 < P.color_off.size(); ++c) {
             pl.batches = P.order + P.color_off[c];
             pl.nb = P.color_off[c + 1] - P.color_off[c];
-            pl.kpb = kpb_for(pl.nb);
             a.plan = pl;
             HIPCHK(launch(a), what);
         }
@@ -1168,7 +1154,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, convec_batch_size(porder), &plan))) return st;
+    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
@@ -1192,7 +1178,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
                                 return launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch", kConvecKpb)))
+                            "convection kernel launch")))
         return st;
     return finish_call("convection kernel");
 }
@@ -1258,7 +1244,7 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
                                     if (fp32_arith) return launch_diffu_fp32(porder, x, g.stream);
                                 return launch_diffu(porder, x, g.stream);
                             },
-                            "diffusion kernel launch", kDiffuKpb)))
+                            "diffusion kernel launch")))
         return st;
     return finish_call("diffusion kernel");
 }

@@ -1,4 +1,4 @@
-"""GPU tests of the column kernels (porder 1..5) at the edges of their batches,
+"""GPU tests of the column kernels (porder 1..8) at the edges of their batches,
 through the C ABI against the CPU oracle: element counts of one, one less
 than a batch, a batch, one more and two batches and one, in both assembly
 modes, FP64 and the FP32 storage forms (the FP64 oracle on the rounded
@@ -13,7 +13,7 @@ from oracle_lib import Oracle, rel_l2
 pytestmark = pytest.mark.gpu
 
 # elements per batch of each order (ColShape<P>::EPB in csrc/msod_columns.h)
-EPB = {1: 64, 2: 28, 3: 16, 4: 10, 5: 3}
+EPB = {1: 64, 2: 28, 3: 16, 4: 10, 5: 7, 6: 5, 7: 4, 8: 3}
 
 
 def on_gpu(prob, convec, diffu, ins):
@@ -30,7 +30,7 @@ def on_gpu(prob, convec, diffu, ins):
 
 
 @pytest.mark.parametrize("mode", [m.ASSEMBLY_ATOMIC, m.ASSEMBLY_COLORED])
-@pytest.mark.parametrize("p", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("p", range(1, 9))
 def test_batch_edges(gpu, p, mode):
     for n in (1, EPB[p] - 1, EPB[p], EPB[p] + 1, 2 * EPB[p] + 1):
         prob = m.box_problem(n, p, ny=1, nz=1, jitter=0.05)
@@ -46,7 +46,7 @@ def test_batch_edges(gpu, p, mode):
             assert rel_l2(g, w) <= 1e-12
 
 
-@pytest.mark.parametrize("p", [2, 4, 5])
+@pytest.mark.parametrize("p", [2, 4, 5, 7, 8])
 def test_fp32_storage_at_a_batch_edge(gpu, p):
     prob = m.box_problem(EPB[p] + 1, p, ny=2, nz=1, jitter=0.05)
     f, t = prob.fp32(), prob.tables
