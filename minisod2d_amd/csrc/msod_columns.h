@@ -145,11 +145,21 @@ __device__ __forceinline__ GeoNode<T> col_geo(const T *geo, uint32_t b, int K, i
     return g;
 }
 
+// Colour of the element e of a batch, within it (coloured mode).
+template <bool COLORED>
+__device__ __forceinline__ int col_color(const Plan &pl, bool active, int64_t e)
+{
+    return COLORED && active ? pl.ecol[e] : 0;
+}
+
 // Adds one slice's five residual values to the batch's node sums sR[c*US + li].
-// Atomic mode: LDS atomics.  Coloured mode: one element after the other, so
-// that the order of the sums is fixed (barriers: uniform control flow).
-template <int P, bool COLORED>
-__device__ __forceinline__ void col_add(double *sR, int US, bool active, int le, uint32_t li, const double (&v)[5])
+// Atomic mode: LDS atomics.  Coloured mode: one colour of the batch's elements
+// (ec, Plan::ecol) after the other, so that the order of the sums is fixed
+// (barriers: uniform control flow).  A row of elements has two colours; one
+// element after the other, ten rounds a slice at order 4, made the coloured pair
+// 15% slower than one node per thread.
+template <bool COLORED>
+__device__ __forceinline__ void col_add(double *sR, int US, bool active, int ec, int rounds, uint32_t li, const double (&v)[5])
 {
     if constexpr (!COLORED) {
         if (active) {
@@ -159,8 +169,8 @@ __device__ __forceinline__ void col_add(double *sR, int US, bool active, int le,
         }
     } else {
 #pragma unroll 1
-        for (int k = 0; k < ColShape<P>::EPB; ++k) {
-            if (active && le == k) {
+        for (int k = 0; k < rounds; ++k) {
+            if (active && ec == k) {
 #pragma unroll
                 for (int c = 0; c < 5; ++c) sR[c * US + li] += v[c];
             }

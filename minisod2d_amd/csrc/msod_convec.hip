@@ -95,6 +95,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
     const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
+    const int ec = col_color<COLORED>(pl, active, (int64_t)b * EPB + le);
     // FP32 state with FP64 outputs comes without a pressure array
     constexpr bool kRecover = sizeof(typename A::F) == 4 && sizeof(typename A::Pt) == 4 && sizeof(typename A::O) == 8;
 
@@ -197,7 +198,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
         sum.finish(dz);
         double v[5];
         sum.values((T)gk.gvol(), ra, Ha, u[k], q[k], v);
-        col_add<P, COLORED>(sR, US, active, le, li, v);
+        col_add<COLORED>(sR, US, active, ec, pl.rounds, li, v);
         __builtin_amdgcn_sched_barrier(0);
     }
     __syncthreads();  // every node sum of the batch done
@@ -237,6 +238,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
     const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
+    const int ec = col_color<COLORED>(pl, active, (int64_t)b * EPB + le);
     constexpr bool kRecover = sizeof(typename A::F) == 4 && sizeof(typename A::Pt) == 4 && sizeof(typename A::O) == 8;
 
     T r[Q], p[Q], H[Q], u[Q][3], q[Q][3];
@@ -372,7 +374,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
         }
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (COLORED)
-            col_add<P, true>(sR, US, active, le, here, v);
+            col_add<true>(sR, US, active, ec, pl.rounds, here, v);
         else if (col_merge<P>(here, I, le, active && (int64_t)b * EPB + le + 1 < a.nelem, v) && active)
             col_scatter(here, v, a.Rmass, a.Rmom, a.Rener, np);
         __builtin_amdgcn_sched_barrier(0);

@@ -59,6 +59,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
     const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
     const int64_t e0 = (int64_t)b * EPB;
     const bool active = t < LANES && e0 + le < a.nelem;
+    const int ec = col_color<COLORED>(pl, active, e0 + le);
 
     uint32_t gn[Q];
 #pragma unroll
@@ -279,7 +280,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
     for (int k = 0; k < Q; ++k) {
         const double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                              (double)(W[k][1] + kappa[k] * W[k][2])};
-        col_add<P, COLORED>(sR, US, active, le, li[k], v);
+        col_add<COLORED>(sR, US, active, ec, pl.rounds, li[k], v);
     }
     __syncthreads();  // every node sum of the batch done
     col_write<P, COLORED>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
@@ -326,6 +327,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const int64_t e0 = (int64_t)b * EPB;
     const bool active = t < LANES && e0 + le < a.nelem;
+    const int ec = col_color<COLORED>(pl, active, e0 + le);
     const uint32_t *conn = pl.conn + (int64_t)b * Q * LANES + tc;
 
     // mu_e and mu_sgs change lanes in LDS (k_diffu_col)
@@ -538,7 +540,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
         double v[5] = {(double)(c.x * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + c.y * W[k][2])};
         if constexpr (COLORED)
-            col_add<P, true>(sR, US, active, le, at[k], v);
+            col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
         else if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
     }
@@ -590,6 +592,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     const uint32_t b = pl.batches ? uniform(pl.batches)[bs] : bs;
     const int64_t e0 = (int64_t)b * EPB + part * E2;
     const bool active = e0 + le < a.nelem;
+    const int ec = col_color<COLORED>(pl, active, e0 + le);
     const int tc = I + Q * ((int)part * E2 + le + EPB * J), k0 = half * H;
     const uint32_t *conn = pl.conn + ((int64_t)b * Q + k0) * LANES + tc;
     // line_ref of slice j of half h (j a compile-time constant)
@@ -839,7 +842,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
         double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + kappa[k] * W[k][2])};
         if constexpr (COLORED)
-            col_add<P, true>(sR, US, active, le, at[k], v);
+            col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
         else if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
     }

@@ -65,6 +65,8 @@ struct Plan {
     int64_t nb;
     int mode;
     int ustride;  // stride of the node sums: the most nodes of any batch
+    const uint8_t *ecol;  // coloured mode: colour of each element within its batch
+    int rounds;           // and the most colours of any batch
 };
 
 // Kernel arguments.  Storage types: TG for the element-sized arrays (geo;
@@ -148,9 +150,6 @@ hipError_t launch_zero_nodes(TO *Rmass, TO *Rmom, TO *Rener, int64_t npoin, cons
 template <typename T>
 hipError_t launch_build_geo(int porder, const T *He, const T *gpvol, int64_t nelem, const int32_t *l2g, T *geo,
                             hipStream_t s);
-// conn and lidx of the lane layout from element-major ones.
-hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *lidx, int64_t nelem, uint32_t *lconn,
-                             uint16_t *llidx, hipStream_t s);
 // Elements that geo, conn and lidx hold: nelem, padded to whole batches.
 int64_t geo_elems(int porder, int64_t nelem);
 

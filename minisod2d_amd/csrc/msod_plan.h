@@ -13,6 +13,8 @@
 //     alone (colored = false);
 //   * bit 31 of unode marks the first writer of a node: the batch of the
 //     lowest colour holding it;
+//   * a greedy colouring of each batch's elements (ecol), so that the elements
+//     of one colour can add to the batch's node sums together;
 //   * the batches grouped by colour (order, color_off) and the nodes no
 //     element references (unref).
 // Header-only so that a CPU check can compile it on its own.
@@ -37,6 +39,8 @@ struct HostPlan {
     std::vector<uint32_t> order;      // [nbatch]
     std::vector<int64_t> color_off;   // [ncolors+1]
     std::vector<uint32_t> unref;
+    std::vector<uint8_t> ecol;        // [nelem] colour within the batch: elements of one share no node
+    int rounds = 1;                   // most colours of any batch
     bool colored = false;             // colouring built (order, color_off, bit 31 valid)
 };
 
@@ -69,7 +73,7 @@ inline bool build_host_plan(const int32_t *raw, int64_t nelem, int64_t npoin,
         *err = "mesh too large for 32-bit node indices";
         return false;
     }
-    if (B < 1 || (int64_t)B * nn > 65536) {
+    if (B < 1 || B > 64 || (int64_t)B * nn > 65536) {
         *err = "batch too large for 16-bit node positions";
         return false;
     }
@@ -135,6 +139,28 @@ inline bool build_host_plan(const int32_t *raw, int64_t nelem, int64_t npoin,
         *err = "inconsistent batch node lists";
         return false;
     }
+
+    P.ecol.assign(nelem, 0);
+    std::atomic<int> rounds{1};
+    plan_parallel_for(NB, [&](int64_t lo, int64_t hi) {
+        std::vector<uint64_t> used;
+        int most = 1;
+        for (int64_t b = lo; b < hi; ++b) {
+            const int64_t e0 = b * B, e1 = std::min<int64_t>(nelem, e0 + B);
+            used.assign(P.uoff[b + 1] - P.uoff[b], 0u);
+            for (int64_t e = e0; e < e1; ++e) {
+                uint64_t forb = 0;
+                for (int l = 0; l < nn; ++l) forb |= used[P.lidx[e * nn + l]];
+                const int c = __builtin_ctzll(~forb);  // free: a batch has at most 64 elements
+                P.ecol[e] = (uint8_t)c;
+                most = std::max(most, c + 1);
+                for (int l = 0; l < nn; ++l) used[P.lidx[e * nn + l]] |= uint64_t(1) << c;
+            }
+        }
+        int cur = rounds.load();
+        while (cur < most && !rounds.compare_exchange_weak(cur, most)) {}
+    });
+    P.rounds = rounds.load();
 
     // greedy colouring: bit c of mask[node] is set once a batch of colour c
     // holds the node.  Past 32 colours the colouring is abandoned: the

@@ -155,27 +155,12 @@ __global__ void k_build_geo(const T *He, const T *gpvol, int64_t nelem, int64_t 
     }
 }
 
-template <int P>
-__global__ void k_plan_lanes(const uint32_t *conn, const uint16_t *lidx, int64_t nelem, int64_t total, uint32_t *lconn,
-                             uint16_t *llidx)
-{
-    constexpr int NN = (P + 1) * (P + 1) * (P + 1);
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
-        const int64_t e = i / NN, ec = e < nelem ? e : nelem - 1;
-        const int l = (int)(i - e * NN);
-        const ElemEntry<P> en{e, l};
-        lconn[en.entry()] = conn[ec * NN + l];
-        llidx[en.entry()] = lidx[ec * NN + l];
-    }
-}
-
 // The batches' node lists from the connectivity, one workgroup per batch: its
 // nodes are sorted in LDS (bitonic) and the distinct ones numbered in
 // ascending order, as build_host_plan does on the host.  FILL = false:
 // count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
 // unode from uoff, conn and lidx in the lane layout.  Above kNarrowP the atomic
-// kernels read conn alone: no lists (count[b] = 0, the rest null).
+// kernels read conn alone: lists = false (count[b] = 0, the rest null).
 // A first convection at 64^3, p=4 takes 7 ms in all (193 with the host plan).
 constexpr uint32_t kBadBatch = 0x80000000u;
 template <int P>
@@ -183,13 +168,12 @@ struct PlanShape {
     static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
     static constexpr int UMAX = ColShape<P>::UMAX;
     static constexpr int NT = 256;
-    static constexpr bool LISTS = P <= kNarrowP;
     static constexpr int SORT = UMAX <= 512 ? 512 : (UMAX <= 1024 ? 1024 : (UMAX <= 2048 ? 2048 : 4096));
     static constexpr int PER = SORT / NT;
 };
 template <int P, bool FILL>
 __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                                                      const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
+                                                      bool lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
                                                       uint32_t *unode, uint32_t *conn, uint16_t *lidx)
 {
     using S = PlanShape<P>;
@@ -220,7 +204,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     }
     if (bad) atomicAdd(&sbad, bad);
     __syncthreads();
-    if constexpr (!S::LISTS) {
+    if (!lists) {
         if constexpr (!FILL) {
             if (t == 0) count[b] = sbad ? kBadBatch + sbad : 0u;
         } else {
@@ -405,31 +389,19 @@ template hipError_t launch_build_geo<double>(int, const double *, const double *
 template hipError_t launch_build_geo<float>(int, const float *, const float *, int64_t, const int32_t *, float *,
                                             hipStream_t);
 
-hipError_t launch_plan_lanes(int porder, const uint32_t *conn, const uint16_t *lidx, int64_t nelem, uint32_t *lconn,
-                             uint16_t *llidx, hipStream_t s)
-{
-    return with_porder(porder, [&](auto p) {
-        constexpr int NN = (p() + 1) * (p() + 1) * (p() + 1);
-        const int64_t total = geo_elems(p(), nelem) * NN;
-        hipLaunchKernelGGL((k_plan_lanes<p()>), dim3(grid_for(total, 256)), dim3(256), 0, s, conn, lidx, nelem, total,
-                           lconn, llidx);
-        return hipGetLastError();
-    });
-}
-
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
 hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                               const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
+                               bool lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
                                uint32_t *conn, uint16_t *lidx, hipStream_t s)
 {
     return with_porder(porder, [&](auto p) {
         if (B > PlanShape<p()>::UMAX / PlanShape<p()>::NN) return hipErrorInvalidValue;
         const dim3 grid((unsigned)((nelem + B - 1) / B)), block(PlanShape<p()>::NT);
         if (fill)
-            hipLaunchKernelGGL((k_plan_batches<p(), true>), grid, block, 0, s, connec, nelem, npoin, B, l2g, uoff, count,
+            hipLaunchKernelGGL((k_plan_batches<p(), true>), grid, block, 0, s, connec, nelem, npoin, B, lists, l2g, uoff, count,
                                unode, conn, lidx);
         else
-            hipLaunchKernelGGL((k_plan_batches<p(), false>), grid, block, 0, s, connec, nelem, npoin, B, l2g, uoff,
+            hipLaunchKernelGGL((k_plan_batches<p(), false>), grid, block, 0, s, connec, nelem, npoin, B, lists, l2g, uoff,
                                count, unode, conn, lidx);
         return hipGetLastError();
     });
@@ -476,18 +448,21 @@ struct PlanEntry {
     int ustride = 0;  // most distinct nodes of any batch
     uint32_t *conn = nullptr, *uoff = nullptr, *unode = nullptr, *order = nullptr;
     uint16_t *lidx = nullptr;
+    uint8_t *ecol = nullptr;
+    int rounds = 1;
     std::vector<int64_t> color_off;  // batches of colour c: order[color_off[c] .. color_off[c+1])
     uint32_t *unref = nullptr;       // nodes no element references (zeroed per call)
     int64_t nunref = 0;
-    bool host = false;               // built on the host: colours, first writers and unref are there
+    bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
     void release()
     {
         for (void *p : {(void *)conn, (void *)uoff, (void *)unode, (void *)order, (void *)lidx,
-                        (void *)unref})
+                        (void *)unref, (void *)ecol})
             if (p) (void)hipFree(p);
         conn = uoff = unode = order = unref = nullptr;
         lidx = nullptr;
+        ecol = nullptr;
     }
 };
 
@@ -783,7 +758,8 @@ int upload(const std::vector<V> &h, V **d, const char *what)
 
 // Builds the node lists of a mesh's batches on the device: all that the atomic
 // assembly reads of the plan.
-int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
+int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, bool lists,
+                      PlanEntry &P)
 {
     const int64_t nn = (int64_t)ts->l2g.size(), nb = (nelem + B - 1) / B;
     if (npoin > 0x7fffffff || nelem * nn > 0xffffffffLL)
@@ -794,7 +770,7 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
     // feeds the host plan waits for
     HIPCHK(hipStreamSynchronize(nullptr), "plan");
     HIPCHK(hipMalloc((void **)&P.uoff, sizeof(uint32_t) * (nb + 1)), "plan");
-    HIPCHK(launch_plan_batches(ts->porder, false, dconnec, nelem, npoin, B, ts->dl2g, nullptr, P.uoff, nullptr, nullptr,
+    HIPCHK(launch_plan_batches(ts->porder, false, dconnec, nelem, npoin, B, lists, ts->dl2g, nullptr, P.uoff, nullptr, nullptr,
                                nullptr, g.stream),
            "batch counts");
     std::vector<uint32_t> uoff(nb + 1);
@@ -815,22 +791,22 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
                     (long long)npoin);
     const int64_t n = geo_elems(ts->porder, nelem) * nn;
     HIPCHK(hipMalloc((void **)&P.conn, sizeof(uint32_t) * n), "plan");
-    if (ts->porder <= kNarrowP) {
+    if (lists) {
         HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
         HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * uoff[nb]), "plan");
     }
     HIPCHK(hipMemcpyAsync(P.uoff, uoff.data(), sizeof(uint32_t) * (nb + 1), hipMemcpyHostToDevice, g.stream), "plan");
-    HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
+    HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, lists, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
                                P.lidx, g.stream),
            "batch lists");
     HIPCHK(hipStreamSynchronize(g.stream), "batch lists");
     return MSOD_OK;
 }
 
-// Builds the whole plan of a mesh (msod_plan.h), with the colouring, on the
-// host from its connectivity, a device array in the reference layout, and
-// uploads it.
-int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
+// Adds to the device's lists what the coloured assembly needs (msod_plan.h):
+// the colourings, the first writers and the unreferenced nodes, found on the
+// host from the connectivity.
+int build_host_part(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
 {
     const int64_t E = nelem * (int64_t)ts->l2g.size();
     std::vector<int32_t> raw(E);
@@ -840,33 +816,14 @@ int build_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet
     std::string err;
     if (!build_host_plan(raw.data(), nelem, npoin, ts->l2g, B, H, &err))
         return fail(MSOD_ERR_MESH, "%s", err.c_str());
-    std::vector<int32_t>().swap(raw);
-    P.B = H.B;
-    P.nbatch = H.nbatch;
     P.color_off = H.color_off;
     P.colored = H.colored;
-    for (int64_t k = 0; k < H.nbatch; ++k) P.ustride = std::max(P.ustride, (int)(H.uoff[k + 1] - H.uoff[k]));
+    P.rounds = H.rounds;
+    HIPCHK(hipMemcpy(P.unode, H.unode.data(), sizeof(uint32_t) * H.unode.size(), hipMemcpyHostToDevice), "plan upload");
     int st;
-    if ((st = upload(H.conn, &P.conn, "plan upload"))) return st;
-    if ((st = upload(H.lidx, &P.lidx, "plan upload"))) return st;
-    {  // element-major to the lane layout
-        const int64_t n = geo_elems(ts->porder, nelem) * (int64_t)ts->l2g.size();
-        uint32_t *conn = P.conn;
-        uint16_t *lidx = P.lidx;
-        P.conn = nullptr;
-        P.lidx = nullptr;
-        hipError_t e = hipMalloc((void **)&P.conn, sizeof(uint32_t) * n);
-        if (e == hipSuccess) e = hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n);
-        if (e == hipSuccess) e = launch_plan_lanes(ts->porder, conn, lidx, nelem, P.conn, P.lidx, g.stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
-        (void)hipFree(conn);
-        (void)hipFree(lidx);
-        if (e != hipSuccess) return hipfail(e, "plan layout");
-    }
-    if ((st = upload(H.uoff, &P.uoff, "plan upload"))) return st;
-    if ((st = upload(H.unode, &P.unode, "plan upload"))) return st;
     if ((st = upload(H.order, &P.order, "plan upload"))) return st;
     if ((st = upload(H.unref, &P.unref, "plan upload"))) return st;
+    if ((st = upload(H.ecol, &P.ecol, "plan upload"))) return st;
     P.nunref = (int64_t)H.unref.size();
     P.host = true;
     return MSOD_OK;
@@ -919,8 +876,8 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
     P.npoin = npoin;
     P.porder = ts->porder;
     P.l2g = ts->l2g;
-    int st = host ? build_plan(dconnec, nelem, npoin, ts, B, P)
-                  : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, P);
+    int st = build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, host || ts->porder <= kNarrowP, P);
+    if (!st && host) st = build_host_part(dconnec, nelem, npoin, ts, B, P);
     if (st) {
         P.release();
         return st;
@@ -1090,6 +1047,8 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     pl.uoff = P.uoff;
     pl.unode = P.unode;
     pl.ustride = P.ustride;
+    pl.ecol = P.ecol;
+    pl.rounds = P.rounds;
     pl.mode = g.assembly;
     const int64_t NP = a.npoin;
     if (g.assembly == kColored && !P.colored)
