@@ -7,17 +7,19 @@
 // the thread's registers; those along I and J read the slice's values from
 // LDS (2Q sources instead of 3Q).  Everything is unrolled over K, so a
 // source costs its FP64 work and its LDS reads with immediate offsets, and no
-// address arithmetic.
+// address arithmetic.  Up to kNarrowP the batch's node sums are in LDS too; the
+// kernels above it add to the outputs from registers (msod_convec.hip,
+// msod_diffu.hip).
 //
 // Against one node per thread (all three directions from LDS, rolled loops)
 // the FP64 kernels issue a quarter to a third fewer VALU instructions and
 // two thirds (convection) or half (diffusion) of the LDS reads per element
-// node: 128^3 order 4 12.6 -> 10.3 ms (convection) and 12.9 -> 10.3 ms
-// (diffusion); 64^3 1.61 -> 1.33 and 1.77 -> 1.50; order 3, 96^3 2.32 -> 2.03 and
-// 2.42 -> 2.19; order 2, 100^3 1.17 -> 0.83 and 0.99 -> 0.99; order 5, 40^3 0.88 -> 0.64
-// and 0.79 -> 0.76.  What bounds them now: two waves per SIMD (220-256
-// VGPRs), whose FP64 work and LDS reads alone take 7.1 ms (convection, 128^3),
-// then the gathers (2.1 ms more) and the atomics (2.8 ms).
+// node: 128^3 order 4 12.6 -> 10.3 ms (convection) and 12.9 -> 10.7 ms
+// (diffusion); 64^3 1.61 -> 1.33 and 1.77 -> 1.47; order 3, 96^3 2.32 -> 2.01 and
+// 2.42 -> 2.18; order 2, 100^3 1.17 -> 0.83 and 0.99 -> 0.97.  What bounds them now:
+// their traffic at the rate of a large copy (45 GB, 10.4 ms at 128^3), and two
+// waves per SIMD (208-230 VGPRs), whose FP64 work and LDS reads alone take 7.1 ms
+// (convection, 128^3).
 //
 // The launch takes the batches in mesh order, one workgroup each: neighbouring
 // batches run side by side and share lines in L2 (order 4, 128^3 convection:

@@ -18,7 +18,7 @@
 // 1e-16 level.
 //
 // Storage types TG (geometry) and TF (nodal fields), FP64 arithmetic
-// (msod_kernels.h), or TA = float for the FP32-arithmetic form.  Without a
+// (msod_kernels.h); the FP32-arithmetic form is msod_convec_fp32.hip.  Without a
 // pressure array the pressure is recovered as p = (gamma-1)(E - rho|u|^2/2)
 // from the stored state.
 #include "msod_columns.h"
@@ -423,11 +423,6 @@ template <class A>
 hipError_t launch_convec(int porder, const A &a, hipStream_t s)
 {
     return launch_order<A, double>(porder, a, s);
-}
-
-hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s)
-{
-    return launch_order<ConvecArgs<float, float>, float>(porder, a, s);
 }
 
 template hipError_t launch_convec(int, const ConvecArgs<double, double> &, hipStream_t);

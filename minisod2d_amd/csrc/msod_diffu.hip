@@ -18,7 +18,8 @@
 // step 2 publishes one component per direction.
 //
 // Storage types TG (geometry, mu_e, mu_sgs) and TF (nodal fields), FP64
-// arithmetic (msod_kernels.h) or TA = float.  CLOSURE (FP64 storage): mu_sgs is not read but predicted by the learned
+// arithmetic (msod_kernels.h); the FP32-arithmetic form is msod_diffu_fp32.hip.
+// CLOSURE (FP64 storage): mu_sgs is not read but predicted by the learned
 // closure (msod_mlp.h) from the velocity gradient before the stress is
 // formed; its per-wave LDS scratch is the wave's own part of the flux buffer,
 // free between the slice's first barrier and the fluxes.
@@ -902,11 +903,6 @@ template <class A>
 hipError_t launch_diffu(int porder, const A &a, hipStream_t s)
 {
     return launch_order<A, false, double>(porder, a, nullptr, s);
-}
-
-hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
-{
-    return launch_order<DiffuArgs<float, float>, false, float>(porder, a, nullptr, s);
 }
 
 hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp, hipStream_t s)

@@ -50,6 +50,9 @@ enum AssemblyMode { kColored = 0, kAtomic = 1 };
 
 // Elements per batch: ColShape<P>::EPB for run-time porder.
 int batch_size(int porder);
+// Those of the FP32-arithmetic kernels: Shape<P>::BATCH and CShape<P>::BATCH.
+int nodes_batch_size(int porder);
+int nodes_convec_batch_size(int porder);
 
 struct Tables {
     const double *D;      // [q*q]
@@ -67,6 +70,7 @@ struct Plan {
     int ustride;  // stride of the node sums: the most nodes of any batch
     const uint8_t *ecol;  // coloured mode: colour of each element within its batch
     int rounds;           // and the most colours of any batch
+    int kpb;              // FP32 arithmetic (msod_nodes.h): batches per workgroup
 };
 
 // Kernel arguments.  Storage types: TG for the element-sized arrays (geo;

@@ -9,6 +9,7 @@
 #include <rocprofiler-sdk-roctx/roctx.h>
 
 #include "msod_columns.h"
+#include "msod_nodes.h"
 #include "msod_mlp.h"
 #include "msod_plan.h"
 #include "msod_tet.h"
@@ -160,6 +161,30 @@ __global__ void __launch_bounds__(ColShape<P>::NT) k_build_geo(const T *He, cons
 #pragma unroll
         for (int k = 0; k < 5; ++k)
             __builtin_nontemporal_store(GeoPair<T>{v[2 * k], v[2 * k + 1]}, &dst[(K * 5 + k) * S::LANES]);
+    }
+}
+
+// geo of the FP32-arithmetic kernels, element-major (msod_nodes.h).
+__global__ void k_build_geo_nodes(const float *He, const float *gpvol, int64_t nelem, int nn, const int32_t *l2g,
+                                  float *geo)
+{
+    const int64_t total = nelem * nn;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += stride) {
+        const int64_t e = i / nn;
+        const int l = (int)(i - e * nn);
+        const int64_t a = l2g[l];
+        const float *src = He + 9 * (a + (int64_t)nn * e);
+        float v[10];
+#pragma unroll
+        for (int c = 0; c < 9; ++c) v[c] = src[c];
+        v[9] = gpvol[a + (int64_t)nn * e];
+        float *dst = geo + 2 * (e * 5 * nn + l);
+#pragma unroll
+        for (int k = 0; k < 5; ++k) {
+            dst[2 * k * nn] = v[2 * k];
+            dst[2 * k * nn + 1] = v[2 * k + 1];
+        }
     }
 }
 
@@ -374,6 +399,16 @@ int batch_size(int porder)
     return with_porder(porder, [](auto p) { return (int)ColShape<p()>::EPB; });
 }
 
+int nodes_batch_size(int porder)
+{
+    return with_porder(porder, [](auto p) { return (int)Shape<p()>::BATCH; });
+}
+
+int nodes_convec_batch_size(int porder)
+{
+    return with_porder(porder, [](auto p) { return (int)CShape<p()>::BATCH; });
+}
+
 int64_t geo_elems(int porder, int64_t nelem)
 {
     const int64_t B = batch_size(porder);
@@ -395,6 +430,13 @@ template hipError_t launch_build_geo<double>(int, const double *, const double *
                                              hipStream_t);
 template hipError_t launch_build_geo<float>(int, const float *, const float *, int64_t, const int32_t *, float *,
                                             hipStream_t);
+
+static hipError_t launch_build_geo_nodes(const float *He, const float *gpvol, int64_t nelem, int nn, const int32_t *l2g,
+                                         float *geo, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_build_geo_nodes, dim3(grid_for(nelem * nn, 256)), dim3(256), 0, s, He, gpvol, nelem, nn, l2g, geo);
+    return hipGetLastError();
+}
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
 hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
@@ -460,6 +502,7 @@ struct PlanEntry {
     std::vector<int64_t> color_off;  // batches of colour c: order[color_off[c] .. color_off[c+1])
     uint32_t *unref = nullptr;       // nodes no element references (zeroed per call)
     int64_t nunref = 0;
+    bool nodes = false;              // element-major, of the FP32-arithmetic kernels (msod_nodes.h)
     bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
     void release()
@@ -480,7 +523,8 @@ struct DerivedGeo {
     int porder;
     size_t elt;
     std::vector<int32_t> l2g;
-    void *geo;  // He and gpvol, element-major pairs (k_build_geo)
+    bool nodes;  // element-major (msod_nodes.h)
+    void *geo;   // He and gpvol as pairs (k_build_geo)
 };
 
 // A tetrahedral connectivity found valid (every entry in 1..npoin), with
@@ -836,6 +880,33 @@ int build_host_part(const void *dconnec, int64_t nelem, int64_t npoin, const Tab
     return MSOD_OK;
 }
 
+// The plan of the FP32-arithmetic kernels (msod_nodes.h), from the host.
+int build_nodes_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
+{
+    const int64_t E = nelem * (int64_t)ts->l2g.size();
+    std::vector<int32_t> raw(E);
+    HIPCHK(hipMemcpy(raw.data(), dconnec, sizeof(int32_t) * E, hipMemcpyDeviceToHost), "reading connec");
+    HostPlan H;
+    std::string err;
+    if (!build_host_plan(raw.data(), nelem, npoin, ts->l2g, B, H, &err))
+        return fail(MSOD_ERR_MESH, "%s", err.c_str());
+    std::vector<int32_t>().swap(raw);
+    P.B = H.B;
+    P.nbatch = H.nbatch;
+    P.color_off = H.color_off;
+    P.colored = H.colored;
+    int st;
+    if ((st = upload(H.conn, &P.conn, "plan upload"))) return st;
+    if ((st = upload(H.lidx, &P.lidx, "plan upload"))) return st;
+    if ((st = upload(H.uoff, &P.uoff, "plan upload"))) return st;
+    if ((st = upload(H.unode, &P.unode, "plan upload"))) return st;
+    if ((st = upload(H.order, &P.order, "plan upload"))) return st;
+    if ((st = upload(H.unref, &P.unref, "plan upload"))) return st;
+    P.nunref = (int64_t)H.unref.size();
+    P.host = P.nodes = true;
+    return MSOD_OK;
+}
+
 // Layouts derived from device memory outside the data region (version 0) are
 // not reused from call to call: the array may have changed since.
 void drop_unversioned(const void *src)
@@ -859,14 +930,14 @@ void drop_unversioned(const void *src)
 }
 
 int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, const TableSet *ts, int B,
-             const PlanEntry **out)
+             const PlanEntry **out, bool nodes = false)
 {
     if (ver == 0) drop_unversioned(dconnec);
     const bool host = g.assembly == kColored;  // the atomic assembly takes either plan
     for (size_t i = 0; i < g.plans.size(); ++i) {
         PlanEntry &c = g.plans[i];
         if (c.src != dconnec || c.ver != ver || c.nelem != nelem || c.npoin != npoin || c.porder != ts->porder ||
-            c.l2g != ts->l2g || c.B != B)
+            c.l2g != ts->l2g || c.B != B || c.nodes != nodes)
             continue;
         if (c.host || !host) {
             *out = &c;
@@ -883,8 +954,9 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
     P.npoin = npoin;
     P.porder = ts->porder;
     P.l2g = ts->l2g;
-    int st = build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, host || ts->porder <= kNarrowP, P);
-    if (!st && host) st = build_host_part(dconnec, nelem, npoin, ts, B, P);
+    int st = nodes ? build_nodes_plan(dconnec, nelem, npoin, ts, B, P)
+                   : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, host || ts->porder <= kNarrowP, P);
+    if (!st && host && !nodes) st = build_host_part(dconnec, nelem, npoin, ts, B, P);
     if (st) {
         P.release();
         return st;
@@ -900,25 +972,29 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
 
 template <typename T>
 int get_geo(const void *dHe, uint64_t vHe, const void *dVol, uint64_t vVol, int64_t nelem,
-            const TableSet *ts, const T **geo)
+            const TableSet *ts, const T **geo, bool nodes = false)
 {
     if (vHe == 0) drop_unversioned(dHe);
     if (vVol == 0) drop_unversioned(dVol);
     for (auto &c : g.geos)
         if (c.srcHe == dHe && c.srcVol == dVol && c.verHe == vHe && c.verVol == vVol &&
-            c.nelem == nelem && c.porder == ts->porder && c.elt == sizeof(T) && c.l2g == ts->l2g) {
+            c.nelem == nelem && c.porder == ts->porder && c.elt == sizeof(T) && c.l2g == ts->l2g && c.nodes == nodes) {
             *geo = (const T *)c.geo;
             return MSOD_OK;
         }
     const int nn = (int)ts->l2g.size();
-    DerivedGeo c{dHe, dVol, vHe, vVol, nelem, ts->porder, sizeof(T), ts->l2g, nullptr};
-    HIPCHK(hipMalloc(&c.geo, sizeof(T) * 10 * geo_elems(ts->porder, nelem) * nn),
-           "hipMalloc element-major He and gpvol");
-    hipError_t e = launch_build_geo<T>(ts->porder, (const T *)dHe, (const T *)dVol, nelem, ts->dl2g, (T *)c.geo, g.stream);
+    DerivedGeo c{dHe, dVol, vHe, vVol, nelem, ts->porder, sizeof(T), ts->l2g, nodes, nullptr};
+    HIPCHK(hipMalloc(&c.geo, sizeof(T) * 10 * (nodes ? nelem : geo_elems(ts->porder, nelem)) * nn),
+           "hipMalloc He and gpvol");
+    hipError_t e;
+    if (nodes)
+        e = launch_build_geo_nodes((const float *)dHe, (const float *)dVol, nelem, nn, ts->dl2g, (float *)c.geo, g.stream);
+    else
+        e = launch_build_geo<T>(ts->porder, (const T *)dHe, (const T *)dVol, nelem, ts->dl2g, (T *)c.geo, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
     if (e != hipSuccess) {
         (void)hipFree(c.geo);
-        return hipfail(e, "building element-major geometry");
+        return hipfail(e, "building the geometry layout");
     }
     if (g.geos.size() >= kMaxDerived) {
         (void)hipFree(g.geos.front().geo);
@@ -1044,9 +1120,12 @@ int check_sizes(int porder, int nelem, int npoin)
 
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
 // the kernel: one launch per colour, or one launch over all batches in mesh
-// order, where neighbouring batches meet in L2.
+// order, where neighbouring batches meet in L2.  FP32 arithmetic: kpb_max
+// batches a workgroup at most, fewer where that would leave the launch short of
+// 2048 workgroups, and the order of the colours unless natural (one node per
+// thread at 128^3, order 4: convection 12.8 ms, 13.3 in mesh order).
 template <class A, class L>
-int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what)
+int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *what, bool natural = true, int kpb_max = 1)
 {
     Plan pl;
     pl.conn = P.conn;
@@ -1056,6 +1135,9 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     pl.ustride = P.ustride;
     pl.ecol = P.ecol;
     pl.rounds = P.rounds;
+    auto kpb_for = [kpb_max](int64_t nb) {
+        return (int)std::max<int64_t>(1, std::min<int64_t>(kpb_max, nb / 2048));
+    };
     pl.mode = g.assembly;
     const int64_t NP = a.npoin;
     if (g.assembly == kColored && !P.colored)
@@ -1073,14 +1155,16 @@ int run_assembled(A &a, const PlanEntry &P, int timer, L launch, const char *wha
     }
     TimedLaunch tk(timer);
     if (g.assembly == kAtomic) {
-        pl.batches = nullptr;  // mesh order, no list
+        pl.batches = natural ? nullptr : P.order;  // null: mesh order, no list
         pl.nb = P.nbatch;
+        pl.kpb = kpb_for(pl.nb);
         a.plan = pl;
         HIPCHK(launch(a), what);
     } else {
         for (size_t c = 0; c + 1 < P.color_off.size(); ++c) {
             pl.batches = P.order + P.color_off[c];
             pl.nb = P.color_off[c + 1] - P.color_off[c];
+            pl.kpb = kpb_for(pl.nb);
             a.plan = pl;
             HIPCHK(launch(a), what);
         }
@@ -1120,8 +1204,9 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), &plan))) return st;
-    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
+    const int B = fp32_arith ? nodes_convec_batch_size(porder) : batch_size(porder);
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, fp32_arith))) return st;
+    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, fp32_arith))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
     a.nelem = NE;
@@ -1144,7 +1229,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
                                 return launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch")))
+                            "convection kernel launch", !fp32_arith, fp32_arith ? kBatchesPerBlock : 1)))
         return st;
     return finish_call("convection kernel");
 }
@@ -1180,8 +1265,9 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), &plan))) return st;
-    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
+    const int B = fp32_arith ? nodes_batch_size(porder) : batch_size(porder);
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, fp32_arith))) return st;
+    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, fp32_arith))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;
     a.nelem = NE;
