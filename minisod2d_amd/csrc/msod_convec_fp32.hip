@@ -292,19 +292,30 @@ static hipError_t launch_p(const A &a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s)
+template <class A, typename TA>
+static hipError_t launch_order(int porder, const A &a, hipStream_t s)
 {
     switch (porder) {
-    case 1: return launch_p<1, ConvecArgs<float, float>, float>(a, s);
-    case 2: return launch_p<2, ConvecArgs<float, float>, float>(a, s);
-    case 3: return launch_p<3, ConvecArgs<float, float>, float>(a, s);
-    case 4: return launch_p<4, ConvecArgs<float, float>, float>(a, s);
-    case 5: return launch_p<5, ConvecArgs<float, float>, float>(a, s);
-    case 6: return launch_p<6, ConvecArgs<float, float>, float>(a, s);
-    case 7: return launch_p<7, ConvecArgs<float, float>, float>(a, s);
-    case 8: return launch_p<8, ConvecArgs<float, float>, float>(a, s);
+    case 1: return launch_p<1, A, TA>(a, s);
+    case 2: return launch_p<2, A, TA>(a, s);
+    case 3: return launch_p<3, A, TA>(a, s);
+    case 4: return launch_p<4, A, TA>(a, s);
+    case 5: return launch_p<5, A, TA>(a, s);
+    case 6: return launch_p<6, A, TA>(a, s);
+    case 7: return launch_p<7, A, TA>(a, s);
+    case 8: return launch_p<8, A, TA>(a, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s)
+{
+    return launch_order<ConvecArgs<float, float>, float>(porder, a, s);
+}
+
+hipError_t launch_convec_nodes(int porder, const ConvecArgs<double, double> &a, hipStream_t s)
+{
+    return launch_order<ConvecArgs<double, double>, double>(porder, a, s);
 }
 
 }  // namespace msod

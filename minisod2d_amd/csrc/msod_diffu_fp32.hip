@@ -335,19 +335,30 @@ static hipError_t launch_p(const A &a, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
+template <class A, typename TA>
+static hipError_t launch_order(int porder, const A &a, hipStream_t s)
 {
     switch (porder) {
-    case 1: return launch_p<1, DiffuArgs<float, float>, float>(a, s);
-    case 2: return launch_p<2, DiffuArgs<float, float>, float>(a, s);
-    case 3: return launch_p<3, DiffuArgs<float, float>, float>(a, s);
-    case 4: return launch_p<4, DiffuArgs<float, float>, float>(a, s);
-    case 5: return launch_p<5, DiffuArgs<float, float>, float>(a, s);
-    case 6: return launch_p<6, DiffuArgs<float, float>, float>(a, s);
-    case 7: return launch_p<7, DiffuArgs<float, float>, float>(a, s);
-    case 8: return launch_p<8, DiffuArgs<float, float>, float>(a, s);
+    case 1: return launch_p<1, A, TA>(a, s);
+    case 2: return launch_p<2, A, TA>(a, s);
+    case 3: return launch_p<3, A, TA>(a, s);
+    case 4: return launch_p<4, A, TA>(a, s);
+    case 5: return launch_p<5, A, TA>(a, s);
+    case 6: return launch_p<6, A, TA>(a, s);
+    case 7: return launch_p<7, A, TA>(a, s);
+    case 8: return launch_p<8, A, TA>(a, s);
     default: return hipErrorInvalidValue;
     }
+}
+
+hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
+{
+    return launch_order<DiffuArgs<float, float>, float>(porder, a, s);
+}
+
+hipError_t launch_diffu_nodes(int porder, const DiffuArgs<double, double> &a, hipStream_t s)
+{
+    return launch_order<DiffuArgs<double, double>, double>(porder, a, s);
 }
 
 }  // namespace msod

@@ -1,5 +1,6 @@
 // One node per thread: batches, records and assembly of the FP32-arithmetic
-// kernels (msod_convec_fp32.hip, msod_diffu_fp32.hip).
+// kernels (msod_convec_fp32.hip, msod_diffu_fp32.hip), and of the FP64 form in the
+// coloured mode where its launches are short (nodes_for_colors).
 //
 // Their results are FP32 rounding, so another order of the FP32 operations is
 // another result (columns: 9e-7 off in relative L2, 48^3 p=7 3.14 -> 2.5 ms for

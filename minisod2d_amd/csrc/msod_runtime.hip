@@ -164,9 +164,9 @@ __global__ void __launch_bounds__(ColShape<P>::NT) k_build_geo(const T *He, cons
     }
 }
 
-// geo of the FP32-arithmetic kernels, element-major (msod_nodes.h).
-__global__ void k_build_geo_nodes(const float *He, const float *gpvol, int64_t nelem, int nn, const int32_t *l2g,
-                                  float *geo)
+// geo of the kernels with one node per thread, element-major (msod_nodes.h).
+template <typename T>
+__global__ void k_build_geo_nodes(const T *He, const T *gpvol, int64_t nelem, int nn, const int32_t *l2g, T *geo)
 {
     const int64_t total = nelem * nn;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -174,12 +174,12 @@ __global__ void k_build_geo_nodes(const float *He, const float *gpvol, int64_t n
         const int64_t e = i / nn;
         const int l = (int)(i - e * nn);
         const int64_t a = l2g[l];
-        const float *src = He + 9 * (a + (int64_t)nn * e);
-        float v[10];
+        const T *src = He + 9 * (a + (int64_t)nn * e);
+        T v[10];
 #pragma unroll
         for (int c = 0; c < 9; ++c) v[c] = src[c];
         v[9] = gpvol[a + (int64_t)nn * e];
-        float *dst = geo + 2 * (e * 5 * nn + l);
+        T *dst = geo + 2 * (e * 5 * nn + l);
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
             dst[2 * k * nn] = v[2 * k];
@@ -431,11 +431,27 @@ template hipError_t launch_build_geo<double>(int, const double *, const double *
 template hipError_t launch_build_geo<float>(int, const float *, const float *, int64_t, const int32_t *, float *,
                                             hipStream_t);
 
-static hipError_t launch_build_geo_nodes(const float *He, const float *gpvol, int64_t nelem, int nn, const int32_t *l2g,
-                                         float *geo, hipStream_t s)
+template <typename T>
+static hipError_t launch_build_geo_nodes(const T *He, const T *gpvol, int64_t nelem, int nn, const int32_t *l2g, T *geo,
+                                         hipStream_t s)
 {
-    hipLaunchKernelGGL(k_build_geo_nodes, dim3(grid_for(nelem * nn, 256)), dim3(256), 0, s, He, gpvol, nelem, nn, l2g, geo);
+    hipLaunchKernelGGL(k_build_geo_nodes<T>, dim3(grid_for(nelem * nn, 256)), dim3(256), 0, s, He, gpvol, nelem, nn, l2g,
+                       geo);
     return hipGetLastError();
+}
+
+// Coloured mode, FP64: whether one node per thread is the faster form.  Its
+// batches are smaller (4 elements against 10 at order 4): where a colour's column
+// batches are fewer than the CUs, its launches end sooner (6x6x8 order 4
+// convection 98 us against 145, 30^3 order 3 the pair 375 against 430; 40^3 order 4
+// 1329 against 1210).  Above kNarrowP a column batch's sums in LDS leave one or
+// two workgroups per CU (40^3 order 5 2.46 ms against 2.63, 48^3 order 7 9.94
+// against 10.4, 32^3 order 8 5.62 against 6.41), but for order 6 (40^3 4.96 against
+// 4.08).  A box has 8 colours.
+static bool nodes_for_colors(int porder, int64_t nelem)
+{
+    const bool few = nelem < (int64_t)256 * 8 * batch_size(porder);
+    return few || (porder > kNarrowP && porder != 6);
 }
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
@@ -988,7 +1004,7 @@ int get_geo(const void *dHe, uint64_t vHe, const void *dVol, uint64_t vVol, int6
            "hipMalloc He and gpvol");
     hipError_t e;
     if (nodes)
-        e = launch_build_geo_nodes((const float *)dHe, (const float *)dVol, nelem, nn, ts->dl2g, (float *)c.geo, g.stream);
+        e = launch_build_geo_nodes((const T *)dHe, (const T *)dVol, nelem, nn, ts->dl2g, (T *)c.geo, g.stream);
     else
         e = launch_build_geo<T>(ts->porder, (const T *)dHe, (const T *)dVol, nelem, ts->dl2g, (T *)c.geo, g.stream);
     if (e == hipSuccess) e = hipStreamSynchronize(g.stream);
@@ -1120,7 +1136,7 @@ int check_sizes(int porder, int nelem, int npoin)
 
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
 // the kernel: one launch per colour, or one launch over all batches in mesh
-// order, where neighbouring batches meet in L2.  FP32 arithmetic: kpb_max
+// order, where neighbouring batches meet in L2.  One node per thread: kpb_max
 // batches a workgroup at most, fewer where that would leave the launch short of
 // 2048 workgroups, and the order of the colours unless natural (one node per
 // thread at 128^3, order 4: convection 12.8 ms, 13.3 in mesh order).
@@ -1204,9 +1220,11 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    const int B = fp32_arith ? nodes_convec_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, fp32_arith))) return st;
-    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, fp32_arith))) return st;
+    constexpr bool kF64 = std::is_same<ConvecArgs<TG, TF, TO, TU, TP>, ConvecArgs<double, double>>::value;
+    const bool nodes = fp32_arith || (kF64 && g.assembly == kColored && nodes_for_colors(porder, NE));
+    const int B = nodes ? nodes_convec_batch_size(porder) : batch_size(porder);
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, nodes))) return st;
+    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
     a.nelem = NE;
@@ -1227,9 +1245,11 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                 if constexpr (std::is_same<ConvecArgs<TG, TF, TO, TU, TP>,
                                                            ConvecArgs<float, float>>::value)
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
+                                if constexpr (kF64)
+                                    if (nodes) return launch_convec_nodes(porder, x, g.stream);
                                 return launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch", !fp32_arith, fp32_arith ? kBatchesPerBlock : 1)))
+                            "convection kernel launch", !nodes, nodes ? kBatchesPerBlock : 1)))
         return st;
     return finish_call("convection kernel");
 }
@@ -1265,9 +1285,11 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    const int B = fp32_arith ? nodes_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, fp32_arith))) return st;
-    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, fp32_arith))) return st;
+    constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
+    const bool nodes = fp32_arith || (kF64 && !dmlp && g.assembly == kColored && nodes_for_colors(porder, NE));
+    const int B = nodes ? nodes_batch_size(porder) : batch_size(porder);
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, nodes))) return st;
+    if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;
     a.nelem = NE;
@@ -1290,8 +1312,10 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     if ((st = run_assembled(a, *plan, timer,
                             [&](const DiffuArgs<TG, TF, TO, TU> &x) {
                                 using AT = DiffuArgs<TG, TF, TO, TU>;
-                                if constexpr (std::is_same<AT, DiffuArgs<double, double>>::value)
+                                if constexpr (kF64) {
                                     if (dmlp) return launch_diffu_closure(porder, x, dmlp, g.stream);
+                                    if (nodes) return launch_diffu_nodes(porder, x, g.stream);
+                                }
                                 if constexpr (std::is_same<AT, DiffuArgs<float, float>>::value)
                                     if (fp32_arith) return launch_diffu_fp32(porder, x, g.stream);
                                 return launch_diffu(porder, x, g.stream);

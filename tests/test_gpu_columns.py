@@ -73,3 +73,28 @@ def test_fp32_storage_at_a_batch_edge(gpu, p):
                                                                       *D), ins)
         for g, w in zip(got, want):
             assert rel_l2(g, w) <= bar
+
+
+@pytest.mark.parametrize("p,n", [(2, 39), (3, 33), (4, 28), (6, 22)])
+def test_colored_batches_of_a_large_mesh(gpu, p, n):
+    """Enough batches a colour for the column kernels' coloured form (smaller
+    meshes run one node per thread there), against the atomic assembly."""
+    prob = m.box_problem(n, p, jitter=0.05)
+    print(f"[gpu] coloured columns p={p} nelem={prob.nelem}", flush=True)
+    R, D = prob.outputs(), prob.outputs()
+    ins = prob.device_inputs()
+    got = {}
+    m.copyin(*ins)
+    m.create(*R, *D)
+    try:
+        for mode in (m.ASSEMBLY_ATOMIC, m.ASSEMBLY_COLORED):
+            m.set_assembly(mode)
+            m.full_convec_ijk(*prob.convec_args(*R))
+            m.full_diffusion_ijk(*prob.diffu_args(*D))
+            m.update_host(*R, *D)
+            got[mode] = [x.copy() for x in R + D]
+    finally:
+        m.set_assembly(m.ASSEMBLY_DEFAULT)
+        m.delete(*ins, *R, *D)
+    for g, w in zip(got[m.ASSEMBLY_COLORED], got[m.ASSEMBLY_ATOMIC]):
+        assert rel_l2(g, w) <= 1e-12
