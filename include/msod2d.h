@@ -270,9 +270,10 @@ int msod_full_diffusion_ijk_f32split(int porder, int nelem, int npoin, const int
  * full_diffusion_ijk with the reference's full argument lists
  * (elem_convec.f90:198-211, elem_diffu.f90:10-23) in float, Cp and Pr
  * included, and float outputs.  The kernels compute in FP64 from the float
- * inputs and sum each batch's contributions to a node in FP64; each batch's
- * sum is rounded once to float and added with a float atomic (a node shared
- * by k batches takes k roundings), so the errors are the float storage of
+ * inputs and sum the contributions of a workgroup's elements (a batch; half
+ * a batch in the diffusion at porder 7) to a node in FP64; each such sum is
+ * rounded once to float and added with a float atomic (a node shared by k
+ * workgroups takes k roundings), so the errors are the float storage of
  * inputs and outputs and those few additions (the reference at rp = 4
  * rounds inside every product and sum). */
 int msod_full_convec_ijk_r4(int porder, int nelem, int npoin, const int32_t *connec, const float *Ngp,

@@ -219,6 +219,42 @@ __device__ __forceinline__ void col_scatter(uint32_t node, const double (&v)[5],
     unsafeAtomicAdd(Rener + g, (TO)v[4]);
 }
 
+// Orders above kNarrowP with FP32 outputs (atomic mode): a value rounded to float
+// at every element node, as col_scatter would, loses bits where elements of a
+// batch meet.  So nodes that several lanes hold after col_merge are summed in
+// LDS, sR[c*US + li], and each goes out rounded once; the others go out at once,
+// a row of elements whole (33^3 order 5 convection 271 us, 29^3 order 6 305; with
+// the merged nodes in LDS as well 349 and 388, rounded at every node 259 and 302).
+template <typename TO>
+__device__ __forceinline__ void col_add_shared(double *sR, int US, uint32_t li, uint32_t node, const double (&v)[5], TO *Rmass,
+                                               TO *Rmom, TO *Rener, int64_t npoin)
+{
+    if (li == kAlone) {
+        col_scatter(node, v, Rmass, Rmom, Rener, npoin);
+    } else {
+#pragma unroll
+        for (int c = 0; c < 5; ++c)
+            __hip_atomic_fetch_add(&sR[c * US + li], v[c], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+}
+// The shared nodes' sums to the outputs.  Sums of zero change nothing (where a
+// batch is split between workgroups, its list holds the other part's nodes too).
+template <typename TO>
+__device__ __forceinline__ void col_write_shared(const Plan &pl, uint32_t b, const double *sR, int NT, TO *Rmass, TO *Rmom,
+                                                 TO *Rener, int64_t npoin)
+{
+    const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
+    for (uint32_t i = threadIdx.x; i < U; i += NT) {
+        const int64_t g = pl.unode[u0 + i];
+        TO *dst[5] = {Rmass + g, Rmom + g, Rmom + npoin + g, Rmom + 2 * npoin + g, Rener + g};
+#pragma unroll
+        for (int c = 0; c < 5; ++c) {
+            const double v = sR[c * pl.ustride + i];
+            if (v != 0.0) unsafeAtomicAdd(dst[c], (TO)v);
+        }
+    }
+}
+
 // A thread's entries t, t + NT, ... of a batch's node list.
 template <int P>
 __device__ __forceinline__ void col_list(const uint32_t *unode, uint32_t U, uint32_t (&wn)[ColShape<P>::UPT])

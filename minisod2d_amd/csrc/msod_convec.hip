@@ -223,11 +223,12 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
     using T = TA;
     using TG = typename A::G;
     constexpr int Q = S::Q, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
+    constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
     __shared__ V2 sP[4][NT];  // one slice: (r,p) (u0,u1) (u2,q0) (q1,q2)
     __shared__ T sH[NT];      // and H
-    extern __shared__ __attribute__((aligned(16))) double sR[];  // coloured mode: node sums [5][US]
+    extern __shared__ __attribute__((aligned(16))) double sR[];  // coloured mode, FP32 outputs: node sums [5][US]
 
     const Plan &pl = a.plan;
     const int US = pl.ustride, t = threadIdx.x;
@@ -264,7 +265,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
         }
         geo = col_geo<P, true>(a.geo, b, 0, tc);
         col_table<P>(a.tab.D, sD);
-        if constexpr (COLORED)
+        if constexpr (COLORED || SHARED)
             for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
 #pragma unroll
         for (int k = 0; k < Q; ++k) {
@@ -287,7 +288,8 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
     }
     // the next slice's place in the outputs: its node, or (coloured) its
     // position in the batch's list
-    uint32_t at = COLORED ? pl.lidx[(int64_t)b * Q * LANES + tc] : pl.conn[(int64_t)b * Q * LANES + tc];
+    uint32_t at = COLORED ? pl.lidx[(int64_t)b * Q * LANES + tc] : pl.conn[(int64_t)b * Q * LANES + tc], li = 0;
+    if constexpr (SHARED) li = pl.lidx[(int64_t)b * Q * LANES + tc];
     const int sI = tc - I, sJ = tc - J * EPB * Q;
     col_slices<Q>([&](auto kc) __attribute__((always_inline)) {
         constexpr int k = kc();
@@ -367,15 +369,19 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
         next_geo(2);
         double v[5];
         sum.values(gv, ra, Ha, u[k], q[k], v);
-        const uint32_t here = at;
+        const uint32_t here = at, li_here = li;
         if (k + 1 < Q) {
             const int64_t i = ((int64_t)b * Q + k + 1) * LANES + tc;
             at = COLORED ? pl.lidx[i] : pl.conn[i];
+            if constexpr (SHARED) li = pl.lidx[i];
         }
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (COLORED)
+        if constexpr (COLORED) {
             col_add<true>(sR, US, active, ec, pl.rounds, here, v);
-        else if (col_merge<P>(here, I, le, active && (int64_t)b * EPB + le + 1 < a.nelem, v) && active)
+        } else if constexpr (SHARED) {
+            if (col_merge<P>(here, I, le, active && (int64_t)b * EPB + le + 1 < a.nelem, v) && active)
+                col_add_shared(sR, US, li_here, here, v, a.Rmass, a.Rmom, a.Rener, np);
+        } else if (col_merge<P>(here, I, le, active && (int64_t)b * EPB + le + 1 < a.nelem, v) && active)
             col_scatter(here, v, a.Rmass, a.Rmom, a.Rener, np);
         __builtin_amdgcn_sched_barrier(0);
     });
@@ -386,6 +392,10 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
         __syncthreads();
         col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
     }
+    if constexpr (SHARED) {
+        __syncthreads();
+        col_write_shared(pl, b, sR, NT, a.Rmass, a.Rmom, a.Rener, np);
+    }
 }
 
 template <int P, class A, typename TA>
@@ -393,7 +403,8 @@ static hipError_t launch_p(const A &a, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
     const bool atomic = a.plan.mode == kAtomic;
-    const size_t sums = P > kNarrowP && atomic ? 0 : sizeof(double) * 5 * a.plan.ustride;
+    const bool registers = P > kNarrowP && atomic && sizeof(typename A::O) == 8;
+    const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride;
     if constexpr (P > kNarrowP)
         hipLaunchKernelGGL((atomic ? k_convec_wide<P, false, A, TA> : k_convec_wide<P, true, A, TA>),
                            dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);

@@ -306,6 +306,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     using TG = typename A::G;
     constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
     constexpr bool AHEAD = kWideWaves<P, TA> == 1;  // read line sources one ahead of their use
+    constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
     __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
@@ -313,8 +314,8 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
     __shared__ V2 sN[Q][NT];                               // nu, kappa of the thread's nodes
     __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
-    // its fluxes along I (0..2) and J (3..5); in the coloured mode, at the end,
-    // the node sums [5][US]
+    // its fluxes along I (0..2) and J (3..5); in the coloured mode and
+    // with FP32 outputs, at the end, the node sums [5][US]
     extern __shared__ __attribute__((aligned(16))) double sR[];
     V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
 
@@ -526,23 +527,28 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
             if (AHEAD) fc = fn;
         }
     });
-    if constexpr (COLORED) {
+    if constexpr (COLORED || SHARED) {
         __syncthreads();  // the last slice's fluxes are read
         for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
         __syncthreads();
     }
-    uint32_t at[Q];
+    uint32_t at[Q], li[Q];
 #pragma unroll
-    for (int k = 0; k < Q; ++k)
+    for (int k = 0; k < Q; ++k) {
         at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k) * LANES + tc] : conn[k * LANES];
+        li[k] = SHARED ? (uint32_t)pl.lidx[((int64_t)b * Q + k) * LANES + tc] : 0u;
+    }
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
         const V2 c = sN[k][t];
         double v[5] = {(double)(c.x * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + c.y * W[k][2])};
-        if constexpr (COLORED)
+        if constexpr (COLORED) {
             col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
-        else if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+        } else if constexpr (SHARED) {
+            if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+                col_add_shared(sR, US, li[k], at[k], v, a.Rmass, a.Rmom, a.Rener, np);
+        } else if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
     }
     if constexpr (COLORED) {
@@ -551,6 +557,10 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
         col_list<P>(pl.unode + u0, U, wn);
         __syncthreads();
         col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
+    }
+    if constexpr (SHARED) {
+        __syncthreads();
+        col_write_shared(pl, b, sR, NT, a.Rmass, a.Rmom, a.Rener, np);
     }
 }
 
@@ -572,6 +582,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     constexpr int H = Q / 2, HL = E2 * QQ, NT = 2 * HL, PARTS = EPB / E2;
     static_assert(Q % 2 == 0 && HL % 64 == 0 && LANES == EPB * QQ, "whole waves per half");
     constexpr bool AHEAD = true;  // read line sources one ahead of their use
+    constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
     __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
@@ -579,7 +590,8 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
     __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
     // its fluxes along I (0..2), J (3..5) and K (6..8); at the start the columns'
-    // values; in the coloured mode, at the end, the node sums [5][US]
+    // values; in the coloured mode and with FP32 outputs, at the end, the node sums
+    // [5][US]
     extern __shared__ __attribute__((aligned(16))) double sR[];
     V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
 
@@ -829,22 +841,27 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
         }
         __builtin_amdgcn_sched_barrier(0);
     });
-    if constexpr (COLORED) {
+    if constexpr (COLORED || SHARED) {
         __syncthreads();  // the last slice's fluxes are read
         for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
         __syncthreads();
     }
-    uint32_t at[H];
+    uint32_t at[H], li[H];
 #pragma unroll
-    for (int k = 0; k < H; ++k)
+    for (int k = 0; k < H; ++k) {
         at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k0 + k) * LANES + tc] : conn[k * LANES];
+        li[k] = SHARED ? (uint32_t)pl.lidx[((int64_t)b * Q + k0 + k) * LANES + tc] : 0u;
+    }
 #pragma unroll
     for (int k = 0; k < H; ++k) {
         double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + kappa[k] * W[k][2])};
-        if constexpr (COLORED)
+        if constexpr (COLORED) {
             col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
-        else if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+        } else if constexpr (SHARED) {
+            if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
+                col_add_shared(sR, US, li[k], at[k], v, a.Rmass, a.Rmom, a.Rener, np);
+        } else if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
     }
     if constexpr (COLORED) {
@@ -856,6 +873,10 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
             col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
         }
     }
+    if constexpr (SHARED) {
+        __syncthreads();
+        col_write_shared(pl, b, sR, NT, a.Rmass, a.Rmom, a.Rener, np);
+    }
 }
 
 template <int P, class A, bool CLOSURE, typename TA>
@@ -863,20 +884,21 @@ static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
     const bool atomic = a.plan.mode == kAtomic;
-    const size_t sums = sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(TA) * 12 * ColShape<P>::NT;
+    const bool registers = P > kNarrowP && atomic && sizeof(typename A::O) == 8;
+    const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(TA) * 12 * ColShape<P>::NT;
     const dim3 grid((unsigned)a.plan.nb), block(ColShape<P>::NT);
     if constexpr (P == 7) {
         constexpr int E2 = 2, EPB = ColShape<P>::EPB, QQ = ColShape<P>::QQ;
         const size_t part = sizeof(TA) * 2 * 9 * 2 * QQ;  // fluxes per element
         if (atomic)
             hipLaunchKernelGGL((k_diffu_split<P, E2, false, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))),
-                               dim3(2 * E2 * QQ), E2 * part, s, a, mlp);
+                               dim3(2 * E2 * QQ), std::max(E2 * part, sums), s, a, mlp);
         else
             hipLaunchKernelGGL((k_diffu_split<P, EPB, true, A, CLOSURE, TA>), grid, dim3(2 * EPB * QQ),
                                std::max(EPB * part, sums), s, a, mlp);
     } else if constexpr (P > kNarrowP)
         hipLaunchKernelGGL((atomic ? k_diffu_wide<P, false, A, CLOSURE, TA> : k_diffu_wide<P, true, A, CLOSURE, TA>), grid,
-                           block, atomic ? fluxes : std::max(fluxes, sums), s, a, mlp);
+                           block, std::max(fluxes, sums), s, a, mlp);
     else
         hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE, TA> : k_diffu_col<P, true, A, CLOSURE, TA>), grid,
                            block, sums, s, a, mlp);

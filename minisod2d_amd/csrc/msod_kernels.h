@@ -15,10 +15,12 @@
 // Assembly plan (built once per mesh by the runtime).  Elements are grouped
 // into batches of ColShape<P>::EPB consecutive elements, one workgroup each,
 // which sums its elements' contributions to every node of the batch in LDS and
-// writes each of the batch's distinct nodes once (above kNarrowP, in the atomic
-// mode, it adds from registers and needs conn alone):
+// writes each of the batch's distinct nodes once.  Above kNarrowP, in the atomic
+// mode, it adds from registers and needs conn alone; with FP32 outputs the nodes
+// that several element nodes of the batch share are summed in LDS all the same,
+// in FP64, and rounded once (unode lists them alone):
 //   conn          0-based global node of each element node
-//   lidx          position of that node in its batch's node list
+//   lidx          position of that node in its batch's node list (kAlone: not listed)
 //   uoff [nbatch+1]  node list of batch b: unode[uoff[b] .. uoff[b+1])
 //   unode [..]    sorted distinct global nodes of each batch; bit 31 set when
 //                 this batch is the first writer of the node (host plan)
@@ -47,6 +49,7 @@ constexpr int kMaxP = 8;
 // 1.84 -> 2.65), order 5 7%.
 constexpr int kNarrowP = 4;
 enum AssemblyMode { kColored = 0, kAtomic = 1 };
+constexpr uint16_t kAlone = 0xffff;
 
 // Elements per batch: ColShape<P>::EPB for run-time porder.
 int batch_size(int porder);

@@ -192,10 +192,13 @@ __global__ void k_build_geo_nodes(const T *He, const T *gpvol, int64_t nelem, in
 // nodes are sorted in LDS (bitonic) and the distinct ones numbered in
 // ascending order, as build_host_plan does on the host.  FILL = false:
 // count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
-// unode from uoff, conn and lidx in the lane layout.  Above kNarrowP the atomic
-// kernels read conn alone: lists = false (count[b] = 0, the rest null).
+// unode from uoff, conn and lidx in the lane layout.  lists (PlanLists): every
+// node of the batch, those alone that several lanes write after col_merge has
+// taken neighbours' nodes together (the others' lidx is kAlone), or none, for
+// kernels that read conn alone (count[b] = 0, the rest null).
 // A first pair at 64^3, p=4 takes 6 ms in all (191 with the host plan).
 constexpr uint32_t kBadBatch = 0x80000000u;
+enum PlanLists { kListNone = 0, kListAll = 1, kListShared = 2 };
 template <int P>
 struct PlanShape {
     static constexpr int NN = (P + 1) * (P + 1) * (P + 1);
@@ -206,7 +209,7 @@ struct PlanShape {
 };
 template <int P, bool FILL>
 __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                                                      bool lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
+                                                      int lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
                                                       uint32_t *unode, uint32_t *conn, uint16_t *lidx)
 {
     using S = PlanShape<P>;
@@ -233,11 +236,27 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
             bad += !ok && le < ne;
             v[j] = ok ? (uint32_t)(c - 1) : 0u;
         }
-        s[i] = v[j];
+        s[i] = i < n && i % B < ne ? v[j] : 0xffffffffu;
     }
     if (bad) atomicAdd(&sbad, bad);
     __syncthreads();
-    if (!lists) {
+    if (lists == kListShared) {
+        // the left node of each pair that col_merge takes together is not written
+        constexpr int Q = P + 1;
+        bool given[PER];
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+            const int i = t + j * NT, le = i % B, l = i / B;
+            given[j] = i < n && l % Q == 1 && le + 1 < ne && s[i + 1 - B] == v[j] &&
+                       (ElemEntry<P>{e0 + le, l}.lane() & 63) != 63;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < PER; ++j)
+            if (given[j]) s[t + j * NT] = 0xffffffffu;
+        __syncthreads();
+    }
+    if (lists == kListNone) {
         if constexpr (!FILL) {
             if (t == 0) count[b] = sbad ? kBadBatch + sbad : 0u;
         } else {
@@ -269,7 +288,8 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
 #pragma unroll
     for (int j = 0; j < PER; ++j) {
         const int i = t * PER + j;
-        first[j] = s[i] != 0xffffffffu && (i == 0 || s[i] != s[i - 1]);
+        first[j] = s[i] != 0xffffffffu && (i == 0 || s[i] != s[i - 1]) &&
+                   (lists == kListAll || (i + 1 < SORT && s[i] == s[i + 1]));
         c += first[j];
     }
     uint32_t sum = c;
@@ -305,7 +325,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
             }
             const ElemEntry<P> en{e0 + i % B, i / B};
             conn[en.entry()] = v[j];
-            lidx[en.entry()] = (uint16_t)lo;
+            lidx[en.entry()] = lists == kListAll || (U > 0 && su[lo] == v[j]) ? (uint16_t)lo : kAlone;
         }
     }
 }
@@ -456,7 +476,7 @@ static bool nodes_for_colors(int porder, int64_t nelem)
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
 hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                               bool lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
+                               int lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
                                uint32_t *conn, uint16_t *lidx, hipStream_t s)
 {
     return with_porder(porder, [&](auto p) {
@@ -519,6 +539,7 @@ struct PlanEntry {
     uint32_t *unref = nullptr;       // nodes no element references (zeroed per call)
     int64_t nunref = 0;
     bool nodes = false;              // element-major, of the FP32-arithmetic kernels (msod_nodes.h)
+    int lists = kListAll;            // the nodes in unode
     bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
     void release()
@@ -825,7 +846,7 @@ int upload(const std::vector<V> &h, V **d, const char *what)
 
 // Builds the node lists of a mesh's batches on the device: all that the atomic
 // assembly reads of the plan.
-int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, bool lists,
+int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, int lists,
                       PlanEntry &P)
 {
     const int64_t nn = (int64_t)ts->l2g.size(), nb = (nelem + B - 1) / B;
@@ -833,6 +854,7 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
         return fail(MSOD_ERR_MESH, "mesh too large for 32-bit node indices");
     P.B = B;
     P.nbatch = nb;
+    P.lists = lists;
     // connec may come from work on the default stream, which the copy that
     // feeds the host plan waits for
     HIPCHK(hipStreamSynchronize(nullptr), "plan");
@@ -858,9 +880,9 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
                     (long long)npoin);
     const int64_t n = geo_elems(ts->porder, nelem) * nn;
     HIPCHK(hipMalloc((void **)&P.conn, sizeof(uint32_t) * n), "plan");
-    if (lists) {
+    if (lists != kListNone) {
         HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
-        HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * uoff[nb]), "plan");
+        HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * std::max(uoff[nb], 1u)), "plan");
     }
     HIPCHK(hipMemcpyAsync(P.uoff, uoff.data(), sizeof(uint32_t) * (nb + 1), hipMemcpyHostToDevice, g.stream), "plan");
     HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, lists, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
@@ -945,15 +967,17 @@ void drop_unversioned(const void *src)
         }
 }
 
-int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, const TableSet *ts, int B,
+// lists: the node lists that the call's kernels read (kListNone: any plan will do).
+int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, const TableSet *ts, int B, int lists,
              const PlanEntry **out, bool nodes = false)
 {
     if (ver == 0) drop_unversioned(dconnec);
     const bool host = g.assembly == kColored;  // the atomic assembly takes either plan
+    if (host) lists = kListAll;
     for (size_t i = 0; i < g.plans.size(); ++i) {
         PlanEntry &c = g.plans[i];
         if (c.src != dconnec || c.ver != ver || c.nelem != nelem || c.npoin != npoin || c.porder != ts->porder ||
-            c.l2g != ts->l2g || c.B != B || c.nodes != nodes)
+            c.l2g != ts->l2g || c.B != B || c.nodes != nodes || (lists != kListNone && c.lists != lists))
             continue;
         if (c.host || !host) {
             *out = &c;
@@ -971,7 +995,7 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
     P.porder = ts->porder;
     P.l2g = ts->l2g;
     int st = nodes ? build_nodes_plan(dconnec, nelem, npoin, ts, B, P)
-                   : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, host || ts->porder <= kNarrowP, P);
+                   : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, lists, P);
     if (!st && host && !nodes) st = build_host_part(dconnec, nelem, npoin, ts, B, P);
     if (st) {
         P.release();
@@ -1134,6 +1158,13 @@ int check_sizes(int porder, int nelem, int npoin)
     return MSOD_OK;
 }
 
+// Node lists that the column kernels read with outputs of type TO.
+template <typename TO>
+int column_lists(int porder)
+{
+    return porder <= kNarrowP ? kListAll : (sizeof(TO) == 4 ? kListShared : kListNone);
+}
+
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
 // the kernel: one launch per colour, or one launch over all batches in mesh
 // order, where neighbouring batches meet in L2.  One node per thread: kpb_max
@@ -1223,7 +1254,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     constexpr bool kF64 = std::is_same<ConvecArgs<TG, TF, TO, TU, TP>, ConvecArgs<double, double>>::value;
     const bool nodes = fp32_arith || (kF64 && g.assembly == kColored && nodes_for_colors(porder, NE));
     const int B = nodes ? nodes_convec_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, nodes))) return st;
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, nodes ? kListAll : column_lists<TO>(porder), &plan, nodes))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
@@ -1288,7 +1319,7 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
     const bool nodes = fp32_arith || (kF64 && !dmlp && g.assembly == kColored && nodes_for_colors(porder, NE));
     const int B = nodes ? nodes_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, &plan, nodes))) return st;
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, nodes ? kListAll : column_lists<TO>(porder), &plan, nodes))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;
@@ -1437,7 +1468,7 @@ int closure_elem_common(int porder, int nelem, int npoin, const int32_t *connec,
     if ((st = resolve(u, sizeof(double) * 3 * NP, "u", &du, &vx))) return st;
     const PlanEntry *plan;
     const double *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), &plan))) return st;
+    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), kListNone, &plan))) return st;
     if ((st = get_geo<double>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
     a = ClosureElemArgs{};
     a.nelem = NE;
