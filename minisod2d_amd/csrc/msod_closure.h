@@ -35,5 +35,7 @@ hipError_t launch_residual_error(const double *Rmom, const double *Rener, const 
 // Diffusion with mu_sgs from the MLP, evaluated inside the kernel (FP64).
 hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp,
                                 hipStream_t s);
+hipError_t launch_diffu_closure_nodes(int porder, const DiffuArgs<double, double> &a, const float *mlp,
+                                      hipStream_t s);
 
 }  // namespace msod

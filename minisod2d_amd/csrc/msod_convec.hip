@@ -18,7 +18,7 @@
 // 1e-16 level.
 //
 // Storage types TG (geometry) and TF (nodal fields), FP64 arithmetic
-// (msod_kernels.h); the FP32-arithmetic form is msod_convec_fp32.hip.  Without a
+// (msod_kernels.h); the FP32-arithmetic form is msod_convec_nodes.hip.  Without a
 // pressure array the pressure is recovered as p = (gamma-1)(E - rho|u|^2/2)
 // from the stored state.
 #include "msod_columns.h"

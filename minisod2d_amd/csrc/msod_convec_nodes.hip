@@ -1,6 +1,5 @@
-// Convective residual with FP32 gathers, fluxes and sweeps (FP64 pressure
-// recovery, node sums and assembly); msod_convec.hip names the reference it
-// stands for, msod_nodes.h says why it has a kernel of its own.
+// Convective residual with one node per thread (msod_convec.hip names the
+// reference it stands for); msod_nodes.h says which calls take it.
 //
 // One workgroup per batch of CShape<P>::BATCH elements, processed in passes of
 // CShape<P>::EPB elements with one thread per element node.  Per pass:
@@ -28,7 +27,7 @@
 // (write_batch_nodes: plain store / read-add-store per colour, or FP64 atomics).
 //
 // Storage types TG (geometry) and TF (nodal fields), FP64 arithmetic
-// throughout (msod_kernels.h).  Without a pressure array the pressure is
+// (msod_kernels.h), or FP32 in the gathers, fluxes and sweeps (TA).  Without a pressure array the pressure is
 // recovered as p = (gamma-1)(E - rho|u|^2/2) from the stored state.
 #include "msod_nodes.h"
 
@@ -313,9 +312,16 @@ hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hip
     return launch_order<ConvecArgs<float, float>, float>(porder, a, s);
 }
 
-hipError_t launch_convec_nodes(int porder, const ConvecArgs<double, double> &a, hipStream_t s)
+template <class A>
+hipError_t launch_convec_nodes(int porder, const A &a, hipStream_t s)
 {
-    return launch_order<ConvecArgs<double, double>, double>(porder, a, s);
+    return launch_order<A, double>(porder, a, s);
 }
+
+template hipError_t launch_convec_nodes(int, const ConvecArgs<double, double> &, hipStream_t);
+template hipError_t launch_convec_nodes(int, const ConvecArgs<float, float> &, hipStream_t);
+template hipError_t launch_convec_nodes(int, const ConvecArgs<float, double> &, hipStream_t);
+template hipError_t launch_convec_nodes(int, const ConvecArgs<float, float, float> &, hipStream_t);
+template hipError_t launch_convec_nodes(int, const ConvecSplitArgs &, hipStream_t);
 
 }  // namespace msod

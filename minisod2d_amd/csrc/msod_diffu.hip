@@ -18,7 +18,7 @@
 // step 2 publishes one component per direction.
 //
 // Storage types TG (geometry, mu_e, mu_sgs) and TF (nodal fields), FP64
-// arithmetic (msod_kernels.h); the FP32-arithmetic form is msod_diffu_fp32.hip.
+// arithmetic (msod_kernels.h); the FP32-arithmetic form is msod_diffu_nodes.hip.
 // CLOSURE (FP64 storage): mu_sgs is not read but predicted by the learned
 // closure (msod_mlp.h) from the velocity gradient before the stress is
 // formed; its per-wave LDS scratch is the wave's own part of the flux buffer,

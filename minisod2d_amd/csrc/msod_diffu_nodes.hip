@@ -1,6 +1,5 @@
-// Diffusive residual with FP32 gathers, gradients, fluxes and sweeps (FP64 node
-// sums and assembly); msod_diffu.hip names the reference it stands for,
-// msod_nodes.h says why it has a kernel of its own.
+// Diffusive residual with one node per thread (counterpart of full_diffusion_ijk,
+// src/kernels/sources/elem_diffu.f90:10-197); msod_nodes.h says which calls take it.
 //
 // One workgroup per batch of Shape<P>::BATCH elements, passes of
 // Shape<P>::EPB elements with one thread per element node.  Per pass:
@@ -24,8 +23,16 @@
 // written once (write_batch_nodes).
 //
 // Storage types TG (geometry, mu_e, mu_sgs) and TF (nodal fields), FP64
-// arithmetic throughout (msod_kernels.h).
+// arithmetic (msod_kernels.h), or FP32 in the gradients, fluxes and sweeps (TA).
+// CLOSURE (FP64 storage): mu_sgs is not read but predicted per element node by
+// the learned closure (msod_mlp.h) from the pass-1 velocity gradient, evaluated
+// with bf16 MFMA inside the kernel before the stress is formed; its LDS scratch
+// overlays the field buffers between the passes.
+#include <type_traits>
+
 #include "msod_nodes.h"
+#include "msod_mlp.h"
+#include "msod_closure.h"
 
 namespace msod {
 
@@ -55,7 +62,7 @@ __device__ __forceinline__ void diffu_fetch(const A &a, uint32_t gnode, DiffuNod
 // lines (and pages) per load; here ME neighbouring lanes read ME
 // consecutive elements of one node, and the batches that follow in mesh
 // order reuse the lines.
-template <int NN, int ME, int NT, class A, typename TG = typename A::G>
+template <int NN, int ME, int NT, bool CLOSURE, class A, typename TG = typename A::G>
 __device__ __forceinline__ void diffu_stage_mu(const A &a, int64_t e0, TG (*sMu)[ME][NN])
 {
     // every load unconditional and issued before any LDS write (entries past
@@ -75,7 +82,7 @@ __device__ __forceinline__ void diffu_stage_mu(const A &a, int64_t e0, TG (*sMu)
         const int64_t e = e0 + i % ME < a.nelem ? e0 + i % ME : a.nelem - 1;
         const int64_t ge = e + a.nelem * (int64_t)gl[k];  // reference layout (nelem,ngaus)
         v0[k] = a.mu_e[ge];
-        v1[k] = a.mu_sgs ? a.mu_sgs[ge] : (TG)0;  // NULL: closure fallback
+        v1[k] = (!CLOSURE && a.mu_sgs) ? a.mu_sgs[ge] : (TG)0;  // NULL: closure fallback
     }
 #pragma unroll
     for (int k = 0; k < IT; ++k) {
@@ -87,28 +94,47 @@ __device__ __forceinline__ void diffu_stage_mu(const A &a, int64_t e0, TG (*sMu)
     }
 }
 
-template <int P, class A, typename TA = double>
-__global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
+// Launch bound in waves per SIMD.  The closure form is bounded to 3
+// workgroups per CU: the compiler then keeps the MFMA accumulators in VGPRs
+// (about 148 in all) instead of 188 VGPRs and 32 AGPRs, 3 waves per SIMD
+// instead of 2 (4.7 against 6.2 ms at 96^3 p=3).  512-thread workgroups with
+// FP32 element arrays and FP64 arithmetic: 6, three workgroups per CU (their
+// LDS fits three), at 80 VGPRs with 20 B of spills per lane (48^3 p=7: FP32
+// split 3.96 -> 3.45 ms, every input in FP32 4.21 -> 3.41 ms); the FP64 form
+// spilled 28 B there and ran slower (3.61 -> 3.90 ms), so it keeps two.
+template <int P, typename TG, typename TA, bool CLOSURE>
+constexpr int diffu_waves()
+{
+    return CLOSURE ? (Shape<P>::NT == 256 ? 3 : 1)
+                   : (Shape<P>::NT == 512 && sizeof(TG) < sizeof(TA) ? 6 : 1);
+}
+
+template <int P, class A, bool CLOSURE, typename TA = double>
+__global__ void __launch_bounds__(Shape<P>::NT, (diffu_waves<P, typename A::G, TA, CLOSURE>())) k_diffu(A a, const float *mlp)
 {
     using TG = typename A::G;
     using S = Shape<P>;
     using T = TA;  // arithmetic: FP64, or FP32 for the FP32-arithmetic form (node sums stay FP64)
     constexpr int Q = S::Q, NN = S::NN, EPB = S::EPB, UMAX = S::UMAX;
     // one buffer of node records (sN) serves pass 1 (rho, T, u) and pass 2
-    // (fluxes of one direction)
+    // (fluxes of one direction); the MLP scratch of the closure overlays it
+    // between the two
     constexpr size_t kRec = sizeof(T) * EPB * 6 * NN;
-    constexpr size_t kBuf = kRec;
+    constexpr size_t kScr = CLOSURE ? (size_t)(S::NT / 64) * 4 * 256 * sizeof(short) : 0;
+    constexpr size_t kBuf = kRec > kScr ? kRec : kScr;
     __shared__ T sD[Q * Q];
     __shared__ __attribute__((aligned(16))) unsigned char sbuf[kBuf];
     __shared__ double sR[5][UMAX];
     // mu_e, mu_sgs of the batch, staged once; of the pass, staged per pass,
     // where the batch's would cost a workgroup per CU (four fit 160 KB of LDS)
-    constexpr size_t kLdsRest = sizeof(T) * Q * Q + kBuf + sizeof(double) * 5 * UMAX;
+    constexpr size_t kLdsRest = sizeof(T) * Q * Q + kBuf + sizeof(double) * 5 * UMAX +
+                                (CLOSURE ? sizeof(MlpShared) : 0);
     constexpr size_t kLdsCu = 160 * 1024 / 4;
     constexpr bool kMuPerPass = kLdsRest + 2 * sizeof(TG) * S::BATCH * NN > kLdsCu &&
                                 kLdsRest + 2 * sizeof(TG) * EPB * NN <= kLdsCu;
     constexpr int ME = kMuPerPass ? EPB : S::BATCH;
     __shared__ TG sMu[2][ME][NN];
+    __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
     // node-major records of 6 values (pass 1: rho, T, u0, u1, u2, unused;
     // pass 2: the contravariant fluxes of one direction), read in pairs: in
     // FP64 three ds_read_b128 per source instead of ds_read2_b64 pairs
@@ -170,7 +196,7 @@ __global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
                 const int64_t em = b * S::BATCH + i % ME < a.nelem ? b * S::BATCH + i % ME : a.nelem - 1;
                 const int64_t ge = em + a.nelem * (int64_t)gl[k];
                 v0[k] = a.mu_e[ge];
-                v1[k] = a.mu_sgs ? a.mu_sgs[ge] : (TG)0;
+                v1[k] = (!CLOSURE && a.mu_sgs) ? a.mu_sgs[ge] : (TG)0;
             }
         }
         for (uint32_t i = t; i < U; i += blockDim.x)
@@ -188,6 +214,7 @@ __global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
             }
         }
     }
+    if constexpr (CLOSURE) mlp_stage(smlp, mlp);
 
 #pragma unroll
     for (int pass = 0; pass < S::NPASS; ++pass) {
@@ -195,7 +222,7 @@ __global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
         const bool active = (le < EPB) && (e < a.nelem);
         T r = 0, muf = 0, mue = 0, mus = 0, uu[3] = {0, 0, 0};
         // the previous pass read its sMu entries before its pass-2 barriers
-        if (kMuPerPass) diffu_stage_mu<NN, ME, NT>(a, b * S::BATCH + pass * EPB, sMu);
+        if (kMuPerPass) diffu_stage_mu<NN, ME, NT, CLOSURE>(a, b * S::BATCH + pass * EPB, sMu);
         __syncthreads();  // previous pass done with sN (and sR zeroed, sMu staged)
         if (active) {
             r = cur.r;
@@ -260,6 +287,22 @@ __global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
                     G[2][i] += hid * aU2;
                 }
             }
+        }
+        if constexpr (CLOSURE) {
+            __syncthreads();  // every pass-1 sweep over sN done: the MLP scratch overlays it
+            float f[kMlpIn];
+            if (active) {
+                T hinv[3][3];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+#pragma unroll
+                    for (int d = 0; d < 3; ++d) hinv[i][d] = (T)gn.he(i + 3 * d);
+                mlp_features<T>(G, r, uu, hinv, f);
+            } else
+#pragma unroll
+                for (int k = 0; k < kMlpIn; ++k) f[k] = smlp.mean[k];
+            const float z3 = mlp_forward_z3(smlp, f, reinterpret_cast<short *>(sbuf) + (t >> 6) * 4 * 256);
+            mus = active ? (T)(smlp.scale * softplusf_(z3)) : (T)0;
         }
         if (active) {
             const T divU = G[0][0] + G[1][1] + G[2][2];
@@ -327,38 +370,50 @@ __global__ void __launch_bounds__(Shape<P>::NT, 1) k_diffu(A a)
     write_batch_nodes<UMAX, NT>(pl.mode, wn, U, sR, a.Rmass, a.Rmom, a.Rener, a.npoin);
 }
 
-template <int P, class A, typename TA>
-static hipError_t launch_p(const A &a, hipStream_t s)
+template <int P, class A, bool CLOSURE, typename TA>
+static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
-    hipLaunchKernelGGL((k_diffu<P, A, TA>), dim3((unsigned)a.plan.nb), dim3(Shape<P>::NT), 0, s, a);
+    hipLaunchKernelGGL((k_diffu<P, A, CLOSURE, TA>), dim3((unsigned)a.plan.nb), dim3(Shape<P>::NT), 0, s, a, mlp);
     return hipGetLastError();
 }
 
-template <class A, typename TA>
-static hipError_t launch_order(int porder, const A &a, hipStream_t s)
+template <class A, bool CLOSURE, typename TA>
+static hipError_t launch_order(int porder, const A &a, const float *mlp, hipStream_t s)
 {
     switch (porder) {
-    case 1: return launch_p<1, A, TA>(a, s);
-    case 2: return launch_p<2, A, TA>(a, s);
-    case 3: return launch_p<3, A, TA>(a, s);
-    case 4: return launch_p<4, A, TA>(a, s);
-    case 5: return launch_p<5, A, TA>(a, s);
-    case 6: return launch_p<6, A, TA>(a, s);
-    case 7: return launch_p<7, A, TA>(a, s);
-    case 8: return launch_p<8, A, TA>(a, s);
+    case 1: return launch_p<1, A, CLOSURE, TA>(a, mlp, s);
+    case 2: return launch_p<2, A, CLOSURE, TA>(a, mlp, s);
+    case 3: return launch_p<3, A, CLOSURE, TA>(a, mlp, s);
+    case 4: return launch_p<4, A, CLOSURE, TA>(a, mlp, s);
+    case 5: return launch_p<5, A, CLOSURE, TA>(a, mlp, s);
+    case 6: return launch_p<6, A, CLOSURE, TA>(a, mlp, s);
+    case 7: return launch_p<7, A, CLOSURE, TA>(a, mlp, s);
+    case 8: return launch_p<8, A, CLOSURE, TA>(a, mlp, s);
     default: return hipErrorInvalidValue;
     }
 }
 
 hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s)
 {
-    return launch_order<DiffuArgs<float, float>, float>(porder, a, s);
+    return launch_order<DiffuArgs<float, float>, false, float>(porder, a, nullptr, s);
 }
 
-hipError_t launch_diffu_nodes(int porder, const DiffuArgs<double, double> &a, hipStream_t s)
+template <class A>
+hipError_t launch_diffu_nodes(int porder, const A &a, hipStream_t s)
 {
-    return launch_order<DiffuArgs<double, double>, double>(porder, a, s);
+    return launch_order<A, false, double>(porder, a, nullptr, s);
 }
+
+hipError_t launch_diffu_closure_nodes(int porder, const DiffuArgs<double, double> &a, const float *mlp, hipStream_t s)
+{
+    return launch_order<DiffuArgs<double, double>, true, double>(porder, a, mlp, s);
+}
+
+template hipError_t launch_diffu_nodes(int, const DiffuArgs<double, double> &, hipStream_t);
+template hipError_t launch_diffu_nodes(int, const DiffuArgs<float, float> &, hipStream_t);
+template hipError_t launch_diffu_nodes(int, const DiffuArgs<float, double> &, hipStream_t);
+template hipError_t launch_diffu_nodes(int, const DiffuArgs<float, float, float> &, hipStream_t);
+template hipError_t launch_diffu_nodes(int, const DiffuSplitArgs &, hipStream_t);
 
 }  // namespace msod

@@ -142,9 +142,11 @@ hipError_t launch_diffu(int porder, const A &a, hipStream_t s);
 // assembly and (convection) pressure recovery.
 hipError_t launch_convec_fp32(int porder, const ConvecArgs<float, float> &a, hipStream_t s);
 hipError_t launch_diffu_fp32(int porder, const DiffuArgs<float, float> &a, hipStream_t s);
-// The FP64 form with one node per thread (msod_nodes.h).
-hipError_t launch_convec_nodes(int porder, const ConvecArgs<double, double> &a, hipStream_t s);
-hipError_t launch_diffu_nodes(int porder, const DiffuArgs<double, double> &a, hipStream_t s);
+// The kernels with one node per thread (msod_nodes.h), FP64 arithmetic.
+template <class A>
+hipError_t launch_convec_nodes(int porder, const A &a, hipStream_t s);
+template <class A>
+hipError_t launch_diffu_nodes(int porder, const A &a, hipStream_t s);
 
 // Zero Rmass (n), Rmom (3n), Rener (n).
 hipError_t launch_zero_outputs(double *Rmass, double *Rmom, double *Rener, int64_t n,

@@ -1,14 +1,15 @@
-// One node per thread: batches, records and assembly of the FP32-arithmetic
-// kernels (msod_convec_fp32.hip, msod_diffu_fp32.hip), and of the FP64 form in the
-// coloured mode where its launches are short (nodes_for_colors).
-//
-// Their results are FP32 rounding, so another order of the FP32 operations is
-// another result (columns: 9e-7 off in relative L2, 48^3 p=7 3.14 -> 2.5 ms for
-// the diffusion).  They keep their order, and with it their own layouts,
-// element-major with the element-local node index l,
+// One node per thread: batches, records and assembly of the kernels in
+// msod_convec_nodes.hip and msod_diffu_nodes.hip.  They serve
+//   * the FP32-arithmetic form: its results are FP32 rounding, so another order
+//     of the FP32 operations is another result (columns: 9e-7 off in relative L2,
+//     48^3 p=7 3.14 -> 2.5 ms for the diffusion);
+//   * the coloured mode where its launches are short (nodes_for_colors), and
+//     where the batches of the column kernels, up to five times as large, need
+//     more than 32 colours (elements in little spatial order).
+// Their layouts are element-major with the element-local node index l,
 //   geo   [nelem][5][nn][2]  GeoNode's five pairs
 //   conn, lidx  [nelem][nn]
-// and their own plan: the host's (msod_plan.h), whose batches hold
+// and their plan is the host's (msod_plan.h), whose batches hold
 // Shape<P>::BATCH elements (convection CShape<P>::BATCH).  A workgroup takes
 // kpb consecutive batches of the launch's list.
 #pragma once

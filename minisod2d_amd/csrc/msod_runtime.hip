@@ -1165,6 +1165,22 @@ int column_lists(int porder)
     return porder <= kNarrowP ? kListAll : (sizeof(TO) == 4 ? kListShared : kListNone);
 }
 
+// The plan of a call: of the kernels with one node per thread (batches of NB
+// elements) where *nodes says so, of the column kernels otherwise.  *nodes is set
+// where those turn out not to suit the mesh: in the coloured mode, when their
+// batches need more than 32 colours.
+template <typename TO>
+int choose_plan(const void *dc, uint64_t vc, int64_t NE, int64_t NP, const TableSet *ts, int NB, bool *nodes,
+                const PlanEntry **plan)
+{
+    if (!*nodes) {
+        const int st = get_plan(dc, vc, NE, NP, ts, batch_size(ts->porder), column_lists<TO>(ts->porder), plan);
+        if (st) return st;
+        *nodes = g.assembly == kColored && !(*plan)->colored;
+    }
+    return *nodes ? get_plan(dc, vc, NE, NP, ts, NB, kListAll, plan, true) : MSOD_OK;
+}
+
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
 // the kernel: one launch per colour, or one launch over all batches in mesh
 // order, where neighbouring batches meet in L2.  One node per thread: kpb_max
@@ -1252,9 +1268,8 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     const PlanEntry *plan;
     const TG *geo;
     constexpr bool kF64 = std::is_same<ConvecArgs<TG, TF, TO, TU, TP>, ConvecArgs<double, double>>::value;
-    const bool nodes = fp32_arith || (kF64 && g.assembly == kColored && nodes_for_colors(porder, NE));
-    const int B = nodes ? nodes_convec_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, nodes ? kListAll : column_lists<TO>(porder), &plan, nodes))) return st;
+    bool nodes = fp32_arith || (kF64 && g.assembly == kColored && nodes_for_colors(porder, NE));
+    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
@@ -1276,9 +1291,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                 if constexpr (std::is_same<ConvecArgs<TG, TF, TO, TU, TP>,
                                                            ConvecArgs<float, float>>::value)
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
-                                if constexpr (kF64)
-                                    if (nodes) return launch_convec_nodes(porder, x, g.stream);
-                                return launch_convec(porder, x, g.stream);
+                                return nodes ? launch_convec_nodes(porder, x, g.stream) : launch_convec(porder, x, g.stream);
                             },
                             "convection kernel launch", !nodes, nodes ? kBatchesPerBlock : 1)))
         return st;
@@ -1317,9 +1330,8 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     const PlanEntry *plan;
     const TG *geo;
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
-    const bool nodes = fp32_arith || (kF64 && !dmlp && g.assembly == kColored && nodes_for_colors(porder, NE));
-    const int B = nodes ? nodes_batch_size(porder) : batch_size(porder);
-    if ((st = get_plan(dc, vc, NE, NP, ts, B, nodes ? kListAll : column_lists<TO>(porder), &plan, nodes))) return st;
+    bool nodes = fp32_arith || (kF64 && !dmlp && g.assembly == kColored && nodes_for_colors(porder, NE));
+    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;
@@ -1343,13 +1355,13 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     if ((st = run_assembled(a, *plan, timer,
                             [&](const DiffuArgs<TG, TF, TO, TU> &x) {
                                 using AT = DiffuArgs<TG, TF, TO, TU>;
-                                if constexpr (kF64) {
-                                    if (dmlp) return launch_diffu_closure(porder, x, dmlp, g.stream);
-                                    if (nodes) return launch_diffu_nodes(porder, x, g.stream);
-                                }
+                                if constexpr (kF64)
+                                    if (dmlp)
+                                        return nodes ? launch_diffu_closure_nodes(porder, x, dmlp, g.stream)
+                                                     : launch_diffu_closure(porder, x, dmlp, g.stream);
                                 if constexpr (std::is_same<AT, DiffuArgs<float, float>>::value)
                                     if (fp32_arith) return launch_diffu_fp32(porder, x, g.stream);
-                                return launch_diffu(porder, x, g.stream);
+                                return nodes ? launch_diffu_nodes(porder, x, g.stream) : launch_diffu(porder, x, g.stream);
                             },
                             "diffusion kernel launch")))
         return st;
