@@ -405,10 +405,12 @@ static hipError_t launch_p(const A &a, hipStream_t s)
     const bool atomic = a.plan.mode == kAtomic;
     const bool registers = P > kNarrowP && atomic && sizeof(typename A::O) == 8;
     const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride;
-    if constexpr (P > kNarrowP)
-        hipLaunchKernelGGL((atomic ? k_convec_wide<P, false, A, TA> : k_convec_wide<P, true, A, TA>),
+    if constexpr (P > kNarrowP) {
+        if constexpr (P != 6)
+            if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
+        hipLaunchKernelGGL((atomic || P != 6 ? k_convec_wide<P, false, A, TA> : k_convec_wide<P, P == 6, A, TA>),
                            dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
-    else
+    } else
         hipLaunchKernelGGL((atomic ? k_convec_col<P, false, A, TA> : k_convec_col<P, true, A, TA>),
                            dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
     return hipGetLastError();

@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
 // Orders above kNarrowP: the same walk, whose columns (r, T, u and the six sums)
 // take up to 198 VGPRs.  nu and kappa wait in LDS for the end, mu_fluid is
 // gathered a slice ahead, and the gradients replace the line derivatives one
-// field at a time.  The atomic mode adds to the outputs from the registers
+// field at a time.  They add to the outputs from the registers
 // (col_merge, col_scatter).  Against one node per thread: 40^3 order 6 1.86 ->
 // 1.21 ms (1.32 with the line sources read one ahead: spills); 32^3 order 8,
 // with one wave per SIMD, 2.40 -> 1.88 (two waves and 80 spilled VGPRs: 2.61);
@@ -298,7 +298,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
 template <int P, typename TA>
 constexpr int kWideWaves = P == 8 && sizeof(TA) == 8 ? 1 : 2;  // per SIMD
 
-template <int P, bool COLORED, class A, bool CLOSURE, typename TA>
+template <int P, class A, bool CLOSURE, typename TA>
 __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_wide(A a, const float *mlp)
 {
     using S = ColShape<P>;
@@ -306,7 +306,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     using TG = typename A::G;
     constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
     constexpr bool AHEAD = kWideWaves<P, TA> == 1;  // read line sources one ahead of their use
-    constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
+    constexpr bool SHARED = sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
     __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
@@ -314,8 +314,8 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
     __shared__ V2 sN[Q][NT];                               // nu, kappa of the thread's nodes
     __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
-    // its fluxes along I (0..2) and J (3..5); in the coloured mode and
-    // with FP32 outputs, at the end, the node sums [5][US]
+    // its fluxes along I (0..2) and J (3..5); with FP32 outputs, at
+    // the end, the node sums [5][US]
     extern __shared__ __attribute__((aligned(16))) double sR[];
     V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
 
@@ -329,7 +329,6 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const int64_t e0 = (int64_t)b * EPB;
     const bool active = t < LANES && e0 + le < a.nelem;
-    const int ec = col_color<COLORED>(pl, active, e0 + le);
     const uint32_t *conn = pl.conn + (int64_t)b * Q * LANES + tc;
 
     // mu_e and mu_sgs change lanes in LDS (k_diffu_col)
@@ -527,7 +526,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
             if (AHEAD) fc = fn;
         }
     });
-    if constexpr (COLORED || SHARED) {
+    if constexpr (SHARED) {
         __syncthreads();  // the last slice's fluxes are read
         for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
         __syncthreads();
@@ -535,7 +534,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     uint32_t at[Q], li[Q];
 #pragma unroll
     for (int k = 0; k < Q; ++k) {
-        at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k) * LANES + tc] : conn[k * LANES];
+        at[k] = conn[k * LANES];
         li[k] = SHARED ? (uint32_t)pl.lidx[((int64_t)b * Q + k) * LANES + tc] : 0u;
     }
 #pragma unroll
@@ -543,20 +542,11 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
         const V2 c = sN[k][t];
         double v[5] = {(double)(c.x * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + c.y * W[k][2])};
-        if constexpr (COLORED) {
-            col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
-        } else if constexpr (SHARED) {
+        if constexpr (SHARED) {
             if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
                 col_add_shared(sR, US, li[k], at[k], v, a.Rmass, a.Rmom, a.Rener, np);
         } else if (col_merge<P>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
-    }
-    if constexpr (COLORED) {
-        const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
-        uint32_t wn[S::UPT];
-        col_list<P>(pl.unode + u0, U, wn);
-        __syncthreads();
-        col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
     }
     if constexpr (SHARED) {
         __syncthreads();
@@ -569,10 +559,10 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
 // and takes 4.4-4.7 ms at 48^3 (3.7 with one wave per SIMD and no spills).
 // Derivatives along K take the mate's half of the column through LDS once;
 // each slice's K fluxes go to the own nodes and, through LDS, to the mate's.  E2
-// elements of a batch per workgroup (coloured mode: all of them).  48^3: 3.09
+// elements of a batch per workgroup.  48^3: 3.09
 // ms, one node per thread 3.49; with all four elements in a workgroup, alone on
 // its CU, 3.56.
-template <int P, int E2, bool COLORED, class A, bool CLOSURE, typename TA>
+template <int P, int E2, class A, bool CLOSURE, typename TA>
 __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a, const float *mlp)
 {
     using S = ColShape<P>;
@@ -582,7 +572,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     constexpr int H = Q / 2, HL = E2 * QQ, NT = 2 * HL, PARTS = EPB / E2;
     static_assert(Q % 2 == 0 && HL % 64 == 0 && LANES == EPB * QQ, "whole waves per half");
     constexpr bool AHEAD = true;  // read line sources one ahead of their use
-    constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
+    constexpr bool SHARED = sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
     __shared__ V2 sP[2][NT];  // one slice: (r,T) (u0,u1)
@@ -590,8 +580,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     __shared__ TG sMu[2][NT];                              // its mu_e, mu_sgs
     __shared__ typename std::conditional<CLOSURE, MlpShared, char>::type smlp;
     // its fluxes along I (0..2), J (3..5) and K (6..8); at the start the columns'
-    // values; in the coloured mode and with FP32 outputs, at the end, the node sums
-    // [5][US]
+    // values; with FP32 outputs, at the end, the node sums [5][US]
     extern __shared__ __attribute__((aligned(16))) double sR[];
     V2(*sF)[NT] = reinterpret_cast<V2(*)[NT]>(sR);
 
@@ -605,7 +594,6 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     const uint32_t b = pl.batches ? uniform(pl.batches)[bs] : bs;
     const int64_t e0 = (int64_t)b * EPB + part * E2;
     const bool active = e0 + le < a.nelem;
-    const int ec = col_color<COLORED>(pl, active, e0 + le);
     const int tc = I + Q * ((int)part * E2 + le + EPB * J), k0 = half * H;
     const uint32_t *conn = pl.conn + ((int64_t)b * Q + k0) * LANES + tc;
     // line_ref of slice j of half h (j a compile-time constant)
@@ -841,7 +829,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
         }
         __builtin_amdgcn_sched_barrier(0);
     });
-    if constexpr (COLORED || SHARED) {
+    if constexpr (SHARED) {
         __syncthreads();  // the last slice's fluxes are read
         for (int i = t; i < 5 * US; i += NT) sR[i] = 0.0;
         __syncthreads();
@@ -849,29 +837,18 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     uint32_t at[H], li[H];
 #pragma unroll
     for (int k = 0; k < H; ++k) {
-        at[k] = COLORED ? (uint32_t)pl.lidx[((int64_t)b * Q + k0 + k) * LANES + tc] : conn[k * LANES];
+        at[k] = conn[k * LANES];
         li[k] = SHARED ? (uint32_t)pl.lidx[((int64_t)b * Q + k0 + k) * LANES + tc] : 0u;
     }
 #pragma unroll
     for (int k = 0; k < H; ++k) {
         double v[5] = {(double)(nu[k] * W[k][0]), (double)W[k][3], (double)W[k][4], (double)W[k][5],
                        (double)(W[k][1] + kappa[k] * W[k][2])};
-        if constexpr (COLORED) {
-            col_add<true>(sR, US, active, ec, pl.rounds, at[k], v);
-        } else if constexpr (SHARED) {
+        if constexpr (SHARED) {
             if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
                 col_add_shared(sR, US, li[k], at[k], v, a.Rmass, a.Rmom, a.Rener, np);
         } else if (col_merge<P, E2>(at[k], I, le, active && e0 + le + 1 < a.nelem, v) && active)
             col_scatter(at[k], v, a.Rmass, a.Rmom, a.Rener, np);
-    }
-    if constexpr (COLORED) {
-        const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
-        __syncthreads();
-        if (t < S::NT) {
-            uint32_t wn[S::UPT];
-            col_list<P>(pl.unode + u0, U, wn);
-            col_write<P, true>(sR, US, wn, U, a.Rmass, a.Rmom, a.Rener, np);
-        }
     }
     if constexpr (SHARED) {
         __syncthreads();
@@ -887,21 +864,22 @@ static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
     const bool registers = P > kNarrowP && atomic && sizeof(typename A::O) == 8;
     const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(TA) * 12 * ColShape<P>::NT;
     const dim3 grid((unsigned)a.plan.nb), block(ColShape<P>::NT);
+    if constexpr (P > kNarrowP)
+        if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
     if constexpr (P == 7) {
         constexpr int E2 = 2, EPB = ColShape<P>::EPB, QQ = ColShape<P>::QQ;
         const size_t part = sizeof(TA) * 2 * 9 * 2 * QQ;  // fluxes per element
-        if (atomic)
-            hipLaunchKernelGGL((k_diffu_split<P, E2, false, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))),
-                               dim3(2 * E2 * QQ), std::max(E2 * part, sums), s, a, mlp);
-        else
-            hipLaunchKernelGGL((k_diffu_split<P, EPB, true, A, CLOSURE, TA>), grid, dim3(2 * EPB * QQ),
-                               std::max(EPB * part, sums), s, a, mlp);
-    } else if constexpr (P > kNarrowP)
-        hipLaunchKernelGGL((atomic ? k_diffu_wide<P, false, A, CLOSURE, TA> : k_diffu_wide<P, true, A, CLOSURE, TA>), grid,
-                           block, std::max(fluxes, sums), s, a, mlp);
-    else
+        hipLaunchKernelGGL((k_diffu_split<P, E2, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))), dim3(2 * E2 * QQ),
+                           std::max(E2 * part, sums), s, a, mlp);
+    } else if constexpr (P > kNarrowP) {
+        hipLaunchKernelGGL((k_diffu_wide<P, A, CLOSURE, TA>), grid, block, std::max(fluxes, sums), s, a, mlp);
+    } else if constexpr (CLOSURE && P == 4) {
+        if (!atomic) return hipErrorInvalidValue;
+        hipLaunchKernelGGL((k_diffu_col<P, false, A, CLOSURE, TA>), grid, block, sums, s, a, mlp);
+    } else {
         hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE, TA> : k_diffu_col<P, true, A, CLOSURE, TA>), grid,
                            block, sums, s, a, mlp);
+    }
     return hipGetLastError();
 }
 

@@ -460,18 +460,37 @@ static hipError_t launch_build_geo_nodes(const T *He, const T *gpvol, int64_t ne
     return hipGetLastError();
 }
 
-// Coloured mode, FP64: whether one node per thread is the faster form.  Its
-// batches are smaller (4 elements against 10 at order 4): where a colour's column
-// batches are fewer than the CUs, its launches end sooner (6x6x8 order 4
-// convection 98 us against 145, 30^3 order 3 the pair 375 against 430; 40^3 order 4
-// 1329 against 1210).  Above kNarrowP a column batch's sums in LDS leave one or
-// two workgroups per CU (40^3 order 5 2.46 ms against 2.63, 48^3 order 7 9.94
-// against 10.4, 32^3 order 8 5.62 against 6.41), but for order 6 (40^3 4.96 against
-// 4.08).  A box has 8 colours.
-static bool nodes_for_colors(int porder, int64_t nelem)
+// Coloured mode: whether one node per thread is the faster form.  Its batches
+// are smaller (4 elements against 10 at order 4) and its sums need fewer rounds,
+// so a launch of few batches ends sooner; the columns move less and compute
+// less.  w: column batches of one colour, of a box's eight.  Times in us, nodes |
+// columns, FP64 (the FP32-storage forms lie within 10% of the same ratios):
+//   convection  order 2  13x11x9 68 | 81, 20^3 113 | 82, 104x90x97 1457 | 1303
+//               order 3  8^3 63 | 80, 13x11x9 102 | 99, 39x35x29 249 | 240, 96^3 3536 | 2973
+//               order 4  16^3 139 | 207, 28^3 275 | 292, 32^3 374 | 318, 64^3 2590 | 2083
+//               order 6  11^3 173 | 322, 18^3 322 | 316, 40^3 2679 | 1568
+//               orders 5, 7, 8: their sums in LDS leave one or two workgroups per CU
+//               (25^3 order 7 0.96 of the speed, 22^3 order 8 0.77, order 5 0.95-1.10)
+//   diffusion   order 2  13x11x9 68 | 86, 33x29x27 132 | 119, 48^3 212 | 238, 80^3 820 | 846
+//               order 3  13x11x9 105 | 107, 16^3 123 | 81, 39x35x29 248 | 265, 96^3 3443 | 2937
+//               order 4  32^3 303 | 377, 40^3 569 | 595, 53x49x51 1295 | 1210, 80^3 4628 | 3722
+//               (FP32 outputs 53x49x51 882 | 940, 80^3 2864 | 2841)
+//               order 6  29^3 887 | 1120; orders 5, 7, 8 0.4-0.8 of the speed
+//   closure     order 3  8^3 122 | 142, 13x11x9 184 | 172, 64^3 1487 | 1264
+//               order 4  40^3 0.69 of the speed (columns spill), 5 to 8 0.4-0.8
+// Where a row of the table has both, the line is drawn between its sizes.
+enum Kernel { kConvec, kDiffu, kClosure };
+static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 {
-    const bool few = nelem < (int64_t)256 * 8 * batch_size(porder);
-    return few || (porder > kNarrowP && porder != 6);
+    const int64_t w = nelem / (8 * batch_size(porder));
+    switch (porder) {
+    case 1: return false;
+    case 2: return w < 8 || (k == kDiffu && w >= 256);
+    case 3: return w < (k == kDiffu ? 16 : 8) || (k == kDiffu && w >= 256 && w < 2048);
+    case 4: return k == kConvec ? w < 320 : k == kClosure || out32 || w < 1500;
+    case 6: return k != kConvec || w < 128;
+    default: return true;
+    }
 }
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
@@ -1267,8 +1286,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    constexpr bool kF64 = std::is_same<ConvecArgs<TG, TF, TO, TU, TP>, ConvecArgs<double, double>>::value;
-    bool nodes = fp32_arith || (kF64 && g.assembly == kColored && nodes_for_colors(porder, NE));
+    bool nodes = fp32_arith || (g.assembly == kColored && nodes_for_colors(kConvec, porder, NE, sizeof(TO) == 4));
     if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
@@ -1330,7 +1348,8 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     const PlanEntry *plan;
     const TG *geo;
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
-    bool nodes = fp32_arith || (kF64 && !dmlp && g.assembly == kColored && nodes_for_colors(porder, NE));
+    bool nodes = fp32_arith || (g.assembly == kColored &&
+                                nodes_for_colors(dmlp ? kClosure : kDiffu, porder, NE, sizeof(TO) == 4));
     if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
