@@ -1,8 +1,9 @@
 // Assembly plan of a mesh (host code, no HIP): the data the kernels' write
-// phase uses (layout described in msod_kernels.h), for the coloured assembly;
-// the atomic one has its node lists from the device (k_plan_batches in
-// msod_runtime.hip, the same lists).  Built once per mesh from
-// the reference connectivity connec(nelem,nnode) (1-based, Fortran layout):
+// phase uses (layout described in msod_kernels.h).  The library builds the node
+// lists on the device (k_plan_batches in msod_runtime.hip) and only colours here,
+// for the coloured assembly; build_host_plan makes the whole plan, as the CPU
+// checks read it, from the reference connectivity connec(nelem,nnode) (1-based,
+// Fortran layout):
 //   * batches of B consecutive elements;
 //   * the sorted distinct nodes of every batch (unode, offsets uoff) and the
 //     position of every element node in its batch's list (lidx);
@@ -61,6 +62,44 @@ void plan_parallel_for(int64_t n, F f)
     }
     for (auto &t : th) t.join();
 }
+
+// Entry of node l of element e in the lane layout of msod_columns.h (l in its
+// order: ascending along each line), batches of B elements, q nodes a line.
+inline int64_t lane_entry(int q, int B, int64_t e, int l)
+{
+    return (e / B * q + l / (q * q)) * B * q * q + l % q + q * (e % B + B * (l / q % q));
+}
+
+// Colours of the elements of each batch: nodes that two of them share have the
+// same position in the batch's list, lidx(e, l).
+template <class F>
+void color_elements(HostPlan &P, int64_t nelem, int nn, const F &lidx)
+{
+    P.ecol.assign(nelem, 0);
+    std::atomic<int> rounds{1};
+    plan_parallel_for(P.nbatch, [&](int64_t lo, int64_t hi) {
+        std::vector<uint64_t> used;
+        int most = 1;
+        for (int64_t b = lo; b < hi; ++b) {
+            const int64_t e0 = b * P.B, e1 = std::min<int64_t>(nelem, e0 + P.B);
+            used.assign(P.uoff[b + 1] - P.uoff[b], 0u);
+            for (int64_t e = e0; e < e1; ++e) {
+                uint64_t forb = 0;
+                for (int l = 0; l < nn; ++l) forb |= used[lidx(e, l)];
+                const int c = __builtin_ctzll(~forb);  // free: a batch has at most 64 elements
+                P.ecol[e] = (uint8_t)c;
+                most = std::max(most, c + 1);
+                for (int l = 0; l < nn; ++l) used[lidx(e, l)] |= uint64_t(1) << c;
+            }
+        }
+        int cur = rounds.load();
+        while (cur < most && !rounds.compare_exchange_weak(cur, most)) {}
+    });
+    P.rounds = rounds.load();
+}
+
+// Colours of the batches, first writers and unreferenced nodes, from the lists.
+inline void color_batches(HostPlan &P, int64_t npoin);
 
 // raw: connec(nelem,nnode) as stored by the reference; l2g[l]: 0-based Gmsh
 // node of lexicographic node l.  Returns false with a message in *err.
@@ -140,28 +179,14 @@ inline bool build_host_plan(const int32_t *raw, int64_t nelem, int64_t npoin,
         return false;
     }
 
-    P.ecol.assign(nelem, 0);
-    std::atomic<int> rounds{1};
-    plan_parallel_for(NB, [&](int64_t lo, int64_t hi) {
-        std::vector<uint64_t> used;
-        int most = 1;
-        for (int64_t b = lo; b < hi; ++b) {
-            const int64_t e0 = b * B, e1 = std::min<int64_t>(nelem, e0 + B);
-            used.assign(P.uoff[b + 1] - P.uoff[b], 0u);
-            for (int64_t e = e0; e < e1; ++e) {
-                uint64_t forb = 0;
-                for (int l = 0; l < nn; ++l) forb |= used[P.lidx[e * nn + l]];
-                const int c = __builtin_ctzll(~forb);  // free: a batch has at most 64 elements
-                P.ecol[e] = (uint8_t)c;
-                most = std::max(most, c + 1);
-                for (int l = 0; l < nn; ++l) used[P.lidx[e * nn + l]] |= uint64_t(1) << c;
-            }
-        }
-        int cur = rounds.load();
-        while (cur < most && !rounds.compare_exchange_weak(cur, most)) {}
-    });
-    P.rounds = rounds.load();
+    color_elements(P, nelem, nn, [&](int64_t e, int l) { return P.lidx[e * nn + l]; });
+    color_batches(P, npoin);
+    return true;
+}
 
+inline void color_batches(HostPlan &P, int64_t npoin)
+{
+    const int64_t NB = P.nbatch;
     // greedy colouring: bit c of mask[node] is set once a batch of colour c
     // holds the node.  Past 32 colours the colouring is abandoned: the
     // atomic assembly does not need it.
@@ -194,7 +219,7 @@ inline bool build_host_plan(const int32_t *raw, int64_t nelem, int64_t npoin,
         P.order.resize(NB);
         for (int64_t b = 0; b < NB; ++b) P.order[b] = (uint32_t)b;
         P.colored = false;
-        return true;
+        return;
     }
     plan_parallel_for(NB, [&](int64_t lo, int64_t hi) {
         for (int64_t b = lo; b < hi; ++b) {
@@ -213,7 +238,6 @@ inline bool build_host_plan(const int32_t *raw, int64_t nelem, int64_t npoin,
     std::vector<int64_t> pos(P.color_off.begin(), P.color_off.end() - 1);
     for (int64_t b = 0; b < NB; ++b) P.order[pos[color[b]]++] = (uint32_t)b;
     P.colored = true;
-    return true;
 }
 
 }  // namespace msod

@@ -192,7 +192,8 @@ __global__ void k_build_geo_nodes(const T *He, const T *gpvol, int64_t nelem, in
 // nodes are sorted in LDS (bitonic) and the distinct ones numbered in
 // ascending order, as build_host_plan does on the host.  FILL = false:
 // count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
-// unode from uoff, conn and lidx in the lane layout.  lists (PlanLists): every
+// unode from uoff, conn and lidx in the lane layout or (lanes = false)
+// element-major (msod_nodes.h).  lists (PlanLists): every
 // node of the batch, those alone that several lanes write after col_merge has
 // taken neighbours' nodes together (the others' lidx is kAlone), or none, for
 // kernels that read conn alone (count[b] = 0, the rest null).
@@ -209,8 +210,8 @@ struct PlanShape {
 };
 template <int P, bool FILL>
 __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                                                      int lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
-                                                      uint32_t *unode, uint32_t *conn, uint16_t *lidx)
+                                                      int lists, bool lanes, const int32_t *l2g, const uint32_t *uoff,
+                                                      uint32_t *count, uint32_t *unode, uint32_t *conn, uint16_t *lidx)
 {
     using S = PlanShape<P>;
     constexpr int NN = S::NN, NT = S::NT, SORT = S::SORT, PER = S::PER;
@@ -323,9 +324,12 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
                 const uint32_t m = (lo + hi) / 2;
                 (su[m] <= v[j] ? lo : hi) = m;
             }
-            const ElemEntry<P> en{e0 + i % B, i / B};
-            conn[en.entry()] = v[j];
-            lidx[en.entry()] = lists == kListAll || (U > 0 && su[lo] == v[j]) ? (uint16_t)lo : kAlone;
+            const int64_t e = e0 + i % B;
+            const int l = i / B;
+            if (!lanes && i % B >= ne) continue;
+            const int64_t at = lanes ? ElemEntry<P>{e, l}.entry() : e * NN + l;
+            conn[at] = v[j];
+            lidx[at] = lists == kListAll || (U > 0 && su[lo] == v[j]) ? (uint16_t)lo : kAlone;
         }
     }
 }
@@ -495,18 +499,18 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
 hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
-                               int lists, const int32_t *l2g, const uint32_t *uoff, uint32_t *count, uint32_t *unode,
-                               uint32_t *conn, uint16_t *lidx, hipStream_t s)
+                               int lists, bool lanes, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
+                               uint32_t *unode, uint32_t *conn, uint16_t *lidx, hipStream_t s)
 {
     return with_porder(porder, [&](auto p) {
         if (B > PlanShape<p()>::UMAX / PlanShape<p()>::NN) return hipErrorInvalidValue;
         const dim3 grid((unsigned)((nelem + B - 1) / B)), block(PlanShape<p()>::NT);
         if (fill)
-            hipLaunchKernelGGL((k_plan_batches<p(), true>), grid, block, 0, s, connec, nelem, npoin, B, lists, l2g, uoff, count,
-                               unode, conn, lidx);
-        else
-            hipLaunchKernelGGL((k_plan_batches<p(), false>), grid, block, 0, s, connec, nelem, npoin, B, lists, l2g, uoff,
+            hipLaunchKernelGGL((k_plan_batches<p(), true>), grid, block, 0, s, connec, nelem, npoin, B, lists, lanes, l2g, uoff,
                                count, unode, conn, lidx);
+        else
+            hipLaunchKernelGGL((k_plan_batches<p(), false>), grid, block, 0, s, connec, nelem, npoin, B, lists, lanes, l2g,
+                               uoff, count, unode, conn, lidx);
         return hipGetLastError();
     });
 }
@@ -557,7 +561,7 @@ struct PlanEntry {
     std::vector<int64_t> color_off;  // batches of colour c: order[color_off[c] .. color_off[c+1])
     uint32_t *unref = nullptr;       // nodes no element references (zeroed per call)
     int64_t nunref = 0;
-    bool nodes = false;              // element-major, of the FP32-arithmetic kernels (msod_nodes.h)
+    bool nodes = false;              // element-major (msod_nodes.h)
     int lists = kListAll;            // the nodes in unode
     bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
@@ -863,11 +867,13 @@ int upload(const std::vector<V> &h, V **d, const char *what)
     return MSOD_OK;
 }
 
-// Builds the node lists of a mesh's batches on the device: all that the atomic
-// assembly reads of the plan.
+// Builds the node lists of a mesh's batches on the device (P.nodes: for the
+// kernels with one node per thread): all that the atomic assembly reads of the
+// plan, but for the order of the colours (msod_full_convec_ijk_fp32).
 int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, int lists,
                       PlanEntry &P)
 {
+    const bool lanes = !P.nodes;
     const int64_t nn = (int64_t)ts->l2g.size(), nb = (nelem + B - 1) / B;
     if (npoin > 0x7fffffff || nelem * nn > 0xffffffffLL)
         return fail(MSOD_ERR_MESH, "mesh too large for 32-bit node indices");
@@ -878,8 +884,8 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
     // feeds the host plan waits for
     HIPCHK(hipStreamSynchronize(nullptr), "plan");
     HIPCHK(hipMalloc((void **)&P.uoff, sizeof(uint32_t) * (nb + 1)), "plan");
-    HIPCHK(launch_plan_batches(ts->porder, false, dconnec, nelem, npoin, B, lists, ts->dl2g, nullptr, P.uoff, nullptr, nullptr,
-                               nullptr, g.stream),
+    HIPCHK(launch_plan_batches(ts->porder, false, dconnec, nelem, npoin, B, lists, lanes, ts->dl2g, nullptr, P.uoff, nullptr,
+                               nullptr, nullptr, g.stream),
            "batch counts");
     std::vector<uint32_t> uoff(nb + 1);
     HIPCHK(hipMemcpyAsync(uoff.data() + 1, P.uoff, sizeof(uint32_t) * nb, hipMemcpyDeviceToHost, g.stream),
@@ -897,15 +903,15 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
     if (bad)
         return fail(MSOD_ERR_MESH, "connec holds %lld node numbers outside 1..npoin (npoin=%lld)", (long long)bad,
                     (long long)npoin);
-    const int64_t n = geo_elems(ts->porder, nelem) * nn;
+    const int64_t n = (lanes ? geo_elems(ts->porder, nelem) : nelem) * nn;
     HIPCHK(hipMalloc((void **)&P.conn, sizeof(uint32_t) * n), "plan");
     if (lists != kListNone) {
         HIPCHK(hipMalloc((void **)&P.lidx, sizeof(uint16_t) * n), "plan");
         HIPCHK(hipMalloc((void **)&P.unode, sizeof(uint32_t) * std::max(uoff[nb], 1u)), "plan");
     }
     HIPCHK(hipMemcpyAsync(P.uoff, uoff.data(), sizeof(uint32_t) * (nb + 1), hipMemcpyHostToDevice, g.stream), "plan");
-    HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, lists, ts->dl2g, P.uoff, nullptr, P.unode, P.conn,
-                               P.lidx, g.stream),
+    HIPCHK(launch_plan_batches(ts->porder, true, dconnec, nelem, npoin, B, lists, lanes, ts->dl2g, P.uoff, nullptr, P.unode,
+                               P.conn, P.lidx, g.stream),
            "batch lists");
     HIPCHK(hipStreamSynchronize(g.stream), "batch lists");
     return MSOD_OK;
@@ -913,54 +919,36 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
 
 // Adds to the device's lists what the coloured assembly needs (msod_plan.h):
 // the colourings, the first writers and the unreferenced nodes, found on the
-// host from the connectivity.
-int build_host_part(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
+// host from those lists.
+int build_host_part(PlanEntry &P)
 {
-    const int64_t E = nelem * (int64_t)ts->l2g.size();
-    std::vector<int32_t> raw(E);
-    HIPCHK(hipMemcpy(raw.data(), dconnec, sizeof(int32_t) * E, hipMemcpyDeviceToHost),
-           "reading connec");
     HostPlan H;
-    std::string err;
-    if (!build_host_plan(raw.data(), nelem, npoin, ts->l2g, B, H, &err))
-        return fail(MSOD_ERR_MESH, "%s", err.c_str());
+    H.B = P.B;
+    H.nbatch = P.nbatch;
+    H.uoff.resize(P.nbatch + 1);
+    HIPCHK(hipStreamSynchronize(g.stream), "plan");  // kernels may be reading the lists
+    HIPCHK(hipMemcpy(H.uoff.data(), P.uoff, sizeof(uint32_t) * H.uoff.size(), hipMemcpyDeviceToHost), "reading the batch lists");
+    H.unode.resize(H.uoff.back());
+    HIPCHK(hipMemcpy(H.unode.data(), P.unode, sizeof(uint32_t) * H.unode.size(), hipMemcpyDeviceToHost), "reading the batch lists");
+    int st;
+    if (!P.nodes) {  // the column kernels add a batch's elements by colour
+        const int q = P.porder + 1, qq = q * q;
+        const int64_t lanes = (int64_t)P.B * qq;
+        H.lidx.resize(P.nbatch * q * lanes);
+        HIPCHK(hipMemcpy(H.lidx.data(), P.lidx, sizeof(uint16_t) * H.lidx.size(), hipMemcpyDeviceToHost),
+               "reading the batch lists");
+        color_elements(H, P.nelem, q * qq, [&](int64_t e, int l) { return H.lidx[lane_entry(q, P.B, e, l)]; });
+        if ((st = upload(H.ecol, &P.ecol, "plan upload"))) return st;
+    }
+    color_batches(H, P.npoin);
     P.color_off = H.color_off;
     P.colored = H.colored;
     P.rounds = H.rounds;
     HIPCHK(hipMemcpy(P.unode, H.unode.data(), sizeof(uint32_t) * H.unode.size(), hipMemcpyHostToDevice), "plan upload");
-    int st;
     if ((st = upload(H.order, &P.order, "plan upload"))) return st;
     if ((st = upload(H.unref, &P.unref, "plan upload"))) return st;
-    if ((st = upload(H.ecol, &P.ecol, "plan upload"))) return st;
     P.nunref = (int64_t)H.unref.size();
     P.host = true;
-    return MSOD_OK;
-}
-
-// The plan of the FP32-arithmetic kernels (msod_nodes.h), from the host.
-int build_nodes_plan(const void *dconnec, int64_t nelem, int64_t npoin, const TableSet *ts, int B, PlanEntry &P)
-{
-    const int64_t E = nelem * (int64_t)ts->l2g.size();
-    std::vector<int32_t> raw(E);
-    HIPCHK(hipMemcpy(raw.data(), dconnec, sizeof(int32_t) * E, hipMemcpyDeviceToHost), "reading connec");
-    HostPlan H;
-    std::string err;
-    if (!build_host_plan(raw.data(), nelem, npoin, ts->l2g, B, H, &err))
-        return fail(MSOD_ERR_MESH, "%s", err.c_str());
-    std::vector<int32_t>().swap(raw);
-    P.B = H.B;
-    P.nbatch = H.nbatch;
-    P.color_off = H.color_off;
-    P.colored = H.colored;
-    int st;
-    if ((st = upload(H.conn, &P.conn, "plan upload"))) return st;
-    if ((st = upload(H.lidx, &P.lidx, "plan upload"))) return st;
-    if ((st = upload(H.uoff, &P.uoff, "plan upload"))) return st;
-    if ((st = upload(H.unode, &P.unode, "plan upload"))) return st;
-    if ((st = upload(H.order, &P.order, "plan upload"))) return st;
-    if ((st = upload(H.unref, &P.unref, "plan upload"))) return st;
-    P.nunref = (int64_t)H.unref.size();
-    P.host = P.nodes = true;
     return MSOD_OK;
 }
 
@@ -986,25 +974,26 @@ void drop_unversioned(const void *src)
         }
 }
 
-// lists: the node lists that the call's kernels read (kListNone: any plan will do).
+// lists: the node lists that the call's kernels read (kListNone: any plan will
+// do).  host: with the colours (the atomic assembly takes either plan).
 int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, const TableSet *ts, int B, int lists,
-             const PlanEntry **out, bool nodes = false)
+             bool host, const PlanEntry **out, bool nodes = false)
 {
     if (ver == 0) drop_unversioned(dconnec);
-    const bool host = g.assembly == kColored;  // the atomic assembly takes either plan
     if (host) lists = kListAll;
     for (size_t i = 0; i < g.plans.size(); ++i) {
         PlanEntry &c = g.plans[i];
         if (c.src != dconnec || c.ver != ver || c.nelem != nelem || c.npoin != npoin || c.porder != ts->porder ||
             c.l2g != ts->l2g || c.B != B || c.nodes != nodes || (lists != kListNone && c.lists != lists))
             continue;
-        if (c.host || !host) {
-            *out = &c;
-            return MSOD_OK;
+        int st = MSOD_OK;
+        if (host && !c.host && (st = build_host_part(c))) {
+            c.release();  // hipFree waits for the work queued
+            g.plans.erase(g.plans.begin() + i);
+            return st;
         }
-        c.release();  // hipFree waits for the work queued
-        g.plans.erase(g.plans.begin() + i);
-        break;
+        *out = &c;
+        return MSOD_OK;
     }
     PlanEntry P;
     P.src = dconnec;
@@ -1013,9 +1002,9 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
     P.npoin = npoin;
     P.porder = ts->porder;
     P.l2g = ts->l2g;
-    int st = nodes ? build_nodes_plan(dconnec, nelem, npoin, ts, B, P)
-                   : build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, lists, P);
-    if (!st && host && !nodes) st = build_host_part(dconnec, nelem, npoin, ts, B, P);
+    P.nodes = nodes;
+    int st = build_device_plan((const int32_t *)dconnec, nelem, npoin, ts, B, lists, P);
+    if (!st && host) st = build_host_part(P);
     if (st) {
         P.release();
         return st;
@@ -1185,19 +1174,21 @@ int column_lists(int porder)
 }
 
 // The plan of a call: of the kernels with one node per thread (batches of NB
-// elements) where *nodes says so, of the column kernels otherwise.  *nodes is set
-// where those turn out not to suit the mesh: in the coloured mode, when their
-// batches need more than 32 colours.
+// elements) where *nodes says so, of the column kernels otherwise.  natural: the
+// atomic launch takes the batches in mesh order.  *nodes is set where columns
+// turn out not to suit the mesh: in the coloured mode, when their batches need
+// more than 32 colours.
 template <typename TO>
-int choose_plan(const void *dc, uint64_t vc, int64_t NE, int64_t NP, const TableSet *ts, int NB, bool *nodes,
+int choose_plan(const void *dc, uint64_t vc, int64_t NE, int64_t NP, const TableSet *ts, int NB, bool natural, bool *nodes,
                 const PlanEntry **plan)
 {
+    const bool colored = g.assembly == kColored;
     if (!*nodes) {
-        const int st = get_plan(dc, vc, NE, NP, ts, batch_size(ts->porder), column_lists<TO>(ts->porder), plan);
+        const int st = get_plan(dc, vc, NE, NP, ts, batch_size(ts->porder), column_lists<TO>(ts->porder), colored, plan);
         if (st) return st;
-        *nodes = g.assembly == kColored && !(*plan)->colored;
+        *nodes = colored && !(*plan)->colored;
     }
-    return *nodes ? get_plan(dc, vc, NE, NP, ts, NB, kListAll, plan, true) : MSOD_OK;
+    return *nodes ? get_plan(dc, vc, NE, NP, ts, NB, kListAll, colored || !natural, plan, true) : MSOD_OK;
 }
 
 // Zero-fill (atomic mode) or unreferenced-node zeroing (coloured mode), then
@@ -1287,7 +1278,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     const PlanEntry *plan;
     const TG *geo;
     bool nodes = fp32_arith || (g.assembly == kColored && nodes_for_colors(kConvec, porder, NE, sizeof(TO) == 4));
-    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), &nodes, &plan))) return st;
+    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), !fp32_arith, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
@@ -1311,7 +1302,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
                                     if (fp32_arith) return launch_convec_fp32(porder, x, g.stream);
                                 return nodes ? launch_convec_nodes(porder, x, g.stream) : launch_convec(porder, x, g.stream);
                             },
-                            "convection kernel launch", !nodes, nodes ? kBatchesPerBlock : 1)))
+                            "convection kernel launch", !fp32_arith, nodes ? kBatchesPerBlock : 1)))
         return st;
     return finish_call("convection kernel");
 }
@@ -1350,7 +1341,7 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
     bool nodes = fp32_arith || (g.assembly == kColored &&
                                 nodes_for_colors(dmlp ? kClosure : kDiffu, porder, NE, sizeof(TO) == 4));
-    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), &nodes, &plan))) return st;
+    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), true, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;
@@ -1499,7 +1490,7 @@ int closure_elem_common(int porder, int nelem, int npoin, const int32_t *connec,
     if ((st = resolve(u, sizeof(double) * 3 * NP, "u", &du, &vx))) return st;
     const PlanEntry *plan;
     const double *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), kListNone, &plan))) return st;
+    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), kListNone, false, &plan))) return st;
     if ((st = get_geo<double>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
     a = ClosureElemArgs{};
     a.nelem = NE;
