@@ -497,6 +497,38 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
     }
 }
 
+// Default mode: whether one node per thread is the faster form.  With fewer column
+// batches (nb) than CUs a launch lasts as long as one workgroup, which walks its
+// slices one after the other; the former kernels' workgroups hold fewer elements
+// and work on all of their nodes at once.  Whole calls in us, nodes | columns,
+// FP64 (the FP32-storage forms cross within 30% of the same nb):
+//   order  convection               diffusion
+//   3      nb 32 31.3|32.0, 63 32.7|32.7, 99 34.3|33.9    32 32.6|33.4, 99 36.0|35.5
+//   4      1 31.5|33.8, 65 34.6|36.4, 100 37.5|37.1       1 32.8|35.8, 65 35.9|38.3, 100 38.1|39.0
+//   5      1 32.8|35.8, 31 35.2|36.5, 64 37.8|36.8        1 33.8|41.2, 129 44.5|45.9, 191 50.2|49.3
+//   6      1 36.6|39.2, 30 39.5|39.9, 51 41.4|40.2        1 32.3|46.3, 103 45.1|51.6, 130 53.8|54.6
+//   8      1 47.6|52.6, 60 55.2|55.4, 98 60.1|58.8        1 40.0|52.5, 60 47.6|55.4, 98 63.1|60.0
+// Orders 1, 2 and 7 (two threads a column in the diffusion) are faster as columns
+// from the first element on.
+static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
+{
+    const int64_t nb = (nelem + batch_size(porder) - 1) / batch_size(porder);
+    switch (porder) {
+    case 3: return nb < 48;
+    case 4: return nb < 88;
+    case 5: return nb < (k == kConvec ? 48 : 150);
+    case 6: return nb < (k == kConvec ? 24 : 128);
+    case 8: return nb < 80;
+    default: return false;
+    }
+}
+
+// Whether a call starts out with the kernels with one node per thread.
+static bool take_nodes(Kernel k, int mode, int porder, int64_t nelem, bool out32)
+{
+    return mode == kColored ? nodes_for_colors(k, porder, nelem, out32) : nodes_for_atomics(k, porder, nelem);
+}
+
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
 hipError_t launch_plan_batches(int porder, bool fill, const int32_t *connec, int64_t nelem, int64_t npoin, int B,
                                int lists, bool lanes, const int32_t *l2g, const uint32_t *uoff, uint32_t *count,
@@ -1277,7 +1309,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     if ((st = resolve(Rener, sizeof(TO) * NP, "Rener", &dRe, &vx))) return st;
     const PlanEntry *plan;
     const TG *geo;
-    bool nodes = fp32_arith || (g.assembly == kColored && nodes_for_colors(kConvec, porder, NE, sizeof(TO) == 4));
+    bool nodes = fp32_arith || take_nodes(kConvec, g.assembly, porder, NE, sizeof(TO) == 4);
     if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), !fp32_arith, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
@@ -1339,8 +1371,7 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     const PlanEntry *plan;
     const TG *geo;
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
-    bool nodes = fp32_arith || (g.assembly == kColored &&
-                                nodes_for_colors(dmlp ? kClosure : kDiffu, porder, NE, sizeof(TO) == 4));
+    bool nodes = fp32_arith || take_nodes(dmlp ? kClosure : kDiffu, g.assembly, porder, NE, sizeof(TO) == 4);
     if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), true, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
