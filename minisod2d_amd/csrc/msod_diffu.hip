@@ -866,16 +866,15 @@ static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
     const dim3 grid((unsigned)a.plan.nb), block(ColShape<P>::NT);
     if constexpr (P > kNarrowP)
         if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
-    if constexpr (P == 7) {
+    if constexpr (CLOSURE && (P == 4 || P == 5 || P == 8)) {
+        return hipErrorInvalidValue;  // and there (nodes_for_atomics)
+    } else if constexpr (P == 7) {
         constexpr int E2 = 2, EPB = ColShape<P>::EPB, QQ = ColShape<P>::QQ;
         const size_t part = sizeof(TA) * 2 * 9 * 2 * QQ;  // fluxes per element
         hipLaunchKernelGGL((k_diffu_split<P, E2, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))), dim3(2 * E2 * QQ),
                            std::max(E2 * part, sums), s, a, mlp);
     } else if constexpr (P > kNarrowP) {
         hipLaunchKernelGGL((k_diffu_wide<P, A, CLOSURE, TA>), grid, block, std::max(fluxes, sums), s, a, mlp);
-    } else if constexpr (CLOSURE && P == 4) {
-        if (!atomic) return hipErrorInvalidValue;
-        hipLaunchKernelGGL((k_diffu_col<P, false, A, CLOSURE, TA>), grid, block, sums, s, a, mlp);
     } else {
         hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE, TA> : k_diffu_col<P, true, A, CLOSURE, TA>), grid,
                            block, sums, s, a, mlp);

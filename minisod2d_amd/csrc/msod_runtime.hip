@@ -480,7 +480,8 @@ static hipError_t launch_build_geo_nodes(const T *He, const T *gpvol, int64_t ne
 //               order 4  32^3 303 | 377, 40^3 569 | 595, 53x49x51 1295 | 1210, 80^3 4628 | 3722
 //               (FP32 outputs 53x49x51 882 | 940, 80^3 2864 | 2841)
 //               order 6  29^3 887 | 1120; orders 5, 7, 8 0.4-0.8 of the speed
-//   closure     order 3  8^3 122 | 142, 13x11x9 184 | 172, 64^3 1487 | 1264
+//   closure     order 2  13x11x9 124 | 141, 33x29x27 223 | 186, 80^3 1321 | 1095
+//               order 3  8^3 122 | 142, 13x11x9 184 | 172, 64^3 1487 | 1264
 //               order 4  40^3 0.69 of the speed (columns spill), 5 to 8 0.4-0.8
 // Where a row of the table has both, the line is drawn between its sizes.
 enum Kernel { kConvec, kDiffu, kClosure };
@@ -509,10 +510,27 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 //   6      1 36.6|39.2, 30 39.5|39.9, 51 41.4|40.2        1 32.3|46.3, 103 45.1|51.6, 130 53.8|54.6
 //   8      1 47.6|52.6, 60 55.2|55.4, 98 60.1|58.8        1 40.0|52.5, 60 47.6|55.4, 98 63.1|60.0
 // Orders 1, 2 and 7 (two threads a column in the diffusion) are faster as columns
-// from the first element on.
+// from the first element on.  With the network's features and weights the columns
+// run out of registers from order 4 on (13 spilled at order 4, 33 at 5, 70 at 6) and
+// have a CU to themselves at order 8:
+//   closure  order 3  nb 256 68|71, 326 76|80, 500 88|83, 5952 398|386
+//            order 4  35 61|72, 521 103|141, 5932 530|819
+//            order 5  35 63|81, 515 122|145, 5950 718|836
+//            order 6  130 90|104, 200 105|109, 267 129|124, 5959 1614|1203
+//            order 7  63 66|73, 128 77|81, 162 89|84, 6098 996|960
+//            order 8  34 66|99, 789 276|324, 2940 845|878, 6084 1671|1674, 19773 5244|5185
 static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
 {
     const int64_t nb = (nelem + batch_size(porder) - 1) / batch_size(porder);
+    if (k == kClosure) switch (porder) {
+        case 3: return nb < 400;
+        case 4:
+        case 5:
+        case 8: return true;
+        case 6: return nb < 220;
+        case 7: return nb < 140;
+        default: return false;
+        }
     switch (porder) {
     case 3: return nb < 48;
     case 4: return nb < 88;
