@@ -21,9 +21,9 @@
 // waves per SIMD (208-230 VGPRs), whose FP64 work and LDS reads alone take 7.1 ms
 // (convection, 128^3).
 //
-// The launch takes the batches in mesh order, one workgroup each: neighbouring
-// batches run side by side and share lines in L2 (order 4, 128^3 convection:
-// 15.9 ms in colour order).  A workgroup that walked several batches with the
+// The launch takes the batches in mesh order (xcd_runs), one workgroup each:
+// neighbouring batches run side by side and share lines in L2 (order 4, 128^3
+// convection: 15.9 ms in colour order).  A workgroup that walked several batches with the
 // next one's gathers in flight was slower (128^3 14.6-15.5 ms): its waits for
 // the gathers wait for the atomics issued after them as well.
 //
@@ -96,6 +96,23 @@ template <typename T>
 __device__ __forceinline__ Uniform<T> uniform(const T *p)
 {
     return (Uniform<T>)p;
+}
+
+// Workgroup i's batch (xcd_range's purpose): every XCD takes runs of kXcdRun
+// neighbouring batches in turn, so that all XCDs stay in one region of the mesh,
+// whose lines they find in the memory-side cache.  With one eighth of the mesh
+// per XCD they do not where consecutive elements leave the rows of nodes and each
+// line is read again a plane of elements later: elements ordered along z, order 4,
+// 40^3 convection 805 us, in runs of 32 622 (256: 624, 2048: 804, 1: 604), diffusion
+// 753 and 611; 62^3 3122 and 2081; 39^3 order 7 2886 and 2010.  Elements along the
+// rows: 62^3 order 4 1277 and 1194, 128^3 11.05 and 10.60 ms, 25^3 112 and 111 us; order
+// 7 diffusion 39^3 1767 and 1753 (runs of 1: 1876).
+__device__ __forceinline__ uint32_t xcd_runs(uint32_t i, uint32_t n)
+{
+    constexpr uint32_t kXcd = 8, kXcdRun = 32;
+    const uint32_t x = i % kXcd, k = i / kXcd, whole = n / (kXcd * kXcdRun) * (kXcd * kXcdRun);
+    if (i < whole) return k / kXcdRun * (kXcd * kXcdRun) + x * kXcdRun + k % kXcdRun;
+    return whole + xcd_range(i - whole, n - whole);
 }
 
 // One thread's place in its batch.

@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
     const int tc = th.tc, le = th.le, I = th.I, J = th.J;
     const int64_t np = a.npoin;
     const auto D = uniform(a.tab.D);
-    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t slot = xcd_runs(blockIdx.x, gridDim.x);
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
     const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
@@ -236,7 +236,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
     const int tc = th.tc, le = th.le, I = th.I, J = th.J;
     const int64_t np = a.npoin;
     const auto D = uniform(a.tab.D);
-    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t slot = xcd_runs(blockIdx.x, gridDim.x);
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const bool active = t < LANES && (int64_t)b * EPB + le < a.nelem;
     const int ec = col_color<COLORED>(pl, active, (int64_t)b * EPB + le);

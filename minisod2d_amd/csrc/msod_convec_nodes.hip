@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(CShape<P>::NT, (convec_waves<P, TA, typename A
     constexpr int NT = S::NT, UPT = (UMAX + NT - 1) / NT;
 
     const Plan &pl = a.plan;
-    const int64_t first = (int64_t)xcd_slot(blockIdx.x, gridDim.x) * pl.kpb;
+    const int64_t first = (int64_t)xcd_range(blockIdx.x, gridDim.x) * pl.kpb;
     const int nbat = (int)(pl.nb - first < pl.kpb ? pl.nb - first : pl.kpb);
     const int npass = nbat * NPASS;  // passes of this block, over its batches
     const int t = threadIdx.x;

@@ -55,7 +55,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
     const int tc = th.tc, le = th.le, I = th.I, J = th.J;
     const int64_t np = a.npoin;
     const auto D = uniform(a.tab.D);
-    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t slot = xcd_runs(blockIdx.x, gridDim.x);
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const uint32_t u0 = uniform(pl.uoff)[b], U = uniform(pl.uoff)[b + 1] - u0;
     const int64_t e0 = (int64_t)b * EPB;
@@ -325,7 +325,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
     const int tc = th.tc, le = th.le, I = th.I, J = th.J;
     const int64_t np = a.npoin;
     const auto D = uniform(a.tab.D);
-    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x);
+    const uint32_t slot = xcd_runs(blockIdx.x, gridDim.x);
     const uint32_t b = pl.batches ? uniform(pl.batches)[slot] : slot;
     const int64_t e0 = (int64_t)b * EPB;
     const bool active = t < LANES && e0 + le < a.nelem;
@@ -590,7 +590,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     const int I = tl % Q, le = tl / Q % E2, J = tl / (Q * E2);
     const int64_t np = a.npoin;
     const auto D = uniform(a.tab.D);
-    const uint32_t slot = xcd_slot(blockIdx.x, gridDim.x), bs = slot / PARTS, part = slot % PARTS;
+    const uint32_t slot = xcd_runs(blockIdx.x, gridDim.x), bs = slot / PARTS, part = slot % PARTS;
     const uint32_t b = pl.batches ? uniform(pl.batches)[bs] : bs;
     const int64_t e0 = (int64_t)b * EPB + part * E2;
     const bool active = e0 + le < a.nelem;

@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(GeomShape<P>::NT) k_elem_jacobian(GeomArgs a)
     __shared__ double sX[EB * (NN + 1) * 3];
     __shared__ double sH[EB * NN * 9];
     const int t = threadIdx.x;
-    const int64_t ec0 = (int64_t)xcd_slot(blockIdx.x, gridDim.x) * EC;
+    const int64_t ec0 = (int64_t)xcd_range(blockIdx.x, gridDim.x) * EC;
     const int nec = (int)(a.nelem - ec0 < EC ? a.nelem - ec0 : EC);
 
     for (int i = t; i < EC * NN; i += NT) {

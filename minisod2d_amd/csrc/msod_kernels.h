@@ -179,11 +179,10 @@ struct GeoNode {
 };
 
 // Blocks of a launch are dealt to the chip's 8 XCDs round robin (block i to
-// XCD i % 8), each XCD with its own L2.  xcd_slot gives every XCD a
-// contiguous range of the launch's batch list, so that batches adjacent in
-// the list (which share nodes and cache lines) meet in the same L2.
-// Bijective on [0, n) for any n.
-__device__ __forceinline__ uint32_t xcd_slot(uint32_t i, uint32_t n)
+// XCD i % 8), each XCD with its own L2.  xcd_range gives every XCD a
+// contiguous range of [0, n), so that neighbours (which share nodes and cache
+// lines) meet in the same L2.  Bijective for any n.
+__device__ __forceinline__ uint32_t xcd_range(uint32_t i, uint32_t n)
 {
     constexpr uint32_t kXcd = 8;
     const uint32_t x = i % kXcd, k = i / kXcd, q = n / kXcd, r = n % kXcd;

@@ -146,7 +146,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT) k_build_geo(const T *He, cons
     using S = ColShape<P>;
     constexpr int Q = S::Q, NN = S::NN;
     const ColThread<P> th(threadIdx.x);
-    const int64_t b = xcd_slot(blockIdx.x, gridDim.x), e = b * S::EPB + th.le, ec = e < nelem ? e : nelem - 1;
+    const int64_t b = xcd_range(blockIdx.x, gridDim.x), e = b * S::EPB + th.le, ec = e < nelem ? e : nelem - 1;
     if (threadIdx.x >= S::LANES) return;
     const int ij = line_ref<P>(th.I) + Q * line_ref<P>(th.J);
     GeoPair<T> *dst = reinterpret_cast<GeoPair<T> *>(geo) + b * Q * 5 * S::LANES + th.tc;
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     __shared__ uint32_t su[SORT];
     __shared__ uint32_t sw[NT / 64], sbad;
     const int t = threadIdx.x;
-    const int64_t b = xcd_slot(blockIdx.x, gridDim.x), e0 = b * B;
+    const int64_t b = xcd_range(blockIdx.x, gridDim.x), e0 = b * B;
     const int ne = (int)(nelem - e0 < B ? nelem - e0 : B);
     const int n = B * NN;  // the layout is padded with copies of the last element
     if (t == 0) sbad = 0;
