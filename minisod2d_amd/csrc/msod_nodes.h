@@ -3,8 +3,9 @@
 //   * the FP32-arithmetic form: its results are FP32 rounding, so another order
 //     of the FP32 operations is another result (columns: 9e-7 off in relative L2,
 //     48^3 p=7 3.14 -> 2.5 ms for the diffusion);
-//   * short launches in the default mode, and the closure's network where the
-//     columns run out of registers (nodes_for_atomics);
+//   * short launches in the default mode, the closure's network where the columns
+//     run out of registers (nodes_for_atomics), and the diffusion of orders 4 and 5
+//     where a batch's elements form no rows (nodes_for_order);
 //   * the coloured mode where they are faster (nodes_for_colors), and where the
 //     batches of the column kernels, up to five times as large, need
 //     more than 32 colours (elements in little spatial order).

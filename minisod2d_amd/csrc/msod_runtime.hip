@@ -191,14 +191,15 @@ __global__ void k_build_geo_nodes(const T *He, const T *gpvol, int64_t nelem, in
 // The batches' node lists from the connectivity, one workgroup per batch: its
 // nodes are sorted in LDS (bitonic) and the distinct ones numbered in
 // ascending order, as build_host_plan does on the host.  FILL = false:
-// count[b] = their number, or kBadBatch + the entries outside 1..npoin.  FILL:
+// count[b] = their number + kPairUnit * the elements that continue the row of
+// nodes (axis I) of the one before, or kBadBatch + the entries outside 1..npoin.  FILL:
 // unode from uoff, conn and lidx in the lane layout or (lanes = false)
 // element-major (msod_nodes.h).  lists (PlanLists): every
 // node of the batch, those alone that several lanes write after col_merge has
 // taken neighbours' nodes together (the others' lidx is kAlone), or none, for
 // kernels that read conn alone (count[b] = 0, the rest null).
 // A first pair at 64^3, p=4 takes 6 ms in all (191 with the host plan).
-constexpr uint32_t kBadBatch = 0x80000000u;
+constexpr uint32_t kBadBatch = 0x80000000u, kPairUnit = 0x10000u;
 enum PlanLists { kListNone = 0, kListAll = 1, kListShared = 2 };
 template <int P>
 struct PlanShape {
@@ -217,12 +218,12 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     constexpr int NN = S::NN, NT = S::NT, SORT = S::SORT, PER = S::PER;
     __shared__ uint32_t s[SORT];
     __shared__ uint32_t su[SORT];
-    __shared__ uint32_t sw[NT / 64], sbad;
+    __shared__ uint32_t sw[NT / 64], sbad, spairs;
     const int t = threadIdx.x;
     const int64_t b = xcd_range(blockIdx.x, gridDim.x), e0 = b * B;
     const int ne = (int)(nelem - e0 < B ? nelem - e0 : B);
     const int n = B * NN;  // the layout is padded with copies of the last element
-    if (t == 0) sbad = 0;
+    if (t == 0) sbad = spairs = 0;
     __syncthreads();
     uint32_t v[PER];
     unsigned bad = 0;
@@ -241,6 +242,12 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     }
     if (bad) atomicAdd(&sbad, bad);
     __syncthreads();
+    if constexpr (!FILL) {
+        // nodes (P,0,0) and (P,P,P) of one element are (0,0,0) and (0,P,P) of the next
+        constexpr int Q = P + 1, far = 1 + Q + Q * Q;
+        if (t + 1 < ne && s[t + B] == s[t + 1] && s[t + B * far] == s[t + 1 + B * (far - 1)]) atomicAdd(&spairs, 1u);
+        __syncthreads();
+    }
     if (lists == kListShared) {
         // the left node of each pair that col_merge takes together is not written
         constexpr int Q = P + 1;
@@ -259,7 +266,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
     }
     if (lists == kListNone) {
         if constexpr (!FILL) {
-            if (t == 0) count[b] = sbad ? kBadBatch + sbad : 0u;
+            if (t == 0) count[b] = sbad ? kBadBatch + sbad : kPairUnit * spairs;
         } else {
 #pragma unroll
             for (int j = 0; j < PER; ++j) {
@@ -307,7 +314,7 @@ __global__ void __launch_bounds__(256) k_plan_batches(const int32_t *connec, int
         U += sw[w];
     }
     if constexpr (!FILL) {
-        if (t == 0) count[b] = sbad ? kBadBatch + sbad : U;
+        if (t == 0) count[b] = sbad ? kBadBatch + sbad : kPairUnit * spairs + U;
     } else {
 #pragma unroll
         for (int j = 0; j < PER; ++j)
@@ -541,6 +548,25 @@ static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
     }
 }
 
+// Default mode, diffusion, once the column plan is known: whether one node per
+// thread is the faster form.  The columns gather a row of elements at a time; with
+// elements in another order, in meshes whose nodes stay in the memory-side cache,
+// the former kernels' three or four waves per SIMD hide more of the gathers.  At
+// order 4 the node sums of a scattered batch (ustride) also leave one workgroup
+// per CU.  In us, nodes | columns, elements along z and in random order:
+//   order 4  25^3 169|186, 40^3 735|621    random: 25^3 194|243, 40^3 686|900, 62^3 FP32 outputs 2336|3017
+//   order 5  21^3 175|204, 33^3 710|685    random: 21^3 182|201, 33^3 662|718, 52^3 3343|3315
+// Orders 2 and 3 lie within 4%, orders 6 and up are faster as columns.
+template <typename TG>
+static bool nodes_for_order(int porder, int64_t nelem, bool rows, int ustride)
+{
+    if (porder == 5) return !rows && nelem * 216 < 12000000;
+    if (porder != 4) return false;
+    constexpr int kLdsCu = 160 * 1024;  // k_diffu_col's static LDS: D, (r,T) (u0,u1), u2, six fluxes, mu
+    const int lds = 25 * 8 + 256 * (2 * 16 + 8 + 6 * 16 + 2 * (int)sizeof(TG)) + 16 + 5 * 8 * ustride;
+    return (!rows && nelem * 125 < 4000000) || 2 * lds > kLdsCu;
+}
+
 // Whether a call starts out with the kernels with one node per thread.
 static bool take_nodes(Kernel k, int mode, int porder, int64_t nelem, bool out32)
 {
@@ -613,6 +639,7 @@ struct PlanEntry {
     int64_t nunref = 0;
     bool nodes = false;              // element-major (msod_nodes.h)
     int lists = kListAll;            // the nodes in unode
+    bool rows = true;                // consecutive elements mostly follow each other along I
     bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
     void release()
@@ -941,15 +968,18 @@ int build_device_plan(const int32_t *dconnec, int64_t nelem, int64_t npoin, cons
     HIPCHK(hipMemcpyAsync(uoff.data() + 1, P.uoff, sizeof(uint32_t) * nb, hipMemcpyDeviceToHost, g.stream),
            "batch counts");
     HIPCHK(hipStreamSynchronize(g.stream), "batch counts");
-    int64_t bad = 0;
+    int64_t bad = 0, pairs = 0;
     for (int64_t b = 1; b <= nb; ++b) {
         if (uoff[b] & kBadBatch) {
             bad += uoff[b] - kBadBatch;
             uoff[b] = 0;
         }
+        pairs += uoff[b] / kPairUnit;
+        uoff[b] %= kPairUnit;
         P.ustride = std::max(P.ustride, (int)uoff[b]);
         uoff[b] += uoff[b - 1];
     }
+    P.rows = 2 * pairs >= nelem - nb;
     if (bad)
         return fail(MSOD_ERR_MESH, "connec holds %lld node numbers outside 1..npoin (npoin=%lld)", (long long)bad,
                     (long long)npoin);
@@ -1227,16 +1257,17 @@ int column_lists(int porder)
 // elements) where *nodes says so, of the column kernels otherwise.  natural: the
 // atomic launch takes the batches in mesh order.  *nodes is set where columns
 // turn out not to suit the mesh: in the coloured mode, when their batches need
-// more than 32 colours.
-template <typename TO>
-int choose_plan(const void *dc, uint64_t vc, int64_t NE, int64_t NP, const TableSet *ts, int NB, bool natural, bool *nodes,
-                const PlanEntry **plan)
+// more than 32 colours, and by nodes_for_order.
+template <typename TG, typename TO>
+int choose_plan(Kernel k, const void *dc, uint64_t vc, int64_t NE, int64_t NP, const TableSet *ts, int NB, bool natural,
+                bool *nodes, const PlanEntry **plan)
 {
     const bool colored = g.assembly == kColored;
     if (!*nodes) {
         const int st = get_plan(dc, vc, NE, NP, ts, batch_size(ts->porder), column_lists<TO>(ts->porder), colored, plan);
         if (st) return st;
-        *nodes = colored && !(*plan)->colored;
+        *nodes = colored ? !(*plan)->colored
+                         : k == kDiffu && nodes_for_order<TG>(ts->porder, NE, (*plan)->rows, (*plan)->ustride);
     }
     return *nodes ? get_plan(dc, vc, NE, NP, ts, NB, kListAll, colored || !natural, plan, true) : MSOD_OK;
 }
@@ -1328,7 +1359,7 @@ int convec_common(int porder, int nelem, int npoin, const int32_t *connec, const
     const PlanEntry *plan;
     const TG *geo;
     bool nodes = fp32_arith || take_nodes(kConvec, g.assembly, porder, NE, sizeof(TO) == 4);
-    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), !fp32_arith, &nodes, &plan))) return st;
+    if ((st = choose_plan<TG, TO>(kConvec, dc, vc, NE, NP, ts, nodes_convec_batch_size(porder), !fp32_arith, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     ConvecArgs<TG, TF, TO, TU, TP> a;
@@ -1389,8 +1420,9 @@ int diffu_common(int porder, int nelem, int npoin, const int32_t *connec, const 
     const PlanEntry *plan;
     const TG *geo;
     constexpr bool kF64 = std::is_same<DiffuArgs<TG, TF, TO, TU>, DiffuArgs<double, double>>::value;
-    bool nodes = fp32_arith || take_nodes(dmlp ? kClosure : kDiffu, g.assembly, porder, NE, sizeof(TO) == 4);
-    if ((st = choose_plan<TO>(dc, vc, NE, NP, ts, nodes_batch_size(porder), true, &nodes, &plan))) return st;
+    const Kernel kernel = dmlp ? kClosure : kDiffu;
+    bool nodes = fp32_arith || take_nodes(kernel, g.assembly, porder, NE, sizeof(TO) == 4);
+    if ((st = choose_plan<TG, TO>(kernel, dc, vc, NE, NP, ts, nodes_batch_size(porder), true, &nodes, &plan))) return st;
     if ((st = get_geo<TG>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
 
     DiffuArgs<TG, TF, TO, TU> a;

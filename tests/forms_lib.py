@@ -21,6 +21,21 @@ def shuffle(prob, perm):
     return prob
 
 
+def rounded(prob, a):
+    """The problem on the form's inputs, widened."""
+    q = m.box_problem(1, prob.porder)
+    for k in ("nelem", "npoin", "connec"):
+        setattr(q, k, getattr(prob, k))
+    for k in ("He", "gpvol", "u", "q", "rho", "pr", "E", "Tem", "mu_fluid", "mu_e", "mu_sgs"):
+        setattr(q, k, np.asfortranarray(getattr(a, k), dtype=np.float64))
+    if a.form == "mixed":
+        q.pr = (q.gamma - 1.0) * (q.E - q.rho * 0.5 * (q.u ** 2).sum(axis=1))
+    if a.form == "r4":
+        q.tables.dlxigp_ip = np.asfortranarray(a.dlx, dtype=np.float64)
+        q.Cp, q.Pr = float(np.float32(q.Cp)), float(np.float32(q.Pr))
+    return q
+
+
 def network(prob, seed=7):
     """Weights near a constant viscosity, standardised by rough scales of the fields."""
     rng = np.random.default_rng(seed)

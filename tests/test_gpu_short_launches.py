@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 import minisod2d_amd as m
-from forms_lib import FORMS, Arrays, network
+from forms_lib import FORMS, Arrays, network, rounded
 from oracle_lib import Oracle, rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -31,21 +31,6 @@ def mesh(p, nelem):
     prob.gpvol = np.asfortranarray(prob.gpvol[:, :, :nelem])
     prob.nelem = nelem
     return prob
-
-
-def rounded(prob, a):
-    """The problem on the form's inputs, widened."""
-    q = m.box_problem(1, prob.porder)
-    for k in ("nelem", "npoin", "connec"):
-        setattr(q, k, getattr(prob, k))
-    for k in ("He", "gpvol", "u", "q", "rho", "pr", "E", "Tem", "mu_fluid", "mu_e", "mu_sgs"):
-        setattr(q, k, np.asfortranarray(getattr(a, k), dtype=np.float64))
-    if a.form == "mixed":
-        q.pr = (q.gamma - 1.0) * (q.E - q.rho * 0.5 * (q.u ** 2).sum(axis=1))
-    if a.form == "r4":
-        q.tables.dlxigp_ip = np.asfortranarray(a.dlx, dtype=np.float64)
-        q.Cp, q.Pr = float(np.float32(q.Cp)), float(np.float32(q.Pr))
-    return q
 
 
 @pytest.mark.parametrize("p,line", LINES)
