@@ -642,6 +642,11 @@ struct PlanEntry {
     bool rows = true;                // consecutive elements mostly follow each other along I
     bool host = false;               // colours, first writers and unref are there (build_host_part)
     bool colored = false;            // batch colouring found (the coloured assembly needs it)
+    bool outdated_by(const PlanEntry &o) const { return src == o.src && ver != o.ver; }
+    bool same_mesh(const PlanEntry &o) const
+    {
+        return src == o.src && ver == o.ver && nelem == o.nelem && npoin == o.npoin && porder == o.porder && l2g == o.l2g;
+    }
     void release()
     {
         for (void *p : {(void *)conn, (void *)uoff, (void *)unode, (void *)order, (void *)lidx,
@@ -662,6 +667,15 @@ struct DerivedGeo {
     std::vector<int32_t> l2g;
     bool nodes;  // element-major (msod_nodes.h)
     void *geo;   // He and gpvol as pairs (k_build_geo)
+    bool outdated_by(const DerivedGeo &o) const
+    {
+        return (srcHe == o.srcHe && verHe != o.verHe) || (srcVol == o.srcVol && verVol != o.verVol);
+    }
+    bool same_mesh(const DerivedGeo &o) const
+    {
+        return srcHe == o.srcHe && srcVol == o.srcVol && verHe == o.verHe && verVol == o.verVol && nelem == o.nelem &&
+               porder == o.porder && elt == o.elt && l2g == o.l2g;
+    }
 };
 
 // A tetrahedral connectivity found valid (every entry in 1..npoin), with
@@ -930,7 +944,33 @@ int get_tables(int porder, const int32_t *invAtoIJK, const int32_t *AtoI, const 
     return MSOD_OK;
 }
 
+// Meshes whose derived layouts are kept: each with as many layouts as its calls
+// take (plans for columns and for one node per thread; geometry of both).
 constexpr size_t kMaxDerived = 4;
+
+// Makes room in v for x: entries of older contents of x's array can never be
+// asked for again; past kMaxDerived meshes the oldest goes, with all its layouts.
+template <class E, class Drop>
+void make_room(std::vector<E> &v, const E &x, const Drop &drop)
+{
+    auto erase_if = [&](auto pred) {
+        for (size_t i = v.size(); i-- > 0;)
+            if (pred(v[i])) {
+                drop(v[i]);
+                v.erase(v.begin() + i);
+            }
+    };
+    erase_if([&](const E &e) { return e.outdated_by(x); });
+    for (;;) {
+        std::vector<const E *> meshes;
+        for (const E &e : v)
+            if (!e.same_mesh(x) && std::none_of(meshes.begin(), meshes.end(), [&](const E *o) { return o->same_mesh(e); }))
+                meshes.push_back(&e);
+        if (meshes.size() < kMaxDerived) return;
+        const E oldest = *meshes.front();
+        erase_if([&](const E &e) { return e.same_mesh(oldest); });
+    }
+}
 
 template <class V>
 int upload(const std::vector<V> &h, V **d, const char *what)
@@ -1089,10 +1129,7 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
         P.release();
         return st;
     }
-    if (g.plans.size() >= kMaxDerived) {
-        g.plans.front().release();
-        g.plans.erase(g.plans.begin());
-    }
+    make_room(g.plans, P, [](PlanEntry &e) { e.release(); });
     g.plans.push_back(std::move(P));
     *out = &g.plans.back();
     return MSOD_OK;
@@ -1124,10 +1161,7 @@ int get_geo(const void *dHe, uint64_t vHe, const void *dVol, uint64_t vVol, int6
         (void)hipFree(c.geo);
         return hipfail(e, "building the geometry layout");
     }
-    if (g.geos.size() >= kMaxDerived) {
-        (void)hipFree(g.geos.front().geo);
-        g.geos.erase(g.geos.begin());
-    }
+    make_room(g.geos, c, [](DerivedGeo &e) { (void)hipFree(e.geo); });
     g.geos.push_back(c);
     *geo = (const T *)c.geo;
     return MSOD_OK;
