@@ -197,9 +197,10 @@ __global__ void __launch_bounds__(256) k_mlp_predict(const float *P, const float
         const float z3 = mlp_z3(s, [&](int mt) {
             const int i = base + 16 * mt + r, ic = i < total ? i : total - 1;
             const int64_t smp = (e0 + ic / nl) * nn + l0 + ic % nl;
-            // lanes of inputs 12..15 read 0..3, standardised to zero
+            // lanes of inputs 12..15 read 0..3 and hold zeros (an infinite
+            // feature times zero would be a NaN)
             const f32x4 f = load_feat4(feat + smp * kMlpIn + (g < 3 ? 4 * g : 0), aligned);
-            return pack_bf16((f - mean) * istd);
+            return g < 3 ? pack_bf16((f - mean) * istd) : s16x4{0, 0, 0, 0};
         });
         const int i = base + lane;
         if (i < total) out[i / nl][i % nl] = (double)(s.scale * softplusf_(z3));
@@ -306,7 +307,7 @@ __global__ void __launch_bounds__(64 * kGW, 2) k_mlp_grad(const float *P, const 
             for (int mt = 0; mt < 4; ++mt) {
                 const bool valid = chunk * 64 + 16 * mt + r < nsamp;
                 xb[mt] = pack_bf16((f[mt] - mean) * istd);
-                if (!valid) xb[mt] = s16x4{0, 0, 0, 0};
+                if (!valid || g == 3) xb[mt] = s16x4{0, 0, 0, 0};
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
                     f32x4 z = mfma16(W1t[t], xb[mt], zero);
