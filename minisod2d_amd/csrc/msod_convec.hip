@@ -72,11 +72,11 @@ struct ConvecSums {
     }
 };
 
-template <int P, bool COLORED, class A, typename TA>
+template <int P, bool COLORED, class A>
 __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
 {
     using S = ColShape<P>;
-    using T = TA;
+    using T = double;
     using TG = typename A::G;
     constexpr int Q = S::Q, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
@@ -216,11 +216,11 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_col(A a)
 // ms, outputs take about a third (2.0 ms of 3.07 without any, 2.4 with plain
 // stores, before neighbours' nodes were merged); the rest is the FP64 work and
 // LDS reads of two waves per SIMD.
-template <int P, bool COLORED, class A, typename TA>
+template <int P, bool COLORED, class A>
 __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
 {
     using S = ColShape<P>;
-    using T = TA;
+    using T = double;
     using TG = typename A::G;
     constexpr int Q = S::Q, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
     constexpr bool SHARED = !COLORED && sizeof(typename A::O) == 4;  // col_add_shared
@@ -398,7 +398,7 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_convec_wide(A a)
     }
 }
 
-template <int P, class A, typename TA>
+template <int P, class A>
 static hipError_t launch_p(const A &a, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
@@ -408,34 +408,28 @@ static hipError_t launch_p(const A &a, hipStream_t s)
     if constexpr (P > kNarrowP) {
         if constexpr (P != 6)
             if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
-        hipLaunchKernelGGL((atomic || P != 6 ? k_convec_wide<P, false, A, TA> : k_convec_wide<P, P == 6, A, TA>),
+        hipLaunchKernelGGL((atomic || P != 6 ? k_convec_wide<P, false, A> : k_convec_wide<P, P == 6, A>),
                            dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
     } else
-        hipLaunchKernelGGL((atomic ? k_convec_col<P, false, A, TA> : k_convec_col<P, true, A, TA>),
+        hipLaunchKernelGGL((atomic ? k_convec_col<P, false, A> : k_convec_col<P, true, A>),
                            dim3((unsigned)a.plan.nb), dim3(ColShape<P>::NT), sums, s, a);
     return hipGetLastError();
-}
-
-template <class A, typename TA>
-static hipError_t launch_order(int porder, const A &a, hipStream_t s)
-{
-    switch (porder) {
-    case 1: return launch_p<1, A, TA>(a, s);
-    case 2: return launch_p<2, A, TA>(a, s);
-    case 3: return launch_p<3, A, TA>(a, s);
-    case 4: return launch_p<4, A, TA>(a, s);
-    case 5: return launch_p<5, A, TA>(a, s);
-    case 6: return launch_p<6, A, TA>(a, s);
-    case 7: return launch_p<7, A, TA>(a, s);
-    case 8: return launch_p<8, A, TA>(a, s);
-    default: return hipErrorInvalidValue;
-    }
 }
 
 template <class A>
 hipError_t launch_convec(int porder, const A &a, hipStream_t s)
 {
-    return launch_order<A, double>(porder, a, s);
+    switch (porder) {
+    case 1: return launch_p<1, A>(a, s);
+    case 2: return launch_p<2, A>(a, s);
+    case 3: return launch_p<3, A>(a, s);
+    case 4: return launch_p<4, A>(a, s);
+    case 5: return launch_p<5, A>(a, s);
+    case 6: return launch_p<6, A>(a, s);
+    case 7: return launch_p<7, A>(a, s);
+    case 8: return launch_p<8, A>(a, s);
+    default: return hipErrorInvalidValue;
+    }
 }
 
 template hipError_t launch_convec(int, const ConvecArgs<double, double> &, hipStream_t);

@@ -32,11 +32,11 @@
 
 namespace msod {
 
-template <int P, bool COLORED, class A, bool CLOSURE, typename TA>
+template <int P, bool COLORED, class A, bool CLOSURE>
 __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const float *mlp)
 {
     using S = ColShape<P>;
-    using T = TA;
+    using T = double;
     using TG = typename A::G;
     constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
     constexpr int LA = 2;  // line sources read ahead of their use (3 and 4: no faster; order 5 spills)
@@ -295,17 +295,17 @@ __global__ void __launch_bounds__(ColShape<P>::NT, 2) k_diffu_col(A a, const flo
 // 1.21 ms (1.32 with the line sources read one ahead: spills); 32^3 order 8,
 // with one wave per SIMD, 2.40 -> 1.88 (two waves and 80 spilled VGPRs: 2.61);
 // order 5, against the kernel above with LDS sums, 64^3 3.08 -> 2.64.
-template <int P, typename TA>
-constexpr int kWideWaves = P == 8 && sizeof(TA) == 8 ? 1 : 2;  // per SIMD
+template <int P>
+constexpr int kWideWaves = P == 8 ? 1 : 2;  // per SIMD
 
-template <int P, class A, bool CLOSURE, typename TA>
-__global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_wide(A a, const float *mlp)
+template <int P, class A, bool CLOSURE>
+__global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P>)) k_diffu_wide(A a, const float *mlp)
 {
     using S = ColShape<P>;
-    using T = TA;
+    using T = double;
     using TG = typename A::G;
     constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES, NT = S::NT;
-    constexpr bool AHEAD = kWideWaves<P, TA> == 1;  // read line sources one ahead of their use
+    constexpr bool AHEAD = kWideWaves<P> == 1;  // read line sources one ahead of their use
     constexpr bool SHARED = sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
@@ -562,16 +562,15 @@ __global__ void __launch_bounds__(ColShape<P>::NT, (kWideWaves<P, TA>)) k_diffu_
 // elements of a batch per workgroup.  48^3: 3.09
 // ms, one node per thread 3.49; with all four elements in a workgroup, alone on
 // its CU, 3.56.
-template <int P, int E2, class A, bool CLOSURE, typename TA>
+template <int P, int E2, class A, bool CLOSURE>
 __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a, const float *mlp)
 {
     using S = ColShape<P>;
-    using T = TA;
+    using T = double;
     using TG = typename A::G;
     constexpr int Q = S::Q, QQ = S::QQ, EPB = S::EPB, LANES = S::LANES;
     constexpr int H = Q / 2, HL = E2 * QQ, NT = 2 * HL, PARTS = EPB / E2;
     static_assert(Q % 2 == 0 && HL % 64 == 0 && LANES == EPB * QQ, "whole waves per half");
-    constexpr bool AHEAD = true;  // read line sources one ahead of their use
     constexpr bool SHARED = sizeof(typename A::O) == 4;  // col_add_shared
     struct alignas(2 * sizeof(T)) V2 { T x, y; };
     __shared__ T sD[Q * Q];
@@ -699,8 +698,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
 #pragma unroll
         for (int s = 0; s < 2 * Q; ++s) {
             const int d = s < Q ? 0 : 1;
-            if (AHEAD && s + 1 < 2 * Q) nxt = read_source(s + 1);
-            if (!AHEAD && s > 0) cur = read_source(s);
+            if (s + 1 < 2 * Q) nxt = read_source(s + 1);
             x[d][0] += cur.D * cur.a.x;
             x[d][1] += cur.D * cur.a.y;
             x[d][2] += cur.D * cur.b.x;
@@ -708,7 +706,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
             x[d][4] += cur.D * cur.c;
             asm volatile("" : "+v"(x[d][0]), "+v"(x[d][1]), "+v"(x[d][2]), "+v"(x[d][3]), "+v"(x[d][4]));
             __builtin_amdgcn_sched_barrier(0);
-            if (AHEAD) cur = nxt;
+            cur = nxt;
         }
         // x[.][f] becomes the gradient: grad rho, grad T, G[c][i] = x[i][2 + c]
 #pragma unroll
@@ -800,8 +798,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
         Flux fc = read_flux(0), fn = fc;
 #pragma unroll
         for (int s = 0; s < 2 * Q; ++s) {
-            if (AHEAD && s + 1 < 2 * Q) fn = read_flux(s + 1);
-            if (!AHEAD && s > 0) fc = read_flux(s);
+            if (s + 1 < 2 * Q) fn = read_flux(s + 1);
             W[k][0] += fc.D * fc.a.x;
             W[k][1] += fc.D * fc.a.y;
             W[k][2] += fc.D * fc.b.x;
@@ -811,7 +808,7 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
 #pragma unroll
             for (int f = 0; f < 6; ++f) asm volatile("" : "+v"(W[k][f]));
             __builtin_amdgcn_sched_barrier(0);
-            if (AHEAD) fc = fn;
+            fc = fn;
         }
         // the mate's slice
         const V2 m0 = sF[6][mate], m1 = sF[7][mate], m2 = sF[8][mate];
@@ -856,13 +853,13 @@ __global__ void __launch_bounds__(2 * E2 * ColShape<P>::QQ, 2) k_diffu_split(A a
     }
 }
 
-template <int P, class A, bool CLOSURE, typename TA>
+template <int P, class A, bool CLOSURE>
 static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
     const bool atomic = a.plan.mode == kAtomic;
     const bool registers = P > kNarrowP && atomic && sizeof(typename A::O) == 8;
-    const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(TA) * 12 * ColShape<P>::NT;
+    const size_t sums = registers ? 0 : sizeof(double) * 5 * a.plan.ustride, fluxes = sizeof(double) * 12 * ColShape<P>::NT;
     const dim3 grid((unsigned)a.plan.nb), block(ColShape<P>::NT);
     if constexpr (P > kNarrowP)
         if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
@@ -870,30 +867,30 @@ static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
         return hipErrorInvalidValue;  // and there (nodes_for_atomics)
     } else if constexpr (P == 7) {
         constexpr int E2 = 2, EPB = ColShape<P>::EPB, QQ = ColShape<P>::QQ;
-        const size_t part = sizeof(TA) * 2 * 9 * 2 * QQ;  // fluxes per element
-        hipLaunchKernelGGL((k_diffu_split<P, E2, A, CLOSURE, TA>), dim3((unsigned)(a.plan.nb * (EPB / E2))), dim3(2 * E2 * QQ),
+        const size_t part = sizeof(double) * 2 * 9 * 2 * QQ;  // fluxes per element
+        hipLaunchKernelGGL((k_diffu_split<P, E2, A, CLOSURE>), dim3((unsigned)(a.plan.nb * (EPB / E2))), dim3(2 * E2 * QQ),
                            std::max(E2 * part, sums), s, a, mlp);
     } else if constexpr (P > kNarrowP) {
-        hipLaunchKernelGGL((k_diffu_wide<P, A, CLOSURE, TA>), grid, block, std::max(fluxes, sums), s, a, mlp);
+        hipLaunchKernelGGL((k_diffu_wide<P, A, CLOSURE>), grid, block, std::max(fluxes, sums), s, a, mlp);
     } else {
-        hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE, TA> : k_diffu_col<P, true, A, CLOSURE, TA>), grid,
+        hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE> : k_diffu_col<P, true, A, CLOSURE>), grid,
                            block, sums, s, a, mlp);
     }
     return hipGetLastError();
 }
 
-template <class A, bool CLOSURE, typename TA>
+template <class A, bool CLOSURE>
 static hipError_t launch_order(int porder, const A &a, const float *mlp, hipStream_t s)
 {
     switch (porder) {
-    case 1: return launch_p<1, A, CLOSURE, TA>(a, mlp, s);
-    case 2: return launch_p<2, A, CLOSURE, TA>(a, mlp, s);
-    case 3: return launch_p<3, A, CLOSURE, TA>(a, mlp, s);
-    case 4: return launch_p<4, A, CLOSURE, TA>(a, mlp, s);
-    case 5: return launch_p<5, A, CLOSURE, TA>(a, mlp, s);
-    case 6: return launch_p<6, A, CLOSURE, TA>(a, mlp, s);
-    case 7: return launch_p<7, A, CLOSURE, TA>(a, mlp, s);
-    case 8: return launch_p<8, A, CLOSURE, TA>(a, mlp, s);
+    case 1: return launch_p<1, A, CLOSURE>(a, mlp, s);
+    case 2: return launch_p<2, A, CLOSURE>(a, mlp, s);
+    case 3: return launch_p<3, A, CLOSURE>(a, mlp, s);
+    case 4: return launch_p<4, A, CLOSURE>(a, mlp, s);
+    case 5: return launch_p<5, A, CLOSURE>(a, mlp, s);
+    case 6: return launch_p<6, A, CLOSURE>(a, mlp, s);
+    case 7: return launch_p<7, A, CLOSURE>(a, mlp, s);
+    case 8: return launch_p<8, A, CLOSURE>(a, mlp, s);
     default: return hipErrorInvalidValue;
     }
 }
@@ -901,12 +898,12 @@ static hipError_t launch_order(int porder, const A &a, const float *mlp, hipStre
 template <class A>
 hipError_t launch_diffu(int porder, const A &a, hipStream_t s)
 {
-    return launch_order<A, false, double>(porder, a, nullptr, s);
+    return launch_order<A, false>(porder, a, nullptr, s);
 }
 
 hipError_t launch_diffu_closure(int porder, const DiffuArgs<double, double> &a, const float *mlp, hipStream_t s)
 {
-    return launch_order<DiffuArgs<double, double>, true, double>(porder, a, mlp, s);
+    return launch_order<DiffuArgs<double, double>, true>(porder, a, mlp, s);
 }
 
 template hipError_t launch_diffu(int, const DiffuArgs<double, double> &, hipStream_t);

@@ -53,7 +53,7 @@ constexpr uint16_t kAlone = 0xffff;
 
 // Elements per batch: ColShape<P>::EPB for run-time porder.
 int batch_size(int porder);
-// Those of the FP32-arithmetic kernels: Shape<P>::BATCH and CShape<P>::BATCH.
+// Those of the kernels with one node per thread: Shape<P>::BATCH and CShape<P>::BATCH.
 int nodes_batch_size(int porder);
 int nodes_convec_batch_size(int porder);
 
@@ -73,7 +73,7 @@ struct Plan {
     int ustride;  // stride of the node sums: the most nodes of any batch
     const uint8_t *ecol;  // coloured mode: colour of each element within its batch
     int rounds;           // and the most colours of any batch
-    int kpb;              // FP32 arithmetic (msod_nodes.h): batches per workgroup
+    int kpb;              // one node per thread (msod_nodes.h): batches per workgroup
 };
 
 // Kernel arguments.  Storage types: TG for the element-sized arrays (geo;

@@ -47,7 +47,6 @@ __device__ __forceinline__ s16x4 pack_bf16(f32x4 v)
     typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
     return __builtin_bit_cast(s16x4, __builtin_convertvector(v, bf16x4));
 }
-__device__ __forceinline__ short f2bf(float f) { return __builtin_bit_cast(short, (__bf16)f); }
 // The hardware reciprocal (1 ulp) instead of a correctly rounded division:
 // the network runs in bf16, whose rounding is 2^-9.
 __device__ __forceinline__ float sigmoidf_(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
