@@ -10,8 +10,9 @@ namespace msod {
 // to mu_sgs at every element node.
 struct ClosureElemArgs {
     int64_t nelem, npoin;
-    const uint32_t *conn;      // [nelem][nn] 0-based nodes
-    const double *geo;  // element-major geometry (GeoNode pairs)
+    bool lanes;                // layout of conn and geo: msod_columns.h, or element-major (msod_nodes.h)
+    const uint32_t *conn;      // 0-based nodes
+    const double *geo;         // GeoNode pairs
     const double *rho, *u, *Tem;
     double Cp;
     const double *rerr;        // [4][npoin]: momentum x, y, z, energy

@@ -508,8 +508,10 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 // Default mode: whether one node per thread is the faster form.  With fewer column
 // batches (nb) than CUs a launch lasts as long as one workgroup, which walks its
 // slices one after the other; the former kernels' workgroups hold fewer elements
-// and work on all of their nodes at once.  Whole calls in us, nodes | columns,
-// FP64 (the FP32-storage forms cross within 30% of the same nb):
+// and work on all of their nodes at once.  With FP32 outputs columns stay: the
+// smaller batches round more partial sums to float (order 4: faces of 4 elements'
+// batches instead of 10).  Whole calls in us, nodes | columns, FP64 (the forms with
+// FP32 storage cross within 30% of the same nb):
 //   order  convection               diffusion
 //   3      nb 32 31.3|32.0, 63 32.7|32.7, 99 34.3|33.9    32 32.6|33.4, 99 36.0|35.5
 //   4      1 31.5|33.8, 65 34.6|36.4, 100 37.5|37.1       1 32.8|35.8, 65 35.9|38.3, 100 38.1|39.0
@@ -526,8 +528,9 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 //            order 6  130 90|104, 200 105|109, 267 129|124, 5959 1614|1203
 //            order 7  63 66|73, 128 77|81, 162 89|84, 6098 996|960
 //            order 8  34 66|99, 789 276|324, 2940 845|878, 6084 1671|1674, 19773 5244|5185
-static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
+static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem, bool out32)
 {
+    if (out32) return false;
     const int64_t nb = (nelem + batch_size(porder) - 1) / batch_size(porder);
     if (k == kClosure) switch (porder) {
         case 3: return nb < 400;
@@ -541,7 +544,7 @@ static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
     switch (porder) {
     case 3: return nb < 48;
     case 4: return nb < 88;
-    case 5: return nb < (k == kConvec ? 48 : 150);
+    case 5: return nb < 80;  // one line, so that a pair needs one layout
     case 6: return nb < (k == kConvec ? 24 : 128);
     case 8: return nb < 80;
     default: return false;
@@ -556,21 +559,22 @@ static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem)
 // per CU.  In us, nodes | columns, elements along z and in random order:
 //   order 4  25^3 169|186, 40^3 735|621    random: 25^3 194|243, 40^3 686|900, 62^3 FP32 outputs 2336|3017
 //   order 5  21^3 175|204, 33^3 710|685    random: 21^3 182|201, 33^3 662|718, 52^3 3343|3315
-// Orders 2 and 3 lie within 4%, orders 6 and up are faster as columns.
+// Orders 2 and 3 lie within 4%, orders 6 and up are faster as columns.  With FP32
+// outputs columns stay where their larger batches save roundings.
 template <typename TG>
-static bool nodes_for_order(int porder, int64_t nelem, bool rows, int ustride)
+static bool nodes_for_order(int porder, int64_t nelem, bool rows, int ustride, bool out32)
 {
-    if (porder == 5) return !rows && nelem * 216 < 12000000;
+    if (porder == 5) return !rows && !out32 && nelem * 216 < 12000000;
     if (porder != 4) return false;
     constexpr int kLdsCu = 160 * 1024;  // k_diffu_col's static LDS: D, (r,T) (u0,u1), u2, six fluxes, mu
     const int lds = 25 * 8 + 256 * (2 * 16 + 8 + 6 * 16 + 2 * (int)sizeof(TG)) + 16 + 5 * 8 * ustride;
-    return (!rows && nelem * 125 < 4000000) || 2 * lds > kLdsCu;
+    return (!rows && !out32 && nelem * 125 < 4000000) || 2 * lds > kLdsCu;
 }
 
 // Whether a call starts out with the kernels with one node per thread.
 static bool take_nodes(Kernel k, int mode, int porder, int64_t nelem, bool out32)
 {
-    return mode == kColored ? nodes_for_colors(k, porder, nelem, out32) : nodes_for_atomics(k, porder, nelem);
+    return mode == kColored ? nodes_for_colors(k, porder, nelem, out32) : nodes_for_atomics(k, porder, nelem, out32);
 }
 
 // k_plan_batches: count (FILL = false, the lists' arrays null) or fill.
@@ -1094,8 +1098,8 @@ void drop_unversioned(const void *src)
         }
 }
 
-// lists: the node lists that the call's kernels read (kListNone: any plan will
-// do).  host: with the colours (the atomic assembly takes either plan).
+// lists: the node lists that the call's kernels read (kListNone: conn alone, any
+// plan will do).  host: with the colours (the atomic assembly takes either plan).
 int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, const TableSet *ts, int B, int lists,
              bool host, const PlanEntry **out, bool nodes = false)
 {
@@ -1115,6 +1119,7 @@ int get_plan(const void *dconnec, uint64_t ver, int64_t nelem, int64_t npoin, co
         *out = &c;
         return MSOD_OK;
     }
+    if (lists == kListNone && (nodes || ts->porder <= kNarrowP)) lists = kListAll;  // as the residuals will ask for
     PlanEntry P;
     P.src = dconnec;
     P.ver = ver;
@@ -1301,7 +1306,7 @@ int choose_plan(Kernel k, const void *dc, uint64_t vc, int64_t NE, int64_t NP, c
         const int st = get_plan(dc, vc, NE, NP, ts, batch_size(ts->porder), column_lists<TO>(ts->porder), colored, plan);
         if (st) return st;
         *nodes = colored ? !(*plan)->colored
-                         : k == kDiffu && nodes_for_order<TG>(ts->porder, NE, (*plan)->rows, (*plan)->ustride);
+                         : k == kDiffu && nodes_for_order<TG>(ts->porder, NE, (*plan)->rows, (*plan)->ustride, sizeof(TO) == 4);
     }
     return *nodes ? get_plan(dc, vc, NE, NP, ts, NB, kListAll, colored || !natural, plan, true) : MSOD_OK;
 }
@@ -1605,9 +1610,18 @@ int closure_elem_common(int porder, int nelem, int npoin, const int32_t *connec,
     if ((st = resolve(u, sizeof(double) * 3 * NP, "u", &du, &vx))) return st;
     const PlanEntry *plan;
     const double *geo;
-    if ((st = get_plan(dc, vc, NE, NP, ts, batch_size(porder), kListNone, false, &plan))) return st;
-    if ((st = get_geo<double>(dHe, vHe, dV, vV, NE, ts, &geo))) return st;
+    // either layout serves: one that is there, else that of the fused diffusion
+    bool nodes = take_nodes(kClosure, g.assembly, porder, NE, false);
+    for (const DerivedGeo &d : g.geos)
+        if (d.same_mesh(DerivedGeo{dHe, dV, vHe, vV, NE, porder, sizeof(double), ts->l2g, false, nullptr})) {
+            nodes = d.nodes;
+            break;
+        }
+    const int B = nodes ? nodes_batch_size(porder) : batch_size(porder);
+    if ((st = get_plan(dc, vc, NE, NP, ts, B, kListNone, false, &plan, nodes))) return st;
+    if ((st = get_geo<double>(dHe, vHe, dV, vV, NE, ts, &geo, nodes))) return st;
     a = ClosureElemArgs{};
+    a.lanes = !nodes;
     a.nelem = NE;
     a.npoin = NP;
     a.conn = plan->conn;

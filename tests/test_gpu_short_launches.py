@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 
 EPB = {3: 16, 4: 10, 5: 7, 6: 5, 8: 3}  # ColShape<P>::EPB in csrc/msod_columns.h
 # column batches from which on a launch takes columns: convection, diffusion
-LINES = [(3, 48), (4, 88), (5, 48), (5, 150), (6, 24), (6, 128), (8, 80)]
+LINES = [(3, 48), (4, 88), (5, 80), (6, 24), (6, 128), (8, 80)]
 
 
 def mesh(p, nelem):
