@@ -522,8 +522,9 @@ static bool nodes_for_colors(Kernel k, int porder, int64_t nelem, bool out32)
 // from the first element on.  With the network's features and weights the columns
 // run out of registers from order 4 on (13 spilled at order 4, 33 at 5, 70 at 6) and
 // have a CU to themselves at order 8:
-//   closure  order 3  nb 256 68|71, 326 76|80, 500 88|83, 5952 398|386
-//            order 4  35 61|72, 521 103|141, 5932 530|819
+//   closure  order 3  the diffusion's line, so that training needs one layout:
+//                     nb 32 60|64, 127 64|67, 256 68|71, 500 88|83
+//            order 4  nb 35 61|72, 521 103|141, 5932 530|819
 //            order 5  35 63|81, 515 122|145, 5950 718|836
 //            order 6  130 90|104, 200 105|109, 267 129|124, 5959 1614|1203
 //            order 7  63 66|73, 128 77|81, 162 89|84, 6098 996|960
@@ -533,13 +534,11 @@ static bool nodes_for_atomics(Kernel k, int porder, int64_t nelem, bool out32)
     if (out32) return false;
     const int64_t nb = (nelem + batch_size(porder) - 1) / batch_size(porder);
     if (k == kClosure) switch (porder) {
-        case 3: return nb < 400;
         case 4:
         case 5:
         case 8: return true;
         case 6: return nb < 220;
         case 7: return nb < 140;
-        default: return false;
         }
     switch (porder) {
     case 3: return nb < 48;
