@@ -69,7 +69,7 @@ int msod_data_present(const void *host);         /* 1 if present, else 0 */
 void *msod_data_deviceptr(const void *host);     /* NULL if not present */
 /* Layouts derived from an array (the assembly plan from connec, the
  * element-major He and gpvol, the TET04 mesh analysis) are cached per array
- * version.  Arrays of the data region change version with
+ * version, for four meshes.  Arrays of the data region change version with
  * msod_data_update_device, msod_data_invalidate and the library's own device
  * routines that write them; the device address of a present array
  * (msod_data_deviceptr) shares its version.  Device memory outside the data
@@ -88,14 +88,17 @@ int msod_data_invalidate(const void *ptr);
 /* ---- execution control -------------------------------------------------- */
 /* How the element contributions meet at shared nodes (no counterpart in the
  * reference, which uses `!$acc atomic update`, elem_convec.f90:414-425).
- * Both modes first sum the contributions of a batch of elements per node in
- * LDS, in a fixed order.
- *   MSOD_ASSEMBLY_ATOMIC (default): one launch over all batches in mesh
- *     order, FP64 atomics of the batch sums into zeroed outputs; the fastest
- *     (neighbouring batches meet in the same L2).
+ *   MSOD_ASSEMBLY_ATOMIC (default): one launch over all batches of elements in
+ *     mesh order, which adds with atomics into zeroed outputs; the fastest
+ *     (neighbouring batches meet in the same L2).  Up to porder 4 a batch's
+ *     contributions to a node are summed in LDS first, above that in registers
+ *     where elements follow each other; with float outputs every sum of a
+ *     batch is formed in FP64 and rounded once (see the rp = 4 entry points).
  *   MSOD_ASSEMBLY_COLORED: batches coloured so that one launch per colour
- *     writes each node without atomics; the summation order is fixed and the
- *     results are bitwise reproducible from run to run. */
+ *     writes each node without atomics; a batch sums in LDS in a fixed order,
+ *     and the results are bitwise reproducible from run to run.  A mesh whose
+ *     batches need more than 32 colours at every batch size the library has
+ *     is refused. */
 enum { MSOD_ASSEMBLY_COLORED = 0, MSOD_ASSEMBLY_ATOMIC = 1 };
 int msod_set_assembly(int mode);
 int msod_set_async(int async);

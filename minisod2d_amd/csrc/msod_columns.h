@@ -9,7 +9,7 @@
 // source costs its FP64 work and its LDS reads with immediate offsets, and no
 // address arithmetic.  Up to kNarrowP the batch's node sums are in LDS too; the
 // kernels above it add to the outputs from registers (msod_convec.hip,
-// msod_diffu.hip).
+// msod_diffu.hip).  msod_nodes.h says which calls take one node per thread instead.
 //
 // Against one node per thread (all three directions from LDS, rolled loops)
 // the FP64 kernels issue a quarter to a third fewer VALU instructions and

@@ -287,6 +287,9 @@ template <int P, class A, typename TA = double>
 static hipError_t launch_p(const A &a, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
+    // order 1: columns with the same batches, but for FP32 arithmetic
+    if constexpr (P == 1 && sizeof(TA) == 8) return hipErrorInvalidValue;
+    else
     hipLaunchKernelGGL((k_convec<P, A, TA>), dim3(plan_blocks(a.plan)), dim3(CShape<P>::NT), 0, s, a);
     return hipGetLastError();
 }

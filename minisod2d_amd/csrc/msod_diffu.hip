@@ -872,6 +872,9 @@ static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
                            std::max(E2 * part, sums), s, a, mlp);
     } else if constexpr (P > kNarrowP) {
         hipLaunchKernelGGL((k_diffu_wide<P, A, CLOSURE>), grid, block, std::max(fluxes, sums), s, a, mlp);
+    } else if constexpr (P == 4 && sizeof(typename A::O) == 4) {
+        if (!atomic) return hipErrorInvalidValue;  // one node per thread there (nodes_for_colors)
+        hipLaunchKernelGGL((k_diffu_col<P, false, A, CLOSURE>), grid, block, sums, s, a, mlp);
     } else {
         hipLaunchKernelGGL((atomic ? k_diffu_col<P, false, A, CLOSURE> : k_diffu_col<P, true, A, CLOSURE>), grid,
                            block, sums, s, a, mlp);

@@ -374,6 +374,9 @@ template <int P, class A, bool CLOSURE, typename TA>
 static hipError_t launch_p(const A &a, const float *mlp, hipStream_t s)
 {
     if (a.plan.nb <= 0) return hipSuccess;
+    // order 1: columns with the same batches, but for FP32 arithmetic
+    if constexpr (P == 1 && sizeof(TA) == 8) return hipErrorInvalidValue;
+    else
     hipLaunchKernelGGL((k_diffu<P, A, CLOSURE, TA>), dim3((unsigned)a.plan.nb), dim3(Shape<P>::NT), 0, s, a, mlp);
     return hipGetLastError();
 }

@@ -91,3 +91,28 @@ def test_the_checker_sees_a_clash(tmp_path):
     prob = m.box_problem(EPB[4], 4, ny=1, nz=1)
     with pytest.raises(AssertionError, match="share a node"):
         rounds(exe, tmp_path, prob.connec, prob.npoin, 4)
+
+
+@pytest.mark.parametrize("shuffled", [False, True])
+@pytest.mark.parametrize("p", range(1, 9))
+def test_whole_plan_with_the_column_batches(checker, tmp_path, p, shuffled):
+    """plan_check.cpp's invariants (tests/test_plan.py) at the column kernels' batch sizes."""
+    exe = os.path.join(HERE, "_build", "plan_check_columns")
+    src = os.path.join(HERE, "plan_check.cpp")
+    if not os.path.exists(exe) or os.path.getmtime(exe) < max(os.path.getmtime(src),
+                                                              os.path.getmtime(os.path.join(CSRC, "msod_plan.h"))):
+        subprocess.run([shutil.which("g++"), "-std=c++17", "-O1", "-g", "-pthread", "-fsanitize=address,undefined",
+                        "-fno-omit-frame-pointer", "-I", CSRC, src, "-o", exe], check=True)
+    n = {1: 9, 2: 7, 3: 5, 4: 4, 5: 4, 6: 3, 7: 3, 8: 2}[p]
+    prob = m.box_problem(n, p, nz=n + 1)
+    connec = prob.connec
+    if shuffled:  # and the nodes of three elements unreferenced
+        connec = connec[np.random.default_rng(p).permutation(prob.nelem)[: prob.nelem - 3]]
+    path = str(tmp_path / "mesh.bin")
+    with open(path, "wb") as fh:
+        np.array([connec.shape[0], prob.npoin], np.int64).tofile(fh)
+        np.array([connec.shape[1], EPB[p]], np.int32).tofile(fh)
+        (prob.tables.invAtoIJK.ravel(order="F") - 1).astype(np.int32).tofile(fh)
+        np.asfortranarray(connec, dtype=np.int32).ravel(order="F").tofile(fh)
+    r = subprocess.run([exe, path], capture_output=True, text=True, env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0"))
+    assert r.returncode == 0 and r.stdout.startswith("OK ncolors="), r.stdout + r.stderr
