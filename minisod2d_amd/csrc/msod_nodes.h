@@ -12,9 +12,9 @@
 // Their layouts are element-major with the element-local node index l,
 //   geo   [nelem][5][nn][2]  GeoNode's five pairs
 //   conn, lidx  [nelem][nn]
-// and their plan is the host's (msod_plan.h), whose batches hold
-// Shape<P>::BATCH elements (convection CShape<P>::BATCH).  A workgroup takes
-// kpb consecutive batches of the launch's list.
+// and their plan's batches hold Shape<P>::BATCH elements (convection
+// CShape<P>::BATCH).  A workgroup takes kpb consecutive batches of the launch's
+// list.
 #pragma once
 
 #include "msod_kernels.h"
